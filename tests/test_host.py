@@ -138,6 +138,31 @@ def test_ring_plan_counts_the_steps_that_cost_something():
             assert plan.live_steps(r, None) == live
 
 
+@pytest.mark.parametrize("starts,want", [
+    ([0, 16, 32, 48], (1, [0])),              # consecutive: one shard
+    ([100, 116, 132, 148], (1, [100])),
+    ([0, 16, 64, 80], (2, [0, 64])),          # two pieces of two shards each
+    ([0, 64, 16, 80], (4, [0, 64, 16, 80])),  # nothing follows on
+])
+def test_consecutive_shards_are_joined(starts, want):
+    q = torch.zeros(1, 64, 1, 64, dtype=torch.bfloat16)
+    pos = torch.cat([torch.arange(16) + s for s in starts])[None]
+    plan = rr._RingPlan(q, q, 4, ra.causal_bias(), {"q_positions": pos}, {"kv_positions": pos})
+    joined = plan.joined()
+    assert (joined.n, joined.q_off) == want and joined.kv_off == joined.q_off
+    assert (joined.Lq, joined.Lk) == (64 // joined.n,) * 2
+    assert plan.n == 4 and plan.joined() is joined and joined.joined() is joined
+    # only one side consecutive, a mask that stays as it is, a shard that would outgrow the tile lists
+    assert rr._RingPlan(q, q, 4, ra.causal_bias(), {"q_positions": pos}, None).joined().n == want[0]
+    ids = torch.zeros(1, 64, dtype=torch.int32)
+    seg = {"q_segment_ids": ids}, {"kv_segment_ids": ids}
+    assert rr._RingPlan(q, q, 4, ra.segment_bias(), *seg).joined().n == 4
+    long = torch.zeros(1, 1, 1, 64, dtype=torch.bfloat16).expand(1, 4 * 32768, 1, 64)
+    ids = torch.zeros(1, 1, dtype=torch.int32).expand(1, 4 * 32768)
+    plan = rr._RingPlan(long, long, 4, ra.causal_bias() + ra.segment_bias(), {"q_segment_ids": ids}, {"kv_segment_ids": ids})
+    assert plan.joined().n == 2
+
+
 def test_ring_plan_with_a_callable_bias_fn():
     # the reference's general form: the callable sees the shards of its kwargs (ring.py:107,186)
     q = torch.zeros(2, 64, 2, 64, dtype=torch.bfloat16)

@@ -263,6 +263,17 @@ int ra_bwd_dkdv_ring(const ra_bwd_step_params* steps, const int32_t* steps_per_p
                      void* dv, int64_t stride_pass, int64_t stride_b, int64_t stride_h, int64_t stride_l,
                      void* stream);
 
+/* One pair of sequences from an empty carry to the finished result: what ra_fwd_ring returns for a
+ * single pass of a single step (ring.py:104-137 with a ring of one shard), with the kernels and the
+ * number of workgroups per row chosen by the pair's size and bias.  Where the keys of a row are
+ * shared by several workgroups their partial results go through `workspace`, a 16-byte aligned
+ * device buffer of at least ra_fwd_pair_workspace(p) bytes (0: none is needed, NULL is fine) that
+ * holds nothing between calls.  The o / m / l fields are not used. */
+int64_t ra_fwd_pair_workspace(const ra_fwd_step_params* p);
+int ra_fwd_pair(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b,
+                int64_t out_stride_h, int64_t out_stride_l, float* lse, void* workspace,
+                int64_t workspace_bytes, void* stream);
+
 /* The elementwise entry points for the shards of n_passes passes in one launch: the fp32 arrays of
  * the passes (carries, accumulators, lse, delta) lie one after another ([n_passes, B, H, L, ...]),
  * pass p reads / writes its strided tensor at an offset of p * stride_pass elements.  With

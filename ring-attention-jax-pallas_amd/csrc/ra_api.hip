@@ -528,11 +528,122 @@ int bwd_dkdv_passes(const ra_bwd_step_params* steps, const std::vector<int>& fir
   return run_passes<ra::QRing>(&ra::QRing::q, entries, live_first, n_passes, set_pass, launch, whole != nullptr);
 }
 
+// ---- one pair of sequences: which kernels, and how many workgroups share a row's keys --------------
+constexpr int kPairSlots = 512;  // workgroups of ra_pair.hip that the chip holds at once: two per compute unit
+constexpr int kPairRowsHost = 128, kPairKeysHost = 64;
+
+struct PairPlan {
+  bool pair;        // the kernels of ra_pair.hip
+  int n_split;      // most workgroups that share a row's keys ...
+  int chunk_tiles;  // ... each of about this many tiles
+};
+
+// Key tiles that one head's query tiles visit (positional terms only): their sum, and the most.
+void count_key_tiles(const ra_bias& bias, int Lq, int Lk, int64_t& total, int& most) {
+  const int ntiles = (Lk + kPairKeysHost - 1) / kPairKeysHost;
+  const ra::BiasArgs b = to_bias(bias);
+  total = 0;
+  most = 0;
+  for (int q0 = 0; q0 < Lq; q0 += kPairRowsHost) {
+    int lo, hi;
+    ra::key_tile_range(b.flags, b.window, b.q_off + q0, b.q_off + std::min(q0 + kPairRowsHost, Lq) - 1, b.kv_off, ntiles,
+                       kPairKeysHost, lo, hi);
+    total += hi - lo;
+    most = std::max(most, hi - lo);
+  }
+}
+
+// The forward kernels.  fwd_step_kernel is the faster one on long stretches of unmasked tiles of a
+// grid that fills the chip: causal / window terms at D = 128 (B=1, H=32, 16384 causal: 1.99 ms against
+// 2.13; 16 heads of 8192 x 8192 unmasked: 0.49 against 0.53).  fwd_pair_kernel is faster or as fast
+// everywhere else - B=2, H=16, 8192 causal: 0.57 both; B=2, H=32, 2048 causal: 0.096 against 0.125; window
+// 1024 of 16384, H=8: 0.099 against 0.116; any term per tile: documents (mean 1024) of 8192, B=2, H=16: 0.29
+// against 0.39, prefix-LM 8192, H=32: 0.68 against 3.0; D = 64: B=2, H=32, 16384 causal: 2.51 against 2.54.
+// The line lies at 96 tiles of 64 keys per workgroup, halfway between the two figures that it separates.
+//
+// A grid below 512 workgroups leaves places on the chip empty: the keys of a row are then shared.
+// Under a mask that leaves all rows about the same number of keys the shares are as many as there
+// are places; under a causal mask a share is 1.5 times the mean work of a place, so that the short
+// rows stay whole (B=1, D=128, causal, unsplit -> split: H=8, 2048: 46 -> 34 us; H=4, 4096: 85 -> 42 us; H=8,
+// 4096: 88 -> 63 us; H=4, 16384: 375 -> 340 us).  At most kMaxSplit shares, and none under kMinChunk tiles, which
+// cost more in partial results (528 bytes per row and share) than they gain.
+constexpr int kMinChunk = 6, kMaxSplit = 64;
+PairPlan plan_fwd_pair(const ra_fwd_step_params& p) {
+  const int rows = (p.Lq + kPairRowsHost - 1) / kPairRowsHost;
+  const int64_t heads = (int64_t)p.B * p.H, wgs = heads * rows;
+  int64_t total;
+  int most;
+  count_key_tiles(p.bias, p.Lq, p.Lk, total, most);
+  PairPlan r{true, 1, std::max(most, 1)};
+  if (kernel_mode(p.bias.flags) == 0 && p.D == 128 && wgs > kPairSlots && total >= 96 * (int64_t)rows) r.pair = false;
+  if (r.pair && wgs <= kPairSlots && most > kMinChunk) {
+    const bool even = total * 20 >= (int64_t)most * rows * 17;
+    const int64_t chunk = even ? (most + kPairSlots / wgs - 1) / (kPairSlots / wgs) : heads * total * 3 / (2 * kPairSlots);
+    r.chunk_tiles = (int)std::min<int64_t>(most, std::max<int64_t>({chunk, kMinChunk, (most + kMaxSplit - 1) / kMaxSplit}));
+    r.n_split = (most + r.chunk_tiles - 1) / r.chunk_tiles;
+  }
+  return r;
+}
+int64_t fwd_part_rows(const ra_fwd_step_params& p, int n_split) { return (int64_t)n_split * p.B * p.H * p.Lq; }
+int64_t fwd_part_bytes(const ra_fwd_step_params& p, int n_split) {
+  return 4 * (fwd_part_rows(p, n_split) * (p.D + 4) + (int64_t)p.B * p.H * ((p.Lq + kPairRowsHost - 1) / kPairRowsHost));
+}
+
 }  // namespace
 
 extern "C" {
 
-int ra_version(void) { return 1006; }
+int ra_version(void) { return 1007; }
+
+int64_t ra_fwd_pair_workspace(const ra_fwd_step_params* p) {
+  if (!p || check_dims(p->B, p->H, p->Lq, p->Lk, p->D)) return 0;
+  const int n = plan_fwd_pair(*p).n_split;
+  return n > 1 ? fwd_part_bytes(*p, n) : 0;
+}
+
+int ra_fwd_pair(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b, int64_t out_stride_h,
+                int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!p) return fail(RA_ERR_NULL, "params is NULL");
+  ra_fwd_step_params c = *p;
+  c.o = c.m = c.l = reinterpret_cast<float*>(uintptr_t(16));  // not used: there is no carry
+  int rc = ra_fwd_step_check(&c);
+  if (rc) return rc;
+  if (!lse) return fail(RA_ERR_NULL, "ra_fwd_pair: lse is NULL");
+  const RingResult r{out, nullptr, lse, out_dtype, 0, out_stride_b, out_stride_h, out_stride_l};
+  if ((rc = check_ring_result("ra_fwd_pair", r))) return rc;
+  const PairPlan plan = plan_fwd_pair(*p);
+  if (!plan.pair) return fwd_passes(p, std::vector<int>{0, 1}, 1, stream, &r);
+  ra::PairFwdArgs a;
+  memset(&a, 0, sizeof(a));
+  a.q = to_arg(p->q);
+  a.k = to_arg(p->k);
+  a.v = to_arg(p->v);
+  a.B = p->B;
+  a.H = p->H;
+  a.Lq = p->Lq;
+  a.Lk = p->Lk;
+  a.scale2 = p->sm_scale * kLog2eHost;
+  a.bias = to_bias(p->bias);
+  a.n_split = plan.n_split;
+  a.chunk_tiles = plan.chunk_tiles;
+  a.out = out;
+  a.out_f32 = out_dtype == RA_DTYPE_F32;
+  a.out_sb = out_stride_b;
+  a.out_sh = out_stride_h;
+  a.out_sl = out_stride_l;
+  a.lse = lse;
+  if (plan.n_split > 1) {
+    const int64_t rows = fwd_part_rows(*p, plan.n_split);
+    if (!workspace || !aligned16(workspace)) return fail(RA_ERR_ALIGN, "ra_fwd_pair: the workspace must be 16-byte aligned");
+    if (workspace_bytes < fwd_part_bytes(*p, plan.n_split))
+      return fail(RA_ERR_SHAPE, "ra_fwd_pair: the workspace is smaller than ra_fwd_pair_workspace()");
+    a.part_o = (float*)workspace;
+    a.part_s = a.part_o + rows * p->D;
+    a.part_n = (int*)(a.part_s + rows * 4);
+  }
+  hipError_t e = ra::launch_fwd_pair(a, p->D, kernel_mode(p->bias.flags), (hipStream_t)stream);
+  return e == hipSuccess ? RA_OK : hip_fail(e, "ra_fwd_pair launch");
+}
 
 const char* ra_last_error(void) { return g_err; }
 

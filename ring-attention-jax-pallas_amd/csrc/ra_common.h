@@ -351,23 +351,27 @@ RA_DEV int classify_pos(int flags, int window, int qlo, int qhi, int klo, int kh
   return (all ? 1 : 0) | (some ? 2 : 0);
 }
 
-RA_DEV int floor_div(int a, int b) { return (a >= 0) ? a / b : -((-a + b - 1) / b); }
-RA_DEV int ceil_div(int a, int b) { return -floor_div(-a, b); }
+// (shared with the host: it sizes the grids)
+#define RA_BOTH __host__ __device__ inline
+RA_BOTH int imin(int a, int b) { return a < b ? a : b; }
+RA_BOTH int imax(int a, int b) { return a > b ? a : b; }
+RA_BOTH int floor_div(int a, int b) { return (a >= 0) ? a / b : -((-a + b - 1) / b); }
+RA_BOTH int ceil_div(int a, int b) { return -floor_div(-a, b); }
 
 // Range [lo, hi) of T-sized tiles on the key side that can hold an unmasked score for
 // queries at positions [qlo, qhi]; keys of tile j are at positions kv_off + T*j + [0, T).
-RA_DEV void key_tile_range(int flags, int window, int qlo, int qhi, int kv_off, int ntiles, int T,
+RA_BOTH void key_tile_range(int flags, int window, int qlo, int qhi, int kv_off, int ntiles, int T,
                            int& lo, int& hi) {
   lo = 0;
   hi = ntiles;
   if (flags & RA_BIAS_PREFIX) return;
-  if (flags & RA_BIAS_CAUSAL) hi = min(hi, floor_div(qhi - kv_off, T) + 1);
+  if (flags & RA_BIAS_CAUSAL) hi = imin(hi, floor_div(qhi - kv_off, T) + 1);
   if (flags & RA_BIAS_WINDOW) {
-    lo = max(lo, ceil_div(qlo - window + 1 - (T - 1) - kv_off, T));
-    if (!(flags & RA_BIAS_CAUSAL)) hi = min(hi, floor_div(qhi + window - 1 - kv_off, T) + 1);
+    lo = imax(lo, ceil_div(qlo - window + 1 - (T - 1) - kv_off, T));
+    if (!(flags & RA_BIAS_CAUSAL)) hi = imin(hi, floor_div(qhi + window - 1 - kv_off, T) + 1);
   }
-  hi = max(hi, 0);
-  lo = min(max(lo, 0), hi);
+  hi = imax(hi, 0);
+  lo = imin(imax(lo, 0), hi);
 }
 
 // Range [lo, hi) of T-sized key tiles in which EVERY score of queries [qlo, qhi] is unmasked by
@@ -435,6 +439,33 @@ RA_DEV void tile_id_range(const int* ids, int t, int L, int& mn, int& mx) {
       mn = min(mn, sid);
       mx = max(mx, sid);
     }
+  }
+}
+
+// Whether some / all tokens of tile t carry a non-zero flag.
+template <int T>
+RA_DEV void tile_flag_range(const int* ids, int t, int L, bool& any, bool& all) {
+  int o = 0, z = 0;
+  const int base = t * T;
+#pragma unroll 8
+  for (int e = 0; e < T; ++e) {
+    const int x = ids[min(base + e, L - 1)];
+    o |= x;
+    z |= (x == 0);
+  }
+  any = o != 0;
+  all = z == 0;
+}
+
+// four elements of a result that is bf16 or fp32
+RA_DEV void store4(void* base, int f32, long long at, const f32x4& x) {
+  if (f32) {
+    *(f32x4*)((float*)base + at) = x;
+  } else {
+    bf16x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = (bf16_t)x[e];
+    *(bf16x4*)((bf16_t*)base + at) = y;
   }
 }
 

@@ -103,6 +103,26 @@ struct QRing {
   const int* kv_pre[kMaxPasses];
 };
 
+// One (query sequence, key sequence) pair on the kernels of ra_pair.hip.
+struct PairFwdArgs {
+  TensorArg q, k, v;
+  int B, H, Lq, Lk;
+  float scale2;  // sm_scale * log2(e)
+  BiasArgs bias;
+  int n_split;   // most workgroups that share a row's keys ...
+  int chunk_tiles;  // ... each of about this many key tiles
+  // where the result goes: partial results of the shares (n_split > 1; part_s: m, l, l of the rounded
+  // probabilities), a carry that is updated in place, or the finished output and logsumexp
+  float *part_o, *part_s;
+  int* part_n;
+  float *o, *m, *l;
+  void* out;
+  int out_f32;
+  long long out_sb, out_sh, out_sl;
+  float* lse;
+};
+hipError_t launch_fwd_pair(const PairFwdArgs& a, int D, int mode, hipStream_t stream);
+
 hipError_t launch_fwd_step(const FwdArgs& a, int D, int mode, hipStream_t stream);
 hipError_t launch_fwd_steps(const FwdArgs& a, const KvRing& ring, int D, int mode, hipStream_t stream);
 hipError_t launch_fwd_init(float* o, float* m, float* l, long long rows, int D, hipStream_t stream);

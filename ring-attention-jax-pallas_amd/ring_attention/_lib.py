@@ -89,6 +89,9 @@ EXPORTS = {
                                  C.c_int64, C.c_int64, C.c_int64, C.c_void_p]),
     "ra_bwd_dkdv_ring": (C.c_int, [C.POINTER(RaBwdStepParams), C.POINTER(C.c_int32), C.c_int32, C.c_void_p,
                                    C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_void_p]),
+    "ra_fwd_pair_workspace": (C.c_int64, [C.POINTER(RaFwdStepParams)]),
+    "ra_fwd_pair": (C.c_int, [C.POINTER(RaFwdStepParams), C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64,
+                              C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p]),
     "ra_fwd_finalize_passes": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_int64,
                                          C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32, C.c_int32,
                                          C.c_int32, C.c_int32, C.c_int32, C.c_void_p]),

@@ -421,10 +421,7 @@ class _RingPlan:
         were shard boundaries, and the host describes one shard pair instead of n * n.  Forward +
         backward: B=2, H=16, 8 x 1024 causal 2.52 -> 2.28 ms; B=2, H=16, D=64, 4 x 1024 causal + ALiBi
         0.73 -> 0.64 ms; fp32 inputs, B=2, H=4, 8 x 256: 3.6 -> 0.19 ms, nearly all of it host code.
-        Prefix-LM masks and documents without a causal mask stay as they are: the first has no
-        straight-line stretches to lengthen (-3 % joined), the second finds two runs of one-id
-        tiles per shard and workgroup, so that fewer shards leave more tiles to the generic
-        iterations (-2 %).  The joined shards stay within what one launch takes under a segment term."""
+        The joined shards stay within what one launch takes under a segment term."""
         got = self.__dict__.get("_joined")
         if got is None:
             got = self._join()
@@ -434,7 +431,7 @@ class _RingPlan:
     def _join(self) -> "_RingPlan":
         n, Lq, Lk = self.n, self.Lq, self.Lk
         fn = self.fn
-        if self.callable is not None or n == 1 or (fn is not None and (fn.prefix or (fn.segments and not fn.causal))):
+        if self.callable is not None or n == 1:
             return self
         segments = fn is not None and fn.segments
         for g in range(n, 1, -1):
@@ -708,9 +705,11 @@ def _pair_forward(q, k, v, plan: "_RingPlan", sm_scale, out_dtype):
     lse = torch.empty((1, B, H, Lq), dtype=torch.float32, device=plan.device)
     p = _lib.RaFwdStepParams(B, H, Lq, plan.Lk, D, sm_scale, _view_blhd(q), _view_blhd(k), _view_blhd(v), None, None,
                              None, plan.pair_bias())
-    _lib.check("ra_fwd_ring", _lib.load().ra_fwd_ring(
-        C.byref(p), _ONE_STEP, 1, out.data_ptr(), _DTYPE_CODE[out_dtype], 0, Lq * H * D, D, H * D, lse.data_ptr(),
-        _stream()))
+    lib = _lib.load()
+    size = lib.ra_fwd_pair_workspace(C.byref(p))
+    ws = torch.empty((size,), dtype=torch.uint8, device=plan.device) if size else None
+    _lib.check("ra_fwd_pair", lib.ra_fwd_pair(C.byref(p), out.data_ptr(), _DTYPE_CODE[out_dtype], Lq * H * D, D, H * D,
+                                              lse.data_ptr(), None if ws is None else ws.data_ptr(), size, _stream()))
     return out, lse
 
 

@@ -152,11 +152,8 @@ def test_consecutive_shards_are_joined(starts, want):
     assert (joined.n, joined.q_off) == want and joined.kv_off == joined.q_off
     assert (joined.Lq, joined.Lk) == (64 // joined.n,) * 2
     assert plan.n == 4 and plan.joined() is joined and joined.joined() is joined
-    # only one side consecutive, a mask that stays as it is, a shard that would outgrow the tile lists
+    # only one side consecutive, a shard that would outgrow the tile lists
     assert rr._RingPlan(q, q, 4, ra.causal_bias(), {"q_positions": pos}, None).joined().n == want[0]
-    ids = torch.zeros(1, 64, dtype=torch.int32)
-    seg = {"q_segment_ids": ids}, {"kv_segment_ids": ids}
-    assert rr._RingPlan(q, q, 4, ra.segment_bias(), *seg).joined().n == 4
     long = torch.zeros(1, 1, 1, 64, dtype=torch.bfloat16).expand(1, 4 * 32768, 1, 64)
     ids = torch.zeros(1, 1, dtype=torch.int32).expand(1, 4 * 32768)
     plan = rr._RingPlan(long, long, 4, ra.causal_bias() + ra.segment_bias(), {"q_segment_ids": ids}, {"kv_segment_ids": ids})

@@ -274,6 +274,16 @@ int ra_fwd_pair(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64
                 int64_t out_stride_h, int64_t out_stride_l, float* lse, void* workspace,
                 int64_t workspace_bytes, void* stream);
 
+/* The gradients of that pair, finished: delta (ring_kernel.py:387-409) and what ra_bwd_dkdv_ring and
+ * ra_bwd_dq_ring store (ring.py:183-210 with a ring of one shard), dk and dv with the same strides.  `out` is
+ * the forward's output.  The workspace (at least ra_bwd_pair_workspace(p) bytes, 16-byte aligned) holds
+ * delta and partial sums; the delta / dq / dk / dv fields of the block are not used. */
+int64_t ra_bwd_pair_workspace(const ra_bwd_step_params* p);
+int ra_bwd_pair(const ra_bwd_step_params* p, const void* out, int32_t out_dtype, int64_t out_stride_b,
+                int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
+                int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
+                int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* The elementwise entry points for the shards of n_passes passes in one launch: the fp32 arrays of
  * the passes (carries, accumulators, lse, delta) lie one after another ([n_passes, B, H, L, ...]),
  * pass p reads / writes its strided tensor at an offset of p * stride_pass elements.  With

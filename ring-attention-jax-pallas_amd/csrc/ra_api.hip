@@ -553,14 +553,21 @@ void count_key_tiles(const ra_bias& bias, int Lq, int Lk, int64_t& total, int& m
   }
 }
 
-// The forward kernels.  fwd_step_kernel is the faster one on long stretches of unmasked tiles of a
-// grid that fills the chip: causal / window terms at D = 128 (B=1, H=32, 16384 causal: 1.99 ms against
-// 2.13; 16 heads of 8192 x 8192 unmasked: 0.49 against 0.53).  fwd_pair_kernel is faster or as fast
-// everywhere else - B=2, H=16, 8192 causal: 0.57 both; B=2, H=32, 2048 causal: 0.096 against 0.125; window
-// 1024 of 16384, H=8: 0.099 against 0.116; any term per tile: documents (mean 1024) of 8192, B=2, H=16: 0.29
-// against 0.39, prefix-LM 8192, H=32: 0.68 against 3.0; D = 64: B=2, H=32, 16384 causal: 2.51 against 2.54.
-// The line lies at 96 tiles of 64 keys per workgroup, halfway between the two figures that it separates.
-//
+// Whether the kernels of ra_fwd.hip / ra_bwd.hip, which hold twice the rows or keys per compute unit and hide all
+// vector work in straight-line stretches, are the faster ones: nothing but positions and ALiBi masks, D = 128, a
+// grid that fills the chip, and at least `tiles` tiles per workgroup on average.  With a list of tiles (documents,
+// prefix, dense block) or D = 64 those of ra_pair.hip are (documents + ALiBi, 32768, H=16: forward 1.1 ms against 1.4,
+// dQ 1.25 against 1.53, dK/dV 1.87 against 1.88; causal documents of mean 1024, 8192, B=2, H=16: 0.29 / 0.22 / 0.30
+// against 0.39 / 0.35 / 0.42; prefix-LM 16384, H=16: 5.6 ms in total against 18; D=64, 32768 causal, H=16: 2.34 / 2.79 /
+// 3.75 against 2.39 / 3.15 / 3.92).
+bool long_stretches(const ra_bias& bias, int D, int64_t wgs, int64_t total, int64_t rows, int tiles) {
+  const bool lists = bias.flags & (RA_BIAS_SEGMENT | RA_BIAS_PREFIX | RA_BIAS_DENSE);
+  return D == 128 && !lists && wgs > kPairSlots && total >= tiles * rows;
+}
+
+// The forward kernels, in 64-key tiles per 128 rows (causal or window, H * B heads; fwd_step_kernel | fwd_pair_kernel):
+// 17 of them (64 heads of 2048) 0.118 | 0.096 ms, 65 (32 of 8192) 0.52 | 0.53, 64 (64 of 4096 x 4096) 0.50 | 0.53, 129 (32 of
+// 16384) 1.92 | 2.10, 257 (32 of 32768) 7.4 | 8.7; with ALiBi, 129 (16 of 16384): 1.18 | 1.21.
 // A grid below 512 workgroups leaves places on the chip empty: the keys of a row are then shared.
 // Under a mask that leaves all rows about the same number of keys the shares are as many as there
 // are places; under a causal mask a share is 1.5 times the mean work of a place, so that the short
@@ -568,6 +575,16 @@ void count_key_tiles(const ra_bias& bias, int Lq, int Lk, int64_t& total, int& m
 // 4096: 88 -> 63 us; H=4, 16384: 375 -> 340 us).  At most kMaxSplit shares, and none under kMinChunk tiles, which
 // cost more in partial results (528 bytes per row and share) than they gain.
 constexpr int kMinChunk = 6, kMaxSplit = 64;
+// How the `wgs` workgroups of one kind of a head's resident tiles, which meet `total` tiles of the other
+// side (`most` at most), share their work (see above).
+void plan_split(PairPlan& r, int64_t heads, int64_t rows, int64_t total, int most, int min_chunk) {
+  const int64_t wgs = heads * rows;
+  if (wgs > kPairSlots || most <= min_chunk) return;
+  const bool even = total * 20 >= (int64_t)most * rows * 17;
+  const int64_t chunk = even ? (most + kPairSlots / wgs - 1) / (kPairSlots / wgs) : heads * total * 3 / (2 * kPairSlots);
+  r.chunk_tiles = (int)std::min<int64_t>(most, std::max<int64_t>({chunk, min_chunk, (most + kMaxSplit - 1) / kMaxSplit}));
+  r.n_split = (most + r.chunk_tiles - 1) / r.chunk_tiles;
+}
 PairPlan plan_fwd_pair(const ra_fwd_step_params& p) {
   const int rows = (p.Lq + kPairRowsHost - 1) / kPairRowsHost;
   const int64_t heads = (int64_t)p.B * p.H, wgs = heads * rows;
@@ -575,14 +592,66 @@ PairPlan plan_fwd_pair(const ra_fwd_step_params& p) {
   int most;
   count_key_tiles(p.bias, p.Lq, p.Lk, total, most);
   PairPlan r{true, 1, std::max(most, 1)};
-  if (kernel_mode(p.bias.flags) == 0 && p.D == 128 && wgs > kPairSlots && total >= 96 * (int64_t)rows) r.pair = false;
-  if (r.pair && wgs <= kPairSlots && most > kMinChunk) {
-    const bool even = total * 20 >= (int64_t)most * rows * 17;
-    const int64_t chunk = even ? (most + kPairSlots / wgs - 1) / (kPairSlots / wgs) : heads * total * 3 / (2 * kPairSlots);
-    r.chunk_tiles = (int)std::min<int64_t>(most, std::max<int64_t>({chunk, kMinChunk, (most + kMaxSplit - 1) / kMaxSplit}));
-    r.n_split = (most + r.chunk_tiles - 1) / r.chunk_tiles;
-  }
+  if (long_stretches(p.bias, p.D, wgs, total, rows, 56)) r.pair = false;
+  if (r.pair) plan_split(r, heads, rows, total, most, kMinChunk);
   return r;
+}
+// dQ, likewise (dq_kernel | dq_pair_kernel): 65 tiles (32 heads of 8192) 0.70 | 0.66 ms, 66 (window 4096 of 65536, H=8) 1.36 |
+// 1.33, 129 (16 of 16384) 1.31 | 1.30, 128 (16 of 8192 x 8192) 0.64 | 0.66, 257 (32 of 32768) 10.1 | 10.4; ALiBi, 129: 1.41 | 1.32.
+PairPlan plan_dq_pair(const ra_bwd_step_params& p) {
+  int64_t total;
+  int most;
+  count_key_tiles(p.bias, p.Lq, p.Lk, total, most);
+  PairPlan r{true, 1, std::max(most, 1)};
+  const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lq + kPairRowsHost - 1) / kPairRowsHost;
+  if (long_stretches(p.bias, p.D, heads * rows, total, rows, 160)) r.pair = false;
+  else plan_split(r, heads, rows, total, most, kMinChunk);
+  return r;
+}
+// dK / dV, in 32-query tiles per 128 keys (dkdv_kernel | dkdv_pair_kernel): 65 (64 heads of 4096) 0.55 | 0.50 ms, 130 (32 of
+// 8192) 0.90 | 0.92, 128 (64 of 4096 x 4096) 0.88 | 0.91, 258 (32 of 16384) 3.4 | 3.6; ALiBi, 258: 1.82 | 1.90.  dkdv_kernel also
+// where there are between one and two and a half slabs per compute unit: dkdv_pair_kernel would hold them all at
+// once, the longest one deciding (16 heads of 4096: 0.13 | 0.16).  Fewer slabs are shared (12 heads of 2048: 0.056 | 0.050).
+PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
+  const int ntiles = (p.Lq + 31) / 32;
+  const ra::BiasArgs b = to_bias(p.bias);
+  int64_t total = 0;
+  int most = 0;
+  for (int k0 = 0; k0 < p.Lk; k0 += kPairRowsHost) {
+    int lo, hi;
+    ra::query_tile_range(b.flags, b.window, b.kv_off + k0, b.kv_off + std::min(k0 + kPairRowsHost, p.Lk) - 1, b.q_off, ntiles, 32, lo, hi);
+    total += hi - lo;
+    most = std::max(most, hi - lo);
+  }
+  PairPlan r{true, 1, std::max(most, 1)};
+  const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lk + kPairRowsHost - 1) / kPairRowsHost, wgs = heads * rows;
+  const bool one_round = wgs > kPairSlots / 2 && wgs <= kPairSlots * 5 / 4;
+  if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, total, rows, one_round ? 0 : 112)) r.pair = false;
+  else plan_split(r, heads, rows, total, most, 2 * kMinChunk);
+  return r;
+}
+// The workspace of ra_bwd_pair: the rows' statistics, then the shares of dQ and of dK and dV.
+struct BwdSpace {
+  int64_t delta, stat, dq_part, dq_n, dkdv_part, dkdv_n, total;  // byte offsets (16-byte aligned) and the size
+};
+BwdSpace bwd_space(const ra_bwd_step_params& p, const PairPlan& dq, const PairPlan& dkdv) {
+  BwdSpace s;
+  int64_t at = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t here = at;
+    at += (bytes + 15) & ~(int64_t)15;
+    return here;
+  };
+  auto tiles = [](int L) { return (int64_t)(L + kPairRowsHost - 1) / kPairRowsHost; };
+  const int64_t heads = (int64_t)p.B * p.H, q_rows = heads * p.Lq, k_rows = heads * p.Lk;
+  s.delta = take(4 * q_rows);
+  s.stat = take(8 * q_rows);
+  s.dq_part = take(dq.n_split > 1 ? 4 * dq.n_split * q_rows * p.D : 0);
+  s.dq_n = take(dq.n_split > 1 ? 4 * heads * tiles(p.Lq) : 0);
+  s.dkdv_part = take(dkdv.n_split > 1 ? 8 * dkdv.n_split * k_rows * p.D : 0);
+  s.dkdv_n = take(dkdv.n_split > 1 ? 4 * heads * tiles(p.Lk) : 0);
+  s.total = at;
+  return s;
 }
 int64_t fwd_part_rows(const ra_fwd_step_params& p, int n_split) { return (int64_t)n_split * p.B * p.H * p.Lq; }
 int64_t fwd_part_bytes(const ra_fwd_step_params& p, int n_split) {
@@ -888,6 +957,66 @@ int ra_bwd_dkdv_ring(const ra_bwd_step_params* steps, const int32_t* steps_per_p
   const RingResult r{dk, dv, nullptr, RA_DTYPE_BF16, stride_pass, stride_b, stride_h, stride_l};
   if ((rc = check_ring_result("ra_bwd_dkdv_ring", r))) return rc;
   return bwd_dkdv_passes(steps, first, n_passes, stream, &r);
+}
+
+int64_t ra_bwd_pair_workspace(const ra_bwd_step_params* p) {
+  if (!p || check_dims(p->B, p->H, p->Lq, p->Lk, p->D)) return 0;
+  return bwd_space(*p, plan_dq_pair(*p), plan_dkdv_pair(*p)).total;
+}
+
+int ra_bwd_pair(const ra_bwd_step_params* p, const void* out, int32_t out_dtype, int64_t out_stride_b,
+                int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
+                int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
+                int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!p) return fail(RA_ERR_NULL, "params is NULL");
+  ra_bwd_step_params c = *p;
+  c.delta = c.dq = c.dk = c.dv = reinterpret_cast<float*>(uintptr_t(16));  // not used: no accumulators
+  int rc = ra_bwd_step_check(&c);
+  if (rc) return rc;
+  const RingResult rq{dq, nullptr, nullptr, RA_DTYPE_BF16, 0, dq_stride_b, dq_stride_h, dq_stride_l};
+  const RingResult rk{dk, dv, nullptr, RA_DTYPE_BF16, 0, dkv_stride_b, dkv_stride_h, dkv_stride_l};
+  if ((rc = check_ring_result("ra_bwd_pair", rq)) || (rc = check_ring_result("ra_bwd_pair", rk))) return rc;
+  if (!dv) return fail(RA_ERR_NULL, "ra_bwd_pair: dv is NULL");
+  const PairPlan plan_q = plan_dq_pair(*p), plan_k = plan_dkdv_pair(*p);
+  const BwdSpace sp = bwd_space(*p, plan_q, plan_k);
+  if (!workspace || !aligned16(workspace)) return fail(RA_ERR_ALIGN, "ra_bwd_pair: the workspace must be 16-byte aligned");
+  if (workspace_bytes < sp.total) return fail(RA_ERR_SHAPE, "ra_bwd_pair: the workspace is smaller than ra_bwd_pair_workspace()");
+  if (!out || !aligned16(out) || (out_stride_b % 8) || (out_stride_h % 8) || (out_stride_l % 8))
+    return fail(RA_ERR_ALIGN, "ra_bwd_pair: out must be 16-byte aligned with strides that are multiples of 8");
+  if (out_dtype != RA_DTYPE_BF16 && out_dtype != RA_DTYPE_F32) return fail(RA_ERR_DTYPE, "unknown out_dtype %d", out_dtype);
+  char* const ws = (char*)workspace;
+  c.delta = (float*)(ws + sp.delta);
+  ra::PairBwdArgs a;
+  memset(&a, 0, sizeof(a));
+  a.a = to_bwd_args(c);
+  a.stat = (const float*)(ws + sp.stat);
+  hipError_t e = ra::launch_pair_stat(out, out_dtype == RA_DTYPE_F32, out_stride_b, out_stride_h, out_stride_l, a.a.dout, c.lse,
+                                      1.0f / a.a.scale_res, (float*)(ws + sp.stat), (float*)(ws + sp.delta), c.B, c.H, c.Lq, c.D,
+                                      (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "ra_bwd_pair launch");
+  const std::vector<int> one{0, 1};
+  const int mode = kernel_mode(c.bias.flags);
+  auto share = [&](const PairPlan& plan, int64_t part, int64_t n, const RingResult& r) {
+    a.n_split = plan.n_split;
+    a.chunk_tiles = plan.chunk_tiles;
+    a.part = plan.n_split > 1 ? (float*)(ws + part) : nullptr;
+    a.part_n = plan.n_split > 1 ? (int*)(ws + n) : nullptr;
+    a.out = r.base;
+    a.out2 = r.base2;
+    a.out_sb = r.stride_b;
+    a.out_sh = r.stride_h;
+    a.out_sl = r.stride_l;
+  };
+  if (plan_k.pair) {
+    share(plan_k, sp.dkdv_part, sp.dkdv_n, rk);
+    if ((e = ra::launch_dkdv_pair(a, c.D, mode, (hipStream_t)stream)) != hipSuccess) return hip_fail(e, "ra_bwd_pair launch");
+  } else if ((rc = bwd_dkdv_passes(&c, one, 1, stream, &rk))) {
+    return rc;
+  }
+  if (!plan_q.pair) return bwd_dq_passes(&c, one, 1, stream, &rq);
+  share(plan_q, sp.dq_part, sp.dq_n, rq);
+  e = ra::launch_dq_pair(a, c.D, mode, (hipStream_t)stream);
+  return e == hipSuccess ? RA_OK : hip_fail(e, "ra_bwd_pair launch");
 }
 
 int ra_bwd_finalize_passes(const float* acc, void* out, int64_t out_stride_pass, int64_t out_stride_b,

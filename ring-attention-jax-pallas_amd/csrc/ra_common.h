@@ -403,18 +403,18 @@ RA_DEV void query_tile_plain_range(int flags, int window, int klo, int khi, int 
 }
 
 // Same for the query side: tiles of queries that can see keys at positions [klo, khi].
-RA_DEV void query_tile_range(int flags, int window, int klo, int khi, int q_off, int ntiles, int T,
+RA_BOTH void query_tile_range(int flags, int window, int klo, int khi, int q_off, int ntiles, int T,
                              int& lo, int& hi) {
   lo = 0;
   hi = ntiles;
   if (flags & RA_BIAS_PREFIX) return;
-  if (flags & RA_BIAS_CAUSAL) lo = max(lo, ceil_div(klo - (T - 1) - q_off, T));
+  if (flags & RA_BIAS_CAUSAL) lo = imax(lo, ceil_div(klo - (T - 1) - q_off, T));
   if (flags & RA_BIAS_WINDOW) {
-    hi = min(hi, floor_div(khi + window - 1 - q_off, T) + 1);
-    if (!(flags & RA_BIAS_CAUSAL)) lo = max(lo, ceil_div(klo - window + 1 - (T - 1) - q_off, T));
+    hi = imin(hi, floor_div(khi + window - 1 - q_off, T) + 1);
+    if (!(flags & RA_BIAS_CAUSAL)) lo = imax(lo, ceil_div(klo - window + 1 - (T - 1) - q_off, T));
   }
-  hi = max(hi, 0);
-  lo = min(max(lo, 0), hi);
+  hi = imax(hi, 0);
+  lo = imin(imax(lo, 0), hi);
 }
 
 // Smallest and largest id of tile t (T tokens) of an id array of length L.  The loads are

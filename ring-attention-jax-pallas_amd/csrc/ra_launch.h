@@ -122,6 +122,22 @@ struct PairFwdArgs {
   float* lse;
 };
 hipError_t launch_fwd_pair(const PairFwdArgs& a, int D, int mode, hipStream_t stream);
+// The gradient of the resident side (dQ; or dK and dV: acc2, out2): shares of a row's sum (n_split > 1),
+// fp32 accumulators that are added to, or the finished bf16 gradient.
+struct PairBwdArgs {
+  BwdArgs a;  // (its dq / dk / dv slots are not used)
+  int n_split, chunk_tiles;
+  const float* stat;  // dK / dV: see pair_stat_kernel
+  float* part;
+  int* part_n;
+  float *acc, *acc2;
+  void *out, *out2;
+  long long out_sb, out_sh, out_sl;
+};
+hipError_t launch_dq_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream);
+hipError_t launch_dkdv_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream);
+hipError_t launch_pair_stat(const void* out, int out_f32, long long sb, long long sh, long long sl, TensorArg dout, const float* lse,
+                            float inv_res, float* stat, float* delta, int B, int H, int Lq, int D, hipStream_t stream);
 
 hipError_t launch_fwd_step(const FwdArgs& a, int D, int mode, hipStream_t stream);
 hipError_t launch_fwd_steps(const FwdArgs& a, const KvRing& ring, int D, int mode, hipStream_t stream);

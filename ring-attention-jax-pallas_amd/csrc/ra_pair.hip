@@ -21,7 +21,7 @@ constexpr int kPairKeys = 64;   // keys per LDS tile
 constexpr int kPairListTiles = 1024;
 
 // what a listed tile must evaluate element by element (bits of a list entry, above the tile index)
-constexpr int kTestShift = 10;
+constexpr int kTestShift = 11;
 constexpr int kTestSegment = 1, kTestPrefix = 2, kTestDense = 4;
 
 // Rows and keys of a workgroup's rectangle as the prefix term sees them: 0 = untouched by the mask,
@@ -45,6 +45,157 @@ RA_DEV void pair_decode(int bid, int BH, int ntile, int& hh, int& piece, int& ti
   piece = t / ntile;
   tile = ntile - 1 - t % ntile;
   hh = spread ? hl * 8 + (bid & 7) : hl;
+}
+
+// Moves ROWS-row tiles of one [L][D] matrix from memory to LDS: each of the four waves takes a quarter of
+// a tile's rows, 1 KiB per instruction.  Lane l fills the l-th 16 bytes of the kilobyte; the permuted
+// layout (tile_off) is obtained by letting it fetch the chunk that belongs there.  From one
+// instruction to another that chunk differs by an XOR: two registers hold what all of them need.
+template <int D, int ROWS>
+struct TileLoader {
+  static constexpr int CPR = D / 8;            // 16-byte chunks per row
+  static constexpr int RPI = 64 / CPR;         // rows per load instruction
+  static constexpr int RPW = ROWS / 4;         // rows per wave
+  static constexpr int NLD = RPW / RPI;        // load instructions per wave and tile
+  const bf16_t* base;
+  long long sl;
+  int L;
+  unsigned row_off;  // byte offset of this lane's row from the first one of an instruction
+  RA_DEV void init(const bf16_t* base_, long long sl_, int L_, int lane) {
+    base = base_;
+    sl = sl_;
+    L = L_;
+    row_off = (unsigned)((long long)(lane / CPR) * sl * 2);
+  }
+  // byte offset inside its row of the chunk that a lane moves with an instruction that starts at row 0 of
+  // a tile, and at `row` (a multiple of RPI)
+  static RA_DEV unsigned first_chunk(int lane) { return (unsigned)(tile_off<D>(lane / CPR, lane % CPR) - (lane / CPR) * (D * 2)); }
+  static RA_DEV unsigned chunk(unsigned first, int row) { return first ^ (16 * (D == 128 ? (row >> 2) & 3 : (row >> 1) & 7)); }
+  RA_DEV void issue(int row0, unsigned dst, int wave, int lane, unsigned first) const {
+    dst += RPW * wave * (D * 2);
+    if (row0 + ROWS <= L) {
+      const bf16_t* sb = base + (long long)(row0 + RPW * wave) * sl;  // wave-uniform: scalar registers
+#pragma unroll
+      for (int t = 0; t < NLD; ++t)
+        global_to_lds16_s(sb + (long long)(RPI * t) * sl, row_off + chunk(first, RPW * wave + RPI * t), dst + RPI * t * (D * 2));
+    } else {  // last, partial tile: rows past the end repeat the last row (masked later)
+#pragma unroll
+      for (int t = 0; t < NLD; ++t) {
+        const int row = RPW * wave + RPI * t;
+        global_to_lds16((const char*)(base + (long long)min(row0 + row + lane / CPR, L - 1) * sl) + chunk(first, row),
+                        dst + RPI * t * (D * 2));
+      }
+    }
+  }
+};
+
+// Per-lane LDS byte offsets of the operand fetches inside a block of 32 rows.  The permutation of a
+// row's chunks is an XOR, and so is the step from one operand to the next: two registers and an XOR
+// per fetch instead of a register per operand, which these kernels do not have.
+template <int D>
+struct FragOffsets {
+  int n0, t0;
+  RA_DEV explicit FragOffsets(int lane) {
+    const int l32 = lane & 31, g = lane >> 5, j = lane & 15;
+    n0 = tile_off<D>(l32, g);
+    const int col = 16 * ((lane >> 4) & 1) + 4 * (j & 3);
+    t0 = tile_off<D>(4 * g + (j >> 2), col >> 3) + ((col & 4) << 1);
+  }
+  RA_DEV FragOffsets opaque() const {  // not to be hoisted out of the loop it is used in
+    FragOffsets r = *this;
+    asm volatile("" : "+v"(r.n0), "+v"(r.t0));
+    return r;
+  }
+  // row l32, head-dim elements 16 ss + 8 g ..: chunk 2 ss + g
+  RA_DEV int nat(int ss) const { return n0 ^ (ss << 5); }
+  // rows 8 h2 + 4 g + j / 4, columns 32 db + ...: chunk 4 db + ...; eight rows further the row's
+  // permutation differs in one bit (D = 128: bit 1, D = 64: bit 2 of the chunk)
+  RA_DEV int tr(int db, int h2) const { return (t0 ^ (db << 6) ^ (h2 * (D == 128 ? 32 : 64))) + h2 * 8 * (D * 2); }
+};
+
+// The list of key tiles that the workgroup's rows [q0, q_hi] have to visit, of the n from j_lo on:
+// tiles that one or the other term rules out are dropped, the others carry the terms that they
+// have to be tested for.  Returns their number.  Called by all four waves.
+template <bool DENSE>
+RA_DEV int list_key_tiles(int Lq, int Lk, const BiasArgs& bs, const int* kv_seg, const int* kv_pre, const unsigned char* dmap,
+                          int q0, int q_hi, bool q_valid, int q_seg, int q_pre, int j_lo, int n, int* s_red,
+                          unsigned char* s_flag, unsigned short* s_list) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool seg_on = kv_seg != nullptr, pre_on = kv_pre != nullptr;
+  const int smin = wave_min(q_valid ? q_seg : 0x7fffffff), smax = wave_max(q_valid ? q_seg : (int)0x80000000);
+  const int any = __any(q_valid && q_pre != 0), all = __all(!q_valid || q_pre != 0);
+  if (lane == 0) {
+    s_red[wave] = smin;
+    s_red[4 + wave] = smax;
+    s_red[8 + wave] = any;
+    s_red[12 + wave] = all;
+  }
+  __syncthreads();
+  const int qmin = min(min(s_red[0], s_red[1]), min(s_red[2], s_red[3]));
+  const int qmax = max(max(s_red[4], s_red[5]), max(s_red[6], s_red[7]));
+  const bool q_any = s_red[8] | s_red[9] | s_red[10] | s_red[11], q_all = s_red[12] & s_red[13] & s_red[14] & s_red[15];
+  for (int i = tid; i < n; i += kPairThreads) {
+    const int j = j_lo + i;
+    int f = 0x80;  // listed
+    if (seg_on) {
+      int kmin, kmax;
+      tile_id_range<kPairKeys>(kv_seg, j, Lk, kmin, kmax);
+      if (kmax < qmin || kmin > qmax) f = 0;
+      else if (kmin != kmax || qmin != qmax) f |= kTestSegment;
+    }
+    if (pre_on && f) {
+      const int klo = bs.kv_off + j * kPairKeys, khi = bs.kv_off + min((j + 1) * kPairKeys, Lk) - 1;
+      if (khi > bs.q_off + q0) {
+        bool k_any, k_all;
+        tile_flag_range<kPairKeys>(kv_pre, j, Lk, k_any, k_all);
+        const int c = prefix_class(bs.q_off + q0, bs.q_off + q_hi, klo, khi, q_any, q_all, k_any, k_all);
+        if (c == 2) f = 0;
+        else if (c == 1) f |= kTestPrefix;
+      }
+    }
+    if constexpr (DENSE) {
+      if (dmap != nullptr && f) {
+        const int bits = dense_map_or(dmap, Lk, q0, q_hi, j * kPairKeys, min((j + 1) * kPairKeys, Lk) - 1);
+        if (!(bits & kMapLive)) f = 0;
+        else if (bits & kMapNonZero) f |= kTestDense;
+      }
+    }
+    s_flag[i] = (unsigned char)f;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int cnt = 0;
+    for (int base = 0; base < n; base += 64) {
+      const int i = base + lane;
+      const int f = (i < n) ? s_flag[i] : 0;
+      const unsigned long long mask = __ballot(f != 0);
+      if (f) s_list[cnt + __popcll(mask & ((1ull << lane) - 1ull))] = (unsigned short)((j_lo + i) | ((f & 7) << kTestShift));
+      cnt += __popcll(mask);
+    }
+    if (lane == 0) s_red[16] = cnt;
+  }
+  __syncthreads();
+  return s_red[16];
+}
+
+// ALiBi on one side of the diagonal: -slope |q - k| = -s (rel - j), with s = +-slope (score units), rel the
+// distance of this lane's query from the tile's first key and j the key's index in the tile, is linear in
+// both positions and enters through the matrix unit as the accumulator's initial value:
+// [j, j, 1, 1, 1] x [s_hi, s_lo, c_hi, c_mid, c_lo], s and c = -s rel split into bf16 words (see
+// fwd_step_kernel).  kb: the 32-key block of the tile.
+RA_DEV f32x16 alibi_one_side(const f32x16& zero, float s, int rel, int kb, int l32, int g) {
+  const float c = -s * (float)rel;
+  bf16x8 bq, rf;
+  bq[0] = (bf16_t)s;
+  bq[1] = (bf16_t)(s - (float)bq[0]);
+  bq[2] = (bf16_t)c;
+  bq[3] = (bf16_t)(c - (float)bq[2]);
+  bq[4] = (bf16_t)((c - (float)bq[2]) - (float)bq[3]);
+  bq[5] = bq[6] = bq[7] = (bf16_t)0.f;
+  rf[0] = rf[1] = (bf16_t)(g == 0 ? (float)(32 * kb + l32) : 0.f);
+  rf[2] = rf[3] = rf[4] = (bf16_t)(g == 0 ? 1.0f : 0.f);
+  rf[5] = rf[6] = rf[7] = (bf16_t)0.f;
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(rf, bq, zero, 0, 0, 0);
 }
 
 // S^T orientation as in fwd_step_kernel: a lane owns one query row and 16 keys of a 32-key block.
@@ -118,65 +269,9 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     if (bs.dense_map) dmap = dense_map_of(bs, b, h, a.H, a.Lq, a.Lk);
   }
   if constexpr (GENERAL) {
-    // tiles that one or the other term rules out are dropped, the others carry the terms that they
-    // have to be tested for
-    const bool seg_on = flags & RA_BIAS_SEGMENT, pre_on = flags & RA_BIAS_PREFIX;
-    use_list = ntiles <= kPairListTiles && (seg_on || pre_on || dmap != nullptr);
-    if (use_list) {
-      const int smin = wave_min(q_valid ? q_seg : 0x7fffffff), smax = wave_max(q_valid ? q_seg : (int)0x80000000);
-      const int any = __any(q_valid && q_pre != 0), all = __all(!q_valid || q_pre != 0);
-      if (lane == 0) {
-        s_red[wave] = smin;
-        s_red[4 + wave] = smax;
-        s_red[8 + wave] = any;
-        s_red[12 + wave] = all;
-      }
-      __syncthreads();
-      const int qmin = min(min(s_red[0], s_red[1]), min(s_red[2], s_red[3]));
-      const int qmax = max(max(s_red[4], s_red[5]), max(s_red[6], s_red[7]));
-      const bool q_any = s_red[8] | s_red[9] | s_red[10] | s_red[11], q_all = s_red[12] & s_red[13] & s_red[14] & s_red[15];
-      for (int j = j_lo + tid; j < j_hi; j += kPairThreads) {
-        int f = 0x80;  // listed
-        if (seg_on) {
-          int kmin, kmax;
-          tile_id_range<kPairKeys>(kv_seg, j, a.Lk, kmin, kmax);
-          if (kmax < qmin || kmin > qmax) f = 0;
-          else if (kmin != kmax || qmin != qmax) f |= kTestSegment;
-        }
-        if (pre_on && f) {
-          const int klo = kv_off + j * kPairKeys, khi = kv_off + min((j + 1) * kPairKeys, a.Lk) - 1;
-          if (khi > q_off + q0) {
-            bool k_any, k_all;
-            tile_flag_range<kPairKeys>(kv_pre, j, a.Lk, k_any, k_all);
-            const int c = prefix_class(q_off + q0, q_off + q_hi, klo, khi, q_any, q_all, k_any, k_all);
-            if (c == 2) f = 0;
-            else if (c == 1) f |= kTestPrefix;
-          }
-        }
-        if constexpr (DENSE) {
-          if (dmap != nullptr && f) {
-            const int bits = dense_map_or(dmap, a.Lk, q0, q_hi, j * kPairKeys, min((j + 1) * kPairKeys, a.Lk) - 1);
-            if (!(bits & kMapLive)) f = 0;
-            else if (bits & kMapNonZero) f |= kTestDense;
-          }
-        }
-        s_flag[j - j_lo] = (unsigned char)f;
-      }
-      __syncthreads();
-      if (wave == 0) {
-        int cnt = 0;
-        for (int base = 0; base < n; base += 64) {
-          const int i = base + lane;
-          const int f = (i < n) ? s_flag[i] : 0;
-          const unsigned long long mask = __ballot(f != 0);
-          if (f) s_list[cnt + __popcll(mask & ((1ull << lane) - 1ull))] = (unsigned short)((j_lo + i) | ((f & 7) << kTestShift));
-          cnt += __popcll(mask);
-        }
-        if (lane == 0) s_red[16] = cnt;
-      }
-      __syncthreads();
-      n = s_red[16];
-    }
+    use_list = ntiles <= kPairListTiles && ((flags & (RA_BIAS_SEGMENT | RA_BIAS_PREFIX)) || dmap != nullptr);
+    if (use_list)
+      n = list_key_tiles<DENSE>(a.Lq, a.Lk, bs, kv_seg, kv_pre, dmap, q0, q_hi, q_valid, q_seg, q_pre, j_lo, n, s_red, s_flag, s_list);
   }
   n = __builtin_amdgcn_readfirstlane(n);
   j_lo = __builtin_amdgcn_readfirstlane(j_lo);
@@ -202,39 +297,16 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     return j_lo + i;
   };
 
-  // ---- global -> LDS: a wave moves 16 of a tile's 64 rows, 1 KiB per instruction -----------------
-  constexpr int CPR = D / 8;         // 16-byte chunks per row
-  constexpr int RPI = 64 / CPR;      // rows per load instruction
-  constexpr int NLD = 16 / RPI;      // load instructions per wave and tile
-  const bf16_t* kbase = a.k.ptr + b * a.k.sb + h * a.k.sh;
-  const bf16_t* vbase = a.v.ptr + b * a.v.sb + h * a.v.sh;
-  // Complete tiles go through a wave-uniform base and per-lane byte offsets from the wave's first row.
-  unsigned k_voff[NLD], v_voff[NLD];
-#pragma unroll
-  for (int t = 0; t < NLD; ++t) {
-    const int row = lane / CPR + RPI * t;
-    const int lc = (tile_off<D>(row, lane % CPR) - row * ROWB) >> 4;  // logical chunk stored at this lane's place
-    k_voff[t] = (unsigned)(((long long)row * a.k.sl + lc * 8) * 2);
-    v_voff[t] = (unsigned)(((long long)row * a.v.sl + lc * 8) * 2);
-  }
-  auto issue = [&](const bf16_t* base, const unsigned (&voff)[NLD], long long sl, int k0, unsigned dst) {
-    if (k0 + kPairKeys <= a.Lk) {
-      const bf16_t* sb = base + (long long)(k0 + 16 * wave) * sl;
-#pragma unroll
-      for (int t = 0; t < NLD; ++t) global_to_lds16_s(sb, voff[t], dst + (16 * wave + RPI * t) * ROWB);
-    } else {  // last, partial tile: rows past the end repeat the last row (masked later)
-#pragma unroll
-      for (int t = 0; t < NLD; ++t) {
-        const int row = 16 * wave + RPI * t + lane / CPR;
-        const int lc = (tile_off<D>(row, lane % CPR) - row * ROWB) >> 4;
-        global_to_lds16(base + (long long)min(k0 + row, a.Lk - 1) * sl + lc * 8, dst + (16 * wave + RPI * t) * ROWB);
-      }
-    }
-  };
+  TileLoader<D, kPairKeys> ldk, ldv;
+  const unsigned first_chunk = TileLoader<D, kPairKeys>::first_chunk(lane);
+  ldk.init(a.k.ptr + b * a.k.sb + h * a.k.sh, a.k.sl, a.Lk, lane);
+  ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, lane);
   auto issue_tile = [&](int j, int buf) {
     const int k0 = j * kPairKeys;
-    issue(kbase, k_voff, a.k.sl, k0, RA_LDS_ADDR(&s_k[0][0]) + buf * TILE_BYTES);
-    issue(vbase, v_voff, a.v.sl, k0, RA_LDS_ADDR(&s_v[0][0]) + buf * TILE_BYTES);
+    unsigned first = first_chunk;
+    asm volatile("" : "+v"(first));  // the XORs are not to be hoisted out of the loop
+    ldk.issue(k0, RA_LDS_ADDR(&s_k[0][0]) + buf * TILE_BYTES, wave, lane, first);
+    ldv.issue(k0, RA_LDS_ADDR(&s_v[0][0]) + buf * TILE_BYTES, wave, lane, first);
     if constexpr (GENERAL) {
       const int kk = min(k0 + lane, a.Lk - 1);
       if (kv_seg && wave == 0) global_to_lds4(kv_seg + kk, RA_LDS_ADDR(&s_seg[0][0]) + buf * (kPairKeys * 4));
@@ -254,20 +326,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   ones2[0] = (bf16_t)1.0f;
   ones2[1] = (bf16_t)1.0f;
 
-  int koff[KS];
-#pragma unroll
-  for (int ss = 0; ss < KS; ++ss) koff[ss] = tile_off<D>(l32, 2 * ss + g);
-  int voff[DB][2];
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int h2 = 0; h2 < 2; ++h2) {
-      const int j = lane & 15;
-      const int vrow = 4 * g + (j >> 2) + 8 * h2;
-      const int vcol = 32 * db + 16 * ((lane >> 4) & 1) + 4 * (j & 3);
-      voff[db][h2] = tile_off<D>(vrow, vcol >> 3) + ((vcol & 4) << 1);
-    }
-
+  const FragOffsets<D> fo(lane);
   const bool wave_on = qw < a.Lq;
   const bool alibi_on = GENERAL && (flags & RA_BIAS_ALIBI);
   const int qlo_w = q_off + qw, qhi_w = q_off + qw + 31;
@@ -283,6 +342,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
       issue_tile(tile_at(i + 1, t1), BUF ^ 1);
     }
     if (!wave_on) return;
+    const FragOffsets<D> fr_off = fo.opaque();
     const int klo = kv_off + kt0, khi = klo + kPairKeys - 1;
     const int cls = classify_pos(flags, bs.window, qlo_w, qhi_w, klo, khi);
     if (cls & 1) return;
@@ -291,34 +351,16 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
 #pragma unroll
     for (int r = 0; r < 16; ++r) S[0][r] = S[1][r] = 0.f;
     if (alibi_on && (khi <= qlo_w || klo >= qhi_w)) {
-      // one side of the diagonal: -slope |q - k| is linear in both positions and enters through the
-      // matrix unit as the accumulators' initial value, split into bf16 words (see fwd_step_kernel)
       alibi_left = false;
-      const float s = khi <= qlo_w ? slope2 : -slope2;
-      const float c = -s * (float)(q_off + qi - klo);
-      bf16x8 bq;
-      bq[0] = (bf16_t)s;
-      bq[1] = (bf16_t)(s - (float)bq[0]);
-      bq[2] = (bf16_t)c;
-      bq[3] = (bf16_t)(c - (float)bq[2]);
-      bq[4] = (bf16_t)((c - (float)bq[2]) - (float)bq[3]);
-      bq[5] = bq[6] = bq[7] = (bf16_t)0.f;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        bf16x8 rf;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) rf[e] = (bf16_t)0.f;
-        rf[0] = rf[1] = (bf16_t)(g == 0 ? (float)(32 * kb + l32) : 0.f);
-        rf[2] = rf[3] = rf[4] = (bf16_t)(g == 0 ? 1.0f : 0.f);
-        S[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(rf, bq, S[kb], 0, 0, 0);
-      }
+      for (int kb = 0; kb < 2; ++kb) S[kb] = alibi_one_side(S[kb], khi <= qlo_w ? slope2 : -slope2, q_off + qi - klo, kb, l32, g);
     }
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int ss = 0; ss < KS; ++ss)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
-        S[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(s_k[BUF] + 32 * kb * ROWB + koff[ss]), qf[ss], S[kb], 0, 0, 0);
+        S[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(s_k[BUF] + 32 * kb * ROWB + fr_off.nat(ss)), qf[ss], S[kb], 0, 0, 0);
     __builtin_amdgcn_s_setprio(0);
     if ((cls & 2) || kt0 + kPairKeys > a.Lk || (GENERAL && (tests || alibi_left))) {
       TileBias tb;
@@ -390,8 +432,8 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     };
     auto v_frag = [&](int op) {
       const int ks = op / DB, db = op % DB;
-      const lds_char* p0 = (const lds_char*)(s_v[BUF] + 16 * ks * ROWB + voff[db][0]);
-      const lds_char* p1 = (const lds_char*)(s_v[BUF] + 16 * ks * ROWB + voff[db][1]);
+      const lds_char* p0 = (const lds_char*)(s_v[BUF] + 16 * ks * ROWB + fr_off.tr(db, 0));
+      const lds_char* p1 = (const lds_char*)(s_v[BUF] + 16 * ks * ROWB + fr_off.tr(db, 1));
       const bf16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)p0);
       const bf16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)p1);
       return __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -524,6 +566,814 @@ __global__ __launch_bounds__(256) void pair_combine_kernel(const PairFwdArgs a) 
   for (int e = 0; e < 4; ++e) o[e] *= inv;
   store4(a.out, a.out_f32, (hh / a.H) * a.out_sb + (hh % a.H) * a.out_sh + (long long)li * a.out_sl + 4 * c, o);
   if (c == 0) a.lse[row] = (l > 0.f) ? (m + __log2f(l)) * kLn2 : RA_NEG_INF;
+}
+
+// ------------------------------------------------------------------------------------------------
+// dQ
+// ------------------------------------------------------------------------------------------------
+// The same split: 128 query rows per workgroup (Q and dO in registers), 64-key tiles of K and V in two
+// LDS buffers, scores transposed (S^T = K Q^T, dP^T = V dO^T) so that dS^T is the B operand of
+// dQ^T = K^T dS^T, whose A operand comes from the K tile through the transposing read.
+template <int D, int MODE>
+__global__ __launch_bounds__(kPairThreads, 2) void dq_pair_kernel(const PairBwdArgs p) {
+  constexpr bool GENERAL = MODE != 0;
+  constexpr bool DENSE = MODE == 2;
+  constexpr int KS = D / 16, DB = D / 32;
+  constexpr int ROWB = D * 2;
+  constexpr int TILE_BYTES = kPairKeys * ROWB;
+  const BwdArgs& a = p.a;
+  __shared__ __attribute__((aligned(16))) char s_k[2][TILE_BYTES];
+  __shared__ __attribute__((aligned(16))) char s_v[2][TILE_BYTES];
+  __shared__ __attribute__((aligned(16))) int s_seg[GENERAL ? 2 : 1][kPairKeys];
+  __shared__ __attribute__((aligned(16))) int s_pre[GENERAL ? 2 : 1][kPairKeys];
+  __shared__ unsigned short s_list[GENERAL ? kPairListTiles : 1];
+  __shared__ unsigned char s_flag[GENERAL ? kPairListTiles : 1];
+  __shared__ int s_red[20];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, g = lane >> 5;
+  const int nqt = (a.Lq + kPairRows - 1) / kPairRows;
+  int hh, split, qt;
+  pair_decode(blockIdx.x, a.B * a.H, nqt, hh, split, qt);
+  const int b = hh / a.H, h = hh % a.H;
+  const int q0 = qt * kPairRows;
+  const int qw = q0 + wave * 32;
+  const int qi = qw + l32;
+  const bool q_valid = qi < a.Lq;
+  const int qi_c = min(qi, a.Lq - 1);
+  const BiasArgs& bs = a.bias;
+  const int flags = bs.flags;
+  const int q_off = bs.q_off, kv_off = bs.kv_off;
+
+  const int ntiles = (a.Lk + kPairKeys - 1) / kPairKeys;
+  const int q_hi = min(q0 + kPairRows, a.Lq) - 1;
+  int j_lo, j_hi;
+  key_tile_range(flags, bs.window, q_off + q0, q_off + q_hi, kv_off, ntiles, kPairKeys, j_lo, j_hi);
+  int n = j_hi - j_lo;
+  if (split > 0 && split * p.chunk_tiles >= n) return;
+
+  // Q carries the power of two below sm_scale * log2(e) (exact in bf16), the residual factor is
+  // applied to the fp32 score (see dkdv_kernel)
+  bf16x8 qf[KS], dof[KS];
+  {
+    const bf16_t* qp = a.q.ptr + b * a.q.sb + h * a.q.sh + (long long)qi_c * a.q.sl + 8 * g;
+    const bf16_t* dp = a.dout.ptr + b * a.dout.sb + h * a.dout.sh + (long long)qi_c * a.dout.sl + 8 * g;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const bf16x8 qr = *(const bf16x8*)(qp + 16 * s);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qf[s][e] = (bf16_t)((float)qr[e] * a.scale_p2);
+      dof[s] = *(const bf16x8*)(dp + 16 * s);
+    }
+  }
+  const long long row = (long long)hh * a.Lq + qi_c;
+  const float Lraw = a.lse[row];
+  const float neg_lse2 = (Lraw == RA_NEG_INF) ? RA_NEG_INF : -Lraw * kLog2e;  // fully masked row: P = 0
+  const float neg_delta = -a.delta[row];
+  int q_seg = 0, q_pre = 0;
+  float slope2 = 0.f;
+  const int* kv_seg = nullptr;
+  const int* kv_pre = nullptr;
+  if constexpr (GENERAL) {
+    if (flags & RA_BIAS_SEGMENT) {
+      q_seg = bs.q_seg[b * bs.q_seg_sb + qi_c];
+      kv_seg = bs.kv_seg + b * bs.kv_seg_sb;
+    }
+    if (flags & RA_BIAS_PREFIX) {
+      q_pre = bs.q_pre[b * bs.q_pre_sb + qi_c];
+      kv_pre = bs.kv_pre + b * bs.kv_pre_sb;
+    }
+    if (flags & RA_BIAS_ALIBI) slope2 = bs.slopes[h] * kLog2e / a.scale_res;
+  }
+  bool use_list = false;
+  const unsigned char* dmap = nullptr;
+  if constexpr (DENSE) {
+    if (bs.dense_map) dmap = dense_map_of(bs, b, h, a.H, a.Lq, a.Lk);
+  }
+  if constexpr (GENERAL) {
+    use_list = ntiles <= kPairListTiles && ((flags & (RA_BIAS_SEGMENT | RA_BIAS_PREFIX)) || dmap != nullptr);
+    if (use_list)
+      n = list_key_tiles<DENSE>(a.Lq, a.Lk, bs, kv_seg, kv_pre, dmap, q0, q_hi, q_valid, q_seg, q_pre, j_lo, n, s_red, s_flag, s_list);
+  }
+  n = __builtin_amdgcn_readfirstlane(n);
+  j_lo = __builtin_amdgcn_readfirstlane(j_lo);
+  const int n_piece = max(1, min(p.n_split, (n + p.chunk_tiles - 1) / p.chunk_tiles));
+  if (split >= n_piece) return;
+  const int i_lo = n * split / n_piece, i_hi = n * (split + 1) / n_piece;
+  int every_test = 0;
+  if constexpr (GENERAL) {
+    if (!use_list && (flags & RA_BIAS_PREFIX)) every_test |= kTestPrefix;
+    if ((flags & RA_BIAS_DENSE) && dmap == nullptr) every_test |= kTestDense;
+  }
+  auto tile_at = [&](int i, int& tests) -> int {
+    if (GENERAL && use_list) {
+      const int e = __builtin_amdgcn_readfirstlane((int)s_list[i]);
+      tests = (e >> kTestShift) | every_test;
+      return e & ((1 << kTestShift) - 1);
+    }
+    tests = every_test;
+    return j_lo + i;
+  };
+  TileLoader<D, kPairKeys> ldk, ldv;
+  const unsigned first_chunk = TileLoader<D, kPairKeys>::first_chunk(lane);
+  ldk.init(a.k.ptr + b * a.k.sb + h * a.k.sh, a.k.sl, a.Lk, lane);
+  ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, lane);
+  auto issue_tile = [&](int j, int buf) {
+    const int k0 = j * kPairKeys;
+    unsigned first = first_chunk;
+    asm volatile("" : "+v"(first));  // the XORs are not to be hoisted out of the loop
+    ldk.issue(k0, RA_LDS_ADDR(&s_k[0][0]) + buf * TILE_BYTES, wave, lane, first);
+    ldv.issue(k0, RA_LDS_ADDR(&s_v[0][0]) + buf * TILE_BYTES, wave, lane, first);
+    if constexpr (GENERAL) {
+      const int kk = min(k0 + lane, a.Lk - 1);
+      if (kv_seg && wave == 0) global_to_lds4(kv_seg + kk, RA_LDS_ADDR(&s_seg[0][0]) + buf * (kPairKeys * 4));
+      if (kv_pre && wave == 1) global_to_lds4(kv_pre + kk, RA_LDS_ADDR(&s_pre[0][0]) + buf * (kPairKeys * 4));
+    }
+  };
+
+  f32x16 acc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
+  const FragOffsets<D> fo(lane);
+  const bool wave_on = qw < a.Lq;
+  const bool alibi_on = GENERAL && (flags & RA_BIAS_ALIBI);
+  const int qlo_w = q_off + qw, qhi_w = q_off + qw + 31;
+
+  auto step = [&](auto buffer, int i) {
+    constexpr int BUF = decltype(buffer)::value;
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // this wave's share of tile i is in LDS
+    __syncthreads();                     // everyone's is, and nobody reads the other buffer any more
+    int tests;
+    const int kt0 = tile_at(i, tests) * kPairKeys;
+    if (i + 1 < i_hi) {
+      int t1;
+      issue_tile(tile_at(i + 1, t1), BUF ^ 1);
+    }
+    if (!wave_on) return;
+    const FragOffsets<D> fr_off = fo.opaque();
+    const int klo = kv_off + kt0, khi = klo + kPairKeys - 1;
+    const int cls = classify_pos(flags, bs.window, qlo_w, qhi_w, klo, khi);
+    if (cls & 1) return;
+    const bool one_side = alibi_on && (khi <= qlo_w || klo >= qhi_w);
+    const bool biased = (cls & 2) || kt0 + kPairKeys > a.Lk || (GENERAL && (tests || (alibi_on && !one_side)));
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      // S^T first, then dP^T with the exp2 of S in its shadow: dP^T takes no registers while the terms
+      // of a biased tile are evaluated
+      constexpr int PF = 3;  // operand fetches in flight ahead of the matrix instruction that uses them
+      f32x16 S;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) S[r] = 0.f;
+      if (one_side) S = alibi_one_side(S, khi <= qlo_w ? slope2 : -slope2, q_off + qi - klo, kb, l32, g);
+      auto nat_frag = [&](const char* tile, int ss) { return *(const bf16x8*)(tile + 32 * kb * ROWB + fr_off.nat(ss)); };
+      __builtin_amdgcn_s_setprio(1);
+      {
+        bf16x8 fr[KS];
+#pragma unroll
+        for (int op = 0; op < PF; ++op) fr[op] = nat_frag(s_k[BUF], op);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int op = 0; op < KS; ++op) {
+          if (op + PF < KS) fr[op + PF] = nat_frag(s_k[BUF], op + PF);
+          S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], qf[op], S, 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      __builtin_amdgcn_s_setprio(0);
+      if (biased) {
+        TileBias tb;
+        tb.flags = (cls & 2) ? (flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) : 0;
+        if constexpr (GENERAL) {
+          if (tests & kTestSegment) tb.flags |= RA_BIAS_SEGMENT;
+          if (tests & kTestPrefix) tb.flags |= RA_BIAS_PREFIX;
+          if (tests & kTestDense) tb.flags |= RA_BIAS_DENSE;
+          if (alibi_on && !one_side) tb.flags |= RA_BIAS_ALIBI;
+        }
+        tb.window = bs.window;
+        tb.slope2 = slope2;
+        tb.dense_mul = kLog2e / a.scale_res;
+        tb.dense = nullptr;
+        tb.dense_vs = 1;
+        tb.dense_vec = 0;
+        const int var0 = kt0 + 32 * kb + 4 * g;
+        tb.var_limit = a.Lk - var0;
+        if (DENSE) {
+          const float* head = bs.dense + b * bs.dense_sb + h * bs.dense_sh;
+          tb.dense_vec = kt0 + kPairKeys <= a.Lk && ((((uintptr_t)head) | ((uintptr_t)bs.dense_sq << 2)) & 15) == 0;
+          tb.dense = head + (long long)qi_c * bs.dense_sq + var0;
+        }
+        apply_bias<true, DENSE, GENERAL>(S, tb, (q_off + qi) - (kv_off + var0), q_seg, q_pre,
+                                         &s_seg[GENERAL ? BUF : 0][32 * kb + 4 * g], &s_pre[GENERAL ? BUF : 0][32 * kb + 4 * g]);
+      }
+      f32x16 P;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) P[r] = neg_delta;
+      {
+        bf16x8 fr[KS];
+#pragma unroll
+        for (int op = 0; op < PF; ++op) fr[op] = nat_frag(s_v[BUF], op);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int op = 0; op < KS; ++op) {
+          if (op + PF < KS) fr[op + PF] = nat_frag(s_v[BUF], op + PF);
+          P = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], dof[op], P, 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 16 / KS; ++e) {
+            float x = fast_exp2(fmaf(S[op * (16 / KS) + e], a.scale_res, neg_lse2));
+            asm volatile("" : "+v"(x));
+            S[op * (16 / KS) + e] = x;
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      // dS in two groups of eight keys per lane: the second one is worked on while the matrix unit
+      // multiplies with the first
+      bf16x8 dsf[2];
+      auto grad = [&](int ks, int e) {  // elements e, e + 1 of group ks
+        bf16x2 pr;
+        pr[0] = (bf16_t)(S[8 * ks + e] * P[8 * ks + e]);
+        pr[1] = (bf16_t)(S[8 * ks + e + 1] * P[8 * ks + e + 1]);
+        unsigned pw = __builtin_bit_cast(unsigned, pr);
+        asm volatile("" : "+v"(pw));
+        pr = __builtin_bit_cast(bf16x2, pw);
+        dsf[ks][e] = pr[0];
+        dsf[ks][e + 1] = pr[1];
+      };
+      auto k_frag = [&](int op) {
+        const int ks = op / DB, db = op % DB;
+        const lds_char* p0 = (const lds_char*)(s_k[BUF] + (32 * kb + 16 * ks) * ROWB + fr_off.tr(db, 0));
+        const lds_char* p1 = (const lds_char*)(s_k[BUF] + (32 * kb + 16 * ks) * ROWB + fr_off.tr(db, 1));
+        const bf16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)p0);
+        const bf16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)p1);
+        return __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
+      };
+      bf16x8 fr[2 * DB];
+#pragma unroll
+      for (int op = 0; op < PF; ++op) fr[op] = k_frag(op);
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) grad(0, e);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int op = 0; op < 2 * DB; ++op) {
+        const int ks = op / DB, db = op % DB;
+        if (op + PF < 2 * DB) fr[op + PF] = k_frag(op + PF);
+        acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], dsf[ks], acc[db], 0, 0, 0);
+        if (ks < 1) {
+#pragma unroll
+          for (int e = 0; e < 8 / DB; e += 2) grad(1, db * (8 / DB) + e);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
+  if (i_lo < i_hi) {
+    int t0;
+    issue_tile(tile_at(i_lo, t0), 0);
+    for (int i = i_lo; i < i_hi; i += 2) {
+      step(std::integral_constant<int, 0>{}, i);
+      if (i + 1 < i_hi) step(std::integral_constant<int, 1>{}, i + 1);
+    }
+  }
+
+  if (p.part_n != nullptr && split == 0 && tid == 0) p.part_n[hh * nqt + qt] = n_piece;
+  if (!q_valid) return;
+  float* fp = nullptr;  // fp32 destination: a share of the sum, or an accumulator
+  if (n_piece > 1) fp = p.part + ((long long)split * ((long long)a.B * a.H * a.Lq) + row) * D;
+  else if (p.acc != nullptr) fp = p.acc + row * D;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int bb = 0; bb < 4; ++bb) {
+      const int d0 = 32 * db + 8 * bb + 4 * g;
+      f32x4 t;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) t[c] = acc[db][4 * bb + c] * a.sm_scale;
+      if (fp != nullptr) {
+        if (n_piece == 1) t += *(const f32x4*)(fp + d0);
+        *(f32x4*)(fp + d0) = t;
+      } else {
+        store4(p.out, 0, b * p.out_sb + h * p.out_sh + (long long)qi * p.out_sl + d0, t);
+      }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+// dK / dV
+// ------------------------------------------------------------------------------------------------
+constexpr int kPairSlab = 128;      // keys per workgroup: 4 waves x 32
+constexpr int kPairQueries = 32;    // queries per LDS tile
+constexpr int kPairQListTiles = 2048;
+
+// The query-side twin of list_key_tiles: the 32-query tiles that the workgroup's keys [k0, k_hi] meet.
+template <bool DENSE>
+RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg, const int* q_pre, const unsigned char* dmap,
+                            int k0, int k_hi, bool k_valid, int k_seg, int k_pre, int j_lo, int n, int* s_red,
+                            unsigned char* s_flag, unsigned short* s_list) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool seg_on = q_seg != nullptr, pre_on = q_pre != nullptr;
+  const int smin = wave_min(k_valid ? k_seg : 0x7fffffff), smax = wave_max(k_valid ? k_seg : (int)0x80000000);
+  const int any = __any(k_valid && k_pre != 0), all = __all(!k_valid || k_pre != 0);
+  if (lane == 0) {
+    s_red[wave] = smin;
+    s_red[4 + wave] = smax;
+    s_red[8 + wave] = any;
+    s_red[12 + wave] = all;
+  }
+  __syncthreads();
+  const int kmin = min(min(s_red[0], s_red[1]), min(s_red[2], s_red[3]));
+  const int kmax = max(max(s_red[4], s_red[5]), max(s_red[6], s_red[7]));
+  const bool k_any = s_red[8] | s_red[9] | s_red[10] | s_red[11], k_all = s_red[12] & s_red[13] & s_red[14] & s_red[15];
+  for (int i = tid; i < n; i += kPairThreads) {
+    const int j = j_lo + i;
+    const int q_last = min((j + 1) * kPairQueries, Lq) - 1;
+    int f = 0x80;  // listed
+    if (seg_on) {
+      int qmin, qmax;
+      tile_id_range<kPairQueries>(q_seg, j, Lq, qmin, qmax);
+      if (qmax < kmin || qmin > kmax) f = 0;
+      else if (qmin != qmax || kmin != kmax) f |= kTestSegment;
+    }
+    if (pre_on && f) {
+      const int qlo = bs.q_off + j * kPairQueries, qhi = bs.q_off + q_last;
+      if (bs.kv_off + k_hi > qlo) {
+        bool q_any, q_all;
+        tile_flag_range<kPairQueries>(q_pre, j, Lq, q_any, q_all);
+        const int c = prefix_class(qlo, qhi, bs.kv_off + k0, bs.kv_off + k_hi, q_any, q_all, k_any, k_all);
+        if (c == 2) f = 0;
+        else if (c == 1) f |= kTestPrefix;
+      }
+    }
+    if constexpr (DENSE) {
+      if (dmap != nullptr && f) {
+        const int bits = dense_map_or(dmap, Lk, j * kPairQueries, q_last, k0, k_hi);
+        if (!(bits & kMapLive)) f = 0;
+        else if (bits & kMapNonZero) f |= kTestDense;
+      }
+    }
+    s_flag[i] = (unsigned char)f;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int cnt = 0;
+    for (int base = 0; base < n; base += 64) {
+      const int i = base + lane;
+      const int f = (i < n) ? s_flag[i] : 0;
+      const unsigned long long mask = __ballot(f != 0);
+      if (f) s_list[cnt + __popcll(mask & ((1ull << lane) - 1ull))] = (unsigned short)((j_lo + i) | ((f & 7) << kTestShift));
+      cnt += __popcll(mask);
+    }
+    if (lane == 0) s_red[16] = cnt;
+  }
+  __syncthreads();
+  return s_red[16];
+}
+
+// 128 keys per workgroup, 32 per wave, two workgroups per compute unit: K operands and the dK / dV
+// accumulators in registers; V, which a second wave per SIMD leaves no registers for at D = 128, in
+// LDS; 32-query tiles of Q and dO in two LDS buffers.  S = Q K^T: a lane owns one key and 16 queries, so
+// that P and dS are the A operands of dV = P^T dO and dK = dS^T Q.  The rows' statistics (stat:
+// -lse log2(e) / scale_res, then -delta, from pair_stat_kernel) are the accumulators' initial values.
+template <int D, int MODE>
+__global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kernel(const PairBwdArgs p) {
+  constexpr bool GENERAL = MODE != 0;
+  constexpr bool DENSE = MODE == 2;
+  constexpr bool VLDS = D == 128;
+  constexpr int KS = D / 16, DB = D / 32;
+  constexpr int ROWB = D * 2;
+  constexpr int TILE_BYTES = kPairQueries * ROWB;
+  const BwdArgs& a = p.a;
+  __shared__ __attribute__((aligned(16))) char s_q[2][TILE_BYTES];
+  __shared__ __attribute__((aligned(16))) char s_do[2][TILE_BYTES];
+  __shared__ __attribute__((aligned(16))) char s_v[VLDS ? kPairSlab * ROWB : 16];
+  __shared__ __attribute__((aligned(16))) float s_stat[2][2][kPairQueries];
+  __shared__ __attribute__((aligned(16))) int s_seg[GENERAL ? 2 : 1][64];  // (a 64-lane load writes 64 words)
+  __shared__ __attribute__((aligned(16))) int s_pre[GENERAL ? 2 : 1][64];
+  __shared__ unsigned short s_list[GENERAL ? kPairQListTiles : 1];
+  __shared__ unsigned char s_flag[GENERAL ? kPairQListTiles : 1];
+  __shared__ int s_red[20];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, g = lane >> 5;
+  const int nkt = (a.Lk + kPairSlab - 1) / kPairSlab;
+  int hh, split, kt;
+  pair_decode(blockIdx.x, a.B * a.H, nkt, hh, split, kt);
+  kt = nkt - 1 - kt;  // under a causal mask the first keys have the most work
+  const int b = hh / a.H, h = hh % a.H;
+  const int k0 = kt * kPairSlab;
+  const int kw = k0 + wave * 32;
+  const int ki = kw + l32;
+  const bool k_valid = ki < a.Lk;
+  const int ki_c = min(ki, a.Lk - 1);
+  const BiasArgs& bs = a.bias;
+  const int flags = bs.flags;
+  const int q_off = bs.q_off, kv_off = bs.kv_off;
+
+  const int ntiles = (a.Lq + kPairQueries - 1) / kPairQueries;
+  const int k_hi = min(k0 + kPairSlab, a.Lk) - 1;
+  int j_lo, j_hi;
+  query_tile_range(flags, bs.window, kv_off + k0, kv_off + k_hi, q_off, ntiles, kPairQueries, j_lo, j_hi);
+  int n = j_hi - j_lo;
+  if (split > 0 && split * p.chunk_tiles >= n) return;
+
+  bf16x8 kf[KS], vf[VLDS ? 1 : KS];
+  {
+    const bf16_t* kp = a.k.ptr + b * a.k.sb + h * a.k.sh + (long long)ki_c * a.k.sl + 8 * g;
+    const bf16_t* vp = a.v.ptr + b * a.v.sb + h * a.v.sh + (long long)ki_c * a.v.sl + 8 * g;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const bf16x8 kr = *(const bf16x8*)(kp + 16 * s);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) kf[s][e] = (bf16_t)((float)kr[e] * a.scale_p2);
+      if constexpr (!VLDS) vf[s] = *(const bf16x8*)(vp + 16 * s);
+    }
+  }
+  int k_seg = 0, k_pre = 0;
+  float slope2 = 0.f;
+  const int* q_seg = nullptr;
+  const int* q_pre = nullptr;
+  if constexpr (GENERAL) {
+    if (flags & RA_BIAS_SEGMENT) {
+      k_seg = bs.kv_seg[b * bs.kv_seg_sb + ki_c];
+      q_seg = bs.q_seg + b * bs.q_seg_sb;
+    }
+    if (flags & RA_BIAS_PREFIX) {
+      k_pre = bs.kv_pre[b * bs.kv_pre_sb + ki_c];
+      q_pre = bs.q_pre + b * bs.q_pre_sb;
+    }
+    if (flags & RA_BIAS_ALIBI) slope2 = bs.slopes[h] * kLog2e / a.scale_res;
+  }
+  bool use_list = false;
+  const unsigned char* dmap = nullptr;
+  if constexpr (DENSE) {
+    if (bs.dense_map) dmap = dense_map_of(bs, b, h, a.H, a.Lq, a.Lk);
+  }
+  if constexpr (GENERAL) {
+    use_list = ntiles <= kPairQListTiles && ((flags & (RA_BIAS_SEGMENT | RA_BIAS_PREFIX)) || dmap != nullptr);
+    if (use_list)
+      n = list_query_tiles<DENSE>(a.Lq, a.Lk, bs, q_seg, q_pre, dmap, k0, k_hi, k_valid, k_seg, k_pre, j_lo, n, s_red, s_flag, s_list);
+  }
+  n = __builtin_amdgcn_readfirstlane(n);
+  j_lo = __builtin_amdgcn_readfirstlane(j_lo);
+  const int n_piece = max(1, min(p.n_split, (n + p.chunk_tiles - 1) / p.chunk_tiles));
+  if (split >= n_piece) return;
+  const int i_lo = n * split / n_piece, i_hi = n * (split + 1) / n_piece;
+  int every_test = 0;
+  if constexpr (GENERAL) {
+    if (!use_list && (flags & RA_BIAS_PREFIX)) every_test |= kTestPrefix;
+    if ((flags & RA_BIAS_DENSE) && dmap == nullptr) every_test |= kTestDense;
+  }
+  auto tile_at = [&](int i, int& tests) -> int {
+    if (GENERAL && use_list) {
+      const int e = __builtin_amdgcn_readfirstlane((int)s_list[i]);
+      tests = (e >> kTestShift) | every_test;
+      return e & ((1 << kTestShift) - 1);
+    }
+    tests = every_test;
+    return j_lo + i;
+  };
+  TileLoader<D, kPairQueries> ldq, ldo;
+  const unsigned first_chunk = TileLoader<D, kPairQueries>::first_chunk(lane);
+  ldq.init(a.q.ptr + b * a.q.sb + h * a.q.sh, a.q.sl, a.Lq, lane);
+  ldo.init(a.dout.ptr + b * a.dout.sb + h * a.dout.sh, a.dout.sl, a.Lq, lane);
+  // lanes 0..31 move -lse of a tile's rows, lanes 32..63 -delta
+  const float* stat = p.stat + (long long)hh * a.Lq + (g ? (long long)a.B * a.H * a.Lq : 0);
+  auto issue_tile = [&](int j, int buf) {
+    const int r0 = j * kPairQueries;
+    unsigned first = first_chunk;
+    asm volatile("" : "+v"(first));  // the XORs are not to be hoisted out of the loop
+    ldq.issue(r0, RA_LDS_ADDR(&s_q[0][0]) + buf * TILE_BYTES, wave, lane, first);
+    ldo.issue(r0, RA_LDS_ADDR(&s_do[0][0]) + buf * TILE_BYTES, wave, lane, first);
+    const int rr = min(r0 + l32, a.Lq - 1);
+    if (wave == 0) global_to_lds4(stat + rr, RA_LDS_ADDR(&s_stat[0][0][0]) + buf * (2 * kPairQueries * 4));
+    if constexpr (GENERAL) {
+      if (q_seg && wave == 1) global_to_lds4(q_seg + rr, RA_LDS_ADDR(&s_seg[0][0]) + buf * 256);
+      if (q_pre && wave == 2) global_to_lds4(q_pre + rr, RA_LDS_ADDR(&s_pre[0][0]) + buf * 256);
+    }
+  };
+
+  f32x16 dk[DB], dv[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dk[db][r] = dv[db][r] = 0.f;
+  const FragOffsets<D> fo(lane);
+  const bool wave_on = kw < a.Lk;
+  const bool alibi_on = GENERAL && (flags & RA_BIAS_ALIBI);
+  const int klo_w = kv_off + kw, khi_w = kv_off + kw + 31;
+
+  auto step = [&](auto buffer, int i) {
+    constexpr int BUF = decltype(buffer)::value;
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // this wave's share of tile i is in LDS
+    __syncthreads();                     // everyone's is, and nobody reads the other buffer any more
+    int tests;
+    const int qt0 = tile_at(i, tests) * kPairQueries;
+    if (i + 1 < i_hi) {
+      int t1;
+      issue_tile(tile_at(i + 1, t1), BUF ^ 1);
+    }
+    if (!wave_on) return;
+    const FragOffsets<D> fr_off = fo.opaque();
+    const int qlo = q_off + qt0, qhi = qlo + kPairQueries - 1;
+    const int cls = classify_pos(flags, bs.window, qlo, qhi, klo_w, khi_w);
+    if (cls & 1) return;
+    const bool one_side = alibi_on && (qlo >= khi_w || qhi <= klo_w);
+    constexpr int PF = 3;  // operand fetches in flight ahead of the matrix instruction that uses them
+    f32x16 S;
+#pragma unroll
+    for (int bb = 0; bb < 4; ++bb) {
+      const f32x4 t = *(const f32x4*)&s_stat[BUF][0][8 * bb + 4 * g];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) S[4 * bb + c] = t[c];
+    }
+    if (one_side) S = alibi_one_side(S, qlo >= khi_w ? -slope2 : slope2, (kv_off + ki) - qlo, 0, l32, g);
+    auto nat_frag = [&](const char* tile, int ss) { return *(const bf16x8*)(tile + fr_off.nat(ss)); };
+    __builtin_amdgcn_s_setprio(1);
+    {
+      bf16x8 fr[KS];
+#pragma unroll
+      for (int op = 0; op < PF; ++op) fr[op] = nat_frag(s_q[BUF], op);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int op = 0; op < KS; ++op) {
+        if (op + PF < KS) fr[op + PF] = nat_frag(s_q[BUF], op + PF);
+        S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], kf[op], S, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __builtin_amdgcn_s_setprio(0);
+    if ((cls & 2) || qt0 + kPairQueries > a.Lq || (GENERAL && (tests || (alibi_on && !one_side)))) {
+      TileBias tb;
+      tb.flags = (cls & 2) ? (flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) : 0;
+      if constexpr (GENERAL) {
+        if (tests & kTestSegment) tb.flags |= RA_BIAS_SEGMENT;
+        if (tests & kTestPrefix) tb.flags |= RA_BIAS_PREFIX;
+        if (tests & kTestDense) tb.flags |= RA_BIAS_DENSE;
+        if (alibi_on && !one_side) tb.flags |= RA_BIAS_ALIBI;
+      }
+      tb.window = bs.window;
+      tb.slope2 = slope2;
+      tb.dense_mul = kLog2e / a.scale_res;
+      tb.dense = nullptr;
+      tb.dense_vs = 1;
+      tb.dense_vec = 0;
+      tb.var_limit = a.Lq - (qt0 + 4 * g);
+      if (DENSE) {
+        tb.dense = bs.dense + b * bs.dense_sb + h * bs.dense_sh + (long long)(qt0 + 4 * g) * bs.dense_sq + ki_c;
+        tb.dense_vs = bs.dense_sq;
+      }
+      apply_bias<false, DENSE, GENERAL>(S, tb, (qlo + 4 * g) - (kv_off + ki), k_seg, k_pre, &s_seg[GENERAL ? BUF : 0][4 * g],
+                                        &s_pre[GENERAL ? BUF : 0][4 * g]);
+    }
+    // dP with exp2(S) in its shadow
+    bf16x8 pf[2], dsf[2];
+    f32x16 P;
+#pragma unroll
+    for (int bb = 0; bb < 4; ++bb) {
+      const f32x4 t = *(const f32x4*)&s_stat[BUF][1][8 * bb + 4 * g];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) P[4 * bb + c] = t[c];
+    }
+    {
+      bf16x8 fr[KS], vr[KS];
+      auto v_op = [&](int op) {
+        if constexpr (VLDS) return *(const bf16x8*)(s_v + 32 * wave * ROWB + fr_off.nat(op));
+        else return vf[op];
+      };
+      constexpr int PFV = 2;
+#pragma unroll
+      for (int op = 0; op < PFV; ++op) {
+        fr[op] = nat_frag(s_do[BUF], op);
+        vr[op] = v_op(op);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int op = 0; op < KS; ++op) {
+        if (op + PFV < KS) {
+          fr[op + PFV] = nat_frag(s_do[BUF], op + PFV);
+          vr[op + PFV] = v_op(op + PFV);
+        }
+        P = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], vr[op], P, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 16 / KS; e += 2) {
+          const int r = op * (16 / KS) + e;
+          float x0 = fast_exp2(S[r] * a.scale_res), x1 = fast_exp2(S[r + 1] * a.scale_res);
+          bf16x2 pr;
+          pr[0] = (bf16_t)x0;
+          pr[1] = (bf16_t)x1;
+          unsigned pw = __builtin_bit_cast(unsigned, pr);
+          asm volatile("" : "+v"(x0), "+v"(x1), "+v"(pw));
+          pr = __builtin_bit_cast(bf16x2, pw);
+          S[r] = x0;
+          S[r + 1] = x1;
+          pf[r >> 3][r & 7] = pr[0];
+          pf[r >> 3][(r & 7) + 1] = pr[1];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    auto tr_frag = [&](const char* tile, int op) {
+      const int ks = op / DB, db = op % DB;
+      const lds_char* p0 = (const lds_char*)(tile + 16 * ks * ROWB + fr_off.tr(db, 0));
+      const lds_char* p1 = (const lds_char*)(tile + 16 * ks * ROWB + fr_off.tr(db, 1));
+      const bf16x4 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)p0);
+      const bf16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)p1);
+      return __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    // dV with dS = P (dP - delta) in its shadow, then dK
+    {
+      constexpr int NOP = 4 * DB;  // the dV products, then the dK products
+      bf16x8 fr[NOP];
+      auto t_op = [&](int op) { return tr_frag(op < 2 * DB ? s_do[BUF] : s_q[BUF], op % (2 * DB)); };
+#pragma unroll
+      for (int op = 0; op < PF; ++op) fr[op] = t_op(op);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int op = 0; op < NOP; ++op) {
+        if (op + PF < NOP) fr[op + PF] = t_op(op + PF);
+        const int o = op % (2 * DB), ks = o / DB, db = o % DB;
+        if (op < 2 * DB) {
+          dv[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pf[ks], fr[op], dv[db], 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 16 / (2 * DB); e += 2) {
+            const int r = op * (16 / (2 * DB)) + e;
+            bf16x2 pr;
+            pr[0] = (bf16_t)(S[r] * P[r]);
+            pr[1] = (bf16_t)(S[r + 1] * P[r + 1]);
+            unsigned pw = __builtin_bit_cast(unsigned, pr);
+            asm volatile("" : "+v"(pw));
+            pr = __builtin_bit_cast(bf16x2, pw);
+            dsf[r >> 3][r & 7] = pr[0];
+            dsf[r >> 3][(r & 7) + 1] = pr[1];
+          }
+        } else {
+          dk[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dsf[ks], fr[op], dk[db], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
+  if (i_lo < i_hi) {
+    if constexpr (VLDS) {
+      TileLoader<D, kPairSlab> ldv;
+      ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, lane);
+      ldv.issue(k0, RA_LDS_ADDR(&s_v[0]), wave, lane, TileLoader<D, kPairSlab>::first_chunk(lane));
+    }
+    int t0;
+    issue_tile(tile_at(i_lo, t0), 0);
+    for (int i = i_lo; i < i_hi; i += 2) {
+      step(std::integral_constant<int, 0>{}, i);
+      if (i + 1 < i_hi) step(std::integral_constant<int, 1>{}, i + 1);
+    }
+  }
+
+  if (p.part_n != nullptr && split == 0 && tid == 0) p.part_n[hh * nkt + kt] = n_piece;
+  // lane l32 holds column 32 db + l32 of rows kw + 4 g + 8 (r / 4) + r % 4
+  const long long rows = (long long)a.B * a.H * a.Lk;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int key = kw + 4 * g + 8 * (r / 4) + (r % 4);
+    if (key >= a.Lk) continue;
+    if (n_piece > 1) {
+      float* fp = p.part + ((long long)split * 2 * rows + (long long)hh * a.Lk + key) * D + l32;
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        fp[32 * db] = dk[db][r] * a.sm_scale;
+        fp[rows * D + 32 * db] = dv[db][r];
+      }
+    } else if (p.acc != nullptr) {
+      float* fk = p.acc + ((long long)hh * a.Lk + key) * D + l32;
+      float* fv = p.acc2 + ((long long)hh * a.Lk + key) * D + l32;
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        fk[32 * db] += dk[db][r] * a.sm_scale;
+        fv[32 * db] += dv[db][r];
+      }
+    } else {
+      const long long at = b * p.out_sb + h * p.out_sh + (long long)key * p.out_sl + l32;
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        ((bf16_t*)p.out)[at + 32 * db] = (bf16_t)(dk[db][r] * a.sm_scale);
+        ((bf16_t*)p.out2)[at + 32 * db] = (bf16_t)dv[db][r];
+      }
+    }
+  }
+}
+
+// What the dK / dV kernel adds to a row's scores: stat[row] = -lse log2(e) / scale_res (-inf for a row without
+// any key: P = 0) and stat[rows + row] = -delta (0 there: its output, and delta with it, is NaN), with
+// delta = rowsum(out * dout).  HBM bound.
+template <typename OutT, int D>
+__global__ __launch_bounds__(256) void pair_stat_kernel(const OutT* out, long long sb, long long sh, long long sl, TensorArg dout,
+                                                        const float* lse, float inv_res, float* stat, float* delta, int B, int H,
+                                                        int Lq) {
+  constexpr int CPR = D / 8;
+  const long long rows = (long long)B * H * Lq;
+  const long long row = (long long)blockIdx.x * (256 / CPR) + threadIdx.x / CPR;
+  const int c = threadIdx.x % CPR;
+  float acc = 0.f;
+  if (row < rows) {
+    const int li = (int)(row % Lq);
+    const long long hh = row / Lq;
+    const int h = (int)(hh % H);
+    const int b = (int)(hh / H);
+    const OutT* op = out + b * sb + h * sh + (long long)li * sl + 8 * c;
+    const bf16_t* dp = dout.ptr + b * dout.sb + h * dout.sh + (long long)li * dout.sl + 8 * c;
+    const bf16x8 dv = *(const bf16x8*)dp;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc += (float)op[e] * (float)dv[e];
+  }
+#pragma unroll
+  for (int o = CPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+  if (row < rows && c == 0) {
+    const float L = lse[row];
+    const bool dead = L == RA_NEG_INF;
+    delta[row] = acc;
+    stat[row] = dead ? RA_NEG_INF : -L * kLog2e * inv_res;
+    stat[rows + row] = dead ? 0.f : -acc;
+  }
+}
+
+// Sum of the shares of rows that were split, added to an accumulator or stored as bf16.
+// `n_out` results of the same rows (dK and dV) lie one after another in a share; grid dimension y.
+template <int D, int ROWS>
+__global__ __launch_bounds__(256) void pair_sum_kernel(const PairBwdArgs p, int n_out, int BH, int H, int L) {
+  constexpr int CPR = D / 4;
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long rows = (long long)BH * L, row = i / CPR;
+  if (row >= rows) return;
+  const int c = (int)(i % CPR), li = (int)(row % L), which = blockIdx.y;
+  const long long hh = row / L;
+  const int n_piece = p.part_n[hh * ((L + ROWS - 1) / ROWS) + li / ROWS];
+  if (n_piece <= 1) return;  // written by its only workgroup
+  f32x4 x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = 0; s < n_piece; ++s) x += *(const f32x4*)(p.part + (((long long)s * n_out + which) * rows + row) * D + 4 * c);
+  float* acc = which ? p.acc2 : p.acc;
+  if (acc != nullptr) *(f32x4*)(acc + row * D + 4 * c) += x;
+  else store4(which ? p.out2 : p.out, 0, (hh / H) * p.out_sb + (hh % H) * p.out_sh + (long long)li * p.out_sl + 4 * c, x);
+}
+
+template <int D, int ROWS>
+static hipError_t launch_pair_sum(const PairBwdArgs& p, int n_out, int L, hipStream_t stream) {
+  const long long n = (long long)p.a.B * p.a.H * L * (D / 4);
+  hipLaunchKernelGGL((pair_sum_kernel<D, ROWS>), dim3((unsigned)((n + 255) / 256), (unsigned)n_out), dim3(256), 0, stream, p, n_out,
+                     p.a.B * p.a.H, p.a.H, L);
+  return hipGetLastError();
+}
+
+template <int D>
+static hipError_t launch_dq_pair_d(const PairBwdArgs& p, int mode, hipStream_t stream) {
+  const BwdArgs& a = p.a;
+  const int nqt = (a.Lq + kPairRows - 1) / kPairRows;
+  dim3 grid((unsigned)(a.B * a.H * p.n_split * nqt)), block(kPairThreads);
+  if (mode == 2) hipLaunchKernelGGL((dq_pair_kernel<D, 2>), grid, block, 0, stream, p);
+  else if (mode == 1) hipLaunchKernelGGL((dq_pair_kernel<D, 1>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((dq_pair_kernel<D, 0>), grid, block, 0, stream, p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || p.n_split == 1) return e;
+  return launch_pair_sum<D, kPairRows>(p, 1, a.Lq, stream);
+}
+
+template <int D>
+static hipError_t launch_dkdv_pair_d(const PairBwdArgs& p, int mode, hipStream_t stream) {
+  const BwdArgs& a = p.a;
+  const int nkt = (a.Lk + kPairSlab - 1) / kPairSlab;
+  dim3 grid((unsigned)(a.B * a.H * p.n_split * nkt)), block(kPairThreads);
+  if (mode == 2) hipLaunchKernelGGL((dkdv_pair_kernel<D, 2>), grid, block, 0, stream, p);
+  else if (mode == 1) hipLaunchKernelGGL((dkdv_pair_kernel<D, 1>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((dkdv_pair_kernel<D, 0>), grid, block, 0, stream, p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || p.n_split == 1) return e;
+  return launch_pair_sum<D, kPairSlab>(p, 2, a.Lk, stream);
+}
+
+hipError_t launch_dkdv_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream) {
+  return D == 128 ? launch_dkdv_pair_d<128>(p, mode, stream) : launch_dkdv_pair_d<64>(p, mode, stream);
+}
+
+hipError_t launch_pair_stat(const void* out, int out_f32, long long sb, long long sh, long long sl, TensorArg dout, const float* lse,
+                            float inv_res, float* stat, float* delta, int B, int H, int Lq, int D, hipStream_t stream) {
+  const long long rows = (long long)B * H * Lq;
+  const int rpb = 256 / (D / 8);
+  dim3 grid((unsigned)((rows + rpb - 1) / rpb)), block(256);
+  if (D == 128) {
+    if (out_f32) hipLaunchKernelGGL((pair_stat_kernel<float, 128>), grid, block, 0, stream, (const float*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
+    else hipLaunchKernelGGL((pair_stat_kernel<bf16_t, 128>), grid, block, 0, stream, (const bf16_t*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
+  } else {
+    if (out_f32) hipLaunchKernelGGL((pair_stat_kernel<float, 64>), grid, block, 0, stream, (const float*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
+    else hipLaunchKernelGGL((pair_stat_kernel<bf16_t, 64>), grid, block, 0, stream, (const bf16_t*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_dq_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream) {
+  return D == 128 ? launch_dq_pair_d<128>(p, mode, stream) : launch_dq_pair_d<64>(p, mode, stream);
 }
 
 template <int D>

@@ -714,24 +714,19 @@ def _pair_forward(q, k, v, plan: "_RingPlan", sm_scale, out_dtype):
 
 
 def _pair_backward(q, k, v, out, lse, do, plan: "_RingPlan", sm_scale):
-    """``_ring_backward_fused`` of a ring of one shard: one description for the three launches."""
+    """``_ring_backward_fused`` of a ring of one shard: one description for all launches."""
     B, H, D, Lq, Lk = plan.B, plan.H, plan.D, plan.Lq, plan.Lk
-    lib, stream = _lib.load(), _stream()
-    delta = torch.empty((1, B, H, Lq), dtype=torch.float32, device=plan.device)
+    lib = _lib.load()
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    ob, ol, oh, _ = out.stride()
-    do_t = _view_blhd(do)
-    _lib.check("ra_bwd_delta_passes", lib.ra_bwd_delta_passes(
-        out.data_ptr(), _DTYPE_CODE[out.dtype], 0, ob, oh, ol, C.byref(do_t), 0, delta.data_ptr(), 1, B, H, Lq, D,
-        stream))
-    p = _lib.RaBwdStepParams(B, H, Lq, Lk, D, sm_scale, _view_blhd(q), _view_blhd(k), _view_blhd(v), do_t,
-                             lse.data_ptr(), delta.data_ptr(), None, None, None, plan.pair_bias())
-    gb, gl, gh, _ = dk.stride()
+    p = _lib.RaBwdStepParams(B, H, Lq, Lk, D, sm_scale, _view_blhd(q), _view_blhd(k), _view_blhd(v), _view_blhd(do),
+                             lse.data_ptr(), None, None, None, None, plan.pair_bias())
+    size = lib.ra_bwd_pair_workspace(C.byref(p))
+    ws = torch.empty((size,), dtype=torch.uint8, device=plan.device)
     assert dk.stride() == dv.stride()
-    _lib.check("ra_bwd_dkdv_ring", lib.ra_bwd_dkdv_ring(C.byref(p), _ONE_STEP, 1, dk.data_ptr(), dv.data_ptr(), 0, gb,
-                                                        gh, gl, stream))
-    gb, gl, gh, _ = dq.stride()
-    _lib.check("ra_bwd_dq_ring", lib.ra_bwd_dq_ring(C.byref(p), _ONE_STEP, 1, dq.data_ptr(), 0, gb, gh, gl, stream))
+    (ob, ol, oh, _), (qb, ql, qh, _), (kb, kl, kh, _) = out.stride(), dq.stride(), dk.stride()
+    _lib.check("ra_bwd_pair", lib.ra_bwd_pair(
+        C.byref(p), out.data_ptr(), _DTYPE_CODE[out.dtype], ob, oh, ol, dq.data_ptr(), qb, qh, ql, dk.data_ptr(),
+        dv.data_ptr(), kb, kh, kl, ws.data_ptr(), size, _stream()))
     return dq, dk, dv
 
 

@@ -80,6 +80,7 @@ extern "C" {
 
 #define RA_DTYPE_BF16 0
 #define RA_DTYPE_F32 1
+#define RA_DTYPE_F16 2 /* ra_convert only */
 
 /* bf16 tensor view [B, H, L, D] with explicit element strides (D contiguous; strides multiples of 8,
  * D <= stride_l <= 2^27). */
@@ -312,6 +313,24 @@ int ra_bwd_finalize_passes(const float* acc, void* out, int64_t out_stride_pass,
 int64_t ra_dense_map_bytes(int64_t stride_b, int64_t stride_h, int32_t B, int32_t H, int32_t Lq, int32_t Lk);
 int ra_dense_map(const float* dense_bias, int64_t stride_b, int64_t stride_h, int64_t stride_q, int32_t B,
                  int32_t H, int32_t Lq, int32_t Lk, uint8_t* map, void* stream);
+
+/* Arrays of rows [B, L, H, d] (strides in elements, the head dimension contiguous) converted between bf16,
+ * fp16 and fp32 (round to nearest even) and between head dims: elements at or beyond src_d read as
+ * zero, elements at or beyond dst_d are not written.  What stands between a caller's arrays and
+ * the bf16 operands of head dim 64 or 128 that the other entry points take - the reference computes
+ * in the caller's dtype and head dim (ring_kernel.py:123-131) - for up to 4 arrays in one launch.  Rows may
+ * have any alignment that their dtype has.  RA_ERR_TOO_LARGE: an array of 2^31 or more chunks of eight
+ * elements per batch row, or more than 65535 batch rows. */
+typedef struct {
+  const void* src;
+  void* dst;
+  int32_t src_dtype, dst_dtype; /* RA_DTYPE_* */
+  int32_t src_d, dst_d;
+  int32_t B, L, H;
+  int64_t src_stride_b, src_stride_l, src_stride_h;
+  int64_t dst_stride_b, dst_stride_l, dst_stride_h;
+} ra_rows;
+int ra_convert(const ra_rows* items, int32_t n_items, void* stream);
 
 /* Host-only, pure: 1 if every score of the (query shard, key/value shard) pair is masked
  * by the positional terms of `bias` (CAUSAL / WINDOW), so that the whole ring step is an

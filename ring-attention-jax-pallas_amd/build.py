@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(CSRC, "build")
 LIB_PATH = os.path.join(HERE, "ring_attention", "libringattn_hip.so")
-SOURCES = ["ra_fwd.hip", "ra_bwd.hip", "ra_pair.hip", "ra_api.hip"]
+SOURCES = ["ra_fwd.hip", "ra_bwd.hip", "ra_pair.hip", "ra_convert.hip", "ra_api.hip"]
 # the matrix-rate probe that bench.py reports next to the roofline: a library of its own, so that
 # the block-step library exports nothing but the block-step ABI
 PROBE_LIB_PATH = os.path.join(HERE, "ring_attention", "libringattn_probe.so")

@@ -662,7 +662,7 @@ int64_t fwd_part_bytes(const ra_fwd_step_params& p, int n_split) {
 
 extern "C" {
 
-int ra_version(void) { return 1007; }
+int ra_version(void) { return 1008; }
 
 int64_t ra_fwd_pair_workspace(const ra_fwd_step_params* p) {
   if (!p || check_dims(p->B, p->H, p->Lq, p->Lk, p->D)) return 0;
@@ -1017,6 +1017,38 @@ int ra_bwd_pair(const ra_bwd_step_params* p, const void* out, int32_t out_dtype,
   share(plan_q, sp.dq_part, sp.dq_n, rq);
   e = ra::launch_dq_pair(a, c.D, mode, (hipStream_t)stream);
   return e == hipSuccess ? RA_OK : hip_fail(e, "ra_bwd_pair launch");
+}
+
+int ra_convert(const ra_rows* items, int32_t n_items, void* stream) {
+  if (n_items < 1 || n_items > ra::kMaxConvert) return fail(RA_ERR_SHAPE, "ra_convert: 1 to %d arrays (got %d)", ra::kMaxConvert, n_items);
+  if (!items) return fail(RA_ERR_NULL, "ra_convert: items is NULL");
+  ra::ConvertArgs a;
+  memset(&a, 0, sizeof(a));
+  for (int i = 0; i < n_items; ++i) {
+    const ra_rows& r = items[i];
+    if (!r.src || !r.dst) return fail(RA_ERR_NULL, "ra_convert: NULL pointer");
+    if (r.B <= 0 || r.L <= 0 || r.H <= 0 || r.src_d <= 0 || r.dst_d <= 0)
+      return fail(RA_ERR_SHAPE, "ra_convert: bad shape B=%d L=%d H=%d d=%d -> %d", r.B, r.L, r.H, r.src_d, r.dst_d);
+    if (r.src_d > 128 || r.dst_d > 128) return fail(RA_ERR_HEAD_DIM, "ra_convert: head dims of at most 128");
+    if (r.B > 65535 || (int64_t)r.H * 16 >= ((int64_t)1 << 31) || (int64_t)r.L * (r.H * 16) >= ((int64_t)1 << 31))
+      return fail(RA_ERR_TOO_LARGE, "ra_convert: too many rows for one launch");
+    for (int dt : {r.src_dtype, r.dst_dtype})
+      if (dt != RA_DTYPE_BF16 && dt != RA_DTYPE_F32 && dt != RA_DTYPE_F16) return fail(RA_ERR_DTYPE, "unknown dtype %d", dt);
+    // eight elements at a time where every chunk of a row starts on a multiple of 16 bytes
+    auto on_chunks = [](const void* p, int dtype, int64_t sb, int64_t sl, int64_t sh) {
+      const int64_t mask = dtype == RA_DTYPE_F32 ? 3 : 7;
+      return aligned16(p) && !((sb | sl | sh) & mask);
+    };
+    if (reinterpret_cast<uintptr_t>(r.src) % (r.src_dtype == RA_DTYPE_F32 ? 4 : 2) ||
+        reinterpret_cast<uintptr_t>(r.dst) % (r.dst_dtype == RA_DTYPE_F32 ? 4 : 2))
+      return fail(RA_ERR_ALIGN, "ra_convert: arrays must be aligned to their elements");
+    a.item[i] = ra::ConvertItem{r.src, r.dst, r.src_dtype, r.dst_dtype, r.src_d, r.dst_d, r.B, r.L, r.H,
+                                on_chunks(r.src, r.src_dtype, r.src_stride_b, r.src_stride_l, r.src_stride_h),
+                                on_chunks(r.dst, r.dst_dtype, r.dst_stride_b, r.dst_stride_l, r.dst_stride_h),
+                                r.src_stride_b, r.src_stride_l, r.src_stride_h, r.dst_stride_b, r.dst_stride_l, r.dst_stride_h};
+  }
+  hipError_t e = ra::launch_convert(a, n_items, (hipStream_t)stream);
+  return e == hipSuccess ? RA_OK : hip_fail(e, "ra_convert launch");
 }
 
 int ra_bwd_finalize_passes(const float* acc, void* out, int64_t out_stride_pass, int64_t out_stride_b,

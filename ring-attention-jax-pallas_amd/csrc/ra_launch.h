@@ -139,6 +139,22 @@ hipError_t launch_dkdv_pair(const PairBwdArgs& p, int D, int mode, hipStream_t s
 hipError_t launch_pair_stat(const void* out, int out_f32, long long sb, long long sh, long long sl, TensorArg dout, const float* lse,
                             float inv_res, float* stat, float* delta, int B, int H, int Lq, int D, hipStream_t stream);
 
+// Arrays of rows that are converted and padded (or cut) to another head dim (ra_convert).
+constexpr int kMaxConvert = 4;
+struct ConvertItem {
+  const void* src;
+  void* dst;
+  int src_dtype, dst_dtype;  // RA_DTYPE_*
+  int src_d, dst_d;
+  int B, L, H;
+  int src_vec, dst_vec;  // whole chunks of eight elements lie on their own alignment
+  long long src_sb, src_sl, src_sh, dst_sb, dst_sl, dst_sh;
+};
+struct ConvertArgs {
+  ConvertItem item[kMaxConvert];
+};
+hipError_t launch_convert(const ConvertArgs& a, int n, hipStream_t stream);
+
 hipError_t launch_fwd_step(const FwdArgs& a, int D, int mode, hipStream_t stream);
 hipError_t launch_fwd_steps(const FwdArgs& a, const KvRing& ring, int D, int mode, hipStream_t stream);
 hipError_t launch_fwd_init(float* o, float* m, float* l, long long rows, int D, hipStream_t stream);

@@ -20,6 +20,8 @@ RA_MAX_SEGMENT_SHARD = 65536  # longest shard that one call takes under a segmen
 RA_MAX_POSITION = (1 << 30) - (1 << 16)  # token positions (offset + index) stay below this
 RA_MAX_ROW_STRIDE = 1 << 27  # elements between two rows of a q / k / v / dO view, at most
 RA_DTYPE_F32 = 1
+RA_DTYPE_F16 = 2  # ra_convert only
+RA_MAX_CONVERT = 4  # arrays per ra_convert
 
 
 class RaTensor(C.Structure):
@@ -96,6 +98,7 @@ EXPORTS = {
     "ra_bwd_pair": (C.c_int, [C.POINTER(RaBwdStepParams), C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64,
                               C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64,
                               C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p]),
+    "ra_convert": (C.c_int, [C.c_char_p, C.c_int32, C.c_void_p]),  # ra_rows blocks, packed
     "ra_fwd_finalize_passes": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_int64,
                                          C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32, C.c_int32,
                                          C.c_int32, C.c_int32, C.c_int32, C.c_void_p]),

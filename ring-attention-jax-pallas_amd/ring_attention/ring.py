@@ -29,6 +29,7 @@ import collections
 import ctypes as C
 import functools
 import math
+import struct
 from dataclasses import dataclass
 from typing import Callable, Optional, Union
 
@@ -130,6 +131,49 @@ def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
     ok = (t.stride(-1) == 1 and all(s % 8 == 0 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0
           and t.shape[-1] <= t.stride(1) <= _lib.RA_MAX_ROW_STRIDE)
     return t if ok else t.contiguous()
+
+
+def _kernel_dim(d: int) -> int:
+    """The head dim that the kernels compute a head dim of ``d`` in."""
+    return 64 if d <= 64 else 128
+
+
+_ROW_DTYPES = {torch.bfloat16: _lib.RA_DTYPE_BF16, torch.float32: _lib.RA_DTYPE_F32, torch.float16: _lib.RA_DTYPE_F16}
+
+
+_ROWS = struct.Struct("PP7i4x6q")  # an ra_rows: packed in one call, where a ctypes block costs 3 us each
+
+
+def _convert(tensors, dtypes, d: int):
+    """[b, l, h, *] tensors as new contiguous [b, l, h, d] ones of the dtypes given: cast, and cut or
+    padded with zeros, in one launch (``ra_convert``).  What that does not take (other dtypes, a head
+    dimension that is not contiguous, more rows than a launch holds) goes through torch."""
+    out, items, n = [], b"", 0
+    dev = tensors[0].device
+    for t, dtype in zip(tensors, dtypes):
+        B, L, H, dt = t.shape
+        o = torch.empty((B, L, H, d), dtype=dtype, device=dev)
+        out.append(o)
+        src, dst = _ROW_DTYPES.get(t.dtype), _ROW_DTYPES.get(dtype)
+        sb, sl, sh, sd = t.stride()
+        if (src is not None and dst is not None and sd == 1 and t.is_cuda and t.device == dev and B < 65536
+                and 0 < B * L * H and L * H < 1 << 27):
+            items += _ROWS.pack(t.data_ptr(), o.data_ptr(), src, dst, dt, d, B, L, H, sb, sl, sh, L * H * d, H * d, d)
+            n += 1
+        else:
+            o.copy_(t[..., :d] if dt >= d else torch.nn.functional.pad(t, (0, d - dt)))
+    if n:
+        _lib.check("ra_convert", _lib.load().ra_convert(items, n, _stream()))
+    return out
+
+
+def _kernel_inputs(tensors, d: int):
+    """``_kernel_ready`` for several tensors at once, padded to the kernels' head dim ``d``."""
+    todo = [t for t in tensors if t.dtype != torch.bfloat16 or t.shape[3] != d]
+    if not todo:
+        return [_kernel_ready(t) for t in tensors]
+    new = iter(_convert(todo, [torch.bfloat16] * len(todo), d))
+    return [next(new) if t.dtype != torch.bfloat16 or t.shape[3] != d else _kernel_ready(t) for t in tensors]
 
 
 # --------------------------------------------------------------------------------------
@@ -316,7 +360,8 @@ class _RingPlan:
 
     def __init__(self, q, k, n, fn: Optional[BiasFn], q_kwargs, kv_kwargs):
         self.n = n
-        self.B, Sq, self.H, self.D = q.shape
+        self.B, Sq, self.H, d = q.shape
+        self.D = _kernel_dim(d)
         Sk = k.shape[1]
         if Sq % n or Sk % n:
             raise ValueError(f"sequence lengths ({Sq}, {Sk}) must be divisible by the ring size {n}")
@@ -905,24 +950,37 @@ class _RingAttentionFn(torch.autograd.Function):
     """custom_vjp of the reference (ring.py:214-243): forward saves (q, k, v, o, L)."""
 
     @staticmethod
-    def forward(ctx, q, k, v, plan, sm_scale, out_dtype, fused):
+    def forward(ctx, q, k, v, plan, sm_scale, out_dtype, final_dtype, fused):
+        """The output has the inputs' head dim and ``final_dtype``; where no gradient will follow it may
+        be the kernels' own (padded, ``out_dtype``), which the caller cuts."""
+        ctx.given = [(t.shape[3], t.dtype) for t in (q, k, v)]
+        d = q.shape[3]
+        q, k, v = _kernel_inputs((q, k, v), plan.D)
         fwd = _ring_forward_fused if fused else _ring_forward
         out, lse = fwd(q, k, v, plan, sm_scale, out_dtype)
         ctx.save_for_backward(q, k, v, out, lse)
         ctx.plan, ctx.sm_scale, ctx.fused = plan, sm_scale, fused
         ctx.mark_non_differentiable(lse)
         ctx.set_materialize_grads(False)  # no zero fill for the logsumexp's gradient
+        if out_dtype != final_dtype or (d != plan.D and any(ctx.needs_input_grad)):
+            out, = _convert([out], [final_dtype], d)
         return out, lse
 
     @staticmethod
     def backward(ctx, do, _dlse):
         q, k, v, out, lse = ctx.saved_tensors
         if do is None:
-            return (None,) * 7
-        do = _kernel_ready(do)
+            return (None,) * 8
+        do, = _kernel_inputs((do,), ctx.plan.D)
         bwd = _ring_backward_fused if ctx.fused else _ring_backward
-        dq, dk, dv = bwd(q, k, v, out, lse, do, ctx.plan, ctx.sm_scale)
-        return dq, dk, dv, None, None, None, None
+        grads = list(bwd(q, k, v, out, lse, do, ctx.plan, ctx.sm_scale))
+        todo = [i for i, (d, dtype) in enumerate(ctx.given)
+                if ctx.needs_input_grad[i] and (d != ctx.plan.D or dtype != torch.bfloat16)]
+        if todo:
+            new = _convert([grads[i] for i in todo], [ctx.given[i][1] for i in todo], ctx.given[0][0])
+            for i, g in zip(todo, new):
+                grads[i] = g
+        return *(g if need else None for g, need in zip(grads, ctx.needs_input_grad)), None, None, None, None, None
 
 
 def ring_attention_with_lse(q, k, v, axis_name, bias_fn: Union[BiasFn, Callable, None] = None, bias_q_kwargs=None,
@@ -948,23 +1006,17 @@ def ring_attention_with_lse(q, k, v, axis_name, bias_fn: Union[BiasFn, Callable,
     in_dtype = q.dtype
     if out_dtype is None:
         out_dtype = torch.float32 if in_dtype == torch.float32 else torch.bfloat16
-    d_pad = 64 if d_true <= 64 else 128
     if d_true > 128:
         raise ValueError("head dims above 128 are not supported")
-    if d_pad != d_true:
-        pad = (0, d_pad - d_true)
-        q, k, v = (torch.nn.functional.pad(x, pad) for x in (q, k, v))
-    q, k, v = _kernel_ready(q), _kernel_ready(k), _kernel_ready(v)
     plan = _plan_for(q, k, _walked_ring_size(n, q.shape[1], k.shape[1], bias_fn), bias_fn, bias_q_kwargs,
                      bias_kv_kwargs)
     fused = _launch_whole_ring(block_impl, plan)
     if fused:
         plan = plan.joined()
-    out, lse = _RingAttentionFn.apply(q, k, v, plan, float(sm_scale), out_dtype, fused)
-    if d_pad != d_true:
+    final_dtype = out_dtype if in_dtype in (torch.float32, torch.bfloat16) else in_dtype
+    out, lse = _RingAttentionFn.apply(q, k, v, plan, float(sm_scale), out_dtype, final_dtype, fused)
+    if out.shape[-1] != d_true:
         out = out[..., :d_true]
-    if in_dtype not in (torch.float32, torch.bfloat16):
-        out = out.to(in_dtype)
     lse_full = lse.permute(1, 2, 0, 3).reshape(plan.B, plan.H, plan.n * plan.Lq)
     return out, lse_full
 

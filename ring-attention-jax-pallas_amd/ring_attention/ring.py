@@ -466,7 +466,7 @@ class _RingPlan:
         were shard boundaries, and the host describes one shard pair instead of n * n.  Forward +
         backward: B=2, H=16, 8 x 1024 causal 2.52 -> 2.28 ms; B=2, H=16, D=64, 4 x 1024 causal + ALiBi
         0.73 -> 0.64 ms; fp32 inputs, B=2, H=4, 8 x 256: 3.6 -> 0.19 ms, nearly all of it host code.
-        The joined shards stay within what one launch takes under a segment term."""
+        The joined shards stay within what one launch takes, with and without a segment term."""
         got = self.__dict__.get("_joined")
         if got is None:
             got = self._join()
@@ -478,9 +478,9 @@ class _RingPlan:
         fn = self.fn
         if self.callable is not None or n == 1:
             return self
-        segments = fn is not None and fn.segments
+        longest = _lib.RA_MAX_SEGMENT_SHARD if fn is not None and fn.segments else _lib.RA_MAX_SHARD
         for g in range(n, 1, -1):
-            if n % g or (segments and g * max(Lq, Lk) > _lib.RA_MAX_SEGMENT_SHARD):
+            if n % g or g * max(Lq, Lk) > longest:
                 continue
             if all(off[r] == off[r - r % g] + (r % g) * L for off, L in ((self.q_off, Lq), (self.kv_off, Lk))
                    for r in range(n)):

@@ -160,6 +160,13 @@ def test_consecutive_shards_are_joined(starts, want):
     assert plan.joined().n == 2
 
 
+def test_joined_shards_stay_within_one_launch():
+    # 4 shards of 2^23 tokens: the library takes two of them as one, not all four
+    long = torch.zeros(1, 1, 1, 64, dtype=torch.bfloat16).expand(1, 4 << 23, 1, 64)
+    plan = rr._RingPlan(long, long, 4, ra.sliding_window_bias(128), None, None)
+    assert (plan.joined().n, plan.joined().Lq) == (2, 1 << 24)
+
+
 def test_ring_plan_with_a_callable_bias_fn():
     # the reference's general form: the callable sees the shards of its kwargs (ring.py:107,186)
     q = torch.zeros(2, 64, 2, 64, dtype=torch.bfloat16)

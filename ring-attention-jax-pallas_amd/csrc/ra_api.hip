@@ -339,6 +339,69 @@ int check_pass_counts(const int32_t* steps_per_pass, int32_t n_passes, std::vect
   return RA_OK;
 }
 
+// ---- steps on a dense block: the kernels of ra_pair.hip, one launch per step ----------------------------
+// What bounds such a step is the block's elementwise term (one fp32 read and add per score), which the long-stretch kernels pay
+// in generic iterations, one workgroup per compute unit with nothing beside it; the pair kernels have a second workgroup
+// there, and leave a carry or accumulator alone whose tiles are all masked.  Forward + backward, long-stretch kernels -> these:
+// document masks (-inf / 0, with their summary) 32768 in 4 shards, H=16, D=128: 18.8 -> 16.0 ms, 5001 in 3, H=16, D=64: 3.42 ->
+// 3.00, 4096, B=4, H=32, D=96: 6.69 -> 4.33, 16384 in 8, H=4: 9.3 -> 8.3; blocks of values (every tile evaluated)
+// 8192, H=32, D=128: 16.7 -> 10.5 ms, 16384 in 4, H=16: 34.6 -> 23.6, 4096, B=2, H=16, D=64: 3.11 -> 2.51; 512 and 2000 tokens in 8
+// shards (host bound): 8.16 -> 8.22 and 8.15 -> 8.23, within the spread of one side (3 %).
+bool dense_steps_on_pair(const ra_bias& b) { return b.flags & RA_BIAS_DENSE; }
+constexpr int kWholeRow = 1 << 30;  // chunk_tiles of rows that are not shared
+
+int fwd_step_on_pair(const ra_fwd_step_params& p, void* stream) {
+  if (ra_step_is_skippable(&p.bias, p.Lq, p.Lk)) return RA_OK;  // identity on the carry
+  ra::PairFwdArgs a;
+  memset(&a, 0, sizeof(a));
+  a.q = to_arg(p.q);
+  a.k = to_arg(p.k);
+  a.v = to_arg(p.v);
+  a.B = p.B;
+  a.H = p.H;
+  a.Lq = p.Lq;
+  a.Lk = p.Lk;
+  a.scale2 = p.sm_scale * kLog2eHost;
+  a.bias = to_bias(p.bias);
+  a.n_split = 1;
+  a.chunk_tiles = kWholeRow;
+  a.o = p.o;
+  a.m = p.m;
+  a.l = p.l;
+  hipError_t e = ra::launch_fwd_pair(a, p.D, kernel_mode(p.bias.flags), (hipStream_t)stream);
+  return e == hipSuccess ? RA_OK : hip_fail(e, "forward step launch");
+}
+
+// parts: 1 = dK and dV, 2 = dQ
+int bwd_step_on_pair(const ra_bwd_step_params& p, int parts, void* stream) {
+  if (ra_step_is_skippable(&p.bias, p.Lq, p.Lk)) return RA_OK;  // contributes nothing
+  ra::PairBwdArgs a;
+  memset(&a, 0, sizeof(a));
+  a.a = to_bwd_args(p);
+  a.n_split = 1;
+  a.chunk_tiles = kWholeRow;
+  hipError_t e = hipSuccess;
+  if (parts & 1) {
+    a.acc = p.dk;
+    a.acc2 = p.dv;
+    e = ra::launch_dkdv_pair(a, p.D, kernel_mode(p.bias.flags), (hipStream_t)stream);
+  }
+  if (e == hipSuccess && (parts & 2)) {
+    a.acc = p.dq;
+    a.acc2 = nullptr;
+    e = ra::launch_dq_pair(a, p.D, kernel_mode(p.bias.flags), (hipStream_t)stream);
+  }
+  return e == hipSuccess ? RA_OK : hip_fail(e, "backward step launch");
+}
+
+// Every step of a single pass takes that route, or none does.
+template <typename P>
+bool all_on_pair(const P* steps, int n_steps) {
+  for (int i = 0; i < n_steps; ++i)
+    if (!dense_steps_on_pair(steps[i].bias)) return false;
+  return n_steps > 0;
+}
+
 int fwd_passes(const ra_fwd_step_params* steps, const std::vector<int>& first, int n_passes, void* stream,
                const RingResult* whole = nullptr) {
   const int total = first.back();
@@ -363,6 +426,11 @@ int fwd_passes(const ra_fwd_step_params* steps, const std::vector<int>& first, i
                                   "(k.ptr, v.ptr, kv_offset, kv_segment_ids, kv_prefix, dense_bias), or from "
                                   "steps[0] in shape, strides or bias terms", i);
     }
+  }
+  if (!whole && n_passes == 1 && all_on_pair(steps, total)) {
+    int rc = RA_OK;
+    for (int i = 0; i < total && !rc; ++i) rc = fwd_step_on_pair(steps[i], stream);
+    return rc;
   }
   ra::FwdArgs a;
   a.q = to_arg(f.q);
@@ -439,6 +507,11 @@ int bwd_dq_passes(const ra_bwd_step_params* steps, const std::vector<int>& first
                                   "steps[0] in shape, strides or bias terms", i);
     }
   }
+  if (!whole && n_passes == 1 && all_on_pair(steps, total)) {
+    int rc = RA_OK;
+    for (int i = 0; i < total && !rc; ++i) rc = bwd_step_on_pair(steps[i], 2, stream);
+    return rc;
+  }
   ra::BwdArgs a = to_bwd_args(f);
   if (whole) {
     a.bias.flags |= ra::kFlagWholeBf16;
@@ -495,6 +568,11 @@ int bwd_dkdv_passes(const ra_bwd_step_params* steps, const std::vector<int>& fir
                                   "dout.ptr, lse, delta, dq, q_offset, q_segment_ids, q_prefix, dense_bias), or from "
                                   "steps[0] in shape, strides or bias terms", i);
     }
+  }
+  if (!whole && n_passes == 1 && all_on_pair(steps, total)) {
+    int rc = RA_OK;
+    for (int i = 0; i < total && !rc; ++i) rc = bwd_step_on_pair(steps[i], 1, stream);
+    return rc;
   }
   ra::BwdArgs a = to_bwd_args(f);
   if (whole) {
@@ -795,6 +873,7 @@ int ra_dense_map(const float* dense_bias, int64_t stride_b, int64_t stride_h, in
 int ra_fwd_step(const ra_fwd_step_params* p, void* stream) {
   int rc = ra_fwd_step_check(p);
   if (rc) return rc;
+  if (dense_steps_on_pair(p->bias)) return fwd_step_on_pair(*p, stream);
   if (ra_step_is_skippable(&p->bias, p->Lq, p->Lk)) return RA_OK;  // identity on the carry
   ra::FwdArgs a;
   a.q = to_arg(p->q);
@@ -888,6 +967,7 @@ int ra_bwd_step_parts(const ra_bwd_step_params* p, int32_t parts, void* stream) 
   int rc = ra_bwd_step_check(p);
   if (rc) return rc;
   if (parts < 1 || parts > 3) return fail(RA_ERR_SHAPE, "parts must be 1, 2 or 3 (got %d)", parts);
+  if (dense_steps_on_pair(p->bias)) return bwd_step_on_pair(*p, parts, stream);
   if (ra_step_is_skippable(&p->bias, p->Lq, p->Lk)) return RA_OK;  // contributes nothing
   const ra::BwdArgs a = to_bwd_args(*p);
   hipError_t e = ra::launch_bwd_step(a, p->D, kernel_mode(p->bias.flags), parts, (hipStream_t)stream);

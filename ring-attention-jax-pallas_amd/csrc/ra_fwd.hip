@@ -1333,18 +1333,29 @@ __global__ void fwd_finalize_kernel(const float* o, const float* m, const float*
 // ------------------------------------------------------------------------------------------------
 namespace ra {
 
-// mode: 0 = causal / window terms only, 1 = any of the per-tile terms, 2 = a dense bias block too
+// mode: 0 = causal / window terms only, 1 = any of the per-tile terms, 2 = a dense bias block too (MULTI only:
+// single steps on a dense block run on fwd_pair_kernel)
 template <bool MULTI, bool WHOLE, typename Shards>
 static hipError_t launch_fwd(const FwdArgs& a, const Shards& sl, int n_pass, int D, int mode, hipStream_t stream) {
   const int nqt = (a.Lq + kFwdRows - 1) / kFwdRows;
   dim3 grid((unsigned)(a.B * a.H * nqt), (unsigned)n_pass), block(kFwdThreads);
   if (D == 128) {
-    if (mode == 2) hipLaunchKernelGGL((fwd_step_kernel<128, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
-    else if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<128, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+    if constexpr (MULTI) {
+      if (mode == 2) {
+        hipLaunchKernelGGL((fwd_step_kernel<128, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+        return hipGetLastError();
+      }
+    }
+    if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<128, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
     else hipLaunchKernelGGL((fwd_step_kernel<128, 0, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
   } else {
-    if (mode == 2) hipLaunchKernelGGL((fwd_step_kernel<64, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
-    else if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<64, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+    if constexpr (MULTI) {
+      if (mode == 2) {
+        hipLaunchKernelGGL((fwd_step_kernel<64, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+        return hipGetLastError();
+      }
+    }
+    if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<64, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
     else hipLaunchKernelGGL((fwd_step_kernel<64, 0, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
   }
   return hipGetLastError();

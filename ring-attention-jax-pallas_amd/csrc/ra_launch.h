@@ -127,7 +127,7 @@ hipError_t launch_fwd_pair(const PairFwdArgs& a, int D, int mode, hipStream_t st
 struct PairBwdArgs {
   BwdArgs a;  // (its dq / dk / dv slots are not used)
   int n_split, chunk_tiles;
-  const float* stat;  // dK / dV: see pair_stat_kernel
+  const float* stat;  // dK / dV: see pair_stat_kernel (nullptr: from a.lse and a.delta)
   float* part;
   int* part_n;
   float *acc, *acc2;

@@ -275,6 +275,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   }
   n = __builtin_amdgcn_readfirstlane(n);
   j_lo = __builtin_amdgcn_readfirstlane(j_lo);
+  if (n == 0 && a.o != nullptr) return;  // identity on the carry
   const int n_piece = max(1, min(a.n_split, (n + a.chunk_tiles - 1) / a.chunk_tiles));
   if (split >= n_piece) return;
   const int i_lo = n * split / n_piece, i_hi = n * (split + 1) / n_piece;
@@ -658,6 +659,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void dq_pair_kernel(const PairBwdA
   }
   n = __builtin_amdgcn_readfirstlane(n);
   j_lo = __builtin_amdgcn_readfirstlane(j_lo);
+  if (n == 0 && p.acc != nullptr) return;  // contributes nothing
   const int n_piece = max(1, min(p.n_split, (n + p.chunk_tiles - 1) / p.chunk_tiles));
   if (split >= n_piece) return;
   const int i_lo = n * split / n_piece, i_hi = n * (split + 1) / n_piece;
@@ -938,7 +940,7 @@ RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg
 // that P and dS are the A operands of dV = P^T dO and dK = dS^T Q.  The rows' statistics (stat:
 // -lse log2(e) / scale_res, then -delta, from pair_stat_kernel) are the accumulators' initial values.
 template <int D, int MODE>
-__global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kernel(const PairBwdArgs p) {
+__global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dkdv_pair_kernel(const PairBwdArgs p) {
   constexpr bool GENERAL = MODE != 0;
   constexpr bool DENSE = MODE == 2;
   constexpr bool VLDS = D == 128;
@@ -1019,6 +1021,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
   }
   n = __builtin_amdgcn_readfirstlane(n);
   j_lo = __builtin_amdgcn_readfirstlane(j_lo);
+  if (n == 0 && p.acc != nullptr) return;  // contributes nothing
   const int n_piece = max(1, min(p.n_split, (n + p.chunk_tiles - 1) / p.chunk_tiles));
   if (split >= n_piece) return;
   const int i_lo = n * split / n_piece, i_hi = n * (split + 1) / n_piece;
@@ -1041,7 +1044,8 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
   ldq.init(a.q.ptr + b * a.q.sb + h * a.q.sh, a.q.sl, a.Lq, lane);
   ldo.init(a.dout.ptr + b * a.dout.sb + h * a.dout.sh, a.dout.sl, a.Lq, lane);
   // lanes 0..31 move -lse of a tile's rows, lanes 32..63 -delta
-  const float* stat = p.stat + (long long)hh * a.Lq + (g ? (long long)a.B * a.H * a.Lq : 0);
+  const bool raw_stat = DENSE && p.stat == nullptr;  // a single step, which has no room for them: from lse and delta, per tile
+  const float* stat = (raw_stat ? (g ? a.delta : a.lse) : p.stat + (g ? (long long)a.B * a.H * a.Lq : 0)) + (long long)hh * a.Lq;
   auto issue_tile = [&](int j, int buf) {
     const int r0 = j * kPairQueries;
     unsigned first = first_chunk;
@@ -1064,6 +1068,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
   const FragOffsets<D> fo(lane);
   const bool wave_on = kw < a.Lk;
   const bool alibi_on = GENERAL && (flags & RA_BIAS_ALIBI);
+  const float lse_mul = -kLog2e / a.scale_res;
   const int klo_w = kv_off + kw, khi_w = kv_off + kw + 31;
 
   auto step = [&](auto buffer, int i) {
@@ -1089,6 +1094,10 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
       const f32x4 t = *(const f32x4*)&s_stat[BUF][0][8 * bb + 4 * g];
 #pragma unroll
       for (int c = 0; c < 4; ++c) S[4 * bb + c] = t[c];
+    }
+    if (raw_stat) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) S[r] = (S[r] == RA_NEG_INF) ? RA_NEG_INF : S[r] * lse_mul;
     }
     if (one_side) S = alibi_one_side(S, qlo >= khi_w ? -slope2 : slope2, (kv_off + ki) - qlo, 0, l32, g);
     auto nat_frag = [&](const char* tile, int ss) { return *(const bf16x8*)(tile + fr_off.nat(ss)); };
@@ -1137,6 +1146,14 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
       const f32x4 t = *(const f32x4*)&s_stat[BUF][1][8 * bb + 4 * g];
 #pragma unroll
       for (int c = 0; c < 4; ++c) P[4 * bb + c] = t[c];
+    }
+    if (raw_stat) {
+#pragma unroll
+      for (int bb = 0; bb < 4; ++bb) {
+        const f32x4 t = *(const f32x4*)&s_stat[BUF][0][8 * bb + 4 * g];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) P[4 * bb + c] = (t[c] == RA_NEG_INF) ? 0.f : -P[4 * bb + c];
+      }
     }
     {
       bf16x8 fr[KS], vr[KS];

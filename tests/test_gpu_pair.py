@@ -8,6 +8,7 @@ import torch
 
 import ring_attention as ra
 from oracle import ring_oracle as R
+from test_gpu_dense_map import _both_ways
 from test_gpu_parity import _check
 
 pytestmark = pytest.mark.gpu
@@ -60,6 +61,32 @@ def test_pair_kernels_at_their_edges(device, Sq, Sk, D, kind):
     B, H = (1, 1) if Sk > 60000 else (2, 2)
     fn, ofn, qkw, kvkw = _bias(kind, B, Sq, Sk, H)
     _check(device, f"pair {kind}", B, Sq, Sk, H, D, 1, fn, ofn, qkw, kvkw, seed=Sq + Sk, impl="pallas")
+
+
+def _spread(where, absolute, q_segment_ids, kv_segment_ids):
+    """A dense block of values and -inf: rows whose id is a multiple of three see no key whose id is one."""
+    d = q_segment_ids[:, :, None] - kv_segment_ids[:, None, :]
+    return where(d % 3 == 0, float("-inf"), -0.1 * absolute(d))[:, None]
+
+
+@pytest.mark.parametrize("Sq,Sk,D,n", [(1, 1, 64, 1), (33, 63, 128, 1), (129, 65, 64, 1), (387, 195, 128, 3), (64, 520, 64, 2),
+                                       (260, 516, 128, 4)])
+def test_pair_kernels_take_single_steps_on_dense_blocks(device, monkeypatch, Sq, Sk, D, n):
+    # into a carry and fp32 accumulators; rows without a live key in the first shard (n = 1: in all)
+    rng = np.random.default_rng(Sq + Sk)
+    q_ids, k_ids = rng.integers(0, 7, (2, Sq)).astype(np.int32), rng.choice([0, 3, 6, 1], (2, Sk)).astype(np.int32)
+    q_ids[:, 0] = 3
+    k_ids[:, : Sk // n] = 3  # a shard of which these rows see nothing
+    if n == 1:
+        q_ids[:, Sq // 2:] = 4
+    def torch_fn(q_segment_ids, kv_segment_ids):
+        return _spread(torch.where, lambda d: d.abs().float(), q_segment_ids, kv_segment_ids)
+
+    def numpy_fn(q_segment_ids, kv_segment_ids):
+        return _spread(np.where, lambda d: np.abs(d).astype(np.float32), q_segment_ids, kv_segment_ids)
+
+    _both_ways(device, monkeypatch, "dense steps", 2, Sq, Sk, 2, D, n, torch_fn, numpy_fn, {"q_segment_ids": q_ids},
+               {"kv_segment_ids": k_ids}, seed=Sq)
 
 
 def test_a_repeated_call_reads_nothing_of_the_one_before(device):

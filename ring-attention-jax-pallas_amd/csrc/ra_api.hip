@@ -346,7 +346,8 @@ int check_pass_counts(const int32_t* steps_per_pass, int32_t n_passes, std::vect
 // document masks (-inf / 0, with their summary) 32768 in 4 shards, H=16, D=128: 18.8 -> 16.0 ms, 5001 in 3, H=16, D=64: 3.42 ->
 // 3.00, 4096, B=4, H=32, D=96: 6.69 -> 4.33, 16384 in 8, H=4: 9.3 -> 8.3; blocks of values (every tile evaluated)
 // 8192, H=32, D=128: 16.7 -> 10.5 ms, 16384 in 4, H=16: 34.6 -> 23.6, 4096, B=2, H=16, D=64: 3.11 -> 2.51; 512 and 2000 tokens in 8
-// shards (host bound): 8.16 -> 8.22 and 8.15 -> 8.23, within the spread of one side (3 %).
+// shards (host bound): 8.16 -> 8.22 and 8.15 -> 8.23, within the spread of one side (3 %), 810 in 3, H=4: 1.55 -> 1.62 (spread
+// 5 to 11 %; several small steps kept in one launch of the long-stretch kernels made no difference: 1.62).
 bool dense_steps_on_pair(const ra_bias& b) { return b.flags & RA_BIAS_DENSE; }
 constexpr int kWholeRow = 1 << 30;  // chunk_tiles of rows that are not shared
 

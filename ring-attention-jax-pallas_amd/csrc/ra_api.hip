@@ -395,12 +395,19 @@ int bwd_step_on_pair(const ra_bwd_step_params& p, int parts, void* stream) {
   return e == hipSuccess ? RA_OK : hip_fail(e, "backward step launch");
 }
 
-// Every step of a single pass takes that route, or none does.
-template <typename P>
-bool all_on_pair(const P* steps, int n_steps) {
-  for (int i = 0; i < n_steps; ++i)
-    if (!dense_steps_on_pair(steps[i].bias)) return false;
-  return n_steps > 0;
+// The steps of a single pass, one launch each, if they take that route (`taken`; all of them do, or none: a
+// pass has one set of bias terms).  The several-step entry points evaluate whole blocks: only the blocks of
+// a launch differ from step to step, a summary that travels with them describes one of them at most.
+template <typename P, typename Step>
+int steps_on_pair(const P* steps, int n_steps, bool& taken, Step step) {
+  taken = dense_steps_on_pair(steps[0].bias);
+  int rc = RA_OK;
+  for (int i = 0; taken && i < n_steps && !rc; ++i) {
+    P p = steps[i];
+    p.bias.dense_map = nullptr;
+    rc = step(p);
+  }
+  return rc;
 }
 
 int fwd_passes(const ra_fwd_step_params* steps, const std::vector<int>& first, int n_passes, void* stream,
@@ -428,10 +435,10 @@ int fwd_passes(const ra_fwd_step_params* steps, const std::vector<int>& first, i
                                   "steps[0] in shape, strides or bias terms", i);
     }
   }
-  if (!whole && n_passes == 1 && all_on_pair(steps, total)) {
-    int rc = RA_OK;
-    for (int i = 0; i < total && !rc; ++i) rc = fwd_step_on_pair(steps[i], stream);
-    return rc;
+  if (!whole && n_passes == 1) {
+    bool taken;
+    const int rc = steps_on_pair(steps, total, taken, [&](const ra_fwd_step_params& p) { return fwd_step_on_pair(p, stream); });
+    if (taken) return rc;
   }
   ra::FwdArgs a;
   a.q = to_arg(f.q);
@@ -508,10 +515,10 @@ int bwd_dq_passes(const ra_bwd_step_params* steps, const std::vector<int>& first
                                   "steps[0] in shape, strides or bias terms", i);
     }
   }
-  if (!whole && n_passes == 1 && all_on_pair(steps, total)) {
-    int rc = RA_OK;
-    for (int i = 0; i < total && !rc; ++i) rc = bwd_step_on_pair(steps[i], 2, stream);
-    return rc;
+  if (!whole && n_passes == 1) {
+    bool taken;
+    const int rc = steps_on_pair(steps, total, taken, [&](const ra_bwd_step_params& p) { return bwd_step_on_pair(p, 2, stream); });
+    if (taken) return rc;
   }
   ra::BwdArgs a = to_bwd_args(f);
   if (whole) {
@@ -570,10 +577,10 @@ int bwd_dkdv_passes(const ra_bwd_step_params* steps, const std::vector<int>& fir
                                   "steps[0] in shape, strides or bias terms", i);
     }
   }
-  if (!whole && n_passes == 1 && all_on_pair(steps, total)) {
-    int rc = RA_OK;
-    for (int i = 0; i < total && !rc; ++i) rc = bwd_step_on_pair(steps[i], 1, stream);
-    return rc;
+  if (!whole && n_passes == 1) {
+    bool taken;
+    const int rc = steps_on_pair(steps, total, taken, [&](const ra_bwd_step_params& p) { return bwd_step_on_pair(p, 1, stream); });
+    if (taken) return rc;
   }
   ra::BwdArgs a = to_bwd_args(f);
   if (whole) {

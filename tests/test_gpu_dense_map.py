@@ -240,3 +240,43 @@ def test_block_api_takes_a_summary_with_segment_ids(device, monkeypatch):
         for got, ref, nm in zip((dq, dk, dv), ref_g, ("dq", "dk", "dv")):
             mx, fro = _rel(got.permute(0, 2, 1, 3).cpu().numpy(), ref)
             assert mx <= GRAD_TOL and fro <= GRAD_TOL, (nm, on, mx, fro)
+
+
+@pytest.mark.parametrize("fn,passes", [("ra_fwd_steps", False), ("ra_fwd_passes", True), ("ra_bwd_dq_steps", False),
+                                       ("ra_bwd_dq_passes", True), ("ra_bwd_dkdv_steps", False), ("ra_bwd_dkdv_passes", True)])
+def test_several_steps_evaluate_their_blocks_whatever_summary_travels_with_them(device, fn, passes):
+    """The blocks of a several-step call agree in everything but the travelling shard and dense_bias, dense_map
+    among it: a caller who copies one description carries the summary of another block along."""
+    lib = _lib.load()
+    B, H, L, D, n = 1, 2, 160, 64, 2
+    rng = np.random.default_rng(4)
+    q, k, v, do = (_dev(x, device, torch.bfloat16).permute(0, 2, 1, 3) for x in R.make_inputs(4, B, L, n * L, H, D))
+    do = do[:, :, :L]
+    blocks = [_dev(rng.standard_normal((B, 1, L, L)).astype(np.float32), device) for _ in range(n)]
+    nothing_live = torch.zeros((lib.ra_dense_map_bytes(0, 0, B, H, L, L),), dtype=torch.uint8, device=device)
+    lse, delta = torch.full((B, H, L), 5.0, device=device), torch.zeros((B, H, L), device=device)
+    got = []
+    for stale in (False, True):
+        acc = [torch.zeros((B, H, L, D), device=device) for _ in range(3)]
+        m, l = torch.full((B, H, L), -float("inf"), device=device), torch.zeros((B, H, L), device=device)
+        steps, keep = [], []
+        for i in range(n):
+            ki, vi = k[:, :, i * L:(i + 1) * L], v[:, :, i * L:(i + 1) * L]
+            bias = rr.BlockBias(dense=blocks[i])
+            keep.append(bias)
+            if "fwd" in fn:
+                p = rr._fwd_params(q, ki, vi, bias, acc[0], m, l, 0.125)
+            elif "dq" in fn:
+                p = rr._bwd_params(q, ki, vi, do, lse, delta, *acc, bias, 0.125)
+            else:  # the query side travels; the same rows under another block are another shard
+                p = rr._bwd_params(q, k[:, :, :L], v[:, :, :L], do, lse, delta, *acc, bias, 0.125)
+            p.bias.dense_map = nothing_live.data_ptr() if stale else None
+            steps.append(p)
+        arr = (type(steps[0]) * n)(*steps)
+        args = (arr, (C.c_int32 * 1)(n), 1) if passes else (arr, n)
+        _lib.check(fn, getattr(lib, fn)(*args, None))
+        torch.cuda.synchronize()
+        got.append([*acc, m, l])
+    assert any(bool((x != 0).any()) for x in got[0][:3])
+    for x, y in zip(*got):
+        assert torch.equal(x, y)

@@ -79,3 +79,23 @@ def test_calls_equal_the_same_call_on_operands_cast_by_hand(device, dtype, d, gr
             assert (x.grad is not None) == need
             if need:
                 assert x.grad.shape == x.shape and _same(x.grad, y.grad[..., :d].to(dtype))
+
+
+class _Cut(torch.autograd.Function):
+    """Passes its input on and no gradient back."""
+    @staticmethod
+    def forward(ctx, x):
+        return x.clone()
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 72), (torch.float32, 128)])
+def test_a_missing_gradient_of_the_output_counts_as_zero(device, dtype, d):
+    q, k, v = (torch.randn((1, 200, 2, d), device=device, dtype=dtype, requires_grad=True) for _ in range(3))
+    grads = torch.autograd.grad(_Cut.apply(ra.ring_attention(q, k, v, 2)).sum(), (q, k, v))
+    for g, x in zip(grads, (q, k, v)):
+        assert g.shape == x.shape and g.dtype == x.dtype and not g.any()

@@ -478,6 +478,9 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     }
   }
 
+  // a wave without a live score leaves its rows of the carry as they are, unread (m would come back through
+  // two unit conversions, a last bit off)
+  if (a.o != nullptr && __all(l_run == 0.f && lr_run == 0.f)) return;
   const float l_step = half_sum(l_run), lr_step = half_sum(lr_run);
   if (a.part_n != nullptr && split == 0 && tid == 0) a.part_n[hh * nqt + qt] = n_piece;
   if (!q_valid) return;

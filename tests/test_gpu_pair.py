@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import ring_attention as ra
+from ring_attention import bias as bias_module
 from oracle import ring_oracle as R
 from test_gpu_dense_map import _both_ways
 from test_gpu_parity import _check
@@ -95,3 +96,23 @@ def test_a_repeated_call_reads_nothing_of_the_one_before(device):
     first = ra.ring_attention(q, k, v, 1, ra.causal_bias())
     ra.ring_attention(*(torch.full_like(x, float("nan")) for x in (q, k, v)), 1, ra.causal_bias())
     assert torch.equal(ra.ring_attention(q, k, v, 1, ra.causal_bias()), first)
+
+
+@pytest.mark.parametrize("summary", [True, False])
+@pytest.mark.parametrize("D", [64, 128])
+def test_rows_without_a_live_score_keep_their_carry(device, monkeypatch, D, summary):
+    # bit for bit: queries 32..63 and 160..191 (one wave each) see nothing, their neighbours do
+    monkeypatch.setattr(bias_module, "DENSE_SUMMARY", summary)
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn((1, 300, 2, D), generator=g).to(device, torch.bfloat16).permute(0, 2, 1, 3) for _ in range(3))
+    block = torch.randn((1, 1, 300, 300), generator=g)
+    dead = torch.zeros(300, dtype=torch.bool)
+    dead[32:64] = dead[160:192] = True
+    block[:, :, dead] = -float("inf")
+    o = torch.randn((1, 2, 300, D), generator=g).to(device)
+    m, l = torch.randn((1, 2, 300), generator=g).to(device), torch.rand((1, 2, 300), generator=g).to(device) + 0.5
+    before = [x.clone() for x in (o, m, l)]
+    ra.fwd_block(q, k, v, block.to(device), o, m, l, 0.1)
+    for x, was in zip((o, m, l), before):
+        same = (x == was).reshape(1, 2, 300, -1).all(-1).cpu()
+        assert same[:, :, dead].all() and not same[:, :, ~dead].all()

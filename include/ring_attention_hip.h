@@ -209,8 +209,8 @@ int ra_bwd_finalize(const float* acc, void* out, int64_t out_stride_b, int64_t o
  * memory at once - an emulated ring on one GPU, or a ring whose next shards have already
  * arrived.  Steps whose scores are all masked (ra_step_is_skippable) are dropped; more than 16
  * remaining steps are split into several launches.  Steps on a dense bias block
- * (RA_BIAS_DENSE) are one launch each, with the carry or accumulator in memory in between; their
- * summaries (ra_bias.dense_map) are not read.
+ * (RA_BIAS_DENSE) are one launch each where that is faster, with the carry or accumulator in memory in
+ * between; their summaries (ra_bias.dense_map) are not read.
  *  - ra_fwd_steps and ra_bwd_dq_steps: one query shard against several key/value shards.  The
  *    blocks must agree in everything but k.ptr, v.ptr, bias.kv_offset, bias.kv_segment_ids,
  *    bias.kv_prefix and bias.dense_bias (and, for the backward, dk and dv, which are not

@@ -349,6 +349,17 @@ int check_pass_counts(const int32_t* steps_per_pass, int32_t n_passes, std::vect
 // shards (host bound): 8.16 -> 8.22 and 8.15 -> 8.23, within the spread of one side (3 %), 810 in 3, H=4: 1.55 -> 1.62 (spread
 // 5 to 11 %; several small steps kept in one launch of the long-stretch kernels made no difference: 1.62).
 bool dense_steps_on_pair(const ra_bias& b) { return b.flags & RA_BIAS_DENSE; }
+// dK and dV only where their slabs are more than one per compute unit: a lone workgroup has nothing beside it there either,
+// and dkdv_kernel the longer pipeline.  dkdv_kernel | dkdv_pair_kernel, D=64, us, at 16 slabs (256 tokens, H=8) values 27 | 31,
+// documents of 300 17 | 21, a causal mask 22 | 25; at 256 (2048, H=16) 168 | 193, 61 | 67, 55 | 104; at 512 (2048, H=32) 329 | 217,
+// 115 | 74, 95 | 104.  D=128 at 256: 192 | 222, 71 | 77, 72 | 122; at 512: 377 | 258, 134 | 87, 125 | 129.
+bool dkdv_on_pair(const ra_bwd_step_params& p) { return (int64_t)p.B * p.H * ((p.Lk + 127) / 128) > 256; }
+// Four and more steps of a single tile of rows and keys stay one launch of the long-stretch kernels, which keep their
+// state in registers from step to step: launching is what such steps cost.  One launch | one per step: ra_fwd_steps, 8 steps of
+// 64 x 64, H=4, D=64: 60 | 76 us, of 128 x 128 80 | 93, of 192 x 192 124 | 118; ra_bwd_dq_steps 64 | 80, 85 | 97, 128 | 122.
+// 4 steps of 128 x 128: 44 | 47, 2 of them 26 | 24.
+template <typename P>
+bool one_tile_steps(const P& p, int n_steps) { return n_steps >= 4 && p.Lq <= 128 && p.Lk <= 128; }
 constexpr int kWholeRow = 1 << 30;  // chunk_tiles of rows that are not shared
 
 int fwd_step_on_pair(const ra_fwd_step_params& p, void* stream) {
@@ -382,7 +393,9 @@ int bwd_step_on_pair(const ra_bwd_step_params& p, int parts, void* stream) {
   a.n_split = 1;
   a.chunk_tiles = kWholeRow;
   hipError_t e = hipSuccess;
-  if (parts & 1) {
+  if ((parts & 1) && !dkdv_on_pair(p)) {
+    e = ra::launch_bwd_step(a.a, p.D, kernel_mode(p.bias.flags), 1, (hipStream_t)stream);
+  } else if (parts & 1) {
     a.acc = p.dk;
     a.acc2 = p.dv;
     e = ra::launch_dkdv_pair(a, p.D, kernel_mode(p.bias.flags), (hipStream_t)stream);
@@ -395,14 +408,12 @@ int bwd_step_on_pair(const ra_bwd_step_params& p, int parts, void* stream) {
   return e == hipSuccess ? RA_OK : hip_fail(e, "backward step launch");
 }
 
-// The steps of a single pass, one launch each, if they take that route (`taken`; all of them do, or none: a
-// pass has one set of bias terms).  The several-step entry points evaluate whole blocks: only the blocks of
+// The steps of a single pass on dense blocks, one launch each.  The several-step entry points evaluate whole blocks: only the blocks of
 // a launch differ from step to step, a summary that travels with them describes one of them at most.
 template <typename P, typename Step>
-int steps_on_pair(const P* steps, int n_steps, bool& taken, Step step) {
-  taken = dense_steps_on_pair(steps[0].bias);
+int steps_on_pair(const P* steps, int n_steps, Step step) {
   int rc = RA_OK;
-  for (int i = 0; taken && i < n_steps && !rc; ++i) {
+  for (int i = 0; i < n_steps && !rc; ++i) {
     P p = steps[i];
     p.bias.dense_map = nullptr;
     rc = step(p);
@@ -435,11 +446,8 @@ int fwd_passes(const ra_fwd_step_params* steps, const std::vector<int>& first, i
                                   "steps[0] in shape, strides or bias terms", i);
     }
   }
-  if (!whole && n_passes == 1) {
-    bool taken;
-    const int rc = steps_on_pair(steps, total, taken, [&](const ra_fwd_step_params& p) { return fwd_step_on_pair(p, stream); });
-    if (taken) return rc;
-  }
+  if (!whole && n_passes == 1 && dense_steps_on_pair(f.bias) && !one_tile_steps(f, total))
+    return steps_on_pair(steps, total, [&](const ra_fwd_step_params& p) { return fwd_step_on_pair(p, stream); });
   ra::FwdArgs a;
   a.q = to_arg(f.q);
   a.k = to_arg(f.k);
@@ -515,11 +523,8 @@ int bwd_dq_passes(const ra_bwd_step_params* steps, const std::vector<int>& first
                                   "steps[0] in shape, strides or bias terms", i);
     }
   }
-  if (!whole && n_passes == 1) {
-    bool taken;
-    const int rc = steps_on_pair(steps, total, taken, [&](const ra_bwd_step_params& p) { return bwd_step_on_pair(p, 2, stream); });
-    if (taken) return rc;
-  }
+  if (!whole && n_passes == 1 && dense_steps_on_pair(f.bias) && !one_tile_steps(f, total))
+    return steps_on_pair(steps, total, [&](const ra_bwd_step_params& p) { return bwd_step_on_pair(p, 2, stream); });
   ra::BwdArgs a = to_bwd_args(f);
   if (whole) {
     a.bias.flags |= ra::kFlagWholeBf16;
@@ -577,11 +582,9 @@ int bwd_dkdv_passes(const ra_bwd_step_params* steps, const std::vector<int>& fir
                                   "steps[0] in shape, strides or bias terms", i);
     }
   }
-  if (!whole && n_passes == 1) {
-    bool taken;
-    const int rc = steps_on_pair(steps, total, taken, [&](const ra_bwd_step_params& p) { return bwd_step_on_pair(p, 1, stream); });
-    if (taken) return rc;
-  }
+  // (few slabs stay one launch: 8 steps of 512 x 512, H=32, D=128: 388 us | 498 on dkdv_pair_kernel; 1024 x 1024, H=64: 1496 | 1149)
+  if (!whole && n_passes == 1 && dense_steps_on_pair(f.bias) && dkdv_on_pair(f))
+    return steps_on_pair(steps, total, [&](const ra_bwd_step_params& p) { return bwd_step_on_pair(p, 1, stream); });
   ra::BwdArgs a = to_bwd_args(f);
   if (whole) {
     a.bias.flags |= ra::kFlagWholeBf16;

@@ -2054,17 +2054,19 @@ hipError_t launch_bwd_delta(const void* out, int out_f32, long long sp, long lon
   return hipGetLastError();
 }
 
-// mode: 0 or 1 (steps on a dense block run on dq_pair_kernel and dkdv_pair_kernel)
+// mode: as for launch_fwd_steps; 2 for dK / dV only (dQ steps on a dense block run on dq_pair_kernel)
 hipError_t launch_bwd_step(const BwdArgs& a, int D, int mode, int parts, hipStream_t stream) {
   if (parts & 1) {
     const int keys_wg = 128;
     const int nkt = (a.Lk + keys_wg - 1) / keys_wg;
     dim3 grid((unsigned)(a.B * a.H * nkt)), block(256);
     if (D == 128) {
-      if (mode == 1) hipLaunchKernelGGL((dkdv_kernel<128, 1, false>), grid, block, 0, stream, a, NoShardList{});
+      if (mode == 2) hipLaunchKernelGGL((dkdv_kernel<128, 2, false>), grid, block, 0, stream, a, NoShardList{});
+      else if (mode == 1) hipLaunchKernelGGL((dkdv_kernel<128, 1, false>), grid, block, 0, stream, a, NoShardList{});
       else hipLaunchKernelGGL((dkdv_kernel<128, 0, false>), grid, block, 0, stream, a, NoShardList{});
     } else {
-      if (mode == 1) hipLaunchKernelGGL((dkdv_kernel<64, 1, false>), grid, block, 0, stream, a, NoShardList{});
+      if (mode == 2) hipLaunchKernelGGL((dkdv_kernel<64, 2, false>), grid, block, 0, stream, a, NoShardList{});
+      else if (mode == 1) hipLaunchKernelGGL((dkdv_kernel<64, 1, false>), grid, block, 0, stream, a, NoShardList{});
       else hipLaunchKernelGGL((dkdv_kernel<64, 0, false>), grid, block, 0, stream, a, NoShardList{});
     }
     hipError_t e = hipGetLastError();

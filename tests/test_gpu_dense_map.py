@@ -280,3 +280,49 @@ def test_several_steps_evaluate_their_blocks_whatever_summary_travels_with_them(
     assert any(bool((x != 0).any()) for x in got[0][:3])
     for x, y in zip(*got):
         assert torch.equal(x, y)
+
+
+def _masked_values(rng, B, Lq, Lk):
+    d = rng.standard_normal((B, 1, Lq, Lk)).astype(np.float32)
+    d[rng.random((B, 1, Lq, Lk)) < 0.3] = -np.inf
+    d[:, :, :, 0] = 0.0  # every row sees a key
+    return d
+
+
+# both sides of the rules that choose kernels for steps on dense blocks: four and more steps of one tile, 256 key slabs
+@pytest.mark.parametrize("L,n,H", [(128, 4, 2), (129, 4, 2), (128, 3, 2), (16, 9, 2), (40, 2, 256), (40, 2, 257)])
+def test_dense_steps_on_both_sides_of_the_kernel_rules(device, L, n, H):
+    B, D, scale = 1, 64, 0.125
+    rng = np.random.default_rng(L + n)
+    q, k, v, do = R.make_inputs(L, B, L, n * L, H, D)
+    hq, hk, hv, hdo = (np.ascontiguousarray(np.transpose(x, (0, 2, 1, 3))) for x in (q, k, v, do))
+    hdo = hdo[:, :, :L]
+    tq, tk, tv, tdo = (_dev(x, device, torch.bfloat16) for x in (hq, hk, hv, hdo))
+    blocks = [_masked_values(rng, B, L, L) for _ in range(n)]
+    biases = [rr.BlockBias(dense=_dev(b, device)) for b in blocks]
+    kv = [(tk[:, :, i * L:(i + 1) * L], tv[:, :, i * L:(i + 1) * L]) for i in range(n)]
+    f64 = lambda x: x.astype(np.float64)
+    hkv = [(f64(hk[:, :, i * L:(i + 1) * L]), f64(hv[:, :, i * L:(i + 1) * L])) for i in range(n)]
+    state = np.zeros((B, H, L, D)), np.full((B, H, L), -np.inf), np.zeros((B, H, L))
+    for (k_, v_), b in zip(hkv, blocks):
+        state = R.fwd_block(f64(hq), k_, v_, f64(b), *state, scale)
+    want, lse = state[0] / state[2][..., None], state[1] + np.log(state[2])
+    o, m, l = rr.fwd_blocks(tq, kv, biases, *rr.init_carry(B, H, L, D, device), scale)
+    assert np.abs((o / l[..., None]).cpu().numpy() - want).max() <= OUT_TOL
+    assert np.abs((m + l.log()).cpu().numpy() - lse).max() <= LSE_TOL
+    grads = [R.bwd_block(f64(hq), k_, v_, f64(b), want, lse, f64(hdo), scale) for (k_, v_), b in zip(hkv, blocks)]
+    tlse = _dev(lse.astype(np.float32), device)
+    delta = _dev((want * f64(hdo)).sum(-1).astype(np.float32), device)
+    zeros = lambda: torch.zeros((B, H, L, D), device=device)
+    dq, dk, dv = zeros(), zeros(), zeros()
+    rr._bwd_steps("dq", [(tq, *x, tdo, tlse, delta, dq, dk, dv, b) for x, b in zip(kv, biases)], scale)
+    assert max(_rel(dq.cpu().numpy(), sum(g[0] for g in grads))) <= GRAD_TOL
+    # the query side travels: the same rows under every block meet the first shard
+    rr._bwd_steps("dkdv", [(tq, *kv[0], tdo, tlse, delta, dq, dk, dv, b) for b in biases], scale)
+    first = [R.bwd_block(f64(hq), *hkv[0], f64(b), want, lse, f64(hdo), scale) for b in blocks]
+    for got, i in ((dk, 1), (dv, 2)):
+        assert max(_rel(got.cpu().numpy(), sum(g[i] for g in first))) <= GRAD_TOL
+    dq, dk, dv = zeros(), zeros(), zeros()
+    rr._bwd_step(tq, *kv[1], tdo, tlse, delta, dq, dk, dv, biases[1], scale)
+    for got, ref in zip((dq, dk, dv), grads[1]):
+        assert max(_rel(got.cpu().numpy(), ref)) <= GRAD_TOL

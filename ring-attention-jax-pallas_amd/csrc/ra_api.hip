@@ -120,6 +120,7 @@ ra::BiasArgs to_bias(const ra_bias& b) {
   r.dense_sh = b.dense_stride_h;
   r.dense_sq = b.dense_stride_q;
   r.dense_map = (b.flags & RA_BIAS_DENSE) ? b.dense_map : nullptr;
+  r.plain_rule = 0;
   return r;
 }
 
@@ -130,6 +131,23 @@ int kernel_mode(int flags) {
 }
 
 constexpr float kLog2eHost = 1.4426950408889634f;
+
+ra::FwdArgs to_fwd_args(const ra_fwd_step_params& p) {
+  ra::FwdArgs a;
+  a.q = to_arg(p.q);
+  a.k = to_arg(p.k);
+  a.v = to_arg(p.v);
+  a.o = p.o;
+  a.m = p.m;
+  a.l = p.l;
+  a.B = p.B;
+  a.H = p.H;
+  a.Lq = p.Lq;
+  a.Lk = p.Lk;
+  a.scale2 = p.sm_scale * kLog2eHost;
+  a.bias = to_bias(p.bias);
+  return a;
+}
 
 ra::BwdArgs to_bwd_args(const ra_bwd_step_params& p) {
   ra::BwdArgs a;
@@ -353,13 +371,28 @@ bool dense_steps_on_pair(const ra_bias& b) { return b.flags & RA_BIAS_DENSE; }
 // and dkdv_kernel the longer pipeline.  dkdv_kernel | dkdv_pair_kernel, D=64, us, at 16 slabs (256 tokens, H=8) values 27 | 31,
 // documents of 300 17 | 21, a causal mask 22 | 25; at 256 (2048, H=16) 168 | 193, 61 | 67, 55 | 104; at 512 (2048, H=32) 329 | 217,
 // 115 | 74, 95 | 104.  D=128 at 256: 192 | 222, 71 | 77, 72 | 122; at 512: 377 | 258, 134 | 87, 125 | 129.
-bool dkdv_on_pair(const ra_bwd_step_params& p) { return (int64_t)p.B * p.H * ((p.Lk + 127) / 128) > 256; }
+int64_t key_slabs(const ra_bwd_step_params& p) { return (int64_t)p.B * p.H * ((p.Lk + 127) / 128); }
+bool dkdv_on_pair(const ra_bwd_step_params& p) { return key_slabs(p) > 256; }
 // Four and more steps of a single tile of rows and keys stay one launch of the long-stretch kernels, which keep their
 // state in registers from step to step: launching is what such steps cost.  One launch | one per step: ra_fwd_steps, 8 steps of
 // 64 x 64, H=4, D=64: 60 | 76 us, of 128 x 128 80 | 93, of 192 x 192 124 | 118; ra_bwd_dq_steps 64 | 80, 85 | 97, 128 | 122.
 // 4 steps of 128 x 128: 44 | 47, 2 of them 26 | 24.
 template <typename P>
 bool one_tile_steps(const P& p, int n_steps) { return n_steps >= 4 && p.Lq <= 128 && p.Lk <= 128; }
+// Blocks of 8192 and more a side (dK and dV: of 4096 too while all slabs have their place at once) that are mostly zeros, tiles
+// without a term to evaluate, are what the long-stretch kernels are faster at, and the pair kernels at all others: there both are
+// launched and the block's summary, if it comes with one, says in every workgroup which of them runs.  The number is mostly_plain's one_in:
+// of a causal mask's cells one in 64 is of another kind at 4096 tokens, one in 128 at 8192, of documents of 2000 tokens one
+// in 30 to 60 at any length.  fwd_step_kernel | fwd_pair_kernel | both launched, us: all zeros 8192, H=16, D=64 409 | 454 | 413, D=128 596 | 667 |
+// 614, a causal mask of 16384, H=8, D=64 394 | 460 | 405; documents of 300 in 8192, H=16, D=64 | 95 | 103.  dkdv_kernel | dkdv_pair_kernel | both:
+// all zeros 8192, H=16, D=64 565 | 838 | 585, D=128 930 | 1115 | 943, a causal mask 344 | 461 | 358 and 526 | 602 | 535, of 4096, H=16, D=64
+// 112 | 192 | 119; documents of 300 in 8192, H=16 181 | 130 | 142.  A training call under a causal mask from a callable, 32768 tokens in 4
+// shards, H=16, D=64: 19.1 ms on the long-stretch kernels, 21.2 on the pair kernels, 19.1 with the choice; under causal documents of 2000 15.1, 13.8, 14.2.
+constexpr int kFwdPlain = 200, kDkdvPlain = 50;
+bool choose_by_content(const ra_bias& b, int64_t workgroups, int Lq, int Lk, bool small) {
+  const int side = std::min(Lq, Lk);
+  return b.dense_map && (side >= 8192 || (small && side >= 4096 && workgroups <= 512));
+}
 constexpr int kWholeRow = 1 << 30;  // chunk_tiles of rows that are not shared
 
 int fwd_step_on_pair(const ra_fwd_step_params& p, void* stream) {
@@ -380,7 +413,14 @@ int fwd_step_on_pair(const ra_fwd_step_params& p, void* stream) {
   a.o = p.o;
   a.m = p.m;
   a.l = p.l;
-  hipError_t e = ra::launch_fwd_pair(a, p.D, kernel_mode(p.bias.flags), (hipStream_t)stream);
+  const int mode = kernel_mode(p.bias.flags), rule = choose_by_content(p.bias, 0, p.Lq, p.Lk, false) ? kFwdPlain : 0;
+  a.bias.plain_rule = -rule;
+  hipError_t e = ra::launch_fwd_pair(a, p.D, mode, (hipStream_t)stream);
+  if (e == hipSuccess && rule) {
+    ra::FwdArgs f = to_fwd_args(p);
+    f.bias.plain_rule = rule;
+    e = ra::launch_fwd_step(f, p.D, mode, (hipStream_t)stream);
+  }
   return e == hipSuccess ? RA_OK : hip_fail(e, "forward step launch");
 }
 
@@ -392,18 +432,25 @@ int bwd_step_on_pair(const ra_bwd_step_params& p, int parts, void* stream) {
   a.a = to_bwd_args(p);
   a.n_split = 1;
   a.chunk_tiles = kWholeRow;
+  const int mode = kernel_mode(p.bias.flags);
   hipError_t e = hipSuccess;
-  if ((parts & 1) && !dkdv_on_pair(p)) {
-    e = ra::launch_bwd_step(a.a, p.D, kernel_mode(p.bias.flags), 1, (hipStream_t)stream);
-  } else if (parts & 1) {
-    a.acc = p.dk;
-    a.acc2 = p.dv;
-    e = ra::launch_dkdv_pair(a, p.D, kernel_mode(p.bias.flags), (hipStream_t)stream);
+  if (parts & 1) {
+    const bool pair = dkdv_on_pair(p);
+    const int rule = pair && choose_by_content(p.bias, key_slabs(p), p.Lq, p.Lk, true) ? kDkdvPlain : 0;
+    if (pair) {
+      a.acc = p.dk;
+      a.acc2 = p.dv;
+      a.a.bias.plain_rule = -rule;
+      e = ra::launch_dkdv_pair(a, p.D, mode, (hipStream_t)stream);
+      a.a.bias.plain_rule = rule;
+    }
+    if (e == hipSuccess && (!pair || rule)) e = ra::launch_bwd_step(a.a, p.D, mode, 1, (hipStream_t)stream);
+    a.a.bias.plain_rule = 0;
   }
   if (e == hipSuccess && (parts & 2)) {
     a.acc = p.dq;
     a.acc2 = nullptr;
-    e = ra::launch_dq_pair(a, p.D, kernel_mode(p.bias.flags), (hipStream_t)stream);
+    e = ra::launch_dq_pair(a, p.D, mode, (hipStream_t)stream);
   }
   return e == hipSuccess ? RA_OK : hip_fail(e, "backward step launch");
 }
@@ -448,19 +495,7 @@ int fwd_passes(const ra_fwd_step_params* steps, const std::vector<int>& first, i
   }
   if (!whole && n_passes == 1 && dense_steps_on_pair(f.bias) && !one_tile_steps(f, total))
     return steps_on_pair(steps, total, [&](const ra_fwd_step_params& p) { return fwd_step_on_pair(p, stream); });
-  ra::FwdArgs a;
-  a.q = to_arg(f.q);
-  a.k = to_arg(f.k);
-  a.v = to_arg(f.v);
-  a.o = f.o;
-  a.m = f.m;
-  a.l = f.l;
-  a.B = f.B;
-  a.H = f.H;
-  a.Lq = f.Lq;
-  a.Lk = f.Lk;
-  a.scale2 = f.sm_scale * kLog2eHost;
-  a.bias = to_bias(f.bias);
+  ra::FwdArgs a = to_fwd_args(f);
   if (whole) {
     a.bias.flags |= whole->dtype == RA_DTYPE_F32 ? ra::kFlagWholeF32 : ra::kFlagWholeBf16;
     a.out_sb = whole->stride_b;  // in the slots of the carry pointers, which have no use here
@@ -886,19 +921,7 @@ int ra_fwd_step(const ra_fwd_step_params* p, void* stream) {
   if (rc) return rc;
   if (dense_steps_on_pair(p->bias)) return fwd_step_on_pair(*p, stream);
   if (ra_step_is_skippable(&p->bias, p->Lq, p->Lk)) return RA_OK;  // identity on the carry
-  ra::FwdArgs a;
-  a.q = to_arg(p->q);
-  a.k = to_arg(p->k);
-  a.v = to_arg(p->v);
-  a.o = p->o;
-  a.m = p->m;
-  a.l = p->l;
-  a.B = p->B;
-  a.H = p->H;
-  a.Lq = p->Lq;
-  a.Lk = p->Lk;
-  a.scale2 = p->sm_scale * kLog2eHost;
-  a.bias = to_bias(p->bias);
+  const ra::FwdArgs a = to_fwd_args(*p);
   hipError_t e = ra::launch_fwd_step(a, p->D, kernel_mode(p->bias.flags), (hipStream_t)stream);
   return e == hipSuccess ? RA_OK : hip_fail(e, "ra_fwd_step launch");
 }

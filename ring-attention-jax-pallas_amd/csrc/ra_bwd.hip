@@ -113,6 +113,9 @@ __global__ __launch_bounds__(256) void dkdv_kernel(
   const int kw = k0 + wave * 32;
   const BiasArgs& bs = a.bias;
   const int flags = bs.flags;
+  if constexpr (DENSE && !MULTI) {
+    if (left_to_the_other<NT>(bs, b, h, a.H, a.Lq, a.Lk, s_red)) return;
+  }
   const bool wave_on = kw < a.Lk;
   // the key/value side of this workgroup's pass
   auto pass_kv_off = [&]() -> int { if constexpr (MULTI) return ring.kv_off[blockIdx.y]; else return bs.kv_off; };
@@ -1250,48 +1253,27 @@ __global__ __launch_bounds__(kDqThreads) void dq_kernel(
   int cons_hi = n_act, cons2_hi = 0;
   bool wg_one_doc = true;
   const bool seg_on = GENERAL && (flags & RA_BIAS_SEGMENT);
-  // A dense block that comes with its summary is listed the same way: tiles in which the
-  // workgroup's rows hold nothing but -inf are left out, tiles of zeros have no term to evaluate,
-  // the rest is evaluated element by element.  (Single-step launches only.)
-  const unsigned char* dmap = nullptr;
-  if constexpr (DENSE && !MULTI) {
-    if (bs.dense_map) dmap = dense_map_of(bs, b, h, a.H, a.Lq, a.Lk);
-  }
-  if ((GENERAL && (flags & RA_BIAS_SEGMENT)) || (DENSE && dmap != nullptr)) {
+  if (seg_on) {
     use_list = true;
-    int qmin = 0, qmax = 0;
-    if (seg_on) {
-      int smin = q_valid ? q_seg : 0x7fffffff, smax = q_valid ? q_seg : (int)0x80000000;
-      smin = wave_min(smin);
-      smax = wave_max(smax);
-      if (lane == 0) {
-        s_red[wave] = smin;
-        s_red[8 + wave] = smax;
-      }
-      __syncthreads();
-      qmin = s_red[0];
-      qmax = s_red[8];
+    int smin = q_valid ? q_seg : 0x7fffffff, smax = q_valid ? q_seg : (int)0x80000000;
+    smin = wave_min(smin);
+    smax = wave_max(smax);
+    if (lane == 0) {
+      s_red[wave] = smin;
+      s_red[8 + wave] = smax;
+    }
+    __syncthreads();
+    int qmin = s_red[0], qmax = s_red[8];
 #pragma unroll
-      for (int w = 1; w < 8; ++w) {
-        qmin = min(qmin, s_red[w]);
-        qmax = max(qmax, s_red[8 + w]);
-      }
+    for (int w = 1; w < 8; ++w) {
+      qmin = min(qmin, s_red[w]);
+      qmax = max(qmax, s_red[8 + w]);
     }
     for (int j = j_lo + tid; j < j_hi; j += kDqThreads) {
-      int f = 1;
-      if (seg_on) {
-        int kmin, kmax;
-        tile_id_range<kDqKeyTile>(kv_seg, j, a.Lk, kmin, kmax);
-        const bool act = !(kmax < qmin || kmin > qmax);
-        f = act ? ((kmin == kmax) ? 1 : 3) : 0;
-      }
-      if constexpr (DENSE) {
-        if (dmap != nullptr && f != 0) {
-          const int bits = dense_map_or(dmap, a.Lk, q0, q_rows_hi, j * kDqKeyTile, min((j + 1) * kDqKeyTile, a.Lk) - 1);
-          f = (bits & kMapLive) ? ((bits & kMapNonZero) ? 3 : f) : 0;
-        }
-      }
-      s_flag[j - j_lo] = f;
+      int kmin, kmax;
+      tile_id_range<kDqKeyTile>(kv_seg, j, a.Lk, kmin, kmax);
+      const bool act = !(kmax < qmin || kmin > qmax);
+      s_flag[j - j_lo] = act ? ((kmin == kmax) ? 1 : 3) : 0;
     }
     wg_one_doc = qmin == qmax;
     __syncthreads();
@@ -1425,12 +1407,8 @@ __global__ __launch_bounds__(kDqThreads) void dq_kernel(
     return classify_pos(flags, bs.window, q_off + qw, q_off + qw + 31, kv_off + kt0,
                         kv_off + kt0 + kDqKeyTile - 1);
   };
-  // terms that every tile must evaluate; a dense block with a summary is read only in the tiles
-  // that the list marks (segbit)
-  int tile_terms = RA_BIAS_ALIBI | RA_BIAS_PREFIX | RA_BIAS_DENSE;
-  if constexpr (DENSE) {
-    if (dmap != nullptr) tile_terms &= ~RA_BIAS_DENSE;
-  }
+  // terms that every tile must evaluate
+  constexpr int tile_terms = RA_BIAS_ALIBI | RA_BIAS_PREFIX | RA_BIAS_DENSE;
   auto needs_bias = [&](int kt0, int segbit, int cls) -> bool {
     bool nb = (cls & 2) || (kt0 + kDqKeyTile > a.Lk);
     if (GENERAL) nb = nb || (flags & tile_terms) || segbit;
@@ -1480,7 +1458,7 @@ __global__ __launch_bounds__(kDqThreads) void dq_kernel(
     tb.flags = (cls & 2) ? (flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) : 0;
     if (GENERAL) {
       tb.flags |= flags & tile_terms;
-      if (segbit) tb.flags |= DENSE ? (flags & (RA_BIAS_SEGMENT | RA_BIAS_DENSE)) : RA_BIAS_SEGMENT;
+      if (segbit) tb.flags |= RA_BIAS_SEGMENT;
     }
     tb.window = bs.window;
     tb.slope2 = slope2;

@@ -44,6 +44,9 @@ struct BiasArgs {
   // bit 0 = the cell holds a value other than -inf, bit 1 = it holds a value other than 0;
   // [B|1, H|1, ceil(Lq / 32), ceil(Lk / 32)], broadcast like the block itself
   const unsigned char* dense_map;
+  // A step with a summary that is launched on both kinds of kernel: > 0 = run if the block is mostly plain by this
+  // measure (see mostly_plain), < 0 = run if it is not, 0 = run.
+  int plain_rule;
 };
 
 constexpr int kMapCell = 32;  // queries and keys per cell of a dense block's summary
@@ -63,6 +66,49 @@ RA_DEV int dense_map_or(const unsigned char* mp, int Lk, int q_lo, int q_hi, int
   for (int r = q_lo / kMapCell; r <= q_hi / kMapCell; ++r)
     for (int c = k_lo / kMapCell; c <= k_hi / kMapCell; ++c) bits |= mp[(long long)r * ncols + c];
   return bits;
+}
+
+// Whether fewer than one in `one_in` of the live cells of a summary holds a value other than 0, in a sample of
+// whole rows of cells, about 1024 cells or one row.  The same sample and answer in every workgroup of every
+// kernel.  Called by all NT threads; red: two words per wave.
+template <int NT>
+RA_DEV bool mostly_plain(const unsigned char* mp, int Lq, int Lk, int one_in, int* red) {
+  const int rows = (Lq + kMapCell - 1) / kMapCell, cols = (Lk + kMapCell - 1) / kMapCell;
+  const int every = max(1, min(rows, rows * cols / 1024)), first = every / 2;
+  const int n = (rows - first + every - 1) / every * cols;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int live = 0, other = 0;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < n; i += NT) {
+    const int r = i / cols;
+    const int c = mp[(long long)(first + r * every) * cols + (i - r * cols)];
+    live += c & kMapLive;
+    other += c == (kMapLive | kMapNonZero);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    live += __shfl_xor(live, o, 64);
+    other += __shfl_xor(other, o, 64);
+  }
+  if (lane == 0) {
+    red[2 * wave] = live;
+    red[2 * wave + 1] = other;
+  }
+  __syncthreads();
+  live = other = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) {
+    live += red[2 * w];
+    other += red[2 * w + 1];
+  }
+  __syncthreads();
+  return (long long)other * one_in < live;
+}
+// ... and whether a kernel of that kind leaves a step to the other one.
+template <int NT>
+RA_DEV bool left_to_the_other(const BiasArgs& bs, int b, int h, int H, int Lq, int Lk, int* red) {
+  if (bs.plain_rule == 0) return false;
+  return mostly_plain<NT>(dense_map_of(bs, b, h, H, Lq, Lk), Lq, Lk, abs(bs.plain_rule), red) != (bs.plain_rule > 0);
 }
 
 struct TensorArg {

@@ -79,6 +79,9 @@ __global__ __launch_bounds__(kFwdThreads) void fwd_step_kernel(
   const int qi_c = min(qi, a.Lq - 1);
   const BiasArgs& bs = a.bias;
   const int flags = bs.flags;
+  if constexpr (DENSE && !MULTI) {
+    if (left_to_the_other<kFwdThreads>(bs, b, h, a.H, a.Lq, a.Lk, s_red)) return;
+  }
   // the query side of this workgroup's pass (read from the argument block where it is needed:
   // nothing of it is carried through the loops)
   auto pass_q_off = [&]() -> int { if constexpr (MULTI) return ring.q_off[blockIdx.y]; else return bs.q_off; };
@@ -1333,29 +1336,18 @@ __global__ void fwd_finalize_kernel(const float* o, const float* m, const float*
 // ------------------------------------------------------------------------------------------------
 namespace ra {
 
-// mode: 0 = causal / window terms only, 1 = any of the per-tile terms, 2 = a dense bias block too (MULTI only:
-// single steps on a dense block run on fwd_pair_kernel)
+// mode: 0 = causal / window terms only, 1 = any of the per-tile terms, 2 = a dense bias block too
 template <bool MULTI, bool WHOLE, typename Shards>
 static hipError_t launch_fwd(const FwdArgs& a, const Shards& sl, int n_pass, int D, int mode, hipStream_t stream) {
   const int nqt = (a.Lq + kFwdRows - 1) / kFwdRows;
   dim3 grid((unsigned)(a.B * a.H * nqt), (unsigned)n_pass), block(kFwdThreads);
   if (D == 128) {
-    if constexpr (MULTI) {
-      if (mode == 2) {
-        hipLaunchKernelGGL((fwd_step_kernel<128, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
-        return hipGetLastError();
-      }
-    }
-    if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<128, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+    if (mode == 2) hipLaunchKernelGGL((fwd_step_kernel<128, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+    else if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<128, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
     else hipLaunchKernelGGL((fwd_step_kernel<128, 0, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
   } else {
-    if constexpr (MULTI) {
-      if (mode == 2) {
-        hipLaunchKernelGGL((fwd_step_kernel<64, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
-        return hipGetLastError();
-      }
-    }
-    if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<64, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+    if (mode == 2) hipLaunchKernelGGL((fwd_step_kernel<64, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+    else if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<64, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
     else hipLaunchKernelGGL((fwd_step_kernel<64, 0, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
   }
   return hipGetLastError();

@@ -229,6 +229,9 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   const int qi_c = min(qi, a.Lq - 1);
   const BiasArgs& bs = a.bias;
   const int flags = bs.flags;
+  if constexpr (DENSE) {
+    if (left_to_the_other<kPairThreads>(bs, b, h, a.H, a.Lq, a.Lk, s_red)) return;
+  }
   const int q_off = bs.q_off, kv_off = bs.kv_off;
 
   // ---- the key tiles of this workgroup ----------------------------------------------------------
@@ -976,6 +979,9 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
   const int ki_c = min(ki, a.Lk - 1);
   const BiasArgs& bs = a.bias;
   const int flags = bs.flags;
+  if constexpr (DENSE) {
+    if (left_to_the_other<kPairThreads>(bs, b, h, a.H, a.Lq, a.Lk, s_red)) return;
+  }
   const int q_off = bs.q_off, kv_off = bs.kv_off;
 
   const int ntiles = (a.Lq + kPairQueries - 1) / kPairQueries;

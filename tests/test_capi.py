@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from oracle import ring_oracle as R
-from ring_attention import _lib
+from ring_attention import _lib, ring
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "ring_attention_hip.h")
@@ -273,6 +273,77 @@ def test_multi_step_entry_points_validate_before_any_gpu_call(lib):
         assert fn(arr, 2, None) == 0
 
 
+def _pair_fwd(lib, mutate=None, **kw):
+    p = _good_fwd()
+    p.o = p.m = p.l = None  # not used
+    if mutate:
+        mutate(p)
+    a = {**dict(out=0x1000, dtype=_lib.RA_DTYPE_BF16, sb=64 * 256, sh=128, sl=256, lse=0x2000, ws=0x3000, size=1 << 30), **kw}
+    return lib.ra_fwd_pair(C.byref(p), a["out"], a["dtype"], a["sb"], a["sh"], a["sl"], a["lse"], a["ws"], a["size"], None)
+
+
+def test_fwd_pair_rejects_bad_arguments_without_a_gpu(lib):
+    def long(p):  # 1 x 2 heads of 64 rows against 4096 keys: shared by several workgroups
+        p.Lk = 4096
+
+    assert lib.ra_fwd_pair(None, 0x1000, 0, 8, 8, 8, 0x2000, None, 0, None) == -1
+    for kw, code in ((dict(out=None), -1), (dict(lse=None), -1), (dict(dtype=5), -7), (dict(dtype=_lib.RA_DTYPE_F16), -7),
+                     (dict(out=0x1004), -4), (dict(out=0x1008, dtype=_lib.RA_DTYPE_F32), -4), (dict(sl=254), -4),
+                     (dict(mutate=lambda p: setattr(p, "D", 96)), -3), (dict(mutate=lambda p: setattr(p.k, "ptr", None)), -1),
+                     (dict(mutate=lambda p: setattr(p.bias, "flags", 64)), -5),
+                     (dict(mutate=long, ws=None), -4), (dict(mutate=long, ws=0x3008), -4), (dict(mutate=long, size=1000), -2)):
+        assert _pair_fwd(lib, **kw) == code, kw
+        assert lib.ra_last_error() != b""
+    p = _good_fwd()
+    assert lib.ra_fwd_pair_workspace(C.byref(p)) == 0
+    long(p)
+    size = lib.ra_fwd_pair_workspace(C.byref(p))
+    assert size > 0 and size % 4 == 0
+    assert _pair_fwd(lib, mutate=long, size=size - 1) == -2
+    p.D = 96
+    assert lib.ra_fwd_pair_workspace(C.byref(p)) == 0 and lib.ra_fwd_pair_workspace(None) == 0
+
+
+def test_bwd_pair_rejects_bad_arguments_without_a_gpu(lib):
+    good = dict(out=0x1000, dtype=_lib.RA_DTYPE_BF16, os=(64 * 128, 64, 128), dq=0x4000, qs=(64 * 128, 64, 128), dk=0x5000, dv=0x6000,
+                ks=(64 * 128, 64, 128), ws=0x7000, size=1 << 30)
+
+    def call(mutate=None, **kw):
+        p = _good_bwd()
+        p.delta = p.dq = p.dk = p.dv = None  # not used
+        if mutate:
+            mutate(p)
+        a = {**good, **kw}
+        return lib.ra_bwd_pair(C.byref(p), a["out"], a["dtype"], *a["os"], a["dq"], *a["qs"], a["dk"], a["dv"], *a["ks"], a["ws"],
+                               a["size"], None)
+
+    need = lib.ra_bwd_pair_workspace(C.byref(_good_bwd()))
+    assert need >= 12 * 2 * 64 and lib.ra_bwd_pair_workspace(None) == 0
+    for kw, code in ((dict(out=None), -4), (dict(out=0x1008), -4), (dict(os=(64 * 128, 60, 128)), -4), (dict(dtype=3), -7),
+                     (dict(dtype=_lib.RA_DTYPE_F16), -7), (dict(dq=None), -1), (dict(dk=None), -1), (dict(dv=None), -1),
+                     (dict(dq=0x4004), -4), (dict(dv=0x6004), -4), (dict(ks=(64 * 128, 64, 126)), -4), (dict(ws=None), -4),
+                     (dict(ws=0x7008), -4), (dict(size=need - 1), -2), (dict(mutate=lambda p: setattr(p, "lse", None)), -1),
+                     (dict(mutate=lambda p: setattr(p.dout, "stride_h", 3)), -4), (dict(mutate=lambda p: setattr(p, "Lk", 0)), -2)):
+        assert call(**kw) == code, kw
+        assert lib.ra_last_error() != b""
+
+
+def _rows(**kw):
+    a = {**dict(src=0x1000, dst=0x2000, sd=_lib.RA_DTYPE_F32, dd=_lib.RA_DTYPE_BF16, d=96, to=128, B=1, L=4, H=2), **kw}
+    return ring._ROWS.pack(a["src"], a["dst"], a["sd"], a["dd"], a["d"], a["to"], a["B"], a["L"], a["H"], 0, 192, 96, 0, 256, 128)
+
+
+def test_convert_rejects_bad_arguments_without_a_gpu(lib):
+    assert lib.ra_convert(None, 1, None) == -1
+    for n in (0, -1, _lib.RA_MAX_CONVERT + 1):
+        assert lib.ra_convert(_rows() * 5, n, None) == -2
+    for kw, code in ((dict(src=0), -1), (dict(dst=0), -1), (dict(B=0), -2), (dict(L=-1), -2), (dict(H=0), -2), (dict(d=0), -2),
+                     (dict(to=129), -3), (dict(d=256), -3), (dict(sd=3), -7), (dict(dd=-1), -7), (dict(src=0x1002), -4),
+                     (dict(dst=0x2001), -4), (dict(B=65536), -8), (dict(L=1 << 26), -8), (dict(H=1 << 27), -8)):
+        assert lib.ra_convert(_rows(**kw), 1, None) == code, kw
+        assert lib.ra_convert(_rows() + _rows(**kw), 2, None) == code, kw  # every array is checked before anything is launched
+
+
 def test_header_is_plain_c(tmp_path):
     """include/ring_attention_hip.h must compile as C99 on its own (no HIP, no C++)."""
     import shutil
@@ -281,7 +352,9 @@ def test_header_is_plain_c(tmp_path):
     if gcc is None:
         pytest.skip("no gcc")
     src = tmp_path / "hdr.c"
-    src.write_text('#include "ring_attention_hip.h"\n'
+    src.write_text('#include "ring_attention_hip.h"\n#include <stddef.h>\n'
+                   f"typedef char size_of_ra_rows[sizeof(ra_rows) == {ring._ROWS.size} ? 1 : -1];\n"
+                   "typedef char place_of_strides[offsetof(ra_rows, src_stride_b) == 48 ? 1 : -1];\n"
                    "int main(void) { ra_fwd_step_params p; (void)p; return RA_OK; }\n")
     res = subprocess.run([gcc, "-std=c99", "-Wall", "-Wextra", "-pedantic", "-Werror", "-fsyntax-only",
                           "-I", os.path.join(ROOT, "include"), str(src)], capture_output=True, text=True)

@@ -2,15 +2,17 @@
 edges of their 128-row and 64-key tiles, single rows, rows whose keys several workgroups share (evenly, and
 under masks that leave rows of different lengths, down to none), every bias term on the tile lists, and key
 sequences longer than a list.  Tolerances as in test_gpu_parity.py."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 import ring_attention as ra
-from ring_attention import bias as bias_module
+from ring_attention import _lib, bias as bias_module, ring as rr
 from oracle import ring_oracle as R
 from test_gpu_dense_map import _both_ways
-from test_gpu_parity import _check
+from test_gpu_parity import GRAD_TOL, LSE_TOL, OUT_TOL, _check, _dev, _rel
 
 pytestmark = pytest.mark.gpu
 
@@ -90,12 +92,69 @@ def test_pair_kernels_take_single_steps_on_dense_blocks(device, monkeypatch, Sq,
                {"kv_segment_ids": k_ids}, seed=Sq)
 
 
-def test_a_repeated_call_reads_nothing_of_the_one_before(device):
-    # the workspace of shared rows comes back from the allocator with the last call's partial results
-    q, k, v, _ = (torch.from_numpy(x).to(device, torch.bfloat16) for x in R.make_inputs(1, 1, 300, 300, 2, 64))
-    first = ra.ring_attention(q, k, v, 1, ra.causal_bias())
-    ra.ring_attention(*(torch.full_like(x, float("nan")) for x in (q, k, v)), 1, ra.causal_bias())
-    assert torch.equal(ra.ring_attention(q, k, v, 1, ra.causal_bias()), first)
+def _spaces(Sq, Sk, H, D, flags):
+    """The workspaces of a forward and a backward call (B = 1) in bytes."""
+    f, b = _lib.RaFwdStepParams(), _lib.RaBwdStepParams()
+    for p in (f, b):
+        p.B, p.H, p.Lq, p.Lk, p.D, p.sm_scale, p.bias.flags = 1, H, Sq, Sk, D, 0.1, flags
+    return _lib.load().ra_fwd_pair_workspace(C.byref(f)), _lib.load().ra_bwd_pair_workspace(C.byref(b))
+
+
+# rows of q and of k that share their work; q alone; k alone
+@pytest.mark.parametrize("Sq,Sk,causal", [(2048, 2048, True), (64, 4096, False), (4096, 64, False)])
+def test_a_repeated_call_reads_nothing_of_the_one_before(device, Sq, Sk, causal):
+    # the workspaces come back from the allocator with the last call's statistics and partial results
+    H, D = 2, 64
+    forward, backward = _spaces(Sq, Sk, H, D, _lib.RA_BIAS_CAUSAL if causal else 0)
+    assert (forward > 0) == (Sk > 64)
+    shares = (8 * Sq * (Sk > 64) + 16 * Sk * (Sq > 64)) * H * D  # two shares of dq, of dk and dv, at least
+    assert backward >= 12 * H * Sq + shares
+    q, k, v, do = (torch.from_numpy(x).to(device, torch.bfloat16) for x in R.make_inputs(1, 1, Sq, Sk, H, D))
+
+    def call(*inputs):
+        q, k, v, do = inputs
+        q, k, v = (x.clone().requires_grad_(True) for x in (q, k, v))
+        out, lse = ra.ring_attention_with_lse(q, k, v, 1, ra.causal_bias() if causal else None)
+        return out.detach(), lse, *torch.autograd.grad(out, (q, k, v), do)
+
+    first = call(q, k, v, do)
+    call(*(torch.full_like(x, float("nan")) for x in (q, k, v, do)))
+    for a, b in zip(call(q, k, v, do), first):
+        assert torch.isfinite(b).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("Lq,Lk,D,summary", [(100, 3000, 64, True), (3000, 100, 128, True), (1000, 1000, 128, False)])
+def test_finished_pairs_on_a_dense_block(device, Lq, Lk, D, summary):
+    """ra_fwd_pair and ra_bwd_pair with RA_BIAS_DENSE, rows or keys shared, against the oracle."""
+    H, scale = 2, 1 / np.sqrt(D)
+    rng = np.random.default_rng(Lq)
+    q, k, v, do = R.make_inputs(Lq, 1, Lq, Lk, H, D)
+    block = rng.standard_normal((1, 1, Lq, Lk)).astype(np.float32)
+    block[:, :, :, Lk // 3: Lk // 2] = -np.inf
+    block[:, :, Lq // 2:] = 0.0
+    tq, tk, tv, tdo = (_dev(x, device, torch.bfloat16) for x in (q, k, v, do))
+    out, lse = torch.empty((1, Lq, H, D), device=device), torch.empty((1, H, Lq), device=device)
+    grads = [torch.empty_like(x) for x in (tq, tk, tv)]
+    lib, view = _lib.load(), rr._view_blhd
+    dense = rr.BlockBias(dense=_dev(block, device))
+    bias = dense.to_struct(tq.device, summary=summary)
+    f = _lib.RaFwdStepParams(1, H, Lq, Lk, D, scale, view(tq), view(tk), view(tv), None, None, None, bias)
+    size = lib.ra_fwd_pair_workspace(C.byref(f))
+    b = _lib.RaBwdStepParams(1, H, Lq, Lk, D, scale, view(tq), view(tk), view(tv), view(tdo), lse.data_ptr(), None, None, None,
+                             None, bias)
+    size_b = lib.ra_bwd_pair_workspace(C.byref(b))
+    assert size_b > 12 * H * Lq and (size > 0) == (Lk > 500)
+    ws = torch.empty((max(size, size_b),), dtype=torch.uint8, device=device)
+    _lib.check("ra_fwd_pair", lib.ra_fwd_pair(C.byref(f), out.data_ptr(), _lib.RA_DTYPE_F32, Lq * H * D, D, H * D, lse.data_ptr(),
+                                              ws.data_ptr(), size, None))
+    _lib.check("ra_bwd_pair", lib.ra_bwd_pair(
+        C.byref(b), out.data_ptr(), _lib.RA_DTYPE_F32, Lq * H * D, D, H * D, grads[0].data_ptr(), Lq * H * D, D, H * D,
+        grads[1].data_ptr(), grads[2].data_ptr(), Lk * H * D, D, H * D, ws.data_ptr(), size_b, None))
+    torch.cuda.synchronize()
+    want, want_lse = R.mha_dense(q, k, v, block)
+    assert np.abs(out.cpu().numpy() - want).max() <= OUT_TOL and np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_TOL
+    for got, ref in zip(grads, R.mha_dense_grads(q, k, v, do, block)):
+        assert max(_rel(got.float().cpu().numpy(), ref)) <= GRAD_TOL
 
 
 @pytest.mark.parametrize("summary", [True, False])

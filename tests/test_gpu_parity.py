@@ -620,9 +620,29 @@ def _fused_cases():
 
 @pytest.mark.parametrize("name", sorted(_fused_cases()))
 def test_fused_ring_pass(device, name):
-    """block_impl="hip_fused": all ring passes in one launch, the kernels walk the shards
-    themselves.  Same oracle, same tolerances as the launch-per-step path."""
+    """block_impl="hip_fused": consecutive shards are joined and launched as one pair.  Same oracle,
+    same tolerances as the launch-per-step path."""
     _check(device, "fused " + name, impl="hip_fused", **_fused_cases()[name])
+
+
+@pytest.mark.parametrize("name", sorted(_fused_cases()))
+def test_whole_ring_launches_walk_the_shards(device, monkeypatch, name):
+    """The same cases with their shards left apart (calls join consecutive shards to one pair, which has kernels of its
+    own): what shards with gaps between their positions and long rings under a segment term run on.  Twenty shards are
+    more than a launch of finished passes takes and go through the split entry points."""
+    case = _fused_cases()[name]
+    monkeypatch.setattr(rr._RingPlan, "joined", lambda plan: plan)
+    for fn in ("_pair_forward", "_pair_backward"):
+        monkeypatch.setattr(rr, fn, None)
+    tried = []
+    check = rr._lib.check
+    monkeypatch.setattr(rr._lib, "check", lambda what, rc: (tried.append(what), check(what, rc))[1])
+    rr.clear_plan_cache()
+    _check(device, "whole ring " + name, impl="hip_fused", **case)
+    rr.clear_plan_cache()
+    split = case["n"] > 16
+    assert ("ra_fwd_passes" in tried) == split == ("ra_bwd_dkdv_passes" in tried)
+    assert ("ra_fwd_ring" in tried) != split and ("ra_bwd_dq_ring" in tried) != split
 
 
 def test_pass_entry_points_equal_launches_per_pass(device):

@@ -122,11 +122,12 @@ typedef struct ra_bias {
   /* Optional (NULL: none) with RA_BIAS_DENSE: the block's summary as written by ra_dense_map().
    * The reference hands its kernels the whole block and they read all of it
    * (ring_kernel.py:75-85); the blocks a bias_fn returns are mostly masks (ring_test.py:226-246:
-   * 0 or -inf), so ra_fwd_step / ra_bwd_step take the summary to leave out the tiles whose part of
-   * the block is -inf throughout (they contribute exp(-inf) = 0, exactly) and to read the block
-   * only in tiles that hold a value other than 0.  Results are those without a summary.  It must
-   * describe this block (same strides and shape); the several-step entry points evaluate the
-   * whole block and do not read it.  Shards of at most RA_MAX_SEGMENT_SHARD tokens. */
+   * 0 or -inf), so ra_fwd_step / ra_bwd_step and ra_fwd_pair / ra_bwd_pair take the summary to leave out
+   * the tiles whose part of the block is -inf throughout (they contribute exp(-inf) = 0, exactly), to
+   * read the block only in tiles that hold a value other than 0, and to choose between kernels for a
+   * large block.  Results are those without a summary, up to rounding.  It must
+   * describe this block (same strides and shape); the several-step and whole-ring entry points evaluate
+   * the whole block and do not read it.  Shards of at most RA_MAX_SEGMENT_SHARD tokens. */
   const uint8_t* dense_map;
 } ra_bias;
 

@@ -1346,7 +1346,7 @@ __global__ __launch_bounds__(256) void pair_stat_kernel(const OutT* out, long lo
   }
 }
 
-// Sum of the shares of rows that were split, added to an accumulator or stored as bf16.
+// Sum of the shares of rows that were split, stored as bf16.
 // `n_out` results of the same rows (dK and dV) lie one after another in a share; grid dimension y.
 template <int D, int ROWS>
 __global__ __launch_bounds__(256) void pair_sum_kernel(const PairBwdArgs p, int n_out, int BH, int H, int L) {
@@ -1361,9 +1361,7 @@ __global__ __launch_bounds__(256) void pair_sum_kernel(const PairBwdArgs p, int 
   f32x4 x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int s = 0; s < n_piece; ++s) x += *(const f32x4*)(p.part + (((long long)s * n_out + which) * rows + row) * D + 4 * c);
-  float* acc = which ? p.acc2 : p.acc;
-  if (acc != nullptr) *(f32x4*)(acc + row * D + 4 * c) += x;
-  else store4(which ? p.out2 : p.out, 0, (hh / H) * p.out_sb + (hh % H) * p.out_sh + (long long)li * p.out_sl + 4 * c, x);
+  store4(which ? p.out2 : p.out, 0, (hh / H) * p.out_sb + (hh % H) * p.out_sh + (long long)li * p.out_sl + 4 * c, x);
 }
 
 template <int D, int ROWS>

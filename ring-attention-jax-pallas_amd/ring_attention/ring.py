@@ -102,14 +102,11 @@ def _stream() -> C.c_void_p:
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
-_ONE_STEP = (C.c_int32 * 1)(1)  # steps_per_pass of a launch with a single pass of a single step
-
-
 @functools.lru_cache(maxsize=64)
-def _array_type(struct, size: int):
-    """``struct * size``.  ctypes holds array types by weak reference only and builds a dropped one
+def _array_type(block, size: int):
+    """``block * size``.  ctypes holds array types by weak reference only and builds a dropped one
     again (35 us each, five of them per forward + backward)."""
-    return struct * size
+    return block * size
 
 
 def _require_gpu(t: torch.Tensor) -> None:
@@ -182,8 +179,8 @@ def _kernel_inputs(tensors, d: int):
 def _bias_struct(bias, device, shape=None, summary=True) -> _lib.RaBias:
     """``bias`` is None, a ``BlockBias`` or a dense additive array ``[b, h | 1, lq, lk]`` - the
     form the reference's block functions take (ring_kernel.py:127,206).  ``summary``: a dense
-    block travels with its summary (``ra_dense_map``); the single-step launches read it, the
-    several-step launches do not, so their callers pass False."""
+    block travels with its summary (``ra_dense_map``); the single-step entry points read it, the
+    several-step ones evaluate whole blocks, so their callers pass False."""
     if bias is None:
         return _lib.RaBias()
     if isinstance(bias, torch.Tensor):
@@ -234,10 +231,11 @@ def _fwd_params(q, k, v, bias, o, m, l, sm_scale, summary=False) -> _lib.RaFwdSt
 
 
 def fwd_blocks(q, kvs, biases, o, m, l, sm_scale: float):
-    """Several consecutive ring steps of one query shard in ONE launch: equivalent to
+    """Several consecutive ring steps of one query shard in one call: equivalent to
     ``fwd_block(q, k, v, bias, o, m, l, sm_scale)`` for every ``(k, v)`` of ``kvs`` with the bias
-    of the same index, in that order (the loop ring.py:104-132), with the step's running state
-    kept in registers between the shards.  The shards share their shape and strides."""
+    of the same index, in that order (the loop ring.py:104-132).  One launch with the step's running
+    state in registers between the shards, or, on dense blocks of more than a tile, one launch per step
+    through the carry; dense blocks are read whole.  The shards share their shape and strides."""
     _require_gpu(q)
     lib = _lib.load()
     steps = _array_type(_lib.RaFwdStepParams, len(kvs))()
@@ -317,7 +315,8 @@ def _bwd_step(q, k, v, do, lse, delta, dq, dk, dv, bias, sm_scale, parts=3):
 def _bwd_steps(which: str, step_args, sm_scale):
     """``step_args``: one ``(q, k, v, do, lse, delta, dq, dk, dv, bias)`` tuple per ring step, as
     for ``_bwd_step``; ``which`` is ``"dq"`` (one query shard, several key/value shards) or
-    ``"dkdv"`` (one key/value shard, several query shards).  One launch for all of them."""
+    ``"dkdv"`` (one key/value shard, several query shards).  One launch for all of them or, on dense
+    blocks, one per step where that is faster (see ``fwd_blocks``)."""
     lib = _lib.load()
     steps = _array_type(_lib.RaBwdStepParams, len(step_args))()
     keep = []  # the bias structs point into tensors that must outlive the call
@@ -463,10 +462,16 @@ class _RingPlan:
         shards whose positions follow on from each other are contiguous in memory too: such a ring
         is the ring of fewer, longer shards (one, for a sequence cut into n pieces in order) up to
         the order of the fp32 sums.  A kernel then runs its straight-line stretches through what
-        were shard boundaries, and the host describes one shard pair instead of n * n.  Forward +
-        backward: B=2, H=16, 8 x 1024 causal 2.52 -> 2.28 ms; B=2, H=16, D=64, 4 x 1024 causal + ALiBi
-        0.73 -> 0.64 ms; fp32 inputs, B=2, H=4, 8 x 256: 3.6 -> 0.19 ms, nearly all of it host code.
-        The joined shards stay within what one launch takes, with and without a segment term."""
+        were shard boundaries, and the host describes one shard pair instead of n * n, which also
+        has kernels of its own (``ra_fwd_pair``).  Forward + backward, unjoined -> joined: B=2, H=16, 8 x 1024 causal
+        2.48 -> 2.11 ms; D=64, 4 x 1024 causal + ALiBi 0.73 -> 0.44; fp32 inputs, B=2, H=4, 8 x 256 of packed documents
+        4.0 -> 0.25, nearly all of it host code.
+        The joined shards stay within what one launch takes, with and without a segment term.  Where
+        that leaves several of them, on the kernels of the whole ring (131072 tokens as 2 shards instead of 8, H=8, D=128):
+        documents of mean 300 6.9 -> 5.8 ms, 2048 16.3 -> 15.7, with ALiBi 16.3 -> 15.0, causal 8.7 -> 8.1, prefix-LM + documents
+        29.8 -> 28.9; documents of mean 16384 are even (eight drawn packings: 494 -> 497 ms, 272 -> 293 with H=4).
+        A prefix-LM mask over 131072 tokens as one shard, past the capacity of the pair kernels' tile lists: H=4, D=128
+        300 -> 197 ms, D=64 222 -> 144."""
         got = self.__dict__.get("_joined")
         if got is None:
             got = self._join()
@@ -648,8 +653,8 @@ def _plan_for(q, k, n, bias_fn, q_kwargs, kv_kwargs) -> "_RingPlan":
     return plan
 
 
-# A callable's dense blocks are [b, h | 1, lq, lk] fp32 each: the several-step launches below take
-# as many of them per launch as fit this many bytes (and at most 16, what one launch walks).
+# A callable's dense blocks are [b, h | 1, lq, lk] fp32 each: the several-step calls below take
+# as many of them per call as fit this many bytes (and at most 16, what one launch walks).
 _DENSE_BLOCKS_BYTES = 1 << 30
 
 
@@ -673,8 +678,8 @@ def _row_chunks(plan: "_RingPlan", r: int):
 
 def _ring_forward_rows(q, k, v, plan: "_RingPlan", sm_scale, out_dtype, timer=_NO_TIMER):
     """The several-step launch scheme for a callable ``bias_fn``: one query shard at a time, its
-    ring steps in launches of up to 16 (``ra_fwd_steps``, the step's running state in registers
-    between the shards), so that only the dense blocks of one launch are alive."""
+    ring steps in calls of up to 16 (``ra_fwd_steps``), so that only the dense blocks of one call
+    are alive."""
     n, B, H, D, Lq, Lk = plan.n, plan.B, plan.H, plan.D, plan.Lq, plan.Lk
     dev = q.device
     out = torch.empty((B, n * Lq, H, D), dtype=out_dtype, device=dev)
@@ -694,7 +699,7 @@ def _ring_forward_rows(q, k, v, plan: "_RingPlan", sm_scale, out_dtype, timer=_N
 
 def _ring_backward_rows(q, k, v, out, lse, do, plan: "_RingPlan", sm_scale, timer=_NO_TIMER):
     """Backward twin of ``_ring_forward_rows``: every dense block is built ONCE and serves both
-    halves of its step - the dQ product of its query shard (one launch per chunk of blocks,
+    halves of its step - the dQ product of its query shard (one call per chunk of blocks,
     ``ra_bwd_dq_steps``) and the dK / dV products of its key/value shard (one launch per block,
     into that shard's fp32 accumulators)."""
     n, B, H, D, Lq, Lk = plan.n, plan.B, plan.H, plan.D, plan.Lq, plan.Lk

@@ -582,7 +582,7 @@ __global__ __launch_bounds__(256) void pair_combine_kernel(const PairFwdArgs a) 
 // LDS buffers, scores transposed (S^T = K Q^T, dP^T = V dO^T) so that dS^T is the B operand of
 // dQ^T = K^T dS^T, whose A operand comes from the K tile through the transposing read.
 template <int D, int MODE>
-__global__ __launch_bounds__(kPairThreads, 2) void dq_pair_kernel(const PairBwdArgs p) {
+__global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dq_pair_kernel(const PairBwdArgs p) {
   constexpr bool GENERAL = MODE != 0;
   constexpr bool DENSE = MODE == 2;
   constexpr int KS = D / 16, DB = D / 32;
@@ -941,18 +941,19 @@ RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg
 }
 
 // 128 keys per workgroup, 32 per wave, two workgroups per compute unit: K operands and the dK / dV
-// accumulators in registers; V, which a second wave per SIMD leaves no registers for at D = 128, in
-// LDS; 32-query tiles of Q and dO in two LDS buffers.  S = Q K^T: a lane owns one key and 16 queries, so
+// accumulators in registers; V, which a second (D = 128) or third (D = 64) wave per SIMD leaves no registers
+// for, in LDS; 32-query tiles of Q and dO in two LDS buffers.  S = Q K^T: a lane owns one key and 16 queries, so
 // that P and dS are the A operands of dV = P^T dO and dK = dS^T Q.  The rows' statistics (stat:
 // -lse log2(e) / scale_res, then -delta, from pair_stat_kernel) are the accumulators' initial values.
-// Three workgroups per compute unit at D = 64 without a dense block, although 168 registers spill 5 (MODE 0) and 12 (MODE 1)
-// of them: whole backward passes with two | three, 32768 causal, H=16 7.23 | 6.95 ms, 4096 causal, B=2, H=16 269 | 261 us,
-// unmasked 491 | 486, documents of 1000 in 16384 560 | 568, causal + ALiBi 346 | 360.
+// Three workgroups per compute unit at D = 64 without a dense block: 168 registers hold everything once V is in LDS.
+// With V in registers too 5 (MODE 0) and 12 (MODE 1) of them spill, and a reload inside the loop waits for the tile loads
+// that were just issued: causal + ALiBi, 4096, B=2, H=16, 240 us against 189; causal documents of 2175 in 48128, B=2, H=4, 636
+// against 531.
 template <int D, int MODE>
 __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dkdv_pair_kernel(const PairBwdArgs p) {
   constexpr bool GENERAL = MODE != 0;
   constexpr bool DENSE = MODE == 2;
-  constexpr bool VLDS = D == 128;
+  constexpr bool VLDS = D == 128 || MODE != 2;
   constexpr int KS = D / 16, DB = D / 32;
   constexpr int ROWB = D * 2;
   constexpr int TILE_BYTES = kPairQueries * ROWB;

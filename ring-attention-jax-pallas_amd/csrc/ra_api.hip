@@ -751,6 +751,7 @@ PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
   const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lk + kPairRowsHost - 1) / kPairRowsHost, wgs = heads * rows;
   const bool one_round = wgs > kPairSlots / 2 && wgs <= kPairSlots * 5 / 4;
   if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, total, rows, one_round ? 0 : 112)) r.pair = false;
+  else if (heads * p.Lq >= (int64_t)1 << 30) r.pair = false;  // one 32-bit offset reaches both statistics of a row
   else plan_split(r, heads, rows, total, most, 2 * kMinChunk);
   return r;
 }

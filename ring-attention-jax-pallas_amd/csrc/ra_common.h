@@ -245,6 +245,12 @@ RA_DEV void global_to_lds16_s_x2(const void* sbase, unsigned voff0, unsigned vof
   asm volatile("s_mov_b32 m0, %3\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %0\n\tglobal_load_lds_dwordx4 %2, %0 offset:1024"
                : : "s"(sbase), "v"(voff0), "v"(voff1_minus_1k), "s"(lds_addr) : "memory", "m0");
 }
+// ... four pieces, the lanes' offsets less 1, 2 and 3 KiB
+RA_DEV void global_to_lds16_s4(const void* sbase, unsigned v0, unsigned v1, unsigned v2, unsigned v3, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %5\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %0\n\tglobal_load_lds_dwordx4 %2, %0 offset:1024\n\t"
+               "global_load_lds_dwordx4 %3, %0 offset:2048\n\tglobal_load_lds_dwordx4 %4, %0 offset:3072"
+               : : "s"(sbase), "v"(v0), "v"(v1), "v"(v2), "v"(v3), "s"(lds_addr) : "memory", "m0");
+}
 // Workgroup barrier of the straight-line loops, whose only LDS writes are tile loads that the caller
 // counts with vmcnt: nothing is awaited, and LDS reads of this wave may stay in flight across it
 // (__syncthreads() puts a workgroup fence on either side of s_barrier, which orders nothing there).
@@ -252,6 +258,17 @@ RA_DEV void barrier_bare() { asm volatile("s_barrier" ::: "memory"); }
 // one dword per lane: lane l's word lands at lds_addr + 4 l
 RA_DEV void global_to_lds4(const void* gptr, unsigned lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(gptr), "s"(lds_addr) : "memory", "m0");
+}
+RA_DEV void global_to_lds4_s(const void* sbase, unsigned voff, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dword %1, %0" : : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory", "m0");
+}
+// The arguments of a kernel that takes one struct, read again: what only the end of a kernel needs does not
+// have to sit in scalar registers (or, spilled, in vector registers' lanes) through its loop.
+template <typename T>
+RA_DEV const __attribute__((address_space(4))) T* kernel_args() {
+  auto p = (const __attribute__((address_space(4))) T*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
 }
 // LDS byte address of an object declared __shared__
 #define RA_LDS_ADDR(obj) ((unsigned)(uintptr_t)(lds_char*)(obj))

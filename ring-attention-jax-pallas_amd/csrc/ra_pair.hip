@@ -9,6 +9,17 @@
 // work under the other's matrix work - and treat every tile alike, masks included.  The streamed
 // side of a pair can be split over several workgroups whose partial results a second kernel
 // combines.
+//
+// What bounds them is the latency of a wave's step through a tile, with two to four waves per SIMD to cover it: of
+// the wave cycles of documents + ALiBi (D = 128) 44 % issued an instruction, 29 % waited at the barrier or for operands and 26 %
+// for the issue port, and a forward tile took 9 vector and 3.6 scalar instructions per matrix instruction where the
+// softmax needs 6.  Hence everything around the matrix instructions is kept short: what a wave does with
+// a tile follows from a few ranges of tile indexes (WaveTiles) and from the wave's own ids (wave_tests), not the
+// workgroup's; the terms of a masked block are passes of their own (apply_terms); a tile's loads share one base
+// (TileLoader); and nothing that can be computed again stays in a register (opaque_lane, kernel_args), so that no
+// variant spills.  Before | after, us: documents of 2048 + ALiBi, 32768, H=16, D=128: forward 1787 | 1590, dQ 1916 | 1755, dK/dV
+// 2770 | 2410; causal documents of 2175 in 48128, B=2, H=4, D=64: 443 | 325, 476 | 350, 495 | 427; prefix-LM 4096, B=2, H=16, D=128,
+// forward 229 | 194; steps on dense blocks (documents of 2048 in 32768, 4 shards) 10.2 ms | 7.8 a pass.
 #include <type_traits>
 
 #include "ra_launch.h"
@@ -47,43 +58,63 @@ RA_DEV void pair_decode(int bid, int BH, int ntile, int& hh, int& piece, int& ti
   hh = spread ? hl * 8 + (bid & 7) : hl;
 }
 
+// The lane number, not known to the compiler as such: what is computed from it inside a loop is computed
+// there, where it is needed, instead of sitting in a register (or in scratch: a reload waits for the tile
+// loads in flight) through the loop.
+RA_DEV int opaque_lane(int lane) {
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
 // Moves ROWS-row tiles of one [L][D] matrix from memory to LDS: each of the four waves takes a quarter of
 // a tile's rows, 1 KiB per instruction.  Lane l fills the l-th 16 bytes of the kilobyte; the permuted
-// layout (tile_off) is obtained by letting it fetch the chunk that belongs there.  From one
-// instruction to another that chunk differs by an XOR: two registers hold what all of them need.
+// layout (tile_off) is obtained by letting it fetch the chunk that belongs there.  A tile costs one scalar
+// base and one LDS address for up to four instructions: the instruction's offset (1 KiB, 2 KiB, ..)
+// moves both addresses, and what the rows are further apart in memory than in LDS is in the lanes' offsets,
+// a register per instruction.  (With a base and an LDS address of its own per instruction a tile took 50 scalar
+// instructions of a wave's 120.)
 template <int D, int ROWS>
 struct TileLoader {
   static constexpr int CPR = D / 8;            // 16-byte chunks per row
   static constexpr int RPI = 64 / CPR;         // rows per load instruction
   static constexpr int RPW = ROWS / 4;         // rows per wave
   static constexpr int NLD = RPW / RPI;        // load instructions per wave and tile
-  const bf16_t* base;
-  long long sl;
-  int L;
-  unsigned row_off;  // byte offset of this lane's row from the first one of an instruction
-  RA_DEV void init(const bf16_t* base_, long long sl_, int L_, int lane) {
-    base = base_;
-    sl = sl_;
-    L = L_;
-    row_off = (unsigned)((long long)(lane / CPR) * sl * 2);
-  }
-  // byte offset inside its row of the chunk that a lane moves with an instruction that starts at row 0 of
-  // a tile, and at `row` (a multiple of RPI)
-  static RA_DEV unsigned first_chunk(int lane) { return (unsigned)(tile_off<D>(lane / CPR, lane % CPR) - (lane / CPR) * (D * 2)); }
-  static RA_DEV unsigned chunk(unsigned first, int row) { return first ^ (16 * (D == 128 ? (row >> 2) & 3 : (row >> 1) & 7)); }
-  RA_DEV void issue(int row0, unsigned dst, int wave, int lane, unsigned first) const {
-    dst += RPW * wave * (D * 2);
-    if (row0 + ROWS <= L) {
-      const bf16_t* sb = base + (long long)(row0 + RPW * wave) * sl;  // wave-uniform: scalar registers
+  static constexpr int NV = NLD < 16 / RPI ? NLD : 16 / RPI;  // of which so many share a base: 16 rows, whose offsets fit
+                                                              // 32 bits and after which the permutation repeats
+  const char* base;  // this wave's first row of the first tile
+  unsigned rowb;     // bytes from row to row
+  int left;          // rows from there on
+  unsigned voff[NV];
+  RA_DEV void init(const bf16_t* base_, long long sl, int L, int wave, int lane) {
+    rowb = (unsigned)sl * 2;
+    base = (const char*)base_ + (unsigned long long)(RPW * wave) * rowb;
+    left = L - RPW * wave;
 #pragma unroll
-      for (int t = 0; t < NLD; ++t)
-        global_to_lds16_s(sb + (long long)(RPI * t) * sl, row_off + chunk(first, RPW * wave + RPI * t), dst + RPI * t * (D * 2));
-    } else {  // last, partial tile: rows past the end repeat the last row (masked later)
+    for (int t = 0; t < NV; ++t) voff[t] = (unsigned)(lane / CPR + RPI * t) * rowb - 1024 * t + chunk(RPW * wave + RPI * t, lane);
+  }
+  // byte offset inside its row of the chunk that a lane moves with the instruction that starts at `row` of a tile
+  static RA_DEV unsigned chunk(int row, int lane) {
+    const int r = row + lane / CPR;
+    return (unsigned)(tile_off<D>(r, lane % CPR) - r * (D * 2));
+  }
+  // tile of the rows from row0 on, to the LDS address dst of the whole tile
+  RA_DEV void issue(int row0, unsigned dst, int wave, int lane) const {
+    dst += RPW * wave * (D * 2);
+    if (row0 + RPW <= left) {
+      const char* sb = base + (unsigned long long)(unsigned)row0 * rowb;  // wave-uniform: scalar registers
+#pragma unroll
+      for (int t = 0; t < NLD; t += NV) {
+        if constexpr (NV == 4) global_to_lds16_s4(sb, voff[0], voff[1], voff[2], voff[3], dst + RPI * t * (D * 2));
+        else if constexpr (NV == 2) global_to_lds16_s_x2(sb, voff[0], voff[1], dst + RPI * t * (D * 2));
+        else global_to_lds16_s(sb, voff[0], dst + RPI * t * (D * 2));
+        sb += (unsigned long long)(RPI * NV) * rowb;
+      }
+    } else {  // past the end: the last row again (masked later)
+      lane = opaque_lane(lane);
 #pragma unroll
       for (int t = 0; t < NLD; ++t) {
-        const int row = RPW * wave + RPI * t;
-        global_to_lds16((const char*)(base + (long long)min(row0 + row + lane / CPR, L - 1) * sl) + chunk(first, row),
-                        dst + RPI * t * (D * 2));
+        const int row = min(row0 + RPI * t + lane / CPR, left - 1);
+        global_to_lds16(base + (long long)row * (long long)rowb + chunk(RPW * wave + RPI * t, lane), dst + RPI * t * (D * 2));
       }
     }
   }
@@ -113,22 +144,32 @@ struct FragOffsets {
   RA_DEV int tr(int db, int h2) const { return (t0 ^ (db << 6) ^ (h2 * (D == 128 ? 32 : 64))) + h2 * 8 * (D * 2); }
 };
 
+// The segment ids and prefix flags of a wave's 32 rows, as uniform values.
+struct WaveIds {
+  int lo, hi;     // smallest and largest segment id of the wave's rows
+  bool any, all;  // some / every row carries the prefix flag
+  RA_DEV void init(bool valid, int seg, int pre) {
+    lo = __builtin_amdgcn_readfirstlane(wave_min(valid ? seg : 0x7fffffff));
+    hi = __builtin_amdgcn_readfirstlane(wave_max(valid ? seg : (int)0x80000000));
+    any = __any(valid && pre != 0);
+    all = __all(!valid || pre != 0);
+  }
+};
+
 // The list of key tiles that the workgroup's rows [q0, q_hi] have to visit, of the n from j_lo on:
 // tiles that one or the other term rules out are dropped, the others carry the terms that they
 // have to be tested for.  Returns their number.  Called by all four waves.
 template <bool DENSE>
 RA_DEV int list_key_tiles(int Lq, int Lk, const BiasArgs& bs, const int* kv_seg, const int* kv_pre, const unsigned char* dmap,
-                          int q0, int q_hi, bool q_valid, int q_seg, int q_pre, int j_lo, int n, int* s_red,
+                          int q0, int q_hi, const WaveIds& w, int j_lo, int n, int* s_red,
                           unsigned char* s_flag, unsigned short* s_list) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool seg_on = kv_seg != nullptr, pre_on = kv_pre != nullptr;
-  const int smin = wave_min(q_valid ? q_seg : 0x7fffffff), smax = wave_max(q_valid ? q_seg : (int)0x80000000);
-  const int any = __any(q_valid && q_pre != 0), all = __all(!q_valid || q_pre != 0);
   if (lane == 0) {
-    s_red[wave] = smin;
-    s_red[4 + wave] = smax;
-    s_red[8 + wave] = any;
-    s_red[12 + wave] = all;
+    s_red[wave] = w.lo;
+    s_red[4 + wave] = w.hi;
+    s_red[8 + wave] = w.any;
+    s_red[12 + wave] = w.all;
   }
   __syncthreads();
   const int qmin = min(min(s_red[0], s_red[1]), min(s_red[2], s_red[3]));
@@ -178,25 +219,179 @@ RA_DEV int list_key_tiles(int Lq, int Lk, const BiasArgs& bs, const int* kv_seg,
   return s_red[16];
 }
 
-// ALiBi on one side of the diagonal: -slope |q - k| = -s (rel - j), with s = +-slope (score units), rel the
-// distance of this lane's query from the tile's first key and j the key's index in the tile, is linear in
-// both positions and enters through the matrix unit as the accumulator's initial value:
-// [j, j, 1, 1, 1] x [s_hi, s_lo, c_hi, c_mid, c_lo], s and c = -s rel split into bf16 words (see
-// fwd_step_kernel).  kb: the 32-key block of the tile.
-RA_DEV f32x16 alibi_one_side(const f32x16& zero, float s, int rel, int kb, int l32, int g) {
-  const float c = -s * (float)rel;
-  bf16x8 bq, rf;
-  bq[0] = (bf16_t)s;
-  bq[1] = (bf16_t)(s - (float)bq[0]);
-  bq[2] = (bf16_t)c;
-  bq[3] = (bf16_t)(c - (float)bq[2]);
-  bq[4] = (bf16_t)((c - (float)bq[2]) - (float)bq[3]);
-  bq[5] = bq[6] = bq[7] = (bf16_t)0.f;
-  rf[0] = rf[1] = (bf16_t)(g == 0 ? (float)(32 * kb + l32) : 0.f);
-  rf[2] = rf[3] = rf[4] = (bf16_t)(g == 0 ? 1.0f : 0.f);
-  rf[5] = rf[6] = rf[7] = (bf16_t)0.f;
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(rf, bq, zero, 0, 0, 0);
+// ALiBi on one side of the diagonal: -slope |q - k| = s (j - rel), with s = +-slope (score units), rel the
+// distance of this lane's row from the tile's first position and j the index in the tile, enters through the
+// matrix unit as the accumulator's initial value, exactly: [j, 1] x [s, c] with c = -s rel in one fp32 product of
+// depth two.  `j`: alibi_index of the block.  (Split into bf16 words for the bf16 product, s and c took 20
+// vector instructions a tile, of the 200 of a forward tile.)
+RA_DEV float alibi_index(int first, int l32, int g) { return g == 0 ? (float)(first + l32) : 1.0f; }
+RA_DEV float alibi_terms(float s, int rel, int g) { return g == 0 ? s : -s * (float)rel; }
+RA_DEV f32x16 alibi_one_side(const f32x16& init, float j, float terms) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(j, terms, init, 0, 0, 0);
 }
+
+// What the 32 rows of a wave need done for a tile of the streamed side, as ranges of tile indexes: outside of `live`
+// the positional terms mask every score, inside of `plain` none (and the tile is whole); ALiBi is linear
+// for tiles below `past` and from `future` on.
+struct WaveTiles {
+  int live_lo, live_n, plain_lo, plain_n, past, future;
+  template <int T>
+  RA_DEV void sides(int lo, int hi, int off) {  // of rows at positions [lo, hi]; tile 0 starts at position off
+    past = floor_div(lo - off - (T - 1), T) + 1;
+    future = ceil_div(hi - off, T);
+  }
+  RA_DEV bool live(int j) const { return (unsigned)(j - live_lo) < (unsigned)live_n; }
+  RA_DEV bool plain(int j) const { return (unsigned)(j - plain_lo) < (unsigned)plain_n; }
+};
+RA_DEV WaveTiles wave_key_tiles(const BiasArgs& bs, int qlo, int qhi, int Lk) {
+  WaveTiles w;
+  const int flags = bs.flags & ~RA_BIAS_PREFIX;  // (tested for by itself)
+  const int n = (Lk + kPairKeys - 1) / kPairKeys;
+  int hi;
+  key_tile_range(flags, bs.window, qlo, qhi, bs.kv_off, n, kPairKeys, w.live_lo, hi);
+  w.live_n = hi - w.live_lo;
+  key_tile_plain_range(flags, bs.window, qlo, qhi, bs.kv_off, Lk / kPairKeys, kPairKeys, w.plain_lo, hi);
+  w.plain_n = hi - w.plain_lo;
+  w.sides<kPairKeys>(qlo, qhi, bs.kv_off);
+  return w;
+}
+
+// Drops the tests of a tile that hold for none or all of the wave's scores; true: every score is masked.
+// ids, flags: the tile's, one per lane (of a tile of 32 twice).  before: the keys of the tile and the wave's queries (or the other
+// way round) are in causal order throughout; after: none of them is.
+RA_DEV bool wave_tests(int& tests, const WaveIds& w, const int* ids, const int* flags, bool before, bool after, int lane) {
+  lane = opaque_lane(lane);
+  if (tests & kTestSegment) {
+    const int id = ids[lane];
+    if (!__any(id >= w.lo && id <= w.hi)) return true;
+    if (w.lo == w.hi && __all(id == w.lo)) tests &= ~kTestSegment;
+  }
+  if (tests & kTestPrefix) {
+    if (before) {
+      tests &= ~kTestPrefix;
+    } else {
+      const bool f = flags[lane] != 0;
+      if (w.all && __all(f)) tests &= ~kTestPrefix;
+      else if (after && !(w.any && __any(f))) return true;
+    }
+  }
+  return false;
+}
+
+// The terms `todo` (kTest..., kTestPos, kTestAlibi) on one 32x32 block: see apply_bias, whose interval test, id test,
+// prefix test and ALiBi are here one pass over the elements each, taken where the block needs it - most
+// blocks that need one need no other, and a pass is two to four instructions per element where the common
+// form takes five and a scalar one.
+constexpr int kTestPos = 8, kTestAlibi = 16;
+template <bool QFIXED, bool DENSE, bool GENERAL>
+RA_DEV void apply_terms(f32x16& t, int todo, const TileBias& tb, int rel0, int fixed_seg, int fixed_pre, const int* var_seg,
+                        const int* var_pre) {
+  if constexpr (GENERAL) {
+    if (todo & kTestAlibi) {
+      const float slope = -tb.slope2, relf0 = (float)rel0;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float off = (float)(8 * (r / 4) + r % 4);
+        t[r] = fmaf(fabsf(QFIXED ? relf0 - off : relf0 + off), slope, t[r]);
+      }
+    }
+    if constexpr (DENSE) {
+      if (todo & kTestDense) {
+        float dn[16];
+        if (QFIXED && __builtin_amdgcn_readfirstlane(tb.dense_vec)) {
+          // a lane's four keys are 16 contiguous bytes of its row
+#pragma unroll
+          for (int bb = 0; bb < 4; ++bb) {
+            const f32x4 v4 = *(const f32x4*)(tb.dense + 8 * bb);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) dn[4 * bb + c] = v4[c];
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int off = 8 * (r / 4) + r % 4;
+            dn[r] = 0.f;
+            if (off < tb.var_limit) dn[r] = QFIXED ? tb.dense[off] : tb.dense[off * tb.dense_vs];
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) t[r] = fmaf(dn[r], tb.dense_mul, t[r]);
+      }
+    }
+    if (todo & kTestSegment) {
+#pragma unroll
+      for (int bb = 0; bb < 4; ++bb) {
+        const i32x4 vs = *(const i32x4*)(var_seg + 8 * bb);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) t[4 * bb + c] = vs[c] != fixed_seg ? RA_NEG_INF : t[4 * bb + c];
+      }
+    }
+    if (todo & kTestPrefix) {
+      // masked where the key is behind the query's position, unless both carry the flag
+      constexpr int kFar = 1 << 30;
+      const int edge = QFIXED ? rel0 : -rel0, free = fixed_pre != 0 ? (QFIXED ? kFar : -kFar) : edge;
+#pragma unroll
+      for (int bb = 0; bb < 4; ++bb) {
+        const i32x4 vp = *(const i32x4*)(var_pre + 8 * bb);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int off = 8 * bb + c, e = vp[c] != 0 ? free : edge;
+          t[4 * bb + c] = (QFIXED ? off > e : off < e) ? RA_NEG_INF : t[4 * bb + c];
+        }
+      }
+    }
+  }
+  if (todo & kTestPos) {
+    // range limit, causal and window terms: an interval of the element's offset on the varying side
+    const bool causal = tb.flags & RA_BIAS_CAUSAL, window = tb.flags & RA_BIAS_WINDOW;
+    int lo = 0, hi = tb.var_limit - 1;
+    if (QFIXED) {
+      if (causal) hi = min(hi, rel0);
+      if (window) lo = max(lo, rel0 - tb.window + 1);
+      if (window && !causal) hi = min(hi, rel0 + tb.window - 1);
+    } else {
+      if (causal) lo = max(lo, -rel0);
+      if (window) hi = min(hi, tb.window - 1 - rel0);
+      if (window && !causal) lo = max(lo, 1 - rel0 - tb.window);
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[r] = 8 * (r / 4) + r % 4 > hi ? RA_NEG_INF : t[r];
+    if (window || (!QFIXED && causal)) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) t[r] = 8 * (r / 4) + r % 4 < lo ? RA_NEG_INF : t[r];
+    }
+  }
+}
+
+// The tiles of a workgroup one after another: entries of its list, or consecutive ones.  An entry is read two tiles
+// ahead, so that the address of the next tile is there when it is requested.
+struct TileWalk {
+  typedef __attribute__((address_space(3))) const unsigned short lds_entry;
+  lds_entry* list;
+  bool listed;  // (else consecutive tiles)
+  int j_lo, i_hi, every_test, mask;
+  int now, ahead;  // the entry of the current tile (uniform); one of the next tile, as it came from LDS
+  RA_DEV int entry(int i) const {
+    i = min(i, i_hi - 1);
+    return listed ? (int)list[i] : j_lo + i;
+  }
+  RA_DEV void start(bool listed_, const unsigned short* list_, int j_lo_, int i_lo, int i_hi_, int every_test_) {
+    listed = listed_;
+    list = (lds_entry*)list_;
+    j_lo = j_lo_;
+    i_hi = i_hi_;
+    every_test = every_test_;
+    mask = listed_ ? (1 << kTestShift) - 1 : 0x7fffffff;
+    now = __builtin_amdgcn_readfirstlane(entry(i_lo));
+    ahead = entry(i_lo + 1);
+  }
+  RA_DEV int tile() const { return now & mask; }
+  RA_DEV int tests() const { return (now & ~mask) >> kTestShift | every_test; }
+  RA_DEV void next(int i) {  // i: ordinal of the tile that becomes the current one
+    now = __builtin_amdgcn_readfirstlane(ahead);
+    ahead = entry(i + 1);
+  }
+};
 
 // S^T orientation as in fwd_step_kernel: a lane owns one query row and 16 keys of a 32-key block.
 // D is the row pitch of the LDS tiles (64 or 128 elements).
@@ -266,6 +461,8 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     if (flags & RA_BIAS_ALIBI) slope2 = bs.slopes[h] * kLog2e / a.scale2;
   }
 
+  WaveIds ids;
+  if constexpr (GENERAL) ids.init(q_valid, q_seg, q_pre);
   bool use_list = false;
   const unsigned char* dmap = nullptr;
   if constexpr (DENSE) {
@@ -274,7 +471,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   if constexpr (GENERAL) {
     use_list = ntiles <= kPairListTiles && ((flags & (RA_BIAS_SEGMENT | RA_BIAS_PREFIX)) || dmap != nullptr);
     if (use_list)
-      n = list_key_tiles<DENSE>(a.Lq, a.Lk, bs, kv_seg, kv_pre, dmap, q0, q_hi, q_valid, q_seg, q_pre, j_lo, n, s_red, s_flag, s_list);
+      n = list_key_tiles<DENSE>(a.Lq, a.Lk, bs, kv_seg, kv_pre, dmap, q0, q_hi, ids, j_lo, n, s_red, s_flag, s_list);
   }
   n = __builtin_amdgcn_readfirstlane(n);
   j_lo = __builtin_amdgcn_readfirstlane(j_lo);
@@ -291,26 +488,14 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     }
     if ((flags & RA_BIAS_DENSE) && dmap == nullptr) every_test |= kTestDense;
   }
-  auto tile_at = [&](int i, int& tests) -> int {
-    if (GENERAL && use_list) {
-      const int e = __builtin_amdgcn_readfirstlane((int)s_list[i]);
-      tests = (e >> kTestShift) | every_test;
-      return e & ((1 << kTestShift) - 1);
-    }
-    tests = every_test;
-    return j_lo + i;
-  };
 
   TileLoader<D, kPairKeys> ldk, ldv;
-  const unsigned first_chunk = TileLoader<D, kPairKeys>::first_chunk(lane);
-  ldk.init(a.k.ptr + b * a.k.sb + h * a.k.sh, a.k.sl, a.Lk, lane);
-  ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, lane);
+  ldk.init(a.k.ptr + b * a.k.sb + h * a.k.sh, a.k.sl, a.Lk, wave, lane);
+  ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, wave, lane);
   auto issue_tile = [&](int j, int buf) {
     const int k0 = j * kPairKeys;
-    unsigned first = first_chunk;
-    asm volatile("" : "+v"(first));  // the XORs are not to be hoisted out of the loop
-    ldk.issue(k0, RA_LDS_ADDR(&s_k[0][0]) + buf * TILE_BYTES, wave, lane, first);
-    ldv.issue(k0, RA_LDS_ADDR(&s_v[0][0]) + buf * TILE_BYTES, wave, lane, first);
+    ldk.issue(k0, RA_LDS_ADDR(&s_k[0][0]) + buf * TILE_BYTES, wave, lane);
+    ldv.issue(k0, RA_LDS_ADDR(&s_v[0][0]) + buf * TILE_BYTES, wave, lane);
     if constexpr (GENERAL) {
       const int kk = min(k0 + lane, a.Lk - 1);
       if (kv_seg && wave == 0) global_to_lds4(kv_seg + kk, RA_LDS_ADDR(&s_seg[0][0]) + buf * (kPairKeys * 4));
@@ -333,48 +518,67 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   const FragOffsets<D> fo(lane);
   const bool wave_on = qw < a.Lq;
   const bool alibi_on = GENERAL && (flags & RA_BIAS_ALIBI);
-  const int qlo_w = q_off + qw, qhi_w = q_off + qw + 31;
+  const WaveTiles wt = wave_key_tiles(bs, q_off + qw, q_off + qw + 31, a.Lk);
+  TileWalk walk;
 
   auto step = [&](auto buffer, int i) {
     constexpr int BUF = decltype(buffer)::value;
     __builtin_amdgcn_s_waitcnt(0x0f70);  // this wave's share of tile i is in LDS
     __syncthreads();                     // everyone's is, and nobody reads the other buffer any more
-    int tests;
-    const int kt0 = tile_at(i, tests) * kPairKeys;
-    if (i + 1 < i_hi) {
-      int t1;
-      issue_tile(tile_at(i + 1, t1), BUF ^ 1);
-    }
-    if (!wave_on) return;
     const FragOffsets<D> fr_off = fo.opaque();
-    const int klo = kv_off + kt0, khi = klo + kPairKeys - 1;
-    const int cls = classify_pos(flags, bs.window, qlo_w, qhi_w, klo, khi);
-    if (cls & 1) return;
-    f32x16 S[2];
-    bool alibi_left = alibi_on;  // ALiBi still to be added element by element
+    // K operands in the order of use, both key blocks of 16 head-dim elements in turn; the first ones
+    // are on their way while the next tile is requested
+    constexpr int PFK = 4;
+    bf16x8 kf[2 * KS];
+    auto k_frag = [&](int op) { return *(const bf16x8*)(s_k[BUF] + 32 * (op & 1) * ROWB + fr_off.nat(op >> 1)); };
 #pragma unroll
-    for (int r = 0; r < 16; ++r) S[0][r] = S[1][r] = 0.f;
-    if (alibi_on && (khi <= qlo_w || klo >= qhi_w)) {
-      alibi_left = false;
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) S[kb] = alibi_one_side(S[kb], khi <= qlo_w ? slope2 : -slope2, q_off + qi - klo, kb, l32, g);
+    for (int op = 0; op < PFK; ++op) kf[op] = k_frag(op);
+    __builtin_amdgcn_sched_barrier(0);
+    const int j = walk.tile(), kt0 = j * kPairKeys;
+    int tests = walk.tests();
+    if (i + 1 < i_hi) {
+      walk.next(i + 1);
+      issue_tile(walk.tile(), BUF ^ 1);
     }
+    if (!wave_on || !wt.live(j)) return;
+    const bool one_side = alibi_on && (j < wt.past || j >= wt.future);
+    if constexpr (GENERAL) {
+      if (tests && wave_tests(tests, ids, s_seg[BUF], s_pre[BUF], j < wt.past, j > wt.future, lane)) return;
+      if (alibi_on && !one_side) tests |= kTestAlibi;
+    }
+    if (!wt.plain(j)) tests |= kTestPos;
+    f32x16 S[2], zero;
+    float beyond = 0.f;  // what the scores of the second key block lack
+#pragma unroll
+    for (int r = 0; r < 16; ++r) zero[r] = 0.f;
     __builtin_amdgcn_s_setprio(1);
+    if (one_side) {
+      const int at = opaque_lane(lane), l = at & 31, half = at >> 5;
+      // one initial value for both key blocks: the second one's is 32 slopes further, added to its exponents
+      const float s = j < wt.past ? slope2 : -slope2;
+      const f32x16 init = alibi_one_side(zero, alibi_index(0, l, half), alibi_terms(s, q_off + qw + l - (kv_off + kt0), half));
+      beyond = 32.f * s;
+      S[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[0], init, 0, 0, 0);
+      S[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[1], qf[0], init, 0, 0, 0);
+    } else {
+      S[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[0], zero, 0, 0, 0);
+      S[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[1], qf[0], zero, 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    kf[PFK] = k_frag(PFK);
+    kf[PFK + 1] = k_frag(PFK + 1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ss = 0; ss < KS; ++ss)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-        S[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(s_k[BUF] + 32 * kb * ROWB + fr_off.nat(ss)), qf[ss], S[kb], 0, 0, 0);
+    for (int op = 2; op < 2 * KS; ++op) {
+      if (op + PFK < 2 * KS) kf[op + PFK] = k_frag(op + PFK);
+      S[op & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[op], qf[op >> 1], S[op & 1], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     __builtin_amdgcn_s_setprio(0);
-    if ((cls & 2) || kt0 + kPairKeys > a.Lk || (GENERAL && (tests || alibi_left))) {
+    if (tests) {
+      const int at = opaque_lane(lane), g = at >> 5, qi = qw + (at & 31);
       TileBias tb;
-      tb.flags = (cls & 2) ? (flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) : 0;
-      if constexpr (GENERAL) {
-        if (tests & kTestSegment) tb.flags |= RA_BIAS_SEGMENT;
-        if (tests & kTestPrefix) tb.flags |= RA_BIAS_PREFIX;
-        if (tests & kTestDense) tb.flags |= RA_BIAS_DENSE;
-        if (alibi_left) tb.flags |= RA_BIAS_ALIBI;
-      }
+      tb.flags = flags;
       tb.window = bs.window;
       tb.slope2 = slope2;
       tb.dense_mul = kLog2e / a.scale2;
@@ -390,9 +594,9 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
       for (int kb = 0; kb < 2; ++kb) {
         const int var0 = kt0 + 32 * kb + 4 * g;
         tb.var_limit = a.Lk - var0;
-        if (DENSE) tb.dense = head + (long long)qi_c * bs.dense_sq + var0;
-        apply_bias<true, DENSE, GENERAL>(S[kb], tb, (q_off + qi) - (kv_off + var0), q_seg, q_pre,
-                                         &s_seg[GENERAL ? BUF : 0][32 * kb + 4 * g], &s_pre[GENERAL ? BUF : 0][32 * kb + 4 * g]);
+        if (DENSE) tb.dense = head + (long long)min(qi, a.Lq - 1) * bs.dense_sq + var0;
+        apply_terms<true, DENSE, GENERAL>(S[kb], tests, tb, (q_off + qi) - (kv_off + var0), q_seg, q_pre,
+                                          &s_seg[GENERAL ? BUF : 0][32 * kb + 4 * g], &s_pre[GENERAL ? BUF : 0][32 * kb + 4 * g]);
       }
     }
     float mx0 = RA_NEG_INF, mx1 = RA_NEG_INF;
@@ -401,7 +605,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
       mx0 = fmaxf(fmaxf(mx0, S[0][r]), S[0][r + 1]);
       mx1 = fmaxf(fmaxf(mx1, S[1][r]), S[1][r + 1]);
     }
-    const float mx = half_max(fmaxf(mx0, mx1)) * a.scale2;
+    const float mx = half_max(fmaxf(mx0, GENERAL ? mx1 + beyond : mx1)) * a.scale2;
     m_true = fmaxf(m_true, mx);
     if (__any(mx > m_run + 8.0f)) {
       const float m_new = fmaxf(m_run, mx);
@@ -415,14 +619,15 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
         for (int r = 0; r < 16; ++r) oacc[db][r] *= corr;
     }
     const float neg_m = (m_run == RA_NEG_INF) ? 0.f : -m_run;
+    const float neg_m1 = GENERAL ? fmaf(beyond, a.scale2, neg_m) : neg_m;
     // The 32 scores of a lane go through exp2 in four groups of eight, one group per 16 keys of the
     // output product: group ks + 1 is worked on while the matrix unit multiplies with group ks.
     bf16x8 pf[4];
     float rs0 = 0.f, rs1 = 0.f;
     auto soft = [&](int ks, int e) {  // elements e, e + 1 of group ks
       const int r = 8 * (ks & 1) + e;
-      const float p0 = fast_exp2(fmaf(S[ks >> 1][r], a.scale2, neg_m));
-      const float p1 = fast_exp2(fmaf(S[ks >> 1][r + 1], a.scale2, neg_m));
+      const float p0 = fast_exp2(fmaf(S[ks >> 1][r], a.scale2, ks < 2 ? neg_m : neg_m1));
+      const float p1 = fast_exp2(fmaf(S[ks >> 1][r + 1], a.scale2, ks < 2 ? neg_m : neg_m1));
       rs0 += p0;
       rs1 += p1;
       bf16x2 pr;
@@ -473,25 +678,26 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   };
 
   if (i_lo < i_hi) {
-    int t0;
-    issue_tile(tile_at(i_lo, t0), 0);
+    walk.start(GENERAL && use_list, s_list, j_lo, i_lo, i_hi, every_test);
+    issue_tile(walk.tile(), 0);
     for (int i = i_lo; i < i_hi; i += 2) {
       step(std::integral_constant<int, 0>{}, i);
       if (i + 1 < i_hi) step(std::integral_constant<int, 1>{}, i + 1);
     }
   }
 
+  const auto* e = kernel_args<PairFwdArgs>();
   // a wave without a live score leaves its rows of the carry as they are, unread (m would come back through
   // two unit conversions, a last bit off)
-  if (a.o != nullptr && __all(l_run == 0.f && lr_run == 0.f)) return;
+  if (e->o != nullptr && __all(l_run == 0.f && lr_run == 0.f)) return;
   const float l_step = half_sum(l_run), lr_step = half_sum(lr_run);
-  if (a.part_n != nullptr && split == 0 && tid == 0) a.part_n[hh * nqt + qt] = n_piece;
+  if (e->part_n != nullptr && split == 0 && tid == 0) e->part_n[hh * nqt + qt] = n_piece;
   if (!q_valid) return;
-  const long long row = (long long)hh * a.Lq + qi;
+  const long long row = (long long)hh * e->Lq + qi;
   if (n_piece > 1) {
     // a share of the row's keys: combined by pair_combine_kernel
-    const long long prow = (long long)split * ((long long)a.B * a.H * a.Lq) + row;
-    float* op = a.part_o + prow * D + 4 * g;
+    const long long prow = (long long)split * ((long long)e->B * e->H * e->Lq) + row;
+    float* op = e->part_o + prow * D + 4 * g;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -501,15 +707,15 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
         for (int c = 0; c < 4; ++c) t[c] = oacc[db][4 * bb + c];
         *(f32x4*)(op + 32 * db + 8 * bb) = t;
       }
-    if (g == 0) *(f32x4*)(a.part_s + 4 * prow) = (f32x4){m_run, l_step, lr_step, 0.f};
-  } else if (a.o != nullptr) {
+    if (g == 0) *(f32x4*)(e->part_s + 4 * prow) = (f32x4){m_run, l_step, lr_step, 0.f};
+  } else if (e->o != nullptr) {
     // merge into the carry (see fwd_step_kernel)
-    const float m_in = a.m[row] * kLog2e, l_in = a.l[row];
+    const float m_in = e->m[row] * kLog2e, l_in = e->l[row];
     const float m_out = fmaxf(m_true, m_in), m_safe = (m_out == RA_NEG_INF) ? 0.f : m_out;
     const float f_in = fast_exp2(m_in - m_safe);
     const float f_step = (l_step > 0.f) ? fast_exp2(m_run - m_safe) : 0.f;
     const float f_o = f_step * ((lr_step > 0.f) ? l_step / lr_step : 1.f);
-    float* op = a.o + row * D + 4 * g;
+    float* op = e->o + row * D + 4 * g;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -520,12 +726,12 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
         *(f32x4*)(op + 32 * db + 8 * bb) = t;
       }
     if (g == 0) {
-      a.m[row] = m_out * kLn2;
-      a.l[row] = l_in * f_in + l_step * f_step;
+      e->m[row] = m_out * kLn2;
+      e->l[row] = l_in * f_in + l_step * f_step;
     }
   } else {
     const float inv = 1.0f / lr_step;
-    const long long at = b * a.out_sb + h * a.out_sh + (long long)qi * a.out_sl + 4 * g;
+    const long long at = b * e->out_sb + h * e->out_sh + (long long)qi * e->out_sl + 4 * g;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -533,9 +739,9 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
         f32x4 t;
 #pragma unroll
         for (int c = 0; c < 4; ++c) t[c] = oacc[db][4 * bb + c] * inv;
-        store4(a.out, a.out_f32, at + 32 * db + 8 * bb, t);
+        store4(e->out, e->out_f32, at + 32 * db + 8 * bb, t);
       }
-    if (g == 0) a.lse[row] = (l_step > 0.f) ? (m_run + __log2f(l_step)) * kLn2 : RA_NEG_INF;
+    if (g == 0) e->lse[row] = (l_step > 0.f) ? (m_run + __log2f(l_step)) * kLn2 : RA_NEG_INF;
   }
 }
 
@@ -582,7 +788,7 @@ __global__ __launch_bounds__(256) void pair_combine_kernel(const PairFwdArgs a) 
 // LDS buffers, scores transposed (S^T = K Q^T, dP^T = V dO^T) so that dS^T is the B operand of
 // dQ^T = K^T dS^T, whose A operand comes from the K tile through the transposing read.
 template <int D, int MODE>
-__global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dq_pair_kernel(const PairBwdArgs p) {
+__global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(const PairBwdArgs p) {
   constexpr bool GENERAL = MODE != 0;
   constexpr bool DENSE = MODE == 2;
   constexpr int KS = D / 16, DB = D / 32;
@@ -653,6 +859,8 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dq
     }
     if (flags & RA_BIAS_ALIBI) slope2 = bs.slopes[h] * kLog2e / a.scale_res;
   }
+  WaveIds ids;
+  if constexpr (GENERAL) ids.init(q_valid, q_seg, q_pre);
   bool use_list = false;
   const unsigned char* dmap = nullptr;
   if constexpr (DENSE) {
@@ -661,7 +869,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dq
   if constexpr (GENERAL) {
     use_list = ntiles <= kPairListTiles && ((flags & (RA_BIAS_SEGMENT | RA_BIAS_PREFIX)) || dmap != nullptr);
     if (use_list)
-      n = list_key_tiles<DENSE>(a.Lq, a.Lk, bs, kv_seg, kv_pre, dmap, q0, q_hi, q_valid, q_seg, q_pre, j_lo, n, s_red, s_flag, s_list);
+      n = list_key_tiles<DENSE>(a.Lq, a.Lk, bs, kv_seg, kv_pre, dmap, q0, q_hi, ids, j_lo, n, s_red, s_flag, s_list);
   }
   n = __builtin_amdgcn_readfirstlane(n);
   j_lo = __builtin_amdgcn_readfirstlane(j_lo);
@@ -674,25 +882,13 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dq
     if (!use_list && (flags & RA_BIAS_PREFIX)) every_test |= kTestPrefix;
     if ((flags & RA_BIAS_DENSE) && dmap == nullptr) every_test |= kTestDense;
   }
-  auto tile_at = [&](int i, int& tests) -> int {
-    if (GENERAL && use_list) {
-      const int e = __builtin_amdgcn_readfirstlane((int)s_list[i]);
-      tests = (e >> kTestShift) | every_test;
-      return e & ((1 << kTestShift) - 1);
-    }
-    tests = every_test;
-    return j_lo + i;
-  };
   TileLoader<D, kPairKeys> ldk, ldv;
-  const unsigned first_chunk = TileLoader<D, kPairKeys>::first_chunk(lane);
-  ldk.init(a.k.ptr + b * a.k.sb + h * a.k.sh, a.k.sl, a.Lk, lane);
-  ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, lane);
+  ldk.init(a.k.ptr + b * a.k.sb + h * a.k.sh, a.k.sl, a.Lk, wave, lane);
+  ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, wave, lane);
   auto issue_tile = [&](int j, int buf) {
     const int k0 = j * kPairKeys;
-    unsigned first = first_chunk;
-    asm volatile("" : "+v"(first));  // the XORs are not to be hoisted out of the loop
-    ldk.issue(k0, RA_LDS_ADDR(&s_k[0][0]) + buf * TILE_BYTES, wave, lane, first);
-    ldv.issue(k0, RA_LDS_ADDR(&s_v[0][0]) + buf * TILE_BYTES, wave, lane, first);
+    ldk.issue(k0, RA_LDS_ADDR(&s_k[0][0]) + buf * TILE_BYTES, wave, lane);
+    ldv.issue(k0, RA_LDS_ADDR(&s_v[0][0]) + buf * TILE_BYTES, wave, lane);
     if constexpr (GENERAL) {
       const int kk = min(k0 + lane, a.Lk - 1);
       if (kv_seg && wave == 0) global_to_lds4(kv_seg + kk, RA_LDS_ADDR(&s_seg[0][0]) + buf * (kPairKeys * 4));
@@ -708,34 +904,35 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dq
   const FragOffsets<D> fo(lane);
   const bool wave_on = qw < a.Lq;
   const bool alibi_on = GENERAL && (flags & RA_BIAS_ALIBI);
-  const int qlo_w = q_off + qw, qhi_w = q_off + qw + 31;
+  const WaveTiles wt = wave_key_tiles(bs, q_off + qw, q_off + qw + 31, a.Lk);
+  TileWalk walk;
 
   auto step = [&](auto buffer, int i) {
     constexpr int BUF = decltype(buffer)::value;
     __builtin_amdgcn_s_waitcnt(0x0f70);  // this wave's share of tile i is in LDS
     __syncthreads();                     // everyone's is, and nobody reads the other buffer any more
-    int tests;
-    const int kt0 = tile_at(i, tests) * kPairKeys;
-    if (i + 1 < i_hi) {
-      int t1;
-      issue_tile(tile_at(i + 1, t1), BUF ^ 1);
-    }
-    if (!wave_on) return;
     const FragOffsets<D> fr_off = fo.opaque();
-    const int klo = kv_off + kt0, khi = klo + kPairKeys - 1;
-    const int cls = classify_pos(flags, bs.window, qlo_w, qhi_w, klo, khi);
-    if (cls & 1) return;
-    const bool one_side = alibi_on && (khi <= qlo_w || klo >= qhi_w);
-    const bool biased = (cls & 2) || kt0 + kPairKeys > a.Lk || (GENERAL && (tests || (alibi_on && !one_side)));
+    const int j = walk.tile(), kt0 = j * kPairKeys;
+    int tests = walk.tests();
+    if (i + 1 < i_hi) {
+      walk.next(i + 1);
+      issue_tile(walk.tile(), BUF ^ 1);
+    }
+    if (!wave_on || !wt.live(j)) return;
+    const bool one_side = alibi_on && (j < wt.past || j >= wt.future);
+    if constexpr (GENERAL) {
+      if (tests && wave_tests(tests, ids, s_seg[BUF], s_pre[BUF], j < wt.past, j > wt.future, lane)) return;
+      if (alibi_on && !one_side) tests |= kTestAlibi;
+    }
+    if (!wt.plain(j)) tests |= kTestPos;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       // S^T first, then dP^T with the exp2 of S in its shadow: dP^T takes no registers while the terms
       // of a biased tile are evaluated
       constexpr int PF = 3;  // operand fetches in flight ahead of the matrix instruction that uses them
-      f32x16 S;
+      f32x16 S, zero;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) S[r] = 0.f;
-      if (one_side) S = alibi_one_side(S, khi <= qlo_w ? slope2 : -slope2, q_off + qi - klo, kb, l32, g);
+      for (int r = 0; r < 16; ++r) zero[r] = 0.f;
       auto nat_frag = [&](const char* tile, int ss) { return *(const bf16x8*)(tile + 32 * kb * ROWB + fr_off.nat(ss)); };
       __builtin_amdgcn_s_setprio(1);
       {
@@ -743,23 +940,29 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dq
 #pragma unroll
         for (int op = 0; op < PF; ++op) fr[op] = nat_frag(s_k[BUF], op);
         __builtin_amdgcn_sched_barrier(0);
+        if (one_side) {
+          const int at = opaque_lane(lane), l = at & 31, half = at >> 5;
+          S = alibi_one_side(zero, alibi_index(32 * kb, l, half),
+                             alibi_terms(j < wt.past ? slope2 : -slope2, q_off + qw + l - (kv_off + kt0), half));
+          S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[0], qf[0], S, 0, 0, 0);
+        } else {
+          S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[0], qf[0], zero, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fr[PF] = nat_frag(s_k[BUF], PF);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int op = 0; op < KS; ++op) {
+        for (int op = 1; op < KS; ++op) {
           if (op + PF < KS) fr[op + PF] = nat_frag(s_k[BUF], op + PF);
           S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], qf[op], S, 0, 0, 0);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
       __builtin_amdgcn_s_setprio(0);
-      if (biased) {
+      if (tests) {
+        const int at = opaque_lane(lane), g = at >> 5, qi = qw + (at & 31);
         TileBias tb;
-        tb.flags = (cls & 2) ? (flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) : 0;
-        if constexpr (GENERAL) {
-          if (tests & kTestSegment) tb.flags |= RA_BIAS_SEGMENT;
-          if (tests & kTestPrefix) tb.flags |= RA_BIAS_PREFIX;
-          if (tests & kTestDense) tb.flags |= RA_BIAS_DENSE;
-          if (alibi_on && !one_side) tb.flags |= RA_BIAS_ALIBI;
-        }
+        tb.flags = flags;
         tb.window = bs.window;
         tb.slope2 = slope2;
         tb.dense_mul = kLog2e / a.scale_res;
@@ -771,10 +974,10 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dq
         if (DENSE) {
           const float* head = bs.dense + b * bs.dense_sb + h * bs.dense_sh;
           tb.dense_vec = kt0 + kPairKeys <= a.Lk && ((((uintptr_t)head) | ((uintptr_t)bs.dense_sq << 2)) & 15) == 0;
-          tb.dense = head + (long long)qi_c * bs.dense_sq + var0;
+          tb.dense = head + (long long)min(qi, a.Lq - 1) * bs.dense_sq + var0;
         }
-        apply_bias<true, DENSE, GENERAL>(S, tb, (q_off + qi) - (kv_off + var0), q_seg, q_pre,
-                                         &s_seg[GENERAL ? BUF : 0][32 * kb + 4 * g], &s_pre[GENERAL ? BUF : 0][32 * kb + 4 * g]);
+        apply_terms<true, DENSE, GENERAL>(S, tests, tb, (q_off + qi) - (kv_off + var0), q_seg, q_pre,
+                                          &s_seg[GENERAL ? BUF : 0][32 * kb + 4 * g], &s_pre[GENERAL ? BUF : 0][32 * kb + 4 * g]);
       }
       f32x16 P;
 #pragma unroll
@@ -839,19 +1042,20 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dq
   };
 
   if (i_lo < i_hi) {
-    int t0;
-    issue_tile(tile_at(i_lo, t0), 0);
+    walk.start(GENERAL && use_list, s_list, j_lo, i_lo, i_hi, every_test);
+    issue_tile(walk.tile(), 0);
     for (int i = i_lo; i < i_hi; i += 2) {
       step(std::integral_constant<int, 0>{}, i);
       if (i + 1 < i_hi) step(std::integral_constant<int, 1>{}, i + 1);
     }
   }
 
-  if (p.part_n != nullptr && split == 0 && tid == 0) p.part_n[hh * nqt + qt] = n_piece;
+  const auto* e = kernel_args<PairBwdArgs>();
+  if (e->part_n != nullptr && split == 0 && tid == 0) e->part_n[hh * nqt + qt] = n_piece;
   if (!q_valid) return;
   float* fp = nullptr;  // fp32 destination: a share of the sum, or an accumulator
-  if (n_piece > 1) fp = p.part + ((long long)split * ((long long)a.B * a.H * a.Lq) + row) * D;
-  else if (p.acc != nullptr) fp = p.acc + row * D;
+  if (n_piece > 1) fp = e->part + ((long long)split * ((long long)e->a.B * e->a.H * e->a.Lq) + row) * D;
+  else if (e->acc != nullptr) fp = e->acc + row * D;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -859,12 +1063,12 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dq
       const int d0 = 32 * db + 8 * bb + 4 * g;
       f32x4 t;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) t[c] = acc[db][4 * bb + c] * a.sm_scale;
+      for (int c = 0; c < 4; ++c) t[c] = acc[db][4 * bb + c] * e->a.sm_scale;
       if (fp != nullptr) {
         if (n_piece == 1) t += *(const f32x4*)(fp + d0);
         *(f32x4*)(fp + d0) = t;
       } else {
-        store4(p.out, 0, b * p.out_sb + h * p.out_sh + (long long)qi * p.out_sl + d0, t);
+        store4(e->out, 0, b * e->out_sb + h * e->out_sh + (long long)qi * e->out_sl + d0, t);
       }
     }
 }
@@ -879,17 +1083,15 @@ constexpr int kPairQListTiles = 2048;
 // The query-side twin of list_key_tiles: the 32-query tiles that the workgroup's keys [k0, k_hi] meet.
 template <bool DENSE>
 RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg, const int* q_pre, const unsigned char* dmap,
-                            int k0, int k_hi, bool k_valid, int k_seg, int k_pre, int j_lo, int n, int* s_red,
+                            int k0, int k_hi, const WaveIds& w, int j_lo, int n, int* s_red,
                             unsigned char* s_flag, unsigned short* s_list) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool seg_on = q_seg != nullptr, pre_on = q_pre != nullptr;
-  const int smin = wave_min(k_valid ? k_seg : 0x7fffffff), smax = wave_max(k_valid ? k_seg : (int)0x80000000);
-  const int any = __any(k_valid && k_pre != 0), all = __all(!k_valid || k_pre != 0);
   if (lane == 0) {
-    s_red[wave] = smin;
-    s_red[4 + wave] = smax;
-    s_red[8 + wave] = any;
-    s_red[12 + wave] = all;
+    s_red[wave] = w.lo;
+    s_red[4 + wave] = w.hi;
+    s_red[8 + wave] = w.any;
+    s_red[12 + wave] = w.all;
   }
   __syncthreads();
   const int kmin = min(min(s_red[0], s_red[1]), min(s_red[2], s_red[3]));
@@ -945,22 +1147,20 @@ RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg
 // for, in LDS; 32-query tiles of Q and dO in two LDS buffers.  S = Q K^T: a lane owns one key and 16 queries, so
 // that P and dS are the A operands of dV = P^T dO and dK = dS^T Q.  The rows' statistics (stat:
 // -lse log2(e) / scale_res, then -delta, from pair_stat_kernel) are the accumulators' initial values.
-// Three workgroups per compute unit at D = 64 without a dense block: 168 registers hold everything once V is in LDS.
-// With V in registers too 5 (MODE 0) and 12 (MODE 1) of them spill, and a reload inside the loop waits for the tile loads
-// that were just issued: causal + ALiBi, 4096, B=2, H=16, 240 us against 189; causal documents of 2175 in 48128, B=2, H=4, 636
-// against 531.
+// Three workgroups per compute unit at D = 64: 168 registers hold everything once V is in LDS.  With V in registers too 5
+// (MODE 0) and 12 (MODE 1) of them spill, and a reload inside the loop waits for the tile loads that were just issued:
+// causal + ALiBi, 4096, B=2, H=16, 240 us against 189; causal documents of 2175 in 48128, B=2, H=4, 636 against 531.
 template <int D, int MODE>
-__global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dkdv_pair_kernel(const PairBwdArgs p) {
+__global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kernel(const PairBwdArgs p) {
   constexpr bool GENERAL = MODE != 0;
   constexpr bool DENSE = MODE == 2;
-  constexpr bool VLDS = D == 128 || MODE != 2;
   constexpr int KS = D / 16, DB = D / 32;
   constexpr int ROWB = D * 2;
   constexpr int TILE_BYTES = kPairQueries * ROWB;
   const BwdArgs& a = p.a;
   __shared__ __attribute__((aligned(16))) char s_q[2][TILE_BYTES];
   __shared__ __attribute__((aligned(16))) char s_do[2][TILE_BYTES];
-  __shared__ __attribute__((aligned(16))) char s_v[VLDS ? kPairSlab * ROWB : 16];
+  __shared__ __attribute__((aligned(16))) char s_v[kPairSlab * ROWB];
   __shared__ __attribute__((aligned(16))) float s_stat[2][2][kPairQueries];
   __shared__ __attribute__((aligned(16))) int s_seg[GENERAL ? 2 : 1][64];  // (a 64-lane load writes 64 words)
   __shared__ __attribute__((aligned(16))) int s_pre[GENERAL ? 2 : 1][64];
@@ -995,16 +1195,14 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
   int n = j_hi - j_lo;
   if (split > 0 && split * p.chunk_tiles >= n) return;
 
-  bf16x8 kf[KS], vf[VLDS ? 1 : KS];
+  bf16x8 kf[KS];
   {
     const bf16_t* kp = a.k.ptr + b * a.k.sb + h * a.k.sh + (long long)ki_c * a.k.sl + 8 * g;
-    const bf16_t* vp = a.v.ptr + b * a.v.sb + h * a.v.sh + (long long)ki_c * a.v.sl + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const bf16x8 kr = *(const bf16x8*)(kp + 16 * s);
 #pragma unroll
       for (int e = 0; e < 8; ++e) kf[s][e] = (bf16_t)((float)kr[e] * a.scale_p2);
-      if constexpr (!VLDS) vf[s] = *(const bf16x8*)(vp + 16 * s);
     }
   }
   int k_seg = 0, k_pre = 0;
@@ -1022,6 +1220,8 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
     }
     if (flags & RA_BIAS_ALIBI) slope2 = bs.slopes[h] * kLog2e / a.scale_res;
   }
+  WaveIds ids;
+  if constexpr (GENERAL) ids.init(k_valid, k_seg, k_pre);
   bool use_list = false;
   const unsigned char* dmap = nullptr;
   if constexpr (DENSE) {
@@ -1030,7 +1230,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
   if constexpr (GENERAL) {
     use_list = ntiles <= kPairQListTiles && ((flags & (RA_BIAS_SEGMENT | RA_BIAS_PREFIX)) || dmap != nullptr);
     if (use_list)
-      n = list_query_tiles<DENSE>(a.Lq, a.Lk, bs, q_seg, q_pre, dmap, k0, k_hi, k_valid, k_seg, k_pre, j_lo, n, s_red, s_flag, s_list);
+      n = list_query_tiles<DENSE>(a.Lq, a.Lk, bs, q_seg, q_pre, dmap, k0, k_hi, ids, j_lo, n, s_red, s_flag, s_list);
   }
   n = __builtin_amdgcn_readfirstlane(n);
   j_lo = __builtin_amdgcn_readfirstlane(j_lo);
@@ -1043,33 +1243,25 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
     if (!use_list && (flags & RA_BIAS_PREFIX)) every_test |= kTestPrefix;
     if ((flags & RA_BIAS_DENSE) && dmap == nullptr) every_test |= kTestDense;
   }
-  auto tile_at = [&](int i, int& tests) -> int {
-    if (GENERAL && use_list) {
-      const int e = __builtin_amdgcn_readfirstlane((int)s_list[i]);
-      tests = (e >> kTestShift) | every_test;
-      return e & ((1 << kTestShift) - 1);
-    }
-    tests = every_test;
-    return j_lo + i;
-  };
   TileLoader<D, kPairQueries> ldq, ldo;
-  const unsigned first_chunk = TileLoader<D, kPairQueries>::first_chunk(lane);
-  ldq.init(a.q.ptr + b * a.q.sb + h * a.q.sh, a.q.sl, a.Lq, lane);
-  ldo.init(a.dout.ptr + b * a.dout.sb + h * a.dout.sh, a.dout.sl, a.Lq, lane);
+  ldq.init(a.q.ptr + b * a.q.sb + h * a.q.sh, a.q.sl, a.Lq, wave, lane);
+  ldo.init(a.dout.ptr + b * a.dout.sb + h * a.dout.sh, a.dout.sl, a.Lq, wave, lane);
   // lanes 0..31 move -lse of a tile's rows, lanes 32..63 -delta
   const bool raw_stat = DENSE && p.stat == nullptr;  // a single step, which has no room for them: from lse and delta, per tile
-  const float* stat = (raw_stat ? (g ? a.delta : a.lse) : p.stat + (g ? (long long)a.B * a.H * a.Lq : 0)) + (long long)hh * a.Lq;
+  const float* stat = (DENSE ? (raw_stat ? (g ? a.delta : a.lse) : p.stat + (g ? (long long)a.B * a.H * a.Lq : 0)) : p.stat) + (long long)hh * a.Lq;
+  const unsigned to_delta = (unsigned)(a.B * a.H) * (unsigned)a.Lq * 4;  // (below 2^32: plan_dkdv_pair)
   auto issue_tile = [&](int j, int buf) {
     const int r0 = j * kPairQueries;
-    unsigned first = first_chunk;
-    asm volatile("" : "+v"(first));  // the XORs are not to be hoisted out of the loop
-    ldq.issue(r0, RA_LDS_ADDR(&s_q[0][0]) + buf * TILE_BYTES, wave, lane, first);
-    ldo.issue(r0, RA_LDS_ADDR(&s_do[0][0]) + buf * TILE_BYTES, wave, lane, first);
-    const int rr = min(r0 + l32, a.Lq - 1);
-    if (wave == 0) global_to_lds4(stat + rr, RA_LDS_ADDR(&s_stat[0][0][0]) + buf * (2 * kPairQueries * 4));
+    ldq.issue(r0, RA_LDS_ADDR(&s_q[0][0]) + buf * TILE_BYTES, wave, lane);
+    ldo.issue(r0, RA_LDS_ADDR(&s_do[0][0]) + buf * TILE_BYTES, wave, lane);
+    const int row = min(opaque_lane(lane) & 31, a.Lq - 1 - r0);
+    if (wave == 0) {
+      if constexpr (DENSE) global_to_lds4(stat + (r0 + row), RA_LDS_ADDR(&s_stat[0][0][0]) + buf * (2 * kPairQueries * 4));
+      else global_to_lds4_s(stat + r0, 4 * row + (lane >= 32 ? to_delta : 0u), RA_LDS_ADDR(&s_stat[0][0][0]) + buf * (2 * kPairQueries * 4));
+    }
     if constexpr (GENERAL) {
-      if (q_seg && wave == 1) global_to_lds4(q_seg + rr, RA_LDS_ADDR(&s_seg[0][0]) + buf * 256);
-      if (q_pre && wave == 2) global_to_lds4(q_pre + rr, RA_LDS_ADDR(&s_pre[0][0]) + buf * 256);
+      if (q_seg && wave == 1) global_to_lds4_s(q_seg + r0, 4 * row, RA_LDS_ADDR(&s_seg[0][0]) + buf * 256);
+      if (q_pre && wave == 2) global_to_lds4_s(q_pre + r0, 4 * row, RA_LDS_ADDR(&s_pre[0][0]) + buf * 256);
     }
   };
 
@@ -1082,24 +1274,36 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
   const bool wave_on = kw < a.Lk;
   const bool alibi_on = GENERAL && (flags & RA_BIAS_ALIBI);
   const float lse_mul = -kLog2e / a.scale_res;
-  const int klo_w = kv_off + kw, khi_w = kv_off + kw + 31;
+  WaveTiles wt;
+  {
+    const int klo_w = kv_off + kw, khi_w = kv_off + kw + 31, pos_flags = flags & ~RA_BIAS_PREFIX;  // (prefix: tested for by itself)
+    int hi;
+    query_tile_range(pos_flags, bs.window, klo_w, khi_w, q_off, ntiles, kPairQueries, wt.live_lo, hi);
+    wt.live_n = hi - wt.live_lo;
+    query_tile_plain_range(pos_flags, bs.window, klo_w, khi_w, q_off, a.Lq / kPairQueries, kPairQueries, wt.plain_lo, hi);
+    wt.plain_n = hi - wt.plain_lo;
+    wt.sides<kPairQueries>(klo_w, khi_w, q_off);
+  }
+  TileWalk walk;
 
   auto step = [&](auto buffer, int i) {
     constexpr int BUF = decltype(buffer)::value;
     __builtin_amdgcn_s_waitcnt(0x0f70);  // this wave's share of tile i is in LDS
     __syncthreads();                     // everyone's is, and nobody reads the other buffer any more
-    int tests;
-    const int qt0 = tile_at(i, tests) * kPairQueries;
-    if (i + 1 < i_hi) {
-      int t1;
-      issue_tile(tile_at(i + 1, t1), BUF ^ 1);
-    }
-    if (!wave_on) return;
     const FragOffsets<D> fr_off = fo.opaque();
-    const int qlo = q_off + qt0, qhi = qlo + kPairQueries - 1;
-    const int cls = classify_pos(flags, bs.window, qlo, qhi, klo_w, khi_w);
-    if (cls & 1) return;
-    const bool one_side = alibi_on && (qlo >= khi_w || qhi <= klo_w);
+    const int j = walk.tile(), qt0 = j * kPairQueries;
+    int tests = walk.tests();
+    if (i + 1 < i_hi) {
+      walk.next(i + 1);
+      issue_tile(walk.tile(), BUF ^ 1);
+    }
+    if (!wave_on || !wt.live(j)) return;
+    const bool one_side = alibi_on && (j < wt.past || j >= wt.future);
+    if constexpr (GENERAL) {
+      if (tests && wave_tests(tests, ids, s_seg[BUF], s_pre[BUF], j >= wt.future, j < wt.past - 1, lane)) return;
+      if (alibi_on && !one_side) tests |= kTestAlibi;
+    }
+    if (!wt.plain(j)) tests |= kTestPos;
     constexpr int PF = 3;  // operand fetches in flight ahead of the matrix instruction that uses them
     f32x16 S;
 #pragma unroll
@@ -1112,7 +1316,10 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
 #pragma unroll
       for (int r = 0; r < 16; ++r) S[r] = (S[r] == RA_NEG_INF) ? RA_NEG_INF : S[r] * lse_mul;
     }
-    if (one_side) S = alibi_one_side(S, qlo >= khi_w ? -slope2 : slope2, (kv_off + ki) - qlo, 0, l32, g);
+    if (one_side) {
+      const int at = opaque_lane(lane), l = at & 31;
+      S = alibi_one_side(S, alibi_index(0, l, at >> 5), alibi_terms(j < wt.past ? slope2 : -slope2, (kv_off + kw + l) - (q_off + qt0), at >> 5));
+    }
     auto nat_frag = [&](const char* tile, int ss) { return *(const bf16x8*)(tile + fr_off.nat(ss)); };
     __builtin_amdgcn_s_setprio(1);
     {
@@ -1128,15 +1335,10 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
       }
     }
     __builtin_amdgcn_s_setprio(0);
-    if ((cls & 2) || qt0 + kPairQueries > a.Lq || (GENERAL && (tests || (alibi_on && !one_side)))) {
+    if (tests) {
+      const int at = opaque_lane(lane), g = at >> 5, ki = kw + (at & 31);
       TileBias tb;
-      tb.flags = (cls & 2) ? (flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) : 0;
-      if constexpr (GENERAL) {
-        if (tests & kTestSegment) tb.flags |= RA_BIAS_SEGMENT;
-        if (tests & kTestPrefix) tb.flags |= RA_BIAS_PREFIX;
-        if (tests & kTestDense) tb.flags |= RA_BIAS_DENSE;
-        if (alibi_on && !one_side) tb.flags |= RA_BIAS_ALIBI;
-      }
+      tb.flags = flags;
       tb.window = bs.window;
       tb.slope2 = slope2;
       tb.dense_mul = kLog2e / a.scale_res;
@@ -1145,11 +1347,11 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
       tb.dense_vec = 0;
       tb.var_limit = a.Lq - (qt0 + 4 * g);
       if (DENSE) {
-        tb.dense = bs.dense + b * bs.dense_sb + h * bs.dense_sh + (long long)(qt0 + 4 * g) * bs.dense_sq + ki_c;
+        tb.dense = bs.dense + b * bs.dense_sb + h * bs.dense_sh + (long long)(qt0 + 4 * g) * bs.dense_sq + min(ki, a.Lk - 1);
         tb.dense_vs = bs.dense_sq;
       }
-      apply_bias<false, DENSE, GENERAL>(S, tb, (qlo + 4 * g) - (kv_off + ki), k_seg, k_pre, &s_seg[GENERAL ? BUF : 0][4 * g],
-                                        &s_pre[GENERAL ? BUF : 0][4 * g]);
+      apply_terms<false, DENSE, GENERAL>(S, tests, tb, (q_off + qt0 + 4 * g) - (kv_off + ki), k_seg, k_pre, &s_seg[GENERAL ? BUF : 0][4 * g],
+                                         &s_pre[GENERAL ? BUF : 0][4 * g]);
     }
     // dP with exp2(S) in its shadow
     bf16x8 pf[2], dsf[2];
@@ -1170,10 +1372,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
     }
     {
       bf16x8 fr[KS], vr[KS];
-      auto v_op = [&](int op) {
-        if constexpr (VLDS) return *(const bf16x8*)(s_v + 32 * wave * ROWB + fr_off.nat(op));
-        else return vf[op];
-      };
+      auto v_op = [&](int op) { return *(const bf16x8*)(s_v + 32 * wave * ROWB + fr_off.nat(op)); };
       constexpr int PFV = 2;
 #pragma unroll
       for (int op = 0; op < PFV; ++op) {
@@ -1249,28 +1448,27 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
   };
 
   if (i_lo < i_hi) {
-    if constexpr (VLDS) {
-      TileLoader<D, kPairSlab> ldv;
-      ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, lane);
-      ldv.issue(k0, RA_LDS_ADDR(&s_v[0]), wave, lane, TileLoader<D, kPairSlab>::first_chunk(lane));
-    }
-    int t0;
-    issue_tile(tile_at(i_lo, t0), 0);
+    TileLoader<D, kPairSlab> ldv;
+    ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, wave, lane);
+    ldv.issue(k0, RA_LDS_ADDR(&s_v[0]), wave, lane);
+    walk.start(GENERAL && use_list, s_list, j_lo, i_lo, i_hi, every_test);
+    issue_tile(walk.tile(), 0);
     for (int i = i_lo; i < i_hi; i += 2) {
       step(std::integral_constant<int, 0>{}, i);
       if (i + 1 < i_hi) step(std::integral_constant<int, 1>{}, i + 1);
     }
   }
 
-  if (p.part_n != nullptr && split == 0 && tid == 0) p.part_n[hh * nkt + kt] = n_piece;
+  const auto* e = kernel_args<PairBwdArgs>();
+  if (e->part_n != nullptr && split == 0 && tid == 0) e->part_n[hh * nkt + kt] = n_piece;
   // lane l32 holds column 32 db + l32 of rows kw + 4 g + 8 (r / 4) + r % 4
-  const long long rows = (long long)a.B * a.H * a.Lk;
-  if (n_piece == 1 && p.acc != nullptr) {
+  const long long rows = (long long)e->a.B * e->a.H * e->a.Lk;
+  if (n_piece == 1 && e->acc != nullptr) {
     // All loads of an array are issued before the first value is needed (see dkdv_kernel): a block of values, L=256, H=8, D=128,
     // 64.7 us with a load - add - store chain per element, 35.6 without; L=128, H=2, D=64, 36.4 and 19.8.
     auto add_to = [&](float* acc, const f32x16 (&x)[DB], float mul) {
-      float* const at = acc + ((long long)hh * a.Lk + kw + 4 * g) * D + l32;
-      if (kw + 32 <= a.Lk) {  // (wave-uniform)
+      float* const at = acc + ((long long)hh * e->a.Lk + kw + 4 * g) * D + l32;
+      if (kw + 32 <= e->a.Lk) {  // (wave-uniform)
         float old[DB][16];
 #pragma unroll
         for (int r = 0; r < 16; ++r)
@@ -1284,33 +1482,33 @@ __global__ __launch_bounds__(kPairThreads, D == 64 && MODE != 2 ? 3 : 2) void dk
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int row = 8 * (r / 4) + r % 4;
-          if (kw + 4 * g + row >= a.Lk) continue;
+          if (kw + 4 * g + row >= e->a.Lk) continue;
 #pragma unroll
           for (int db = 0; db < DB; ++db) at[row * D + 32 * db] += x[db][r] * mul;
         }
       }
     };
-    add_to(p.acc, dk, a.sm_scale);
-    add_to(p.acc2, dv, 1.0f);
+    add_to(e->acc, dk, e->a.sm_scale);
+    add_to(e->acc2, dv, 1.0f);
     return;
   }
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int key = kw + 4 * g + 8 * (r / 4) + (r % 4);
-    if (key >= a.Lk) continue;
+    if (key >= e->a.Lk) continue;
     if (n_piece > 1) {
-      float* fp = p.part + ((long long)split * 2 * rows + (long long)hh * a.Lk + key) * D + l32;
+      float* fp = e->part + ((long long)split * 2 * rows + (long long)hh * e->a.Lk + key) * D + l32;
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        fp[32 * db] = dk[db][r] * a.sm_scale;
+        fp[32 * db] = dk[db][r] * e->a.sm_scale;
         fp[rows * D + 32 * db] = dv[db][r];
       }
     } else {
-      const long long at = b * p.out_sb + h * p.out_sh + (long long)key * p.out_sl + l32;
+      const long long at = b * e->out_sb + h * e->out_sh + (long long)key * e->out_sl + l32;
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        ((bf16_t*)p.out)[at + 32 * db] = (bf16_t)(dk[db][r] * a.sm_scale);
-        ((bf16_t*)p.out2)[at + 32 * db] = (bf16_t)dv[db][r];
+        ((bf16_t*)e->out)[at + 32 * db] = (bf16_t)(dk[db][r] * e->a.sm_scale);
+        ((bf16_t*)e->out2)[at + 32 * db] = (bf16_t)dv[db][r];
       }
     }
   }

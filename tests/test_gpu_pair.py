@@ -66,6 +66,54 @@ def test_pair_kernels_at_their_edges(device, Sq, Sk, D, kind):
     _check(device, f"pair {kind}", B, Sq, Sk, H, D, 1, fn, ofn, qkw, kvkw, seed=Sq + Sk, impl="pallas")
 
 
+@pytest.mark.parametrize("S,D,kind", [(415, 64, "segments"), (415, 128, "segments"), (300, 128, "segments+causal+alibi"),
+                                      (300, 64, "segments+alibi"), (415, 64, "prefix"), (300, 128, "prefix+segments"),
+                                      (129, 128, "window+segments")])
+def test_each_wave_decides_by_its_own_ids_and_flags(device, S, D, kind):
+    """Ids and flags that change inside, at and across the 32 rows of a wave and the 64 (32) tokens of a tile, in no
+    order; k and q with row strides of their own, v and the gradient with others."""
+    B, H = 2, 2
+    rng = np.random.default_rng(S + D)
+    cuts = (np.arange(S)[None] // np.array([[32], [24]])) % 5  # whole waves and tiles, and shifted ones
+    ids = np.where(rng.random((B, S)) < 0.02, 9, cuts * 7 - 3).astype(np.int32)
+    flags = np.where(rng.random((B, S)) < 0.02, 0, np.array([0, 1, -5, 1, 0])[(cuts * 3) % 5]).astype(np.int32)
+    sl = R.alibi_slopes(H)
+    fn, kw, qkw, kvkw = None, {}, {}, {}
+    for term in kind.split("+"):
+        f, o = {"segments": (ra.segment_bias(), dict(use_segments=True)), "causal": (ra.causal_bias(), dict(causal=True)),
+                "alibi": (ra.alibi_bias(sl), dict(alibi=sl)), "prefix": (ra.prefix_lm_bias(), dict(use_prefix=True)),
+                "window": (ra.sliding_window_bias(40), dict(causal=True, window=40))}[term]
+        fn = f if fn is None else fn + f
+        kw.update(o)
+    if "segments" in kind:
+        qkw["q_segment_ids"], kvkw["kv_segment_ids"] = ids, ids
+    if "prefix" in kind:
+        qkw["q_prefix_mask"], kvkw["kv_prefix_mask"] = flags, flags
+    q, k, v, do = R.make_inputs(S, B, S, S, H, D)
+    at = np.broadcast_to(np.arange(S), (B, S))
+    bias = R.make_bias_fn(**kw)(**qkw, **kvkw, q_positions=at, kv_positions=at)
+    qk = torch.zeros((B, S, 2, H, D), dtype=torch.bfloat16, device=device)
+    qk[:, :, 0], qk[:, :, 1] = _dev(q, device, torch.bfloat16), _dev(k, device, torch.bfloat16)
+    leaves = [x.detach().requires_grad_(True) for x in (qk[:, :, 0], qk[:, :, 1], _dev(v, device, torch.bfloat16))]
+    out, lse = ra.ring_attention_with_lse(*leaves, 1, fn, {a: _dev(x, device) for a, x in qkw.items()},
+                                          {a: _dev(x, device) for a, x in kvkw.items()}, out_dtype=torch.float32)
+    want, want_lse = R.mha_dense(q, k, v, bias)
+    live = np.isfinite(want_lse).transpose(0, 2, 1)
+    assert live.all(axis=2).any() and np.isnan(out.detach().cpu().numpy()[~live]).all()
+    got = out.detach().cpu().numpy()
+    assert np.abs(got - want)[live].max() <= OUT_TOL
+    assert np.abs(lse.cpu().numpy() - want_lse)[np.isfinite(want_lse)].max() <= LSE_TOL
+    rows = live.all(axis=2)
+    do = np.where(rows[:, :, None, None], do, 0.0)
+    bias = np.where(rows[:, None, :, None], bias, 0.0)
+    grads = torch.autograd.grad(out, leaves, _dev(do, device))
+    for g, ref, name in zip(grads, R.mha_dense_grads(q, k, v, do, bias), ("dq", "dk", "dv")):
+        g = g.float().cpu().numpy()
+        if name == "dq":
+            g, ref = g[rows], ref[rows]
+        assert max(_rel(g, ref)) <= GRAD_TOL, name
+
+
 def _spread(where, absolute, q_segment_ids, kv_segment_ids):
     """A dense block of values and -inf: rows whose id is a multiple of three see no key whose id is one."""
     d = q_segment_ids[:, :, None] - kv_segment_ids[:, None, :]

@@ -366,11 +366,16 @@ int check_pass_counts(const int32_t* steps_per_pass, int32_t n_passes, std::vect
 // 8192, H=32, D=128: 16.7 -> 10.5 ms, 16384 in 4, H=16: 34.6 -> 23.6, 4096, B=2, H=16, D=64: 3.11 -> 2.51; 512 and 2000 tokens in 8
 // shards (host bound): 8.16 -> 8.22 and 8.15 -> 8.23, within the spread of one side (3 %), 810 in 3, H=4: 1.55 -> 1.62 (spread
 // 5 to 11 %; several small steps kept in one launch of the long-stretch kernels made no difference: 1.62).
+// What a block's summary says is told to each wave for its own 32 rows or keys and each 32 x 32 block of scores: values are read and
+// added where there are some, and a block that is -inf throughout is not read.  By workgroup and tile | by wave and block, with the
+// pair kernels' shorter steps, us, forward / dQ / dK and dV: documents of 300 in 8192, H=16, D=128 157 / 153 / 233 | 103 / 113 / 175; of 2000
+// 478 / 502 / 633 | 306 / 350 / 488; values 1264 / 1365 / 1949 | 905 / 980 / 1475.
 bool dense_steps_on_pair(const ra_bias& b) { return b.flags & RA_BIAS_DENSE; }
-// dK and dV only where their slabs are more than one per compute unit: a lone workgroup has nothing beside it there either,
-// and dkdv_kernel the longer pipeline.  dkdv_kernel | dkdv_pair_kernel, D=64, us, at 16 slabs (256 tokens, H=8) values 27 | 31,
-// documents of 300 17 | 21, a causal mask 22 | 25; at 256 (2048, H=16) 168 | 193, 61 | 67, 55 | 104; at 512 (2048, H=32) 329 | 217,
-// 115 | 74, 95 | 104.  D=128 at 256: 192 | 222, 71 | 77, 72 | 122; at 512: 377 | 258, 134 | 87, 125 | 129.
+// dK and dV only where their slabs are more than one per compute unit: a lone workgroup has nothing beside it there, and
+// dkdv_kernel the longer pipeline.  dkdv_kernel | dkdv_pair_kernel, us, at 256 slabs (2048, H=16), D=64: a causal mask 53 | 85, zeros
+// 49 | 86, documents of 300 125 | 102, values 169 | 145; D=128 72 | 104, 79 | 110, 149 | 126, 192 | 169; at 512 (2048, H=32), D=64: values
+// 329 | 217, documents 115 | 74, a causal mask 95 | 104.  (Both launched, with the block's content deciding as below, would cost the
+// plain ones a launch, a tenth of these.)
 int64_t key_slabs(const ra_bwd_step_params& p) { return (int64_t)p.B * p.H * ((p.Lk + 127) / 128); }
 bool dkdv_on_pair(const ra_bwd_step_params& p) { return key_slabs(p) > 256; }
 // Four and more steps of a single tile of rows and keys stay one launch of the long-stretch kernels, which keep their
@@ -379,19 +384,19 @@ bool dkdv_on_pair(const ra_bwd_step_params& p) { return key_slabs(p) > 256; }
 // 4 steps of 128 x 128: 44 | 47, 2 of them 26 | 24.
 template <typename P>
 bool one_tile_steps(const P& p, int n_steps) { return n_steps >= 4 && p.Lq <= 128 && p.Lk <= 128; }
-// Blocks of 8192 and more a side (dK and dV: of 4096 too while all slabs have their place at once) that are mostly zeros, tiles
-// without a term to evaluate, are what the long-stretch kernels are faster at, and the pair kernels at all others: there both are
-// launched and the block's summary, if it comes with one, says in every workgroup which of them runs.  The number is mostly_plain's one_in:
-// of a causal mask's cells one in 64 is of another kind at 4096 tokens, one in 128 at 8192, of documents of 2000 tokens one
-// in 30 to 60 at any length.  fwd_step_kernel | fwd_pair_kernel | both launched, us: all zeros 8192, H=16, D=64 409 | 454 | 413, D=128 596 | 667 |
-// 614, a causal mask of 16384, H=8, D=64 394 | 460 | 405; documents of 300 in 8192, H=16, D=64 | 95 | 103.  dkdv_kernel | dkdv_pair_kernel | both:
-// all zeros 8192, H=16, D=64 565 | 838 | 585, D=128 930 | 1115 | 943, a causal mask 344 | 461 | 358 and 526 | 602 | 535, of 4096, H=16, D=64
-// 112 | 192 | 119; documents of 300 in 8192, H=16 181 | 130 | 142.  A training call under a causal mask from a callable, 32768 tokens in 4
-// shards, H=16, D=64: 19.1 ms on the long-stretch kernels, 21.2 on the pair kernels, 19.1 with the choice; under causal documents of 2000 15.1, 13.8, 14.2.
-constexpr int kFwdPlain = 200, kDkdvPlain = 50;
-bool choose_by_content(const ra_bias& b, int64_t workgroups, int Lq, int Lk, bool small) {
+// dK and dV of blocks of 8192 and more a side (of 4096 too while all slabs have their place at once) that are zeros over whole
+// rows, tiles without a term to evaluate, are what dkdv_kernel is faster at, and dkdv_pair_kernel at all others: there both are
+// launched and the block's summary, if it comes with one, says in every workgroup which of them runs (see mostly_plain).  Its one_in:
+// of a causal mask's cells one in 64 is of another kind at 4096 tokens, one in 128 at 8192; documents are told by the last row
+// of cells, which one of them hardly ever fills.  dkdv_kernel | dkdv_pair_kernel, us, H=16: all zeros 8192, D=64 570 | 698, D=128 981 |
+// 1070, a causal mask 352 | 343 and 569 | 603, of 4096 115 | 157 and 165 | 208; documents of 6000 in 8192 1021 | 845 and 827 | 696, of 2000
+// in 4096, D=128, 454 | 349, of 300 in 8192, D=64, 181 | 96.
+// The forward takes fwd_pair_kernel throughout (fwd_step_kernel | fwd_pair_kernel, D=128: all zeros 8192 658 | 667, a causal mask 386 | 382,
+// documents of 6000 in 16384, H=8, 2191 | 912), and so does dQ.
+constexpr int kDkdvPlain = 50;
+bool choose_by_content(const ra_bias& b, int64_t slabs, int Lq, int Lk) {
   const int side = std::min(Lq, Lk);
-  return b.dense_map && (side >= 8192 || (small && side >= 4096 && workgroups <= 512));
+  return b.dense_map && (side >= 8192 || (side >= 4096 && slabs <= 512));
 }
 constexpr int kWholeRow = 1 << 30;  // chunk_tiles of rows that are not shared
 
@@ -413,14 +418,7 @@ int fwd_step_on_pair(const ra_fwd_step_params& p, void* stream) {
   a.o = p.o;
   a.m = p.m;
   a.l = p.l;
-  const int mode = kernel_mode(p.bias.flags), rule = choose_by_content(p.bias, 0, p.Lq, p.Lk, false) ? kFwdPlain : 0;
-  a.bias.plain_rule = -rule;
-  hipError_t e = ra::launch_fwd_pair(a, p.D, mode, (hipStream_t)stream);
-  if (e == hipSuccess && rule) {
-    ra::FwdArgs f = to_fwd_args(p);
-    f.bias.plain_rule = rule;
-    e = ra::launch_fwd_step(f, p.D, mode, (hipStream_t)stream);
-  }
+  hipError_t e = ra::launch_fwd_pair(a, p.D, kernel_mode(p.bias.flags), (hipStream_t)stream);
   return e == hipSuccess ? RA_OK : hip_fail(e, "forward step launch");
 }
 
@@ -436,7 +434,7 @@ int bwd_step_on_pair(const ra_bwd_step_params& p, int parts, void* stream) {
   hipError_t e = hipSuccess;
   if (parts & 1) {
     const bool pair = dkdv_on_pair(p);
-    const int rule = pair && choose_by_content(p.bias, key_slabs(p), p.Lq, p.Lk, true) ? kDkdvPlain : 0;
+    const int rule = pair && choose_by_content(p.bias, key_slabs(p), p.Lq, p.Lk) ? kDkdvPlain : 0;
     if (pair) {
       a.acc = p.dk;
       a.acc2 = p.dv;

@@ -68,41 +68,46 @@ RA_DEV int dense_map_or(const unsigned char* mp, int Lk, int q_lo, int q_hi, int
   return bits;
 }
 
-// Whether fewer than one in `one_in` of the live cells of a summary holds a value other than 0, in a sample of
-// whole rows of cells, about 1024 cells or one row.  The same sample and answer in every workgroup of every
-// kernel.  Called by all NT threads; red: two words per wave.
+// Whether a block is plain for the most part: the last row of cells, which a causal mask leaves whole, is live over
+// seven eighths at least, and fewer than one in `one_in` of the live cells of a summary holds a value other than 0, in a sample
+// of whole rows of cells from that one up, about 1024 cells or one row.  The same sample and answer in every workgroup of
+// every kernel.  Called by all NT threads; red: three words per wave.
 template <int NT>
 RA_DEV bool mostly_plain(const unsigned char* mp, int Lq, int Lk, int one_in, int* red) {
   const int rows = (Lq + kMapCell - 1) / kMapCell, cols = (Lk + kMapCell - 1) / kMapCell;
-  const int every = max(1, min(rows, rows * cols / 1024)), first = every / 2;
-  const int n = (rows - first + every - 1) / every * cols;
+  const int every = max(1, min(rows, rows * cols / 1024));
+  const int n = (rows + every - 1) / every * cols;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int live = 0, other = 0;
+  int live = 0, other = 0, last = 0;
 #pragma unroll 8
   for (int i = threadIdx.x; i < n; i += NT) {
     const int r = i / cols;
-    const int c = mp[(long long)(first + r * every) * cols + (i - r * cols)];
+    const int c = mp[(long long)(rows - 1 - r * every) * cols + (i - r * cols)];
     live += c & kMapLive;
+    last += r == 0 ? c & kMapLive : 0;
     other += c == (kMapLive | kMapNonZero);
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     live += __shfl_xor(live, o, 64);
     other += __shfl_xor(other, o, 64);
+    last += __shfl_xor(last, o, 64);
   }
   if (lane == 0) {
-    red[2 * wave] = live;
-    red[2 * wave + 1] = other;
+    red[3 * wave] = live;
+    red[3 * wave + 1] = other;
+    red[3 * wave + 2] = last;
   }
   __syncthreads();
-  live = other = 0;
+  live = other = last = 0;
 #pragma unroll
   for (int w = 0; w < NT / 64; ++w) {
-    live += red[2 * w];
-    other += red[2 * w + 1];
+    live += red[3 * w];
+    other += red[3 * w + 1];
+    last += red[3 * w + 2];
   }
   __syncthreads();
-  return (long long)other * one_in < live;
+  return 8 * last >= 7 * cols && (long long)other * one_in < live;
 }
 // ... and whether a kernel of that kind leaves a step to the other one.
 template <int NT>

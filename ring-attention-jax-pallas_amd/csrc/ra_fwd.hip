@@ -79,9 +79,6 @@ __global__ __launch_bounds__(kFwdThreads) void fwd_step_kernel(
   const int qi_c = min(qi, a.Lq - 1);
   const BiasArgs& bs = a.bias;
   const int flags = bs.flags;
-  if constexpr (DENSE && !MULTI) {
-    if (left_to_the_other<kFwdThreads>(bs, b, h, a.H, a.Lq, a.Lk, s_red)) return;
-  }
   // the query side of this workgroup's pass (read from the argument block where it is needed:
   // nothing of it is carried through the loops)
   auto pass_q_off = [&]() -> int { if constexpr (MULTI) return ring.q_off[blockIdx.y]; else return bs.q_off; };
@@ -1262,13 +1259,15 @@ __global__ void fwd_init_kernel(float* o, float* m, float* l, long long rows, in
 // Summary of a dense bias block [nb, nh, Lq, Lk] (the strides say where a batch / head starts):
 // one byte per cell of 32 queries x 32 keys, bit 0 = some value of the cell is not -inf, bit 1 =
 // some value is not 0 (elements beyond Lq / Lk count for nothing).  A wave takes 32 rows x 256
-// keys, eight cells: lane l reads keys 4l .. 4l+3 of every row.  HBM bound: the block is read once.
+// keys, eight cells: lane l reads keys 4l .. 4l+3 of every row.  HBM bound: the block is read once, from its end, which whoever
+// built it wrote last and the memory side's cache (256 MB) still holds: 8192 x 8192 behind torch.where 49 us, 5.5 TB/s, from its
+// beginning 61.
 __global__ __launch_bounds__(256) void dense_map_kernel(const float* dense, long long sb, long long sh,
                                                         long long sq, int nh, int Lq, int Lk, unsigned char* map) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ncols = (Lk + kMapCell - 1) / kMapCell, nrows = (Lq + kMapCell - 1) / kMapCell;
   const int cg = blockIdx.x * 4 + wave;  // group of eight cell columns
-  const int rb = blockIdx.y, bh = blockIdx.z;
+  const int rb = nrows - 1 - blockIdx.y, bh = blockIdx.z;
   if (cg * 8 >= ncols) return;
   const float* base = dense + (bh / nh) * sb + (bh % nh) * sh;
   const int k0 = cg * 256 + 4 * lane;
@@ -1341,13 +1340,19 @@ template <bool MULTI, bool WHOLE, typename Shards>
 static hipError_t launch_fwd(const FwdArgs& a, const Shards& sl, int n_pass, int D, int mode, hipStream_t stream) {
   const int nqt = (a.Lq + kFwdRows - 1) / kFwdRows;
   dim3 grid((unsigned)(a.B * a.H * nqt), (unsigned)n_pass), block(kFwdThreads);
+  if (mode == 2) {
+    if constexpr (MULTI) {  // (a single step on a dense block runs on fwd_pair_kernel)
+      if (D == 128) hipLaunchKernelGGL((fwd_step_kernel<128, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+      else hipLaunchKernelGGL((fwd_step_kernel<64, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+      return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+  }
   if (D == 128) {
-    if (mode == 2) hipLaunchKernelGGL((fwd_step_kernel<128, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
-    else if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<128, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+    if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<128, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
     else hipLaunchKernelGGL((fwd_step_kernel<128, 0, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
   } else {
-    if (mode == 2) hipLaunchKernelGGL((fwd_step_kernel<64, 2, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
-    else if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<64, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
+    if (mode == 1) hipLaunchKernelGGL((fwd_step_kernel<64, 1, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
     else hipLaunchKernelGGL((fwd_step_kernel<64, 0, MULTI, WHOLE>), grid, block, 0, stream, a, sl);
   }
   return hipGetLastError();

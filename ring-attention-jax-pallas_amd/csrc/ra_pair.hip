@@ -34,6 +34,12 @@ constexpr int kPairListTiles = 1024;
 // what a listed tile must evaluate element by element (bits of a list entry, above the tile index)
 constexpr int kTestShift = 11;
 constexpr int kTestSegment = 1, kTestPrefix = 2, kTestDense = 4;
+constexpr int kTestPos = 8, kTestAlibi = 16, kTestDead = 32;  // (not in a list: from the wave's own rows)
+// ... and under a dense block what its summary says about the tile, two bits (kMapLive, kMapNonZero) per wave and block of
+// 32 x 32 scores, above them
+constexpr int kCellShift = 16;
+template <bool DENSE>
+using ListEntry = std::conditional_t<DENSE, unsigned, unsigned short>;
 
 // Rows and keys of a workgroup's rectangle as the prefix term sees them: 0 = untouched by the mask,
 // 1 = some score may be masked, 2 = every score is.
@@ -162,7 +168,7 @@ struct WaveIds {
 template <bool DENSE>
 RA_DEV int list_key_tiles(int Lq, int Lk, const BiasArgs& bs, const int* kv_seg, const int* kv_pre, const unsigned char* dmap,
                           int q0, int q_hi, const WaveIds& w, int j_lo, int n, int* s_red,
-                          unsigned char* s_flag, unsigned short* s_list) {
+                          unsigned char* s_flag, ListEntry<DENSE>* s_list) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool seg_on = kv_seg != nullptr, pre_on = kv_pre != nullptr;
   if (lane == 0) {
@@ -196,9 +202,17 @@ RA_DEV int list_key_tiles(int Lq, int Lk, const BiasArgs& bs, const int* kv_seg,
     }
     if constexpr (DENSE) {
       if (dmap != nullptr && f) {
-        const int bits = dense_map_or(dmap, Lk, q0, q_hi, j * kPairKeys, min((j + 1) * kPairKeys, Lk) - 1);
-        if (!(bits & kMapLive)) f = 0;
-        else if (bits & kMapNonZero) f |= kTestDense;
+        // the summary's cells of the four waves' rows, two bits each, first and second key block of the tile
+        const int ncols = (Lk + kMapCell - 1) / kMapCell;
+        unsigned cells = 0;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const int r = q0 / kMapCell + c / 2, col = 2 * j + c % 2;
+          if (r * kMapCell <= q_hi && col < ncols) cells |= (dmap[(long long)r * ncols + col] & 3u) << (2 * c);
+        }
+        if (!(cells & 0x5555)) f = 0;
+        else if (cells & 0xaaaa) f |= kTestDense;
+        s_list[i] = cells;  // (until the entries are written)
       }
     }
     s_flag[i] = (unsigned char)f;
@@ -210,7 +224,12 @@ RA_DEV int list_key_tiles(int Lq, int Lk, const BiasArgs& bs, const int* kv_seg,
       const int i = base + lane;
       const int f = (i < n) ? s_flag[i] : 0;
       const unsigned long long mask = __ballot(f != 0);
-      if (f) s_list[cnt + __popcll(mask & ((1ull << lane) - 1ull))] = (unsigned short)((j_lo + i) | ((f & 7) << kTestShift));
+      unsigned entry = (j_lo + i) | ((f & 7) << kTestShift);
+      if constexpr (DENSE) {
+        if (f) entry |= (dmap != nullptr ? s_list[i] : 0xffffu) << kCellShift;
+        __builtin_amdgcn_wave_barrier();  // (entries land at or below what has been read)
+      }
+      if (f) s_list[cnt + __popcll(mask & ((1ull << lane) - 1ull))] = (ListEntry<DENSE>)entry;
       cnt += __popcll(mask);
     }
     if (lane == 0) s_red[16] = cnt;
@@ -278,14 +297,26 @@ RA_DEV bool wave_tests(int& tests, const WaveIds& w, const int* ids, const int* 
   return false;
 }
 
-// The terms `todo` (kTest..., kTestPos, kTestAlibi) on one 32x32 block: see apply_bias, whose interval test, id test,
+// What the summary says about a block, as tests: nothing to do, values to add, or every score masked.
+RA_DEV int cell_tests(int tests, unsigned cell) {
+  if (!(tests & kTestDense) || cell == (kMapLive | kMapNonZero)) return tests;
+  return (tests & ~kTestDense) | ((cell & kMapLive) ? 0 : kTestDead);
+}
+
+// The terms `todo` (kTest..., kTestPos, kTestAlibi, kTestDead) on one 32x32 block: see apply_bias, whose interval test, id test,
 // prefix test and ALiBi are here one pass over the elements each, taken where the block needs it - most
 // blocks that need one need no other, and a pass is two to four instructions per element where the common
 // form takes five and a scalar one.
-constexpr int kTestPos = 8, kTestAlibi = 16;
 template <bool QFIXED, bool DENSE, bool GENERAL>
 RA_DEV void apply_terms(f32x16& t, int todo, const TileBias& tb, int rel0, int fixed_seg, int fixed_pre, const int* var_seg,
                         const int* var_pre) {
+  if constexpr (DENSE) {
+    if (todo & kTestDead) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) t[r] = RA_NEG_INF;
+      return;
+    }
+  }
   if constexpr (GENERAL) {
     if (todo & kTestAlibi) {
       const float slope = -tb.slope2, relf0 = (float)rel0;
@@ -365,8 +396,9 @@ RA_DEV void apply_terms(f32x16& t, int todo, const TileBias& tb, int rel0, int f
 
 // The tiles of a workgroup one after another: entries of its list, or consecutive ones.  An entry is read two tiles
 // ahead, so that the address of the next tile is there when it is requested.
+template <bool DENSE>
 struct TileWalk {
-  typedef __attribute__((address_space(3))) const unsigned short lds_entry;
+  typedef __attribute__((address_space(3))) const ListEntry<DENSE> lds_entry;
   lds_entry* list;
   bool listed;  // (else consecutive tiles)
   int j_lo, i_hi, every_test, mask;
@@ -375,7 +407,7 @@ struct TileWalk {
     i = min(i, i_hi - 1);
     return listed ? (int)list[i] : j_lo + i;
   }
-  RA_DEV void start(bool listed_, const unsigned short* list_, int j_lo_, int i_lo, int i_hi_, int every_test_) {
+  RA_DEV void start(bool listed_, const ListEntry<DENSE>* list_, int j_lo_, int i_lo, int i_hi_, int every_test_) {
     listed = listed_;
     list = (lds_entry*)list_;
     j_lo = j_lo_;
@@ -386,7 +418,8 @@ struct TileWalk {
     ahead = entry(i_lo + 1);
   }
   RA_DEV int tile() const { return now & mask; }
-  RA_DEV int tests() const { return (now & ~mask) >> kTestShift | every_test; }
+  RA_DEV int tests() const { return ((now & ~mask & 0xffff) >> kTestShift) | every_test; }
+  RA_DEV unsigned cells() const { return listed ? (unsigned)now >> kCellShift : 0xffffu; }
   RA_DEV void next(int i) {  // i: ordinal of the tile that becomes the current one
     now = __builtin_amdgcn_readfirstlane(ahead);
     ahead = entry(i + 1);
@@ -406,7 +439,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   __shared__ __attribute__((aligned(16))) char s_v[2][TILE_BYTES];
   __shared__ __attribute__((aligned(16))) int s_seg[GENERAL ? 2 : 1][kPairKeys];
   __shared__ __attribute__((aligned(16))) int s_pre[GENERAL ? 2 : 1][kPairKeys];
-  __shared__ unsigned short s_list[GENERAL ? kPairListTiles : 1];
+  __shared__ ListEntry<DENSE> s_list[GENERAL ? kPairListTiles : 1];
   __shared__ unsigned char s_flag[GENERAL ? kPairListTiles : 1];
   __shared__ int s_red[20];
 
@@ -424,9 +457,6 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   const int qi_c = min(qi, a.Lq - 1);
   const BiasArgs& bs = a.bias;
   const int flags = bs.flags;
-  if constexpr (DENSE) {
-    if (left_to_the_other<kPairThreads>(bs, b, h, a.H, a.Lq, a.Lk, s_red)) return;
-  }
   const int q_off = bs.q_off, kv_off = bs.kv_off;
 
   // ---- the key tiles of this workgroup ----------------------------------------------------------
@@ -519,7 +549,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   const bool wave_on = qw < a.Lq;
   const bool alibi_on = GENERAL && (flags & RA_BIAS_ALIBI);
   const WaveTiles wt = wave_key_tiles(bs, q_off + qw, q_off + qw + 31, a.Lk);
-  TileWalk walk;
+  TileWalk<DENSE> walk;
 
   auto step = [&](auto buffer, int i) {
     constexpr int BUF = decltype(buffer)::value;
@@ -536,11 +566,20 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     __builtin_amdgcn_sched_barrier(0);
     const int j = walk.tile(), kt0 = j * kPairKeys;
     int tests = walk.tests();
+    bool dead = !wave_on || !wt.live(j);
+    unsigned cells = 0;
+    if constexpr (DENSE) {
+      if (tests & kTestDense) {
+        cells = walk.cells() >> (4 * wave);
+        dead = dead || !(cells & 5);
+        if ((cells & 15) == 5) tests &= ~kTestDense;
+      }
+    }
     if (i + 1 < i_hi) {
       walk.next(i + 1);
       issue_tile(walk.tile(), BUF ^ 1);
     }
-    if (!wave_on || !wt.live(j)) return;
+    if (dead) return;
     const bool one_side = alibi_on && (j < wt.past || j >= wt.future);
     if constexpr (GENERAL) {
       if (tests && wave_tests(tests, ids, s_seg[BUF], s_pre[BUF], j < wt.past, j > wt.future, lane)) return;
@@ -582,9 +621,6 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
       tb.window = bs.window;
       tb.slope2 = slope2;
       tb.dense_mul = kLog2e / a.scale2;
-      tb.dense = nullptr;
-      tb.dense_vs = 1;
-      tb.dense_vec = 0;
       const float* head = nullptr;
       if (DENSE) {
         head = bs.dense + b * bs.dense_sb + h * bs.dense_sh;
@@ -595,8 +631,9 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
         const int var0 = kt0 + 32 * kb + 4 * g;
         tb.var_limit = a.Lk - var0;
         if (DENSE) tb.dense = head + (long long)min(qi, a.Lq - 1) * bs.dense_sq + var0;
-        apply_terms<true, DENSE, GENERAL>(S[kb], tests, tb, (q_off + qi) - (kv_off + var0), q_seg, q_pre,
-                                          &s_seg[GENERAL ? BUF : 0][32 * kb + 4 * g], &s_pre[GENERAL ? BUF : 0][32 * kb + 4 * g]);
+        apply_terms<true, DENSE, GENERAL>(S[kb], DENSE ? cell_tests(tests, (cells >> (2 * kb)) & 3) : tests, tb,
+                                          (q_off + qi) - (kv_off + var0), q_seg, q_pre, &s_seg[GENERAL ? BUF : 0][32 * kb + 4 * g],
+                                          &s_pre[GENERAL ? BUF : 0][32 * kb + 4 * g]);
       }
     }
     float mx0 = RA_NEG_INF, mx1 = RA_NEG_INF;
@@ -799,7 +836,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
   __shared__ __attribute__((aligned(16))) char s_v[2][TILE_BYTES];
   __shared__ __attribute__((aligned(16))) int s_seg[GENERAL ? 2 : 1][kPairKeys];
   __shared__ __attribute__((aligned(16))) int s_pre[GENERAL ? 2 : 1][kPairKeys];
-  __shared__ unsigned short s_list[GENERAL ? kPairListTiles : 1];
+  __shared__ ListEntry<DENSE> s_list[GENERAL ? kPairListTiles : 1];
   __shared__ unsigned char s_flag[GENERAL ? kPairListTiles : 1];
   __shared__ int s_red[20];
 
@@ -905,7 +942,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
   const bool wave_on = qw < a.Lq;
   const bool alibi_on = GENERAL && (flags & RA_BIAS_ALIBI);
   const WaveTiles wt = wave_key_tiles(bs, q_off + qw, q_off + qw + 31, a.Lk);
-  TileWalk walk;
+  TileWalk<DENSE> walk;
 
   auto step = [&](auto buffer, int i) {
     constexpr int BUF = decltype(buffer)::value;
@@ -914,11 +951,20 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
     const FragOffsets<D> fr_off = fo.opaque();
     const int j = walk.tile(), kt0 = j * kPairKeys;
     int tests = walk.tests();
+    bool dead = !wave_on || !wt.live(j);
+    unsigned cells = 0;
+    if constexpr (DENSE) {
+      if (tests & kTestDense) {
+        cells = walk.cells() >> (4 * wave);
+        dead = dead || !(cells & 5);
+        if ((cells & 15) == 5) tests &= ~kTestDense;
+      }
+    }
     if (i + 1 < i_hi) {
       walk.next(i + 1);
       issue_tile(walk.tile(), BUF ^ 1);
     }
-    if (!wave_on || !wt.live(j)) return;
+    if (dead) return;
     const bool one_side = alibi_on && (j < wt.past || j >= wt.future);
     if constexpr (GENERAL) {
       if (tests && wave_tests(tests, ids, s_seg[BUF], s_pre[BUF], j < wt.past, j > wt.future, lane)) return;
@@ -966,9 +1012,6 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
         tb.window = bs.window;
         tb.slope2 = slope2;
         tb.dense_mul = kLog2e / a.scale_res;
-        tb.dense = nullptr;
-        tb.dense_vs = 1;
-        tb.dense_vec = 0;
         const int var0 = kt0 + 32 * kb + 4 * g;
         tb.var_limit = a.Lk - var0;
         if (DENSE) {
@@ -976,8 +1019,9 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
           tb.dense_vec = kt0 + kPairKeys <= a.Lk && ((((uintptr_t)head) | ((uintptr_t)bs.dense_sq << 2)) & 15) == 0;
           tb.dense = head + (long long)min(qi, a.Lq - 1) * bs.dense_sq + var0;
         }
-        apply_terms<true, DENSE, GENERAL>(S, tests, tb, (q_off + qi) - (kv_off + var0), q_seg, q_pre,
-                                          &s_seg[GENERAL ? BUF : 0][32 * kb + 4 * g], &s_pre[GENERAL ? BUF : 0][32 * kb + 4 * g]);
+        apply_terms<true, DENSE, GENERAL>(S, DENSE ? cell_tests(tests, (cells >> (2 * kb)) & 3) : tests, tb,
+                                          (q_off + qi) - (kv_off + var0), q_seg, q_pre, &s_seg[GENERAL ? BUF : 0][32 * kb + 4 * g],
+                                          &s_pre[GENERAL ? BUF : 0][32 * kb + 4 * g]);
       }
       f32x16 P;
 #pragma unroll
@@ -1084,7 +1128,7 @@ constexpr int kPairQListTiles = 2048;
 template <bool DENSE>
 RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg, const int* q_pre, const unsigned char* dmap,
                             int k0, int k_hi, const WaveIds& w, int j_lo, int n, int* s_red,
-                            unsigned char* s_flag, unsigned short* s_list) {
+                            unsigned char* s_flag, ListEntry<DENSE>* s_list) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool seg_on = q_seg != nullptr, pre_on = q_pre != nullptr;
   if (lane == 0) {
@@ -1119,9 +1163,17 @@ RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg
     }
     if constexpr (DENSE) {
       if (dmap != nullptr && f) {
-        const int bits = dense_map_or(dmap, Lk, j * kPairQueries, q_last, k0, k_hi);
-        if (!(bits & kMapLive)) f = 0;
-        else if (bits & kMapNonZero) f |= kTestDense;
+        // the summary's cells of the four waves' keys, two bits each
+        const int ncols = (Lk + kMapCell - 1) / kMapCell;
+        unsigned cells = 0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int col = k0 / kMapCell + c;
+          if (col * kMapCell <= k_hi) cells |= (dmap[(long long)j * ncols + col] & 3u) << (2 * c);
+        }
+        if (!(cells & 0x55)) f = 0;
+        else if (cells & 0xaa) f |= kTestDense;
+        s_list[i] = cells;  // (until the entries are written)
       }
     }
     s_flag[i] = (unsigned char)f;
@@ -1133,7 +1185,12 @@ RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg
       const int i = base + lane;
       const int f = (i < n) ? s_flag[i] : 0;
       const unsigned long long mask = __ballot(f != 0);
-      if (f) s_list[cnt + __popcll(mask & ((1ull << lane) - 1ull))] = (unsigned short)((j_lo + i) | ((f & 7) << kTestShift));
+      unsigned entry = (j_lo + i) | ((f & 7) << kTestShift);
+      if constexpr (DENSE) {
+        if (f) entry |= (dmap != nullptr ? s_list[i] : 0xffffu) << kCellShift;
+        __builtin_amdgcn_wave_barrier();  // (entries land at or below what has been read)
+      }
+      if (f) s_list[cnt + __popcll(mask & ((1ull << lane) - 1ull))] = (ListEntry<DENSE>)entry;
       cnt += __popcll(mask);
     }
     if (lane == 0) s_red[16] = cnt;
@@ -1164,7 +1221,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
   __shared__ __attribute__((aligned(16))) float s_stat[2][2][kPairQueries];
   __shared__ __attribute__((aligned(16))) int s_seg[GENERAL ? 2 : 1][64];  // (a 64-lane load writes 64 words)
   __shared__ __attribute__((aligned(16))) int s_pre[GENERAL ? 2 : 1][64];
-  __shared__ unsigned short s_list[GENERAL ? kPairQListTiles : 1];
+  __shared__ ListEntry<DENSE> s_list[GENERAL ? kPairQListTiles : 1];
   __shared__ unsigned char s_flag[GENERAL ? kPairQListTiles : 1];
   __shared__ int s_red[20];
 
@@ -1284,7 +1341,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
     wt.plain_n = hi - wt.plain_lo;
     wt.sides<kPairQueries>(klo_w, khi_w, q_off);
   }
-  TileWalk walk;
+  TileWalk<DENSE> walk;
 
   auto step = [&](auto buffer, int i) {
     constexpr int BUF = decltype(buffer)::value;
@@ -1293,11 +1350,19 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
     const FragOffsets<D> fr_off = fo.opaque();
     const int j = walk.tile(), qt0 = j * kPairQueries;
     int tests = walk.tests();
+    bool dead = !wave_on || !wt.live(j);
+    if constexpr (DENSE) {
+      if (tests & kTestDense) {
+        const unsigned cell = (walk.cells() >> (2 * wave)) & 3;
+        dead = dead || !(cell & kMapLive);
+        if (cell == kMapLive) tests &= ~kTestDense;
+      }
+    }
     if (i + 1 < i_hi) {
       walk.next(i + 1);
       issue_tile(walk.tile(), BUF ^ 1);
     }
-    if (!wave_on || !wt.live(j)) return;
+    if (dead) return;
     const bool one_side = alibi_on && (j < wt.past || j >= wt.future);
     if constexpr (GENERAL) {
       if (tests && wave_tests(tests, ids, s_seg[BUF], s_pre[BUF], j >= wt.future, j < wt.past - 1, lane)) return;
@@ -1342,16 +1407,13 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
       tb.window = bs.window;
       tb.slope2 = slope2;
       tb.dense_mul = kLog2e / a.scale_res;
-      tb.dense = nullptr;
-      tb.dense_vs = 1;
-      tb.dense_vec = 0;
       tb.var_limit = a.Lq - (qt0 + 4 * g);
       if (DENSE) {
         tb.dense = bs.dense + b * bs.dense_sb + h * bs.dense_sh + (long long)(qt0 + 4 * g) * bs.dense_sq + min(ki, a.Lk - 1);
         tb.dense_vs = bs.dense_sq;
       }
-      apply_terms<false, DENSE, GENERAL>(S, tests, tb, (q_off + qt0 + 4 * g) - (kv_off + ki), k_seg, k_pre, &s_seg[GENERAL ? BUF : 0][4 * g],
-                                         &s_pre[GENERAL ? BUF : 0][4 * g]);
+      apply_terms<false, DENSE, GENERAL>(S, tests, tb, (q_off + qt0 + 4 * g) - (kv_off + ki), k_seg, k_pre,
+                                         &s_seg[GENERAL ? BUF : 0][4 * g], &s_pre[GENERAL ? BUF : 0][4 * g]);
     }
     // dP with exp2(S) in its shadow
     bf16x8 pf[2], dsf[2];

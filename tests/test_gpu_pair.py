@@ -223,3 +223,30 @@ def test_rows_without_a_live_score_keep_their_carry(device, monkeypatch, D, summ
     for x, was in zip((o, m, l), before):
         same = (x == was).reshape(1, 2, 300, -1).all(-1).cpu()
         assert same[:, :, dead].all() and not same[:, :, ~dead].all()
+
+
+@pytest.mark.parametrize("Lq,Lk,D", [(129, 193, 64), (300, 415, 128), (512, 320, 128)])
+def test_each_wave_decides_by_its_own_cells_of_a_summary(device, Lq, Lk, D):
+    # cells of 32 x 32 that are -inf, zero, constant or mixed, in no order; whole rows and columns of cells of one kind
+    H, scale = 2, 1 / np.sqrt(D)
+    rng = np.random.default_rng(Lq + D)
+    nr, nc = -(-Lq // 32), -(-Lk // 32)
+    kinds = rng.integers(0, 4, (nr, nc))
+    kinds[1], kinds[:, 1], kinds[:, 2] = 1, 0, 1
+    grid = np.repeat(np.repeat(kinds, 32, 0), 32, 1)[:Lq, :Lk]
+    values = rng.standard_normal((Lq, Lk)).astype(np.float32)
+    values[values > 1] = -np.inf
+    block = np.select([grid == 0, grid == 1, grid == 2], [np.float32(-np.inf), np.float32(0), np.float32(0.7)], values)[None, None]
+    q, k, v, do = R.make_inputs(Lq, 1, Lq, Lk, H, D)
+    tq, tk, tv, tdo = (_dev(x, device, torch.bfloat16).permute(0, 2, 1, 3) for x in (q, k, v, do))
+    carry = rr.init_carry(1, H, Lq, D, tq.device)
+    ra.fwd_block(tq, tk, tv, _dev(block, device), *carry, scale)
+    out, lse = torch.empty((1, H, Lq, D), device=device), torch.empty((1, H, Lq), device=device)
+    rr.finalize_carry(*carry, out, lse)
+    want, want_lse = R.mha_dense(q, k, v, block)
+    assert np.isfinite(want_lse).all()
+    assert np.abs(out.permute(0, 2, 1, 3).cpu().numpy() - want).max() <= OUT_TOL
+    assert np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_TOL
+    grads = ra.bwd_block(tq, tk, tv, _dev(block, device), out, lse, tdo, scale)
+    for got, ref in zip(grads, R.mha_dense_grads(q, k, v, do, block)):
+        assert max(_rel(got.permute(0, 2, 1, 3).cpu().numpy(), ref)) <= GRAD_TOL

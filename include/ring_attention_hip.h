@@ -288,6 +288,18 @@ int ra_bwd_pair(const ra_bwd_step_params* p, const void* out, int32_t out_dtype,
                 int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same two calls for every head dim that is a multiple of 32 up to 128 (dense blocks at 64 and 128
+ * only). */
+int64_t ra_fwd_whole_workspace(const ra_fwd_step_params* p);
+int ra_fwd_whole(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b,
+                 int64_t out_stride_h, int64_t out_stride_l, float* lse, void* workspace,
+                 int64_t workspace_bytes, void* stream);
+int64_t ra_bwd_whole_workspace(const ra_bwd_step_params* p);
+int ra_bwd_whole(const ra_bwd_step_params* p, const void* out, int32_t out_dtype, int64_t out_stride_b,
+                 int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
+                 int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
+                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* The elementwise entry points for the shards of n_passes passes in one launch: the fp32 arrays of
  * the passes (carries, accumulators, lse, delta) lie one after another ([n_passes, B, H, L, ...]),
  * pass p reads / writes its strided tensor at an offset of p * stride_pass elements.  With

@@ -50,7 +50,8 @@ constexpr int kMaxWindow = 1 << 30;  // wider than any position difference: mask
 constexpr int kMaxLen = 1 << 24;
 constexpr int kMaxSegLen = 65536;  // tile-list capacity of the kernels (1024 tiles x 64)
 
-int check_dims(int B, int H, int Lq, int Lk, int D) {
+// any_dim: the calls on whole sequences, which take every multiple of 32
+int check_dims(int B, int H, int Lq, int Lk, int D, bool any_dim = false) {
   if (B <= 0 || H <= 0 || Lq <= 0 || Lk <= 0)
     return fail(RA_ERR_SHAPE, "B, H, Lq, Lk must be positive (got %d, %d, %d, %d)", B, H, Lq, Lk);
   if (Lq > kMaxLen || Lk > kMaxLen)
@@ -62,7 +63,8 @@ int check_dims(int B, int H, int Lq, int Lk, int D) {
   if ((int64_t)B * H * tiles > 0x7fffffffll)
     return fail(RA_ERR_SHAPE, "B*H*ceil(L/128) = %lld workgroups exceed the grid limit of 2^31-1",
                 (long long)((int64_t)B * H * tiles));
-  if (D != 64 && D != 128) return fail(RA_ERR_HEAD_DIM, "head dim %d unsupported (64 or 128)", D);
+  if (any_dim ? (D < 32 || D > 128 || D % 32) : (D != 64 && D != 128))
+    return fail(RA_ERR_HEAD_DIM, any_dim ? "head dim %d unsupported (32, 64, 96 or 128)" : "head dim %d unsupported (64 or 128)", D);
   return RA_OK;
 }
 
@@ -785,21 +787,31 @@ int64_t fwd_part_bytes(const ra_fwd_step_params& p, int n_split) {
 
 extern "C" {
 
-int ra_version(void) { return 1008; }
+int ra_version(void) { return 1009; }
 
-int64_t ra_fwd_pair_workspace(const ra_fwd_step_params* p) {
-  if (!p || check_dims(p->B, p->H, p->Lq, p->Lk, p->D)) return 0;
+static int64_t fwd_pair_workspace(const ra_fwd_step_params* p, bool any_dim) {
+  if (!p || check_dims(p->B, p->H, p->Lq, p->Lk, p->D, any_dim)) return 0;
   const int n = plan_fwd_pair(*p).n_split;
   return n > 1 ? fwd_part_bytes(*p, n) : 0;
 }
 
-int ra_fwd_pair(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b, int64_t out_stride_h,
-                int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
+// A head dim that only the kernels of ra_pair.hip have, and those without a dense block.
+static bool narrow(int D) { return D != 64 && D != 128; }
+static int check_whole_call(const char* what, int D, const ra_bias& bias) {
+  if (narrow(D) && (bias.flags & RA_BIAS_DENSE))
+    return fail(RA_ERR_HEAD_DIM, "%s: head dim %d with a dense block (64 or 128)", what, D);
+  return RA_OK;
+}
+static int check_fwd_step(const ra_fwd_step_params* p, bool any_dim);
+static int check_bwd_step(const ra_bwd_step_params* p, bool any_dim);
+
+static int fwd_pair(const ra_fwd_step_params* p, bool any_dim, void* out, int32_t out_dtype, int64_t out_stride_b, int64_t out_stride_h,
+                    int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
   if (!p) return fail(RA_ERR_NULL, "params is NULL");
   ra_fwd_step_params c = *p;
   c.o = c.m = c.l = reinterpret_cast<float*>(uintptr_t(16));  // not used: there is no carry
-  int rc = ra_fwd_step_check(&c);
-  if (rc) return rc;
+  int rc = check_fwd_step(&c, any_dim);
+  if (rc || (rc = check_whole_call("ra_fwd_whole", c.D, c.bias))) return rc;
   if (!lse) return fail(RA_ERR_NULL, "ra_fwd_pair: lse is NULL");
   const RingResult r{out, nullptr, lse, out_dtype, 0, out_stride_b, out_stride_h, out_stride_l};
   if ((rc = check_ring_result("ra_fwd_pair", r))) return rc;
@@ -837,6 +849,18 @@ int ra_fwd_pair(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64
   return e == hipSuccess ? RA_OK : hip_fail(e, "ra_fwd_pair launch");
 }
 
+int64_t ra_fwd_pair_workspace(const ra_fwd_step_params* p) { return fwd_pair_workspace(p, false); }
+int64_t ra_fwd_whole_workspace(const ra_fwd_step_params* p) { return fwd_pair_workspace(p, true); }
+
+int ra_fwd_pair(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b, int64_t out_stride_h,
+                int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
+  return fwd_pair(p, false, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, lse, workspace, workspace_bytes, stream);
+}
+int ra_fwd_whole(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b, int64_t out_stride_h,
+                 int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
+  return fwd_pair(p, true, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, lse, workspace, workspace_bytes, stream);
+}
+
 const char* ra_last_error(void) { return g_err; }
 
 int ra_step_is_skippable(const ra_bias* bias, int32_t Lq, int32_t Lk) {
@@ -852,9 +876,9 @@ int ra_step_is_skippable(const ra_bias* bias, int32_t Lq, int32_t Lk) {
   return 0;
 }
 
-int ra_fwd_step_check(const ra_fwd_step_params* p) {
+static int check_fwd_step(const ra_fwd_step_params* p, bool any_dim) {
   if (!p) return fail(RA_ERR_NULL, "params is NULL");
-  int rc = check_dims(p->B, p->H, p->Lq, p->Lk, p->D);
+  int rc = check_dims(p->B, p->H, p->Lq, p->Lk, p->D, any_dim);
   if (rc) return rc;
   if ((rc = check_tensor("q", p->q, p->D))) return rc;
   if ((rc = check_tensor("k", p->k, p->D))) return rc;
@@ -866,9 +890,9 @@ int ra_fwd_step_check(const ra_fwd_step_params* p) {
   return check_bias(p->bias, p->Lq, p->Lk);
 }
 
-int ra_bwd_step_check(const ra_bwd_step_params* p) {
+static int check_bwd_step(const ra_bwd_step_params* p, bool any_dim) {
   if (!p) return fail(RA_ERR_NULL, "params is NULL");
-  int rc = check_dims(p->B, p->H, p->Lq, p->Lk, p->D);
+  int rc = check_dims(p->B, p->H, p->Lq, p->Lk, p->D, any_dim);
   if (rc) return rc;
   if ((rc = check_tensor("q", p->q, p->D))) return rc;
   if ((rc = check_tensor("k", p->k, p->D))) return rc;
@@ -882,6 +906,9 @@ int ra_bwd_step_check(const ra_bwd_step_params* p) {
     return fail(RA_ERR_SHAPE, "sm_scale must be a positive finite number");
   return check_bias(p->bias, p->Lq, p->Lk);
 }
+
+int ra_fwd_step_check(const ra_fwd_step_params* p) { return check_fwd_step(p, false); }
+int ra_bwd_step_check(const ra_bwd_step_params* p) { return check_bwd_step(p, false); }
 
 int ra_fwd_init(float* o, float* m, float* l, int32_t B, int32_t H, int32_t Lq, int32_t D, void* stream) {
   if (!o || !m || !l) return fail(RA_ERR_NULL, "carry pointer (o, m or l) is NULL");
@@ -1072,25 +1099,26 @@ int ra_bwd_dkdv_ring(const ra_bwd_step_params* steps, const int32_t* steps_per_p
   return bwd_dkdv_passes(steps, first, n_passes, stream, &r);
 }
 
-int64_t ra_bwd_pair_workspace(const ra_bwd_step_params* p) {
-  if (!p || check_dims(p->B, p->H, p->Lq, p->Lk, p->D)) return 0;
+static int64_t bwd_pair_workspace(const ra_bwd_step_params* p, bool any_dim) {
+  if (!p || check_dims(p->B, p->H, p->Lq, p->Lk, p->D, any_dim)) return 0;
   return bwd_space(*p, plan_dq_pair(*p), plan_dkdv_pair(*p)).total;
 }
 
-int ra_bwd_pair(const ra_bwd_step_params* p, const void* out, int32_t out_dtype, int64_t out_stride_b,
+static int bwd_pair(const ra_bwd_step_params* p, bool any_dim, const void* out, int32_t out_dtype, int64_t out_stride_b,
                 int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
                 int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
   if (!p) return fail(RA_ERR_NULL, "params is NULL");
   ra_bwd_step_params c = *p;
   c.delta = c.dq = c.dk = c.dv = reinterpret_cast<float*>(uintptr_t(16));  // not used: no accumulators
-  int rc = ra_bwd_step_check(&c);
-  if (rc) return rc;
+  int rc = check_bwd_step(&c, any_dim);
+  if (rc || (rc = check_whole_call("ra_bwd_whole", c.D, c.bias))) return rc;
   const RingResult rq{dq, nullptr, nullptr, RA_DTYPE_BF16, 0, dq_stride_b, dq_stride_h, dq_stride_l};
   const RingResult rk{dk, dv, nullptr, RA_DTYPE_BF16, 0, dkv_stride_b, dkv_stride_h, dkv_stride_l};
   if ((rc = check_ring_result("ra_bwd_pair", rq)) || (rc = check_ring_result("ra_bwd_pair", rk))) return rc;
   if (!dv) return fail(RA_ERR_NULL, "ra_bwd_pair: dv is NULL");
   const PairPlan plan_q = plan_dq_pair(*p), plan_k = plan_dkdv_pair(*p);
+  if (!plan_k.pair && narrow(c.D)) return fail(RA_ERR_TOO_LARGE, "ra_bwd_whole: too many rows");
   const BwdSpace sp = bwd_space(*p, plan_q, plan_k);
   if (!workspace || !aligned16(workspace)) return fail(RA_ERR_ALIGN, "ra_bwd_pair: the workspace must be 16-byte aligned");
   if (workspace_bytes < sp.total) return fail(RA_ERR_SHAPE, "ra_bwd_pair: the workspace is smaller than ra_bwd_pair_workspace()");
@@ -1130,6 +1158,24 @@ int ra_bwd_pair(const ra_bwd_step_params* p, const void* out, int32_t out_dtype,
   share(plan_q, sp.dq_part, sp.dq_n, rq);
   e = ra::launch_dq_pair(a, c.D, mode, (hipStream_t)stream);
   return e == hipSuccess ? RA_OK : hip_fail(e, "ra_bwd_pair launch");
+}
+
+int64_t ra_bwd_pair_workspace(const ra_bwd_step_params* p) { return bwd_pair_workspace(p, false); }
+int64_t ra_bwd_whole_workspace(const ra_bwd_step_params* p) { return bwd_pair_workspace(p, true); }
+
+int ra_bwd_pair(const ra_bwd_step_params* p, const void* out, int32_t out_dtype, int64_t out_stride_b,
+                int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
+                int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
+                int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
+  return bwd_pair(p, false, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h, dq_stride_l, dk, dv, dkv_stride_b,
+                  dkv_stride_h, dkv_stride_l, workspace, workspace_bytes, stream);
+}
+int ra_bwd_whole(const ra_bwd_step_params* p, const void* out, int32_t out_dtype, int64_t out_stride_b,
+                int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
+                int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
+                int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
+  return bwd_pair(p, true, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h, dq_stride_l, dk, dv, dkv_stride_b,
+                  dkv_stride_h, dkv_stride_l, workspace, workspace_bytes, stream);
 }
 
 int ra_convert(const ra_rows* items, int32_t n_items, void* stream) {

@@ -1,5 +1,5 @@
 // Between a caller's arrays (bf16, fp16 or fp32, any head dim up to 128) and the operands of the
-// attention kernels (bf16, head dim 64 or 128): conversion and padding in one pass, several arrays in
+// attention kernels (bf16, head dim 32, 64, 96 or 128): conversion and padding in one pass, several arrays in
 // one launch.
 #include "ra_launch.h"
 

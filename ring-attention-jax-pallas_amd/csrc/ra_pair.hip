@@ -79,7 +79,9 @@ RA_DEV int opaque_lane(int lane) {
 // moves both addresses, and what the rows are further apart in memory than in LDS is in the lanes' offsets,
 // a register per instruction.  (With a base and an LDS address of its own per instruction a tile took 50 scalar
 // instructions of a wave's 120.)
-template <int D, int ROWS>
+// LIVE: the elements of a row that there are to move; the lanes of the rest of the pitch D fetch a chunk that another lane moves
+// too, which nothing reads.
+template <int D, int ROWS, int LIVE = D>
 struct TileLoader {
   static constexpr int CPR = D / 8;            // 16-byte chunks per row
   static constexpr int RPI = 64 / CPR;         // rows per load instruction
@@ -101,7 +103,8 @@ struct TileLoader {
   // byte offset inside its row of the chunk that a lane moves with the instruction that starts at `row` of a tile
   static RA_DEV unsigned chunk(int row, int lane) {
     const int r = row + lane / CPR;
-    return (unsigned)(tile_off<D>(r, lane % CPR) - r * (D * 2));
+    const unsigned c = (unsigned)(tile_off<D>(r, lane % CPR) - r * (D * 2));
+    return LIVE < D && c >= LIVE * 2 ? c - (D - LIVE) * 2 : c;
   }
   // tile of the rows from row0 on, to the LDS address dst of the whole tile
   RA_DEV void issue(int row0, unsigned dst, int wave, int lane) const {
@@ -427,12 +430,17 @@ struct TileWalk {
 };
 
 // S^T orientation as in fwd_step_kernel: a lane owns one query row and 16 keys of a 32-key block.
-// D is the row pitch of the LDS tiles (64 or 128 elements).
-template <int D, int MODE>
+// DL is the head dim, a multiple of 32; the LDS tiles keep a row pitch D of 64 or 128 elements, whose layout both operand
+// fetches know, and what lies beyond DL is neither multiplied nor stored.  Padded to 64 or 128 | in the head dim itself, whole training
+// calls: D=96, 32768 causal, H=16 15.2 | 13.4 ms (padded on the long-stretch kernels), window 4096 4.32 | 3.47, causal 4096, B=2,
+// H=16 659 | 496 us, unmasked 8192 x 16384 3.79 | 3.47 ms; D=32, 32768 causal, H=16 8.2 | 6.0 ms; fp16, D=96, 1047 x 4791, B=2, H=8 283 |
+// 229 us, conversions included.
+template <int DL, int MODE>
 __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwdArgs a) {
   constexpr bool GENERAL = MODE != 0;
   constexpr bool DENSE = MODE == 2;
-  constexpr int KS = D / 16, DB = D / 32;
+  constexpr int D = DL <= 64 ? 64 : 128;  // row pitch of the LDS tiles
+  constexpr int KS = DL / 16, DB = DL / 32;
   constexpr int ROWB = D * 2;
   constexpr int TILE_BYTES = kPairKeys * ROWB;
   __shared__ __attribute__((aligned(16))) char s_k[2][TILE_BYTES];
@@ -519,7 +527,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     if ((flags & RA_BIAS_DENSE) && dmap == nullptr) every_test |= kTestDense;
   }
 
-  TileLoader<D, kPairKeys> ldk, ldv;
+  TileLoader<D, kPairKeys, DL> ldk, ldv;
   ldk.init(a.k.ptr + b * a.k.sb + h * a.k.sh, a.k.sl, a.Lk, wave, lane);
   ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, wave, lane);
   auto issue_tile = [&](int j, int buf) {
@@ -558,7 +566,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     const FragOffsets<D> fr_off = fo.opaque();
     // K operands in the order of use, both key blocks of 16 head-dim elements in turn; the first ones
     // are on their way while the next tile is requested
-    constexpr int PFK = 4;
+    constexpr int PFK = 4 < 2 * KS ? 4 : 2 * KS;
     bf16x8 kf[2 * KS];
     auto k_frag = [&](int op) { return *(const bf16x8*)(s_k[BUF] + 32 * (op & 1) * ROWB + fr_off.nat(op >> 1)); };
 #pragma unroll
@@ -604,9 +612,11 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
       S[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[1], qf[0], zero, 0, 0, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
-    kf[PFK] = k_frag(PFK);
-    kf[PFK + 1] = k_frag(PFK + 1);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (PFK < 2 * KS) {
+      kf[PFK] = k_frag(PFK);
+      kf[PFK + 1] = k_frag(PFK + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int op = 2; op < 2 * KS; ++op) {
       if (op + PFK < 2 * KS) kf[op + PFK] = k_frag(op + PFK);
@@ -698,7 +708,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
       oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], pf[ks], oacc[db], 0, 0, 0);
       if (ks < 3) {
 #pragma unroll
-        for (int e = 0; e < 8 / DB; e += 2) soft(ks + 1, db * (8 / DB) + e);
+        for (int e = 4 * db / DB; e < 4 * (db + 1) / DB; ++e) soft(ks + 1, 2 * e);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -734,7 +744,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   if (n_piece > 1) {
     // a share of the row's keys: combined by pair_combine_kernel
     const long long prow = (long long)split * ((long long)e->B * e->H * e->Lq) + row;
-    float* op = e->part_o + prow * D + 4 * g;
+    float* op = e->part_o + prow * DL + 4 * g;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -752,7 +762,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     const float f_in = fast_exp2(m_in - m_safe);
     const float f_step = (l_step > 0.f) ? fast_exp2(m_run - m_safe) : 0.f;
     const float f_o = f_step * ((lr_step > 0.f) ? l_step / lr_step : 1.f);
-    float* op = e->o + row * D + 4 * g;
+    float* op = e->o + row * DL + 4 * g;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -824,11 +834,12 @@ __global__ __launch_bounds__(256) void pair_combine_kernel(const PairFwdArgs a) 
 // The same split: 128 query rows per workgroup (Q and dO in registers), 64-key tiles of K and V in two
 // LDS buffers, scores transposed (S^T = K Q^T, dP^T = V dO^T) so that dS^T is the B operand of
 // dQ^T = K^T dS^T, whose A operand comes from the K tile through the transposing read.
-template <int D, int MODE>
-__global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(const PairBwdArgs p) {
+template <int DL, int MODE>
+__global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel(const PairBwdArgs p) {
   constexpr bool GENERAL = MODE != 0;
   constexpr bool DENSE = MODE == 2;
-  constexpr int KS = D / 16, DB = D / 32;
+  constexpr int D = DL <= 64 ? 64 : 128;  // row pitch of the LDS tiles
+  constexpr int KS = DL / 16, DB = DL / 32;
   constexpr int ROWB = D * 2;
   constexpr int TILE_BYTES = kPairKeys * ROWB;
   const BwdArgs& a = p.a;
@@ -919,7 +930,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
     if (!use_list && (flags & RA_BIAS_PREFIX)) every_test |= kTestPrefix;
     if ((flags & RA_BIAS_DENSE) && dmap == nullptr) every_test |= kTestDense;
   }
-  TileLoader<D, kPairKeys> ldk, ldv;
+  TileLoader<D, kPairKeys, DL> ldk, ldv;
   ldk.init(a.k.ptr + b * a.k.sb + h * a.k.sh, a.k.sl, a.Lk, wave, lane);
   ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, wave, lane);
   auto issue_tile = [&](int j, int buf) {
@@ -975,7 +986,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
     for (int kb = 0; kb < 2; ++kb) {
       // S^T first, then dP^T with the exp2 of S in its shadow: dP^T takes no registers while the terms
       // of a biased tile are evaluated
-      constexpr int PF = 3;  // operand fetches in flight ahead of the matrix instruction that uses them
+      constexpr int PF = KS < 3 ? KS : 3;  // operand fetches in flight ahead of the matrix instruction that uses them
       f32x16 S, zero;
 #pragma unroll
       for (int r = 0; r < 16; ++r) zero[r] = 0.f;
@@ -995,8 +1006,10 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
           S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[0], qf[0], zero, 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
-        fr[PF] = nat_frag(s_k[BUF], PF);
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (PF < KS) {
+          fr[PF] = nat_frag(s_k[BUF], PF);
+          __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int op = 1; op < KS; ++op) {
           if (op + PF < KS) fr[op + PF] = nat_frag(s_k[BUF], op + PF);
@@ -1036,10 +1049,10 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
           if (op + PF < KS) fr[op + PF] = nat_frag(s_v[BUF], op + PF);
           P = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], dof[op], P, 0, 0, 0);
 #pragma unroll
-          for (int e = 0; e < 16 / KS; ++e) {
-            float x = fast_exp2(fmaf(S[op * (16 / KS) + e], a.scale_res, neg_lse2));
+          for (int e = 16 * op / KS; e < 16 * (op + 1) / KS; ++e) {
+            float x = fast_exp2(fmaf(S[e], a.scale_res, neg_lse2));
             asm volatile("" : "+v"(x));
-            S[op * (16 / KS) + e] = x;
+            S[e] = x;
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -1067,7 +1080,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
       };
       bf16x8 fr[2 * DB];
 #pragma unroll
-      for (int op = 0; op < PF; ++op) fr[op] = k_frag(op);
+      for (int op = 0; op < (PF < 2 * DB ? PF : 2 * DB); ++op) fr[op] = k_frag(op);
 #pragma unroll
       for (int e = 0; e < 8; e += 2) grad(0, e);
       __builtin_amdgcn_sched_barrier(0);
@@ -1078,7 +1091,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
         acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], dsf[ks], acc[db], 0, 0, 0);
         if (ks < 1) {
 #pragma unroll
-          for (int e = 0; e < 8 / DB; e += 2) grad(1, db * (8 / DB) + e);
+          for (int e = 4 * db / DB; e < 4 * (db + 1) / DB; ++e) grad(1, 2 * e);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -1098,8 +1111,8 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dq_pair_kernel(
   if (e->part_n != nullptr && split == 0 && tid == 0) e->part_n[hh * nqt + qt] = n_piece;
   if (!q_valid) return;
   float* fp = nullptr;  // fp32 destination: a share of the sum, or an accumulator
-  if (n_piece > 1) fp = e->part + ((long long)split * ((long long)e->a.B * e->a.H * e->a.Lq) + row) * D;
-  else if (e->acc != nullptr) fp = e->acc + row * D;
+  if (n_piece > 1) fp = e->part + ((long long)split * ((long long)e->a.B * e->a.H * e->a.Lq) + row) * DL;
+  else if (e->acc != nullptr) fp = e->acc + row * DL;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -1207,11 +1220,12 @@ RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg
 // Three workgroups per compute unit at D = 64: 168 registers hold everything once V is in LDS.  With V in registers too 5
 // (MODE 0) and 12 (MODE 1) of them spill, and a reload inside the loop waits for the tile loads that were just issued:
 // causal + ALiBi, 4096, B=2, H=16, 240 us against 189; causal documents of 2175 in 48128, B=2, H=4, 636 against 531.
-template <int D, int MODE>
-__global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kernel(const PairBwdArgs p) {
+template <int DL, int MODE>
+__global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dkdv_pair_kernel(const PairBwdArgs p) {
   constexpr bool GENERAL = MODE != 0;
   constexpr bool DENSE = MODE == 2;
-  constexpr int KS = D / 16, DB = D / 32;
+  constexpr int D = DL <= 64 ? 64 : 128;  // row pitch of the LDS tiles
+  constexpr int KS = DL / 16, DB = DL / 32;
   constexpr int ROWB = D * 2;
   constexpr int TILE_BYTES = kPairQueries * ROWB;
   const BwdArgs& a = p.a;
@@ -1300,7 +1314,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
     if (!use_list && (flags & RA_BIAS_PREFIX)) every_test |= kTestPrefix;
     if ((flags & RA_BIAS_DENSE) && dmap == nullptr) every_test |= kTestDense;
   }
-  TileLoader<D, kPairQueries> ldq, ldo;
+  TileLoader<D, kPairQueries, DL> ldq, ldo;
   ldq.init(a.q.ptr + b * a.q.sb + h * a.q.sh, a.q.sl, a.Lq, wave, lane);
   ldo.init(a.dout.ptr + b * a.dout.sb + h * a.dout.sh, a.dout.sl, a.Lq, wave, lane);
   // lanes 0..31 move -lse of a tile's rows, lanes 32..63 -delta
@@ -1369,7 +1383,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
       if (alibi_on && !one_side) tests |= kTestAlibi;
     }
     if (!wt.plain(j)) tests |= kTestPos;
-    constexpr int PF = 3;  // operand fetches in flight ahead of the matrix instruction that uses them
+    constexpr int PF = KS < 3 ? KS : 3;  // operand fetches in flight ahead of the matrix instruction that uses them
     f32x16 S;
 #pragma unroll
     for (int bb = 0; bb < 4; ++bb) {
@@ -1450,8 +1464,8 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
         }
         P = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], vr[op], P, 0, 0, 0);
 #pragma unroll
-        for (int e = 0; e < 16 / KS; e += 2) {
-          const int r = op * (16 / KS) + e;
+        for (int e = 8 * op / KS; e < 8 * (op + 1) / KS; ++e) {
+          const int r = 2 * e;
           float x0 = fast_exp2(S[r] * a.scale_res), x1 = fast_exp2(S[r + 1] * a.scale_res);
           bf16x2 pr;
           pr[0] = (bf16_t)x0;
@@ -1490,8 +1504,8 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
         if (op < 2 * DB) {
           dv[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pf[ks], fr[op], dv[db], 0, 0, 0);
 #pragma unroll
-          for (int e = 0; e < 16 / (2 * DB); e += 2) {
-            const int r = op * (16 / (2 * DB)) + e;
+          for (int e = 8 * op / (2 * DB); e < 8 * (op + 1) / (2 * DB); ++e) {
+            const int r = 2 * e;
             bf16x2 pr;
             pr[0] = (bf16_t)(S[r] * P[r]);
             pr[1] = (bf16_t)(S[r + 1] * P[r + 1]);
@@ -1510,7 +1524,7 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
   };
 
   if (i_lo < i_hi) {
-    TileLoader<D, kPairSlab> ldv;
+    TileLoader<D, kPairSlab, DL> ldv;
     ldv.init(a.v.ptr + b * a.v.sb + h * a.v.sh, a.v.sl, a.Lk, wave, lane);
     ldv.issue(k0, RA_LDS_ADDR(&s_v[0]), wave, lane);
     walk.start(GENERAL && use_list, s_list, j_lo, i_lo, i_hi, every_test);
@@ -1529,24 +1543,24 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
     // All loads of an array are issued before the first value is needed (see dkdv_kernel): a block of values, L=256, H=8, D=128,
     // 64.7 us with a load - add - store chain per element, 35.6 without; L=128, H=2, D=64, 36.4 and 19.8.
     auto add_to = [&](float* acc, const f32x16 (&x)[DB], float mul) {
-      float* const at = acc + ((long long)hh * e->a.Lk + kw + 4 * g) * D + l32;
+      float* const at = acc + ((long long)hh * e->a.Lk + kw + 4 * g) * DL + l32;
       if (kw + 32 <= e->a.Lk) {  // (wave-uniform)
         float old[DB][16];
 #pragma unroll
         for (int r = 0; r < 16; ++r)
 #pragma unroll
-          for (int db = 0; db < DB; ++db) old[db][r] = at[(8 * (r / 4) + r % 4) * D + 32 * db];
+          for (int db = 0; db < DB; ++db) old[db][r] = at[(8 * (r / 4) + r % 4) * DL + 32 * db];
 #pragma unroll
         for (int r = 0; r < 16; ++r)
 #pragma unroll
-          for (int db = 0; db < DB; ++db) at[(8 * (r / 4) + r % 4) * D + 32 * db] = fmaf(x[db][r], mul, old[db][r]);
+          for (int db = 0; db < DB; ++db) at[(8 * (r / 4) + r % 4) * DL + 32 * db] = fmaf(x[db][r], mul, old[db][r]);
       } else {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int row = 8 * (r / 4) + r % 4;
           if (kw + 4 * g + row >= e->a.Lk) continue;
 #pragma unroll
-          for (int db = 0; db < DB; ++db) at[row * D + 32 * db] += x[db][r] * mul;
+          for (int db = 0; db < DB; ++db) at[row * DL + 32 * db] += x[db][r] * mul;
         }
       }
     };
@@ -1559,11 +1573,11 @@ __global__ __launch_bounds__(kPairThreads, D == 64 ? 3 : 2) void dkdv_pair_kerne
     const int key = kw + 4 * g + 8 * (r / 4) + (r % 4);
     if (key >= e->a.Lk) continue;
     if (n_piece > 1) {
-      float* fp = e->part + ((long long)split * 2 * rows + (long long)hh * e->a.Lk + key) * D + l32;
+      float* fp = e->part + ((long long)split * 2 * rows + (long long)hh * e->a.Lk + key) * DL + l32;
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         fp[32 * db] = dk[db][r] * e->a.sm_scale;
-        fp[rows * D + 32 * db] = dv[db][r];
+        fp[rows * DL + 32 * db] = dv[db][r];
       }
     } else {
       const long long at = b * e->out_sb + h * e->out_sh + (long long)key * e->out_sl + l32;
@@ -1583,12 +1597,12 @@ template <typename OutT, int D>
 __global__ __launch_bounds__(256) void pair_stat_kernel(const OutT* out, long long sb, long long sh, long long sl, TensorArg dout,
                                                         const float* lse, float inv_res, float* stat, float* delta, int B, int H,
                                                         int Lq) {
-  constexpr int CPR = D / 8;
+  constexpr int CPR = D == 96 ? 16 : D / 8;  // lanes per row (a power of two)
   const long long rows = (long long)B * H * Lq;
   const long long row = (long long)blockIdx.x * (256 / CPR) + threadIdx.x / CPR;
   const int c = threadIdx.x % CPR;
   float acc = 0.f;
-  if (row < rows) {
+  if (row < rows && c < D / 8) {
     const int li = (int)(row % Lq);
     const long long hh = row / Lq;
     const int h = (int)(hh % H);
@@ -1636,14 +1650,31 @@ static hipError_t launch_pair_sum(const PairBwdArgs& p, int n_out, int L, hipStr
   return hipGetLastError();
 }
 
+// The kernels of a head dim: a multiple of 32, dense blocks at 64 and 128 only.
+template <typename Launch>
+static hipError_t with_dim(int D, int mode, Launch launch) {
+  if (mode < 0 || mode > 2 || (mode == 2 && D != 64 && D != 128)) return hipErrorInvalidValue;
+  switch (D) {
+    case 32: return launch(std::integral_constant<int, 32>{});
+    case 64: return launch(std::integral_constant<int, 64>{});
+    case 96: return launch(std::integral_constant<int, 96>{});
+    case 128: return launch(std::integral_constant<int, 128>{});
+  }
+  return hipErrorInvalidValue;
+}
+
 template <int D>
 static hipError_t launch_dq_pair_d(const PairBwdArgs& p, int mode, hipStream_t stream) {
   const BwdArgs& a = p.a;
   const int nqt = (a.Lq + kPairRows - 1) / kPairRows;
   dim3 grid((unsigned)(a.B * a.H * p.n_split * nqt)), block(kPairThreads);
-  if (mode == 2) hipLaunchKernelGGL((dq_pair_kernel<D, 2>), grid, block, 0, stream, p);
-  else if (mode == 1) hipLaunchKernelGGL((dq_pair_kernel<D, 1>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((dq_pair_kernel<D, 0>), grid, block, 0, stream, p);
+  if (mode == 2) {
+    if constexpr (D == 64 || D == 128) hipLaunchKernelGGL((dq_pair_kernel<D, 2>), grid, block, 0, stream, p);
+  } else if (mode == 1) {
+    hipLaunchKernelGGL((dq_pair_kernel<D, 1>), grid, block, 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((dq_pair_kernel<D, 0>), grid, block, 0, stream, p);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.n_split == 1) return e;
   return launch_pair_sum<D, kPairRows>(p, 1, a.Lq, stream);
@@ -1654,44 +1685,49 @@ static hipError_t launch_dkdv_pair_d(const PairBwdArgs& p, int mode, hipStream_t
   const BwdArgs& a = p.a;
   const int nkt = (a.Lk + kPairSlab - 1) / kPairSlab;
   dim3 grid((unsigned)(a.B * a.H * p.n_split * nkt)), block(kPairThreads);
-  if (mode == 2) hipLaunchKernelGGL((dkdv_pair_kernel<D, 2>), grid, block, 0, stream, p);
-  else if (mode == 1) hipLaunchKernelGGL((dkdv_pair_kernel<D, 1>), grid, block, 0, stream, p);
-  else hipLaunchKernelGGL((dkdv_pair_kernel<D, 0>), grid, block, 0, stream, p);
+  if (mode == 2) {
+    if constexpr (D == 64 || D == 128) hipLaunchKernelGGL((dkdv_pair_kernel<D, 2>), grid, block, 0, stream, p);
+  } else if (mode == 1) {
+    hipLaunchKernelGGL((dkdv_pair_kernel<D, 1>), grid, block, 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((dkdv_pair_kernel<D, 0>), grid, block, 0, stream, p);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.n_split == 1) return e;
   return launch_pair_sum<D, kPairSlab>(p, 2, a.Lk, stream);
 }
 
 hipError_t launch_dkdv_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream) {
-  return D == 128 ? launch_dkdv_pair_d<128>(p, mode, stream) : launch_dkdv_pair_d<64>(p, mode, stream);
+  return with_dim(D, mode, [&](auto d) { return launch_dkdv_pair_d<d.value>(p, mode, stream); });
 }
 
 hipError_t launch_pair_stat(const void* out, int out_f32, long long sb, long long sh, long long sl, TensorArg dout, const float* lse,
                             float inv_res, float* stat, float* delta, int B, int H, int Lq, int D, hipStream_t stream) {
   const long long rows = (long long)B * H * Lq;
-  const int rpb = 256 / (D / 8);
+  const int rpb = 256 / (D == 96 ? 16 : D / 8);
   dim3 grid((unsigned)((rows + rpb - 1) / rpb)), block(256);
-  if (D == 128) {
-    if (out_f32) hipLaunchKernelGGL((pair_stat_kernel<float, 128>), grid, block, 0, stream, (const float*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
-    else hipLaunchKernelGGL((pair_stat_kernel<bf16_t, 128>), grid, block, 0, stream, (const bf16_t*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
-  } else {
-    if (out_f32) hipLaunchKernelGGL((pair_stat_kernel<float, 64>), grid, block, 0, stream, (const float*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
-    else hipLaunchKernelGGL((pair_stat_kernel<bf16_t, 64>), grid, block, 0, stream, (const bf16_t*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
-  }
-  return hipGetLastError();
+  return with_dim(D, 0, [&](auto d) {
+    if (out_f32) hipLaunchKernelGGL((pair_stat_kernel<float, d.value>), grid, block, 0, stream, (const float*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
+    else hipLaunchKernelGGL((pair_stat_kernel<bf16_t, d.value>), grid, block, 0, stream, (const bf16_t*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
+    return hipGetLastError();
+  });
 }
 
 hipError_t launch_dq_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream) {
-  return D == 128 ? launch_dq_pair_d<128>(p, mode, stream) : launch_dq_pair_d<64>(p, mode, stream);
+  return with_dim(D, mode, [&](auto d) { return launch_dq_pair_d<d.value>(p, mode, stream); });
 }
 
 template <int D>
 static hipError_t launch_fwd_pair_d(const PairFwdArgs& a, int mode, hipStream_t stream) {
   const int nqt = (a.Lq + kPairRows - 1) / kPairRows;
   dim3 grid((unsigned)(a.B * a.H * a.n_split * nqt)), block(kPairThreads);
-  if (mode == 2) hipLaunchKernelGGL((fwd_pair_kernel<D, 2>), grid, block, 0, stream, a);
-  else if (mode == 1) hipLaunchKernelGGL((fwd_pair_kernel<D, 1>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((fwd_pair_kernel<D, 0>), grid, block, 0, stream, a);
+  if (mode == 2) {
+    if constexpr (D == 64 || D == 128) hipLaunchKernelGGL((fwd_pair_kernel<D, 2>), grid, block, 0, stream, a);
+  } else if (mode == 1) {
+    hipLaunchKernelGGL((fwd_pair_kernel<D, 1>), grid, block, 0, stream, a);
+  } else {
+    hipLaunchKernelGGL((fwd_pair_kernel<D, 0>), grid, block, 0, stream, a);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.part_o == nullptr) return e;
   const long long n = (long long)a.B * a.H * a.Lq * (D / 4);
@@ -1700,7 +1736,7 @@ static hipError_t launch_fwd_pair_d(const PairFwdArgs& a, int mode, hipStream_t 
 }
 
 hipError_t launch_fwd_pair(const PairFwdArgs& a, int D, int mode, hipStream_t stream) {
-  return D == 128 ? launch_fwd_pair_d<128>(a, mode, stream) : launch_fwd_pair_d<64>(a, mode, stream);
+  return with_dim(D, mode, [&](auto d) { return launch_fwd_pair_d<d.value>(a, mode, stream); });
 }
 
 }  // namespace ra

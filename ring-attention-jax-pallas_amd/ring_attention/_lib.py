@@ -99,6 +99,13 @@ EXPORTS = {
     "ra_bwd_pair": (C.c_int, [C.POINTER(RaBwdStepParams), C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64,
                               C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64,
                               C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p]),
+    "ra_fwd_whole_workspace": (C.c_int64, [C.POINTER(RaFwdStepParams)]),
+    "ra_fwd_whole": (C.c_int, [C.POINTER(RaFwdStepParams), C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64,
+                               C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p]),
+    "ra_bwd_whole_workspace": (C.c_int64, [C.POINTER(RaBwdStepParams)]),
+    "ra_bwd_whole": (C.c_int, [C.POINTER(RaBwdStepParams), C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64,
+                               C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64,
+                               C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p]),
     "ra_convert": (C.c_int, [C.c_char_p, C.c_int32, C.c_void_p]),  # ra_rows blocks, packed
     "ra_fwd_finalize_passes": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_int64,
                                          C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32, C.c_int32,

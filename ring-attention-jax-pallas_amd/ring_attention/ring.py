@@ -18,7 +18,8 @@ Public names follow the reference (``ring.py:246`` ``ring_attention``, ``ring.py
   [b, h | 1, lq, lk]`` (ring.py:107), whose dense block is materialised per ring step and
   streamed by the kernels.
 * Compute is bf16 on the matrix cores with fp32 carries; other input dtypes are cast on
-  entry and the result is cast back.  Head dims other than 64/128 are zero-padded.
+  entry and the result is cast back.  Head dims are zero-padded to 64 or 128, on whole sequences
+  (``_RingPlan._whole``) to the next multiple of 32.
 
 Everything runs through ``libringattn_hip.so``; if it is missing the import of this module
 succeeds but every call raises.
@@ -360,7 +361,7 @@ class _RingPlan:
     def __init__(self, q, k, n, fn: Optional[BiasFn], q_kwargs, kv_kwargs):
         self.n = n
         self.B, Sq, self.H, d = q.shape
-        self.D = _kernel_dim(d)
+        self.D, self.d_pair = _kernel_dim(d), -(-d // 32) * 32
         Sk = k.shape[1]
         if Sq % n or Sk % n:
             raise ValueError(f"sequence lengths ({Sq}, {Sk}) must be divisible by the ring size {n}")
@@ -463,7 +464,7 @@ class _RingPlan:
         is the ring of fewer, longer shards (one, for a sequence cut into n pieces in order) up to
         the order of the fp32 sums.  A kernel then runs its straight-line stretches through what
         were shard boundaries, and the host describes one shard pair instead of n * n, which also
-        has kernels of its own (``ra_fwd_pair``).  Forward + backward, unjoined -> joined: B=2, H=16, 8 x 1024 causal
+        has kernels of its own (``ra_fwd_whole``).  Forward + backward, unjoined -> joined: B=2, H=16, 8 x 1024 causal
         2.48 -> 2.11 ms; D=64, 4 x 1024 causal + ALiBi 0.73 -> 0.44; fp32 inputs, B=2, H=4, 8 x 256 of packed documents
         4.0 -> 0.25, nearly all of it host code.
         The joined shards stay within what one launch takes, with and without a segment term.  Where
@@ -481,8 +482,10 @@ class _RingPlan:
     def _join(self) -> "_RingPlan":
         n, Lq, Lk = self.n, self.Lq, self.Lk
         fn = self.fn
-        if self.callable is not None or n == 1:
+        if self.callable is not None:
             return self
+        if n == 1:
+            return self._whole()
         longest = _lib.RA_MAX_SEGMENT_SHARD if fn is not None and fn.segments else _lib.RA_MAX_SHARD
         for g in range(n, 1, -1):
             if n % g or g * max(Lq, Lk) > longest:
@@ -493,8 +496,18 @@ class _RingPlan:
                 plan.__dict__.update({a: x for a, x in self.__dict__.items() if not a.startswith("_")})
                 plan.n, plan.Lq, plan.Lk = n // g, g * Lq, g * Lk
                 plan.q_off, plan.kv_off = self.q_off[::g], self.kv_off[::g]
-                return plan
+                return plan._whole() if plan.n == 1 else plan
         return self
+
+    def _whole(self) -> "_RingPlan":
+        """A plan of one shard in the head dim that the whole-sequence calls take: the next multiple of 32
+        (everything else takes 64 and 128)."""
+        if self.D == self.d_pair:
+            return self
+        plan = object.__new__(_RingPlan)
+        plan.__dict__.update({a: x for a, x in self.__dict__.items() if not a.startswith("_")})
+        plan.D = self.d_pair
+        return plan
 
     def pair_bias(self) -> "_lib.RaBias":
         """The bias of a ring of one shard, as the library takes it: the plan holds the arrays."""
@@ -756,10 +769,10 @@ def _pair_forward(q, k, v, plan: "_RingPlan", sm_scale, out_dtype):
     p = _lib.RaFwdStepParams(B, H, Lq, plan.Lk, D, sm_scale, _view_blhd(q), _view_blhd(k), _view_blhd(v), None, None,
                              None, plan.pair_bias())
     lib = _lib.load()
-    size = lib.ra_fwd_pair_workspace(C.byref(p))
+    size = lib.ra_fwd_whole_workspace(C.byref(p))
     ws = torch.empty((size,), dtype=torch.uint8, device=plan.device) if size else None
-    _lib.check("ra_fwd_pair", lib.ra_fwd_pair(C.byref(p), out.data_ptr(), _DTYPE_CODE[out_dtype], Lq * H * D, D, H * D,
-                                              lse.data_ptr(), None if ws is None else ws.data_ptr(), size, _stream()))
+    _lib.check("ra_fwd_whole", lib.ra_fwd_whole(C.byref(p), out.data_ptr(), _DTYPE_CODE[out_dtype], Lq * H * D, D, H * D,
+                                                lse.data_ptr(), None if ws is None else ws.data_ptr(), size, _stream()))
     return out, lse
 
 
@@ -770,11 +783,11 @@ def _pair_backward(q, k, v, out, lse, do, plan: "_RingPlan", sm_scale):
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     p = _lib.RaBwdStepParams(B, H, Lq, Lk, D, sm_scale, _view_blhd(q), _view_blhd(k), _view_blhd(v), _view_blhd(do),
                              lse.data_ptr(), None, None, None, None, plan.pair_bias())
-    size = lib.ra_bwd_pair_workspace(C.byref(p))
+    size = lib.ra_bwd_whole_workspace(C.byref(p))
     ws = torch.empty((size,), dtype=torch.uint8, device=plan.device)
     assert dk.stride() == dv.stride()
     (ob, ol, oh, _), (qb, ql, qh, _), (kb, kl, kh, _) = out.stride(), dq.stride(), dk.stride()
-    _lib.check("ra_bwd_pair", lib.ra_bwd_pair(
+    _lib.check("ra_bwd_whole", lib.ra_bwd_whole(
         C.byref(p), out.data_ptr(), _DTYPE_CODE[out.dtype], ob, oh, ol, dq.data_ptr(), qb, qh, ql, dk.data_ptr(),
         dv.data_ptr(), kb, kh, kl, ws.data_ptr(), size, _stream()))
     return dq, dk, dv

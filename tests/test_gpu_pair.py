@@ -250,3 +250,31 @@ def test_each_wave_decides_by_its_own_cells_of_a_summary(device, Lq, Lk, D):
     grads = ra.bwd_block(tq, tk, tv, _dev(block, device), out, lse, tdo, scale)
     for got, ref in zip(grads, R.mha_dense_grads(q, k, v, do, block)):
         assert max(_rel(got.permute(0, 2, 1, 3).cpu().numpy(), ref)) <= GRAD_TOL
+
+
+@pytest.mark.parametrize("Sq,Sk,D,kind", [
+    (1, 1, 32, "none"), (129, 63, 96, "none"), (257, 3001, 96, "none"), (2048, 2048, 96, "causal"), (1000, 1000, 32, "causal"),
+    (1500, 1500, 80, "window"), (700, 900, 20, "window2"), (1100, 1100, 96, "documents+causal+alibi"), (130, 2500, 32, "documents"),
+    (65, 1900, 65, "alibi"), (1024, 1024, 96, "prefix+documents"), (777, 777, 32, "prefix+window"), (64, 2100, 8, "none"),
+])
+def test_pair_kernels_in_head_dims_of_their_own(device, Sq, Sk, D, kind):
+    # computed in 32 and 96; D = 96 and 32 without padding, as views of a wider array whose other columns are not to be read
+    fn, ofn, qkw, kvkw = _bias(kind, 2, Sq, Sk, 2)
+    _check(device, f"pair {kind}", 2, Sq, Sk, 2, D, 1, fn, ofn, qkw, kvkw, seed=Sq + Sk, impl="pallas")
+
+
+@pytest.mark.parametrize("D", [32, 96])
+def test_narrow_rows_of_a_wider_array(device, D):
+    B, S, H = 1, 300, 2
+    q, k, v, do = R.make_inputs(D, B, S, S, H, D)
+    wide = [torch.full((B, S, H, D + 8), float("nan"), dtype=torch.bfloat16, device=device) for _ in range(4)]
+    for w, x in zip(wide, (q, k, v, do)):
+        w[..., :D] = _dev(x, device, torch.bfloat16)
+    leaves = [w[..., :D].detach().requires_grad_(True) for w in wide[:3]]
+    out, lse = ra.ring_attention_with_lse(*leaves, 1, ra.causal_bias(), out_dtype=torch.float32)
+    bias = R.make_bias_fn(causal=True)(q_positions=np.arange(S)[None], kv_positions=np.arange(S)[None])
+    want, want_lse = R.mha_dense(q, k, v, bias)
+    assert np.abs(out.detach().cpu().numpy() - want).max() <= OUT_TOL and np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_TOL
+    grads = torch.autograd.grad(out, leaves, wide[3][..., :D].float())
+    for g, ref in zip(grads, R.mha_dense_grads(q, k, v, do, bias)):
+        assert max(_rel(g.float().cpu().numpy(), ref)) <= GRAD_TOL

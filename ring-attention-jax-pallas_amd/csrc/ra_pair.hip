@@ -89,6 +89,8 @@ struct TileLoader {
   static constexpr int NLD = RPW / RPI;        // load instructions per wave and tile
   static constexpr int NV = NLD < 16 / RPI ? NLD : 16 / RPI;  // of which so many share a base: 16 rows, whose offsets fit
                                                               // 32 bits and after which the permutation repeats
+  static constexpr int kBack = 1024 * (NV - 1);  // the base lies this far before the rows: the lanes' offsets are unsigned, and
+                                                 // rows may be closer together in memory than in LDS
   const char* base;  // this wave's first row of the first tile
   unsigned rowb;     // bytes from row to row
   int left;          // rows from there on
@@ -98,7 +100,8 @@ struct TileLoader {
     base = (const char*)base_ + (unsigned long long)(RPW * wave) * rowb;
     left = L - RPW * wave;
 #pragma unroll
-    for (int t = 0; t < NV; ++t) voff[t] = (unsigned)(lane / CPR + RPI * t) * rowb - 1024 * t + chunk(RPW * wave + RPI * t, lane);
+    for (int t = 0; t < NV; ++t)
+      voff[t] = (unsigned)(lane / CPR + RPI * t) * rowb + (kBack - 1024 * t) + chunk(RPW * wave + RPI * t, lane);
   }
   // byte offset inside its row of the chunk that a lane moves with the instruction that starts at `row` of a tile
   static RA_DEV unsigned chunk(int row, int lane) {
@@ -110,7 +113,7 @@ struct TileLoader {
   RA_DEV void issue(int row0, unsigned dst, int wave, int lane) const {
     dst += RPW * wave * (D * 2);
     if (row0 + RPW <= left) {
-      const char* sb = base + (unsigned long long)(unsigned)row0 * rowb;  // wave-uniform: scalar registers
+      const char* sb = base + (unsigned long long)(unsigned)row0 * rowb - kBack;  // wave-uniform: scalar registers
 #pragma unroll
       for (int t = 0; t < NLD; t += NV) {
         if constexpr (NV == 4) global_to_lds16_s4(sb, voff[0], voff[1], voff[2], voff[3], dst + RPI * t * (D * 2));

@@ -278,3 +278,11 @@ def test_narrow_rows_of_a_wider_array(device, D):
     grads = torch.autograd.grad(out, leaves, wide[3][..., :D].float())
     for g, ref in zip(grads, R.mha_dense_grads(q, k, v, do, bias)):
         assert max(_rel(g.float().cpu().numpy(), ref)) <= GRAD_TOL
+
+
+@pytest.mark.parametrize("Sq,Sk,D,kind", [(300, 415, 96, "none"), (2048, 130, 32, "none"), (640, 640, 96, "causal"),
+                                          (300, 1000, 32, "documents")])
+def test_one_head_whose_rows_are_closer_together_than_in_lds(device, Sq, Sk, D, kind):
+    # 192 and 64 bytes from row to row, where an LDS tile has 256 and 128
+    fn, ofn, qkw, kvkw = _bias(kind, 1, Sq, Sk, 1)
+    _check(device, f"pair {kind}", 1, Sq, Sk, 1, D, 1, fn, ofn, qkw, kvkw, seed=Sq + Sk, impl="pallas")

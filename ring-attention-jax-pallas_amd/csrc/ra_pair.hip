@@ -244,15 +244,24 @@ RA_DEV int list_key_tiles(int Lq, int Lk, const BiasArgs& bs, const int* kv_seg,
   return s_red[16];
 }
 
-// ALiBi on one side of the diagonal: -slope |q - k| = s (j - rel), with s = +-slope (score units), rel the
-// distance of this lane's row from the tile's first position and j the index in the tile, enters through the
-// matrix unit as the accumulator's initial value, exactly: [j, 1] x [s, c] with c = -s rel in one fp32 product of
-// depth two.  `j`: alibi_index of the block.  (Split into bf16 words for the bf16 product, s and c took 20
-// vector instructions a tile, of the 200 of a forward tile.)
+// ALiBi on one side of the diagonal: -slope |q - k| = s (j - rel), with s = +-slope, rel the distance of this lane's
+// row from the tile's first position and j the index in the tile.  s j enters through the matrix unit as the
+// accumulator's initial value, exactly: an fp32 product of depth two, [j, 1] x [s, c].  The constant -s rel, which
+// far from the diagonal is larger than anything else by orders of magnitude, goes into the exponent where the lane owns the row
+// (forward, dQ): in the accumulator it would cost every score its last bits (logsumexp at a bias of 6200: off by
+// 3.4e-3, and by 6e-4 so).  Under dK / dV it is c, on top of -logsumexp, which it cancels.  (Split into
+// bf16 words for the bf16 product, s and c took 20 vector instructions a tile, of the 200 of a forward tile.)
+// `j`: alibi_index of the block.
 RA_DEV float alibi_index(int first, int l32, int g) { return g == 0 ? (float)(first + l32) : 1.0f; }
-RA_DEV float alibi_terms(float s, int rel, int g) { return g == 0 ? s : -s * (float)rel; }
-RA_DEV f32x16 alibi_one_side(const f32x16& init, float j, float terms) {
-  return __builtin_amdgcn_mfma_f32_32x32x2f32(j, terms, init, 0, 0, 0);
+// -slope rel log2(e), and what that lacks of the product to twice the bits
+RA_DEV float alibi_far(float slope, int rel, float& rest) {
+  constexpr float hi = kLog2e, lo = (float)(1.4426950408889634074 - (double)hi);
+  const float r = (float)rel, x = -slope * r, y = x * hi;
+  rest = fmaf(x, lo, fmaf(x, hi, -y)) + fmaf(-slope, r, -x) * hi;
+  return y;
+}
+RA_DEV f32x16 alibi_one_side(const f32x16& init, float j, float s, float c, int g) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(j, g == 0 ? s : c, init, 0, 0, 0);
 }
 
 // What the 32 rows of a wave need done for a tile of the streamed side, as ranges of tile indexes: outside of `live`
@@ -487,7 +496,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     for (int s = 0; s < KS; ++s) qf[s] = *(const bf16x8*)(qp + 16 * s);
   }
   int q_seg = 0, q_pre = 0;
-  float slope2 = 0.f;
+  float slope = 0.f, slope2 = 0.f;  // slope2: in the units of the scores
   const int* kv_seg = nullptr;
   const int* kv_pre = nullptr;
   if constexpr (GENERAL) {
@@ -499,7 +508,10 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
       q_pre = bs.q_pre[b * bs.q_pre_sb + qi_c];
       kv_pre = bs.kv_pre + b * bs.kv_pre_sb;
     }
-    if (flags & RA_BIAS_ALIBI) slope2 = bs.slopes[h] * kLog2e / a.scale2;
+    if (flags & RA_BIAS_ALIBI) {
+      slope = bs.slopes[h];
+      slope2 = slope * kLog2e / a.scale2;
+    }
   }
 
   WaveIds ids;
@@ -598,7 +610,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     }
     if (!wt.plain(j)) tests |= kTestPos;
     f32x16 S[2], zero;
-    float beyond = 0.f;  // what the scores of the second key block lack
+    float beyond = 0.f, far = 0.f, far_rest = 0.f;  // what the scores of the second key block, and the exponents of all, lack
 #pragma unroll
     for (int r = 0; r < 16; ++r) zero[r] = 0.f;
     __builtin_amdgcn_s_setprio(1);
@@ -606,8 +618,9 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
       const int at = opaque_lane(lane), l = at & 31, half = at >> 5;
       // one initial value for both key blocks: the second one's is 32 slopes further, added to its exponents
       const float s = j < wt.past ? slope2 : -slope2;
-      const f32x16 init = alibi_one_side(zero, alibi_index(0, l, half), alibi_terms(s, q_off + qw + l - (kv_off + kt0), half));
+      const f32x16 init = alibi_one_side(zero, alibi_index(0, l, half), s, 0.f, half);
       beyond = 32.f * s;
+      far = alibi_far(j < wt.past ? slope : -slope, q_off + qw + l - (kv_off + kt0), far_rest);
       S[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[0], init, 0, 0, 0);
       S[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[1], qf[0], init, 0, 0, 0);
     } else {
@@ -655,7 +668,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
       mx0 = fmaxf(fmaxf(mx0, S[0][r]), S[0][r + 1]);
       mx1 = fmaxf(fmaxf(mx1, S[1][r]), S[1][r + 1]);
     }
-    const float mx = half_max(fmaxf(mx0, GENERAL ? mx1 + beyond : mx1)) * a.scale2;
+    const float mx = GENERAL ? fmaf(half_max(fmaxf(mx0, mx1 + beyond)), a.scale2, far) : half_max(fmaxf(mx0, mx1)) * a.scale2;
     m_true = fmaxf(m_true, mx);
     if (__any(mx > m_run + 8.0f)) {
       const float m_new = fmaxf(m_run, mx);
@@ -668,7 +681,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[db][r] *= corr;
     }
-    const float neg_m = (m_run == RA_NEG_INF) ? 0.f : -m_run;
+    const float neg_ref = (m_run == RA_NEG_INF) ? 0.f : -m_run, neg_m = GENERAL ? (neg_ref + far) + far_rest : neg_ref;
     const float neg_m1 = GENERAL ? fmaf(beyond, a.scale2, neg_m) : neg_m;
     // The 32 scores of a lane go through exp2 in four groups of eight, one group per 16 keys of the
     // output product: group ks + 1 is worked on while the matrix unit multiplies with group ks.
@@ -893,10 +906,11 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel
   }
   const long long row = (long long)hh * a.Lq + qi_c;
   const float Lraw = a.lse[row];
-  const float neg_lse2 = (Lraw == RA_NEG_INF) ? RA_NEG_INF : -Lraw * kLog2e;  // fully masked row: P = 0
+  const float neg_lse = (Lraw == RA_NEG_INF) ? RA_NEG_INF : -Lraw;  // fully masked row: P = 0
+  const float neg_lse2 = neg_lse * kLog2e;
   const float neg_delta = -a.delta[row];
   int q_seg = 0, q_pre = 0;
-  float slope2 = 0.f;
+  float slope = 0.f, slope2 = 0.f;  // slope2: in the units of the scores
   const int* kv_seg = nullptr;
   const int* kv_pre = nullptr;
   if constexpr (GENERAL) {
@@ -908,7 +922,10 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel
       q_pre = bs.q_pre[b * bs.q_pre_sb + qi_c];
       kv_pre = bs.kv_pre + b * bs.kv_pre_sb;
     }
-    if (flags & RA_BIAS_ALIBI) slope2 = bs.slopes[h] * kLog2e / a.scale_res;
+    if (flags & RA_BIAS_ALIBI) {
+      slope = bs.slopes[h];
+      slope2 = slope * kLog2e / a.scale_res;
+    }
   }
   WaveIds ids;
   if constexpr (GENERAL) ids.init(q_valid, q_seg, q_pre);
@@ -991,6 +1008,7 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel
       // of a biased tile are evaluated
       constexpr int PF = KS < 3 ? KS : 3;  // operand fetches in flight ahead of the matrix instruction that uses them
       f32x16 S, zero;
+      float neg_row = neg_lse2;  // added to the scores in the exponent
 #pragma unroll
       for (int r = 0; r < 16; ++r) zero[r] = 0.f;
       auto nat_frag = [&](const char* tile, int ss) { return *(const bf16x8*)(tile + 32 * kb * ROWB + fr_off.nat(ss)); };
@@ -1002,8 +1020,10 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel
         __builtin_amdgcn_sched_barrier(0);
         if (one_side) {
           const int at = opaque_lane(lane), l = at & 31, half = at >> 5;
-          S = alibi_one_side(zero, alibi_index(32 * kb, l, half),
-                             alibi_terms(j < wt.past ? slope2 : -slope2, q_off + qw + l - (kv_off + kt0), half));
+          const float s = j < wt.past ? slope2 : -slope2;
+          S = alibi_one_side(zero, alibi_index(32 * kb, l, half), s, 0.f, half);
+          // (the bias and the logsumexp cancel before they are scaled)
+          neg_row = fmaf(j < wt.past ? -slope : slope, (float)(q_off + qw + l - (kv_off + kt0)), neg_lse) * kLog2e;
           S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[0], qf[0], S, 0, 0, 0);
         } else {
           S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[0], qf[0], zero, 0, 0, 0);
@@ -1053,7 +1073,7 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel
           P = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[op], dof[op], P, 0, 0, 0);
 #pragma unroll
           for (int e = 16 * op / KS; e < 16 * (op + 1) / KS; ++e) {
-            float x = fast_exp2(fmaf(S[e], a.scale_res, neg_lse2));
+            float x = fast_exp2(fmaf(S[e], a.scale_res, GENERAL ? neg_row : neg_lse2));
             asm volatile("" : "+v"(x));
             S[e] = x;
           }
@@ -1400,7 +1420,8 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dkdv_pair_kern
     }
     if (one_side) {
       const int at = opaque_lane(lane), l = at & 31;
-      S = alibi_one_side(S, alibi_index(0, l, at >> 5), alibi_terms(j < wt.past ? slope2 : -slope2, (kv_off + kw + l) - (q_off + qt0), at >> 5));
+      const float s = j < wt.past ? slope2 : -slope2;
+      S = alibi_one_side(S, alibi_index(0, l, at >> 5), s, -s * (float)((kv_off + kw + l) - (q_off + qt0)), at >> 5);
     }
     auto nat_frag = [&](const char* tile, int ss) { return *(const bf16x8*)(tile + fr_off.nat(ss)); };
     __builtin_amdgcn_s_setprio(1);

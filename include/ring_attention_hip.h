@@ -80,7 +80,8 @@ extern "C" {
 
 #define RA_DTYPE_BF16 0
 #define RA_DTYPE_F32 1
-#define RA_DTYPE_F16 2 /* ra_convert only */
+#define RA_DTYPE_F16 2 /* ra_convert and the gradients of ra_bwd_whole */
+#define RA_DTYPE_VIA_BF16 16 /* added to the dtype of ra_bwd_whole's gradients: each rounded to bf16 before it is converted */
 
 /* bf16 tensor view [B, H, L, D] with explicit element strides (D contiguous; strides multiples of 8,
  * D <= stride_l <= 2^27). */
@@ -289,14 +290,15 @@ int ra_bwd_pair(const ra_bwd_step_params* p, const void* out, int32_t out_dtype,
                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* The same two calls for every head dim that is a multiple of 32 up to 128 (dense blocks at 64 and 128
- * only). */
+ * only), with the gradients in any of the RA_DTYPE_*; with RA_DTYPE_VIA_BF16 the same bits as ra_bwd_pair's
+ * converted afterwards. */
 int64_t ra_fwd_whole_workspace(const ra_fwd_step_params* p);
 int ra_fwd_whole(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b,
                  int64_t out_stride_h, int64_t out_stride_l, float* lse, void* workspace,
                  int64_t workspace_bytes, void* stream);
 int64_t ra_bwd_whole_workspace(const ra_bwd_step_params* p);
 int ra_bwd_whole(const ra_bwd_step_params* p, const void* out, int32_t out_dtype, int64_t out_stride_b,
-                 int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
+                 int64_t out_stride_h, int64_t out_stride_l, int32_t grad_dtype, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
                  int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
                  int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream);
 

@@ -330,11 +330,12 @@ struct RingResult {
   float* lse;
   int dtype;  // RA_DTYPE_*
   int64_t stride_pass, stride_b, stride_h, stride_l;
+  bool via_bf16 = false;  // gradients: rounded to bf16 before the conversion
 };
 
-int check_ring_result(const char* what, const RingResult& r) {
+int check_ring_result(const char* what, const RingResult& r, bool f16 = false) {
   if (!r.base) return fail(RA_ERR_NULL, "%s: NULL result pointer", what);
-  if (r.dtype != RA_DTYPE_BF16 && r.dtype != RA_DTYPE_F32) return fail(RA_ERR_DTYPE, "unknown out_dtype %d", r.dtype);
+  if (r.dtype != RA_DTYPE_BF16 && r.dtype != RA_DTYPE_F32 && !(f16 && r.dtype == RA_DTYPE_F16)) return fail(RA_ERR_DTYPE, "unknown out_dtype %d", r.dtype);
   if ((r.stride_pass % 4) || (r.stride_b % 4) || (r.stride_h % 4) || (r.stride_l % 4))
     return fail(RA_ERR_ALIGN, "%s: result strides must be multiples of 4 elements", what);
   // the kernels store four elements at a time: 8 bytes of bf16 or 16 bytes of fp32
@@ -342,6 +343,11 @@ int check_ring_result(const char* what, const RingResult& r) {
   if (reinterpret_cast<uintptr_t>(r.base) % al || reinterpret_cast<uintptr_t>(r.base2) % al)
     return fail(RA_ERR_ALIGN, "%s: results must be aligned to four elements (%u bytes)", what, al);
   return RA_OK;
+}
+
+int gradient_flags(const RingResult& r) {
+  const int kind = r.dtype == RA_DTYPE_F32 ? ra::kFlagWholeF32 : r.dtype == RA_DTYPE_F16 ? ra::kFlagWholeF16 : ra::kFlagWholeBf16;
+  return kind | (r.via_bf16 ? ra::kFlagViaBf16 : 0);
 }
 
 char* pass_slice(void* base, const RingResult& r, int p) {
@@ -562,7 +568,7 @@ int bwd_dq_passes(const ra_bwd_step_params* steps, const std::vector<int>& first
     return steps_on_pair(steps, total, [&](const ra_bwd_step_params& p) { return bwd_step_on_pair(p, 2, stream); });
   ra::BwdArgs a = to_bwd_args(f);
   if (whole) {
-    a.bias.flags |= ra::kFlagWholeBf16;
+    a.bias.flags |= gradient_flags(*whole);
     a.out_sb = whole->stride_b;  // in the slots of the accumulator pointers, which have no use here
     a.out_sh = whole->stride_h;
     a.out_sl = whole->stride_l;
@@ -622,7 +628,7 @@ int bwd_dkdv_passes(const ra_bwd_step_params* steps, const std::vector<int>& fir
     return steps_on_pair(steps, total, [&](const ra_bwd_step_params& p) { return bwd_step_on_pair(p, 1, stream); });
   ra::BwdArgs a = to_bwd_args(f);
   if (whole) {
-    a.bias.flags |= ra::kFlagWholeBf16;
+    a.bias.flags |= gradient_flags(*whole);
     a.out_sb = whole->stride_b;  // in the slots of the accumulator pointers, which have no use here
     a.out_sh = whole->stride_h;
     a.out_sl = whole->stride_l;
@@ -663,17 +669,20 @@ struct PairPlan {
 };
 
 // Key tiles that one head's query tiles visit (positional terms only): their sum, and the most.
-void count_key_tiles(const ra_bias& bias, int Lq, int Lk, int64_t& total, int& most) {
+// live: the query tiles that visit any.
+void count_key_tiles(const ra_bias& bias, int Lq, int Lk, int64_t& total, int& most, int* live = nullptr) {
   const int ntiles = (Lk + kPairKeysHost - 1) / kPairKeysHost;
   const ra::BiasArgs b = to_bias(bias);
   total = 0;
   most = 0;
+  if (live) *live = 0;
   for (int q0 = 0; q0 < Lq; q0 += kPairRowsHost) {
     int lo, hi;
     ra::key_tile_range(b.flags, b.window, b.q_off + q0, b.q_off + std::min(q0 + kPairRowsHost, Lq) - 1, b.kv_off, ntiles,
                        kPairKeysHost, lo, hi);
     total += hi - lo;
     most = std::max(most, hi - lo);
+    if (live) *live += hi > lo;
   }
 }
 
@@ -708,6 +717,23 @@ void plan_split(PairPlan& r, int64_t heads, int64_t rows, int64_t total, int mos
   const int64_t chunk = even ? (most + kPairSlots / wgs - 1) / (kPairSlots / wgs) : heads * total * 3 / (2 * kPairSlots);
   r.chunk_tiles = (int)std::min<int64_t>(most, std::max<int64_t>({chunk, min_chunk, (most + kMaxSplit - 1) / kMaxSplit}));
   r.n_split = (most + r.chunk_tiles - 1) / r.chunk_tiles;
+}
+// Whether a single step, into a carry or an accumulator, runs on fwd_pair_kernel (dq_pair_kernel) as well: nothing is shared there.  Under
+// a list of tiles and at D = 64 always, but for even rows that fill the chip once or twice in the forward; else up to a workgroup per compute
+// unit, with uneven rows up to two, and beyond with rows that are short.  fwd_step_kernel | fwd_pair_kernel, then dq_kernel |
+// dq_pair_kernel, us: D=128, a causal diagonal of 1024, H=8, 38 | 25 and 44 | 28, of 2048, H=16, 64 | 46 and 72 | 50, of 4096, H=16, 108 | 96 and 132 | 115,
+// H=32, 189 | 158 and 239 | 194, of 8192, H=16, 273 | 295 and 353 | 367; unmasked 2048, H=16, 61 | 48 and 72 | 55, 4096, H=16, 132 | 142 and 173 | 176;
+// D=64, a diagonal of 4096, H=16, 83 | 68 and 89 | 71, unmasked 85 | 90 and 104 | 102, 8192 314 | 317 and 385 | 373, 16384 1221 | 1215 and 1501 | 1432.
+bool step_on_pair(const ra_bias& bias, int B, int H, int Lq, int Lk, int D, bool forward) {
+  if (bias.flags & (RA_BIAS_SEGMENT | RA_BIAS_PREFIX | RA_BIAS_DENSE)) return true;
+  int64_t total;
+  int most, live;
+  count_key_tiles(bias, Lq, Lk, total, most, &live);
+  const int64_t rows = (Lq + kPairRowsHost - 1) / kPairRowsHost, wgs = (int64_t)B * H * rows;
+  const bool even = total * 20 >= (int64_t)most * rows * 17;
+  if (D == 64) return !(forward && even && wgs > kPairSlots / 2 && total < 192 * rows);
+  if (wgs <= kPairSlots / 2) return true;
+  return wgs <= kPairSlots ? !even : total < 56 * (int64_t)live;
 }
 PairPlan plan_fwd_pair(const ra_fwd_step_params& p) {
   const int rows = (p.Lq + kPairRowsHost - 1) / kPairRowsHost;
@@ -945,8 +971,8 @@ int ra_dense_map(const float* dense_bias, int64_t stride_b, int64_t stride_h, in
 int ra_fwd_step(const ra_fwd_step_params* p, void* stream) {
   int rc = ra_fwd_step_check(p);
   if (rc) return rc;
-  if (dense_steps_on_pair(p->bias)) return fwd_step_on_pair(*p, stream);
   if (ra_step_is_skippable(&p->bias, p->Lq, p->Lk)) return RA_OK;  // identity on the carry
+  if (step_on_pair(p->bias, p->B, p->H, p->Lq, p->Lk, p->D, true)) return fwd_step_on_pair(*p, stream);
   const ra::FwdArgs a = to_fwd_args(*p);
   hipError_t e = ra::launch_fwd_step(a, p->D, kernel_mode(p->bias.flags), (hipStream_t)stream);
   return e == hipSuccess ? RA_OK : hip_fail(e, "ra_fwd_step launch");
@@ -1029,6 +1055,10 @@ int ra_bwd_step_parts(const ra_bwd_step_params* p, int32_t parts, void* stream) 
   if (parts < 1 || parts > 3) return fail(RA_ERR_SHAPE, "parts must be 1, 2 or 3 (got %d)", parts);
   if (dense_steps_on_pair(p->bias)) return bwd_step_on_pair(*p, parts, stream);
   if (ra_step_is_skippable(&p->bias, p->Lq, p->Lk)) return RA_OK;  // contributes nothing
+  if ((parts & 2) && step_on_pair(p->bias, p->B, p->H, p->Lq, p->Lk, p->D, false)) {
+    if ((rc = bwd_step_on_pair(*p, 2, stream))) return rc;
+    if (!(parts &= 1)) return RA_OK;
+  }
   const ra::BwdArgs a = to_bwd_args(*p);
   hipError_t e = ra::launch_bwd_step(a, p->D, kernel_mode(p->bias.flags), parts, (hipStream_t)stream);
   return e == hipSuccess ? RA_OK : hip_fail(e, "ra_bwd_step launch");
@@ -1104,7 +1134,7 @@ static int64_t bwd_pair_workspace(const ra_bwd_step_params* p, bool any_dim) {
   return bwd_space(*p, plan_dq_pair(*p), plan_dkdv_pair(*p)).total;
 }
 
-static int bwd_pair(const ra_bwd_step_params* p, bool any_dim, const void* out, int32_t out_dtype, int64_t out_stride_b,
+static int bwd_pair(const ra_bwd_step_params* p, bool any_dim, int grad_dtype, const void* out, int32_t out_dtype, int64_t out_stride_b,
                 int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
                 int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
@@ -1113,9 +1143,11 @@ static int bwd_pair(const ra_bwd_step_params* p, bool any_dim, const void* out, 
   c.delta = c.dq = c.dk = c.dv = reinterpret_cast<float*>(uintptr_t(16));  // not used: no accumulators
   int rc = check_bwd_step(&c, any_dim);
   if (rc || (rc = check_whole_call("ra_bwd_whole", c.D, c.bias))) return rc;
-  const RingResult rq{dq, nullptr, nullptr, RA_DTYPE_BF16, 0, dq_stride_b, dq_stride_h, dq_stride_l};
-  const RingResult rk{dk, dv, nullptr, RA_DTYPE_BF16, 0, dkv_stride_b, dkv_stride_h, dkv_stride_l};
-  if ((rc = check_ring_result("ra_bwd_pair", rq)) || (rc = check_ring_result("ra_bwd_pair", rk))) return rc;
+  const bool via_bf16 = grad_dtype & RA_DTYPE_VIA_BF16;
+  grad_dtype &= ~RA_DTYPE_VIA_BF16;
+  const RingResult rq{dq, nullptr, nullptr, grad_dtype, 0, dq_stride_b, dq_stride_h, dq_stride_l, via_bf16};
+  const RingResult rk{dk, dv, nullptr, grad_dtype, 0, dkv_stride_b, dkv_stride_h, dkv_stride_l, via_bf16};
+  if ((rc = check_ring_result("ra_bwd_pair", rq, true)) || (rc = check_ring_result("ra_bwd_pair", rk, true))) return rc;
   if (!dv) return fail(RA_ERR_NULL, "ra_bwd_pair: dv is NULL");
   const PairPlan plan_q = plan_dq_pair(*p), plan_k = plan_dkdv_pair(*p);
   if (!plan_k.pair && narrow(c.D)) return fail(RA_ERR_TOO_LARGE, "ra_bwd_whole: too many rows");
@@ -1144,17 +1176,35 @@ static int bwd_pair(const ra_bwd_step_params* p, bool any_dim, const void* out, 
     a.part_n = plan.n_split > 1 ? (int*)(ws + n) : nullptr;
     a.out = r.base;
     a.out2 = r.base2;
+    a.out_dtype = r.dtype;
+    a.via_bf16 = r.via_bf16;
     a.out_sb = r.stride_b;
     a.out_sh = r.stride_h;
     a.out_sl = r.stride_l;
   };
+  // fp32 gradients that lie as the accumulators of a step do are stored by its kernels, which know one pair only and are faster
+  // (dK and dV of a causal diagonal and a full pair of 4096, H=16, D=128: 430 us on the several-shard ones, 417 on
+  // these; 32768 in two shards 5.21 | 5.15 ms and dQ 2.60 | 2.54)
+  auto as_accumulator = [&](const RingResult& r, int L) {
+    return r.dtype == RA_DTYPE_F32 && !r.via_bf16 && aligned16(r.base) && aligned16(r.base2) && r.stride_l == c.D && r.stride_h == (int64_t)L * c.D &&
+           r.stride_b == (int64_t)c.H * L * c.D && mode != 2;
+  };
+  auto one_step = [&](int part) -> int {
+    ra::BwdArgs s = a.a;
+    s.dq = (float*)rq.base;
+    s.dk = (float*)rk.base;
+    s.dv = (float*)rk.base2;
+    s.bias.flags |= ra::kFlagWholeF32;
+    hipError_t err = ra::launch_bwd_step(s, c.D, mode, part, (hipStream_t)stream);
+    return err == hipSuccess ? RA_OK : hip_fail(err, "ra_bwd_pair launch");
+  };
   if (plan_k.pair) {
     share(plan_k, sp.dkdv_part, sp.dkdv_n, rk);
     if ((e = ra::launch_dkdv_pair(a, c.D, mode, (hipStream_t)stream)) != hipSuccess) return hip_fail(e, "ra_bwd_pair launch");
-  } else if ((rc = bwd_dkdv_passes(&c, one, 1, stream, &rk))) {
+  } else if ((rc = as_accumulator(rk, c.Lk) ? one_step(1) : bwd_dkdv_passes(&c, one, 1, stream, &rk))) {
     return rc;
   }
-  if (!plan_q.pair) return bwd_dq_passes(&c, one, 1, stream, &rq);
+  if (!plan_q.pair) return as_accumulator(rq, c.Lq) ? one_step(2) : bwd_dq_passes(&c, one, 1, stream, &rq);
   share(plan_q, sp.dq_part, sp.dq_n, rq);
   e = ra::launch_dq_pair(a, c.D, mode, (hipStream_t)stream);
   return e == hipSuccess ? RA_OK : hip_fail(e, "ra_bwd_pair launch");
@@ -1167,14 +1217,14 @@ int ra_bwd_pair(const ra_bwd_step_params* p, const void* out, int32_t out_dtype,
                 int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
                 int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
-  return bwd_pair(p, false, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h, dq_stride_l, dk, dv, dkv_stride_b,
+  return bwd_pair(p, false, RA_DTYPE_BF16, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h, dq_stride_l, dk, dv, dkv_stride_b,
                   dkv_stride_h, dkv_stride_l, workspace, workspace_bytes, stream);
 }
 int ra_bwd_whole(const ra_bwd_step_params* p, const void* out, int32_t out_dtype, int64_t out_stride_b,
-                int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
+                int64_t out_stride_h, int64_t out_stride_l, int32_t grad_dtype, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
                 int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
-  return bwd_pair(p, true, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h, dq_stride_l, dk, dv, dkv_stride_b,
+  return bwd_pair(p, true, grad_dtype, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h, dq_stride_l, dk, dv, dkv_stride_b,
                   dkv_stride_h, dkv_stride_l, workspace, workspace_bytes, stream);
 }
 

@@ -995,24 +995,31 @@ __global__ __launch_bounds__(256) void dkdv_kernel(
   }
   }  // query shards
   const bool whole_ring = MULTI && (flags & kFlagWhole);
-  if (!whole_ring && tiles_listed == 0) return;  // nothing to add
+  const bool store_only = !MULTI && (flags & kFlagWhole);  // the only step: nothing there to add to
+  if (!whole_ring && !store_only && tiles_listed == 0) return;  // nothing to add
   if constexpr (MULTI) {
     if (whole_ring) {
-      // the gradients of this key slab are complete: bf16, in the caller's layout
-      const long long at = b * a.out_sb + h * a.out_sh + (long long)(kw + 4 * g) * a.out_sl + l32;
-      bf16_t* const dkp = (bf16_t*)ring.dk[blockIdx.y] + at;
-      bf16_t* const dvp = (bf16_t*)ring.dv[blockIdx.y] + at;
+      // the gradients of this key slab are complete: in the caller's dtype and layout
+      auto store = [&](auto like) {
+        using T = decltype(like);
+        const long long at = b * a.out_sb + h * a.out_sh + (long long)(kw + 4 * g) * a.out_sl + l32;
+        T* const dkp = (T*)ring.dk[blockIdx.y] + at;
+        T* const dvp = (T*)ring.dv[blockIdx.y] + at;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int kr = 8 * (r / 4) + (r % 4);
-        if (kw + 4 * g + kr < a.Lk) {
+        for (int r = 0; r < 16; ++r) {
+          const int kr = 8 * (r / 4) + (r % 4);
+          if (kw + 4 * g + kr < a.Lk) {
 #pragma unroll
-          for (int db = 0; db < DB; ++db) {
-            dkp[kr * a.out_sl + 32 * db] = (bf16_t)(dk[db][r] * a.sm_scale);
-            dvp[kr * a.out_sl + 32 * db] = (bf16_t)dv[db][r];
+            for (int db = 0; db < DB; ++db) {
+              dkp[kr * a.out_sl + 32 * db] = (T)round_via(dk[db][r] * a.sm_scale, flags & kFlagViaBf16);
+              dvp[kr * a.out_sl + 32 * db] = (T)round_via(dv[db][r], flags & kFlagViaBf16);
+            }
           }
         }
-      }
+      };
+      if (flags & kFlagWholeF32) store(float{});
+      else if (flags & kFlagWholeF16) store(_Float16{});
+      else store(bf16_t{});
       return;
     }
   }
@@ -1031,7 +1038,16 @@ __global__ __launch_bounds__(256) void dkdv_kernel(
     const int key0 = kw + 4 * g;
     auto add_to = [&](float* p, const f32x16 (&acc)[DB], float mul) {
       float old[DB][16];
-      if (kw + 32 <= a.Lk) {  // the whole wave is in range (wave-uniform): straight-line code
+      if (store_only) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int kr = 8 * (r / 4) + (r % 4);
+          if (key0 + kr < a.Lk) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db) p[kr * D + 32 * db] = acc[db][r] * mul;
+          }
+        }
+      } else if (kw + 32 <= a.Lk) {  // the whole wave is in range (wave-uniform): straight-line code
 #pragma unroll
         for (int r = 0; r < 16; ++r)
 #pragma unroll
@@ -1953,20 +1969,22 @@ __global__ __launch_bounds__(kDqThreads) void dq_kernel(
   }
   }  // key/value shards
   const bool whole_ring = MULTI && (flags & kFlagWhole);
-  if (!whole_ring && tiles_listed == 0) return;  // nothing to add
+  const bool store_only = !MULTI && (flags & kFlagWhole);  // the only step: nothing there to add to
+  if (!whole_ring && !store_only && tiles_listed == 0) return;  // nothing to add
   if constexpr (MULTI) {
     if (whole_ring) {
-      // dQ of these rows is complete: bf16, in the caller's layout
+      // dQ of these rows is complete: in the caller's dtype and layout
       if (q_valid) {
-        bf16_t* dq = (bf16_t*)ring.x0[blockIdx.y] + b * a.out_sb + h * a.out_sh + (long long)qi * a.out_sl + 4 * g;
+        const long long at = b * a.out_sb + h * a.out_sh + (long long)qi * a.out_sl + 4 * g;
+        const int dtype = (flags & kFlagWholeF32) ? RA_DTYPE_F32 : (flags & kFlagWholeF16) ? RA_DTYPE_F16 : RA_DTYPE_BF16;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
           for (int bb = 0; bb < 4; ++bb) {
-            bf16x4 t;
+            f32x4 t;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) t[c] = (bf16_t)(acc[db][4 * bb + c] * a.sm_scale);
-            *(bf16x4*)(dq + 32 * db + 8 * bb) = t;
+            for (int c = 0; c < 4; ++c) t[c] = acc[db][4 * bb + c] * a.sm_scale;
+            store4(ring.x0[blockIdx.y], dtype, at + 32 * db + 8 * bb, round_via(t, flags & kFlagViaBf16));
           }
       }
       return;
@@ -1980,7 +1998,8 @@ __global__ __launch_bounds__(kDqThreads) void dq_kernel(
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int bb = 0; bb < 4; ++bb) {
-        f32x4 t = *(f32x4*)(dq + 32 * db + 8 * bb);
+        f32x4 t = {0.f, 0.f, 0.f, 0.f};
+        if (!store_only) t = *(f32x4*)(dq + 32 * db + 8 * bb);
 #pragma unroll
         for (int c = 0; c < 4; ++c) t[c] += acc[db][4 * bb + c] * a.sm_scale;
         *(f32x4*)(dq + 32 * db + 8 * bb) = t;

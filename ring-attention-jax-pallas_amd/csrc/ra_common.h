@@ -525,16 +525,25 @@ RA_DEV void tile_flag_range(const int* ids, int t, int L, bool& any, bool& all) 
   all = z == 0;
 }
 
-// four elements of a result that is bf16 or fp32
-RA_DEV void store4(void* base, int f32, long long at, const f32x4& x) {
-  if (f32) {
-    *(f32x4*)((float*)base + at) = x;
-  } else {
-    bf16x4 y;
+// an element, and four, of a result in the caller's dtype (RA_DTYPE_*)
+template <typename T>
+RA_DEV void store_as(void* base, long long at, const f32x4& x) {
+  typedef __attribute__((ext_vector_type(4))) T vec;
+  vec y;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] = (bf16_t)x[e];
-    *(bf16x4*)((bf16_t*)base + at) = y;
-  }
+  for (int e = 0; e < 4; ++e) y[e] = (T)x[e];
+  *(vec*)((T*)base + at) = y;
+}
+RA_DEV float round_via(float x, bool bf16) { return bf16 ? (float)(bf16_t)x : x; }
+RA_DEV f32x4 round_via(f32x4 x, bool bf16) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) x[e] = round_via(x[e], bf16);
+  return x;
+}
+RA_DEV void store4(void* base, int dtype, long long at, const f32x4& x) {
+  if (dtype == RA_DTYPE_F32) store_as<float>(base, at, x);
+  else if (dtype == RA_DTYPE_F16) store_as<_Float16>(base, at, x);
+  else store_as<bf16_t>(base, at, x);
 }
 
 // Executed by ONE wave.  `list` holds `cnt` entries (tile index in bits 0..14, bit 15 set when

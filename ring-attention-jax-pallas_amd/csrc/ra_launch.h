@@ -15,7 +15,9 @@ namespace ra {
 // that the argument block does not grow: the kernels' scalar registers are all taken.
 constexpr int kFlagWholeBf16 = 1 << 24;
 constexpr int kFlagWholeF32 = 1 << 25;
-constexpr int kFlagWhole = kFlagWholeBf16 | kFlagWholeF32;
+constexpr int kFlagWholeF16 = 1 << 26;  // (gradients only)
+constexpr int kFlagViaBf16 = 1 << 27;   // (gradients only: rounded to bf16 before the conversion)
+constexpr int kFlagWhole = kFlagWholeBf16 | kFlagWholeF32 | kFlagWholeF16;
 
 struct FwdArgs {
   TensorArg q, k, v;
@@ -123,7 +125,7 @@ struct PairFwdArgs {
 };
 hipError_t launch_fwd_pair(const PairFwdArgs& a, int D, int mode, hipStream_t stream);
 // The gradient of the resident side (dQ; or dK and dV: acc2, out2): shares of a row's sum (n_split > 1),
-// fp32 accumulators that are added to, or the finished bf16 gradient.
+// fp32 accumulators that are added to, or the finished gradient.
 struct PairBwdArgs {
   BwdArgs a;  // (its dq / dk / dv slots are not used)
   int n_split, chunk_tiles;
@@ -132,6 +134,8 @@ struct PairBwdArgs {
   int* part_n;
   float *acc, *acc2;
   void *out, *out2;
+  int out_dtype;  // RA_DTYPE_*
+  int via_bf16;   // round to bf16 before the conversion to it
   long long out_sb, out_sh, out_sl;
 };
 hipError_t launch_dq_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream);

@@ -1148,7 +1148,7 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel
         if (n_piece == 1) t += *(const f32x4*)(fp + d0);
         *(f32x4*)(fp + d0) = t;
       } else {
-        store4(e->out, 0, b * e->out_sb + h * e->out_sh + (long long)qi * e->out_sl + d0, t);
+        store4(e->out, e->out_dtype, b * e->out_sb + h * e->out_sh + (long long)qi * e->out_sl + d0, round_via(t, e->via_bf16));
       }
     }
 }
@@ -1592,26 +1592,37 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dkdv_pair_kern
     add_to(e->acc2, dv, 1.0f);
     return;
   }
+  if (n_piece > 1) {
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int key = kw + 4 * g + 8 * (r / 4) + (r % 4);
-    if (key >= e->a.Lk) continue;
-    if (n_piece > 1) {
+    for (int r = 0; r < 16; ++r) {
+      const int key = kw + 4 * g + 8 * (r / 4) + (r % 4);
+      if (key >= e->a.Lk) continue;
       float* fp = e->part + ((long long)split * 2 * rows + (long long)hh * e->a.Lk + key) * DL + l32;
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         fp[32 * db] = dk[db][r] * e->a.sm_scale;
         fp[rows * DL + 32 * db] = dv[db][r];
       }
-    } else {
+    }
+    return;
+  }
+  auto store = [&](auto like) {
+    using T = decltype(like);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int key = kw + 4 * g + 8 * (r / 4) + (r % 4);
+      if (key >= e->a.Lk) continue;
       const long long at = b * e->out_sb + h * e->out_sh + (long long)key * e->out_sl + l32;
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        ((bf16_t*)e->out)[at + 32 * db] = (bf16_t)(dk[db][r] * e->a.sm_scale);
-        ((bf16_t*)e->out2)[at + 32 * db] = (bf16_t)dv[db][r];
+        ((T*)e->out)[at + 32 * db] = (T)round_via(dk[db][r] * e->a.sm_scale, e->via_bf16);
+        ((T*)e->out2)[at + 32 * db] = (T)round_via(dv[db][r], e->via_bf16);
       }
     }
-  }
+  };
+  if (e->out_dtype == RA_DTYPE_F32) store(float{});
+  else if (e->out_dtype == RA_DTYPE_F16) store(_Float16{});
+  else store(bf16_t{});
 }
 
 // What the dK / dV kernel adds to a row's scores: stat[row] = -lse log2(e) / scale_res (-inf for a row without
@@ -1648,7 +1659,7 @@ __global__ __launch_bounds__(256) void pair_stat_kernel(const OutT* out, long lo
   }
 }
 
-// Sum of the shares of rows that were split, stored as bf16.
+// Sum of the shares of rows that were split, stored in the gradient's dtype.
 // `n_out` results of the same rows (dK and dV) lie one after another in a share; grid dimension y.
 template <int D, int ROWS>
 __global__ __launch_bounds__(256) void pair_sum_kernel(const PairBwdArgs p, int n_out, int BH, int H, int L) {
@@ -1663,7 +1674,8 @@ __global__ __launch_bounds__(256) void pair_sum_kernel(const PairBwdArgs p, int 
   f32x4 x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (int s = 0; s < n_piece; ++s) x += *(const f32x4*)(p.part + (((long long)s * n_out + which) * rows + row) * D + 4 * c);
-  store4(which ? p.out2 : p.out, 0, (hh / H) * p.out_sb + (hh % H) * p.out_sh + (long long)li * p.out_sl + 4 * c, x);
+  store4(which ? p.out2 : p.out, p.out_dtype, (hh / H) * p.out_sb + (hh % H) * p.out_sh + (long long)li * p.out_sl + 4 * c,
+         round_via(x, p.via_bf16));
 }
 
 template <int D, int ROWS>

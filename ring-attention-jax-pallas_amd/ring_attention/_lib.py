@@ -21,7 +21,8 @@ RA_MAX_SEGMENT_SHARD = 65536  # longest shard that one call takes under a segmen
 RA_MAX_POSITION = (1 << 30) - (1 << 16)  # token positions (offset + index) stay below this
 RA_MAX_ROW_STRIDE = 1 << 27  # elements between two rows of a q / k / v / dO view, at most
 RA_DTYPE_F32 = 1
-RA_DTYPE_F16 = 2  # ra_convert only
+RA_DTYPE_F16 = 2  # ra_convert and the gradients of ra_bwd_whole
+RA_DTYPE_VIA_BF16 = 16
 RA_MAX_CONVERT = 4  # arrays per ra_convert
 
 
@@ -103,7 +104,7 @@ EXPORTS = {
     "ra_fwd_whole": (C.c_int, [C.POINTER(RaFwdStepParams), C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64,
                                C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p]),
     "ra_bwd_whole_workspace": (C.c_int64, [C.POINTER(RaBwdStepParams)]),
-    "ra_bwd_whole": (C.c_int, [C.POINTER(RaBwdStepParams), C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64,
+    "ra_bwd_whole": (C.c_int, [C.POINTER(RaBwdStepParams), C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64, C.c_int32,
                                C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64,
                                C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p]),
     "ra_convert": (C.c_int, [C.c_char_p, C.c_int32, C.c_void_p]),  # ra_rows blocks, packed

@@ -336,11 +336,27 @@ def bwd_block(q, k, v, bias: Union[BlockBias, torch.Tensor, None], o, L, do, sm_
     ``bwd_block`` (ring_kernel.py:202-297): all tensors ``[b, h, l, d]``, ``o`` the normalised
     forward output, ``L`` the logsumexp ``[b, h, lq]``.  Returns fp32 ``(dq, dk, dv)``."""
     _require_gpu(q)
-    delta = precompute_delta(o, do)
-    dq = torch.zeros(q.shape, dtype=torch.float32, device=q.device)
-    dk = torch.zeros(k.shape, dtype=torch.float32, device=q.device)
-    dv = torch.zeros(v.shape, dtype=torch.float32, device=q.device)
-    _bwd_step(q, k, v, do, L.contiguous(), delta, dq, dk, dv, bias, sm_scale)
+    if isinstance(bias, torch.Tensor):
+        bias = BlockBias(dense=bias)
+    if bias is not None and bias.dense is not None:  # into accumulators: those kernels read the block's summary
+        delta = precompute_delta(o, do)
+        dq = torch.zeros(q.shape, dtype=torch.float32, device=q.device)
+        dk = torch.zeros(k.shape, dtype=torch.float32, device=q.device)
+        dv = torch.zeros(v.shape, dtype=torch.float32, device=q.device)
+        _bwd_step(q, k, v, do, L.contiguous(), delta, dq, dk, dv, bias, sm_scale)
+        return dq, dk, dv
+    lib = _lib.load()
+    B, H, Lq, D = q.shape
+    dq, dk, dv = (torch.empty(x.shape, dtype=torch.float32, device=q.device) for x in (q, k, v))
+    L = L.contiguous()
+    p = _lib.RaBwdStepParams(B, H, Lq, k.shape[2], D, float(sm_scale), _view_bhld(q), _view_bhld(k), _view_bhld(v), _view_bhld(do),
+                             L.data_ptr(), None, None, None, None, _bias_struct(bias, q.device, (B, H, Lq, k.shape[2])))
+    size = lib.ra_bwd_whole_workspace(C.byref(p))
+    ws = torch.empty((size,), dtype=torch.uint8, device=q.device)
+    (ob, oh, ol, _), (qb, qh, ql, _), (kb, kh, kl, _) = o.stride(), dq.stride(), dk.stride()
+    _lib.check("ra_bwd_whole", lib.ra_bwd_whole(
+        C.byref(p), o.data_ptr(), _DTYPE_CODE[o.dtype], ob, oh, ol, _lib.RA_DTYPE_F32, dq.data_ptr(), qb, qh, ql, dk.data_ptr(),
+        dv.data_ptr(), kb, kh, kl, ws.data_ptr(), size, _stream()))
     return dq, dk, dv
 
 
@@ -776,11 +792,12 @@ def _pair_forward(q, k, v, plan: "_RingPlan", sm_scale, out_dtype):
     return out, lse
 
 
-def _pair_backward(q, k, v, out, lse, do, plan: "_RingPlan", sm_scale):
-    """``_ring_backward_fused`` of a ring of one shard: one description for all launches."""
+def _pair_backward(q, k, v, out, lse, do, plan: "_RingPlan", sm_scale, dtype=torch.bfloat16):
+    """``_ring_backward_fused`` of a ring of one shard: one description for all launches.  ``dtype``: the
+    gradients', of bf16 precision whatever it is."""
     B, H, D, Lq, Lk = plan.B, plan.H, plan.D, plan.Lq, plan.Lk
     lib = _lib.load()
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    dq, dk, dv = (torch.empty_like(x, dtype=dtype) for x in (q, k, v))
     p = _lib.RaBwdStepParams(B, H, Lq, Lk, D, sm_scale, _view_blhd(q), _view_blhd(k), _view_blhd(v), _view_blhd(do),
                              lse.data_ptr(), None, None, None, None, plan.pair_bias())
     size = lib.ra_bwd_whole_workspace(C.byref(p))
@@ -788,7 +805,7 @@ def _pair_backward(q, k, v, out, lse, do, plan: "_RingPlan", sm_scale):
     assert dk.stride() == dv.stride()
     (ob, ol, oh, _), (qb, ql, qh, _), (kb, kl, kh, _) = out.stride(), dq.stride(), dk.stride()
     _lib.check("ra_bwd_whole", lib.ra_bwd_whole(
-        C.byref(p), out.data_ptr(), _DTYPE_CODE[out.dtype], ob, oh, ol, dq.data_ptr(), qb, qh, ql, dk.data_ptr(),
+        C.byref(p), out.data_ptr(), _DTYPE_CODE[out.dtype], ob, oh, ol, _ROW_DTYPES[dtype] | _lib.RA_DTYPE_VIA_BF16, dq.data_ptr(), qb, qh, ql, dk.data_ptr(),
         dv.data_ptr(), kb, kh, kl, ws.data_ptr(), size, _stream()))
     return dq, dk, dv
 
@@ -990,10 +1007,16 @@ class _RingAttentionFn(torch.autograd.Function):
         if do is None:  # nothing came back for the output: gradients of zero, as materialised ones give
             do = torch.zeros(out.shape, dtype=torch.bfloat16, device=out.device)
         do, = _kernel_inputs((do,), ctx.plan.D)
-        bwd = _ring_backward_fused if ctx.fused else _ring_backward
-        grads = list(bwd(q, k, v, out, lse, do, ctx.plan, ctx.sm_scale))
+        plan = ctx.plan
+        d_true, dtype = ctx.given[0]
+        if (ctx.fused and plan.n == 1 and plan.callable is None and d_true == plan.D and dtype in _ROW_DTYPES
+                and all(given[1] == dtype for given in ctx.given)):
+            grads = list(_pair_backward(q, k, v, out, lse, do, plan, ctx.sm_scale, dtype))  # as the caller wants them
+        else:
+            bwd = _ring_backward_fused if ctx.fused else _ring_backward
+            grads = list(bwd(q, k, v, out, lse, do, plan, ctx.sm_scale))
         todo = [i for i, (d, dtype) in enumerate(ctx.given)
-                if ctx.needs_input_grad[i] and (d != ctx.plan.D or dtype != torch.bfloat16)]
+                if ctx.needs_input_grad[i] and (d != plan.D or dtype != grads[i].dtype)]
         if todo:
             new = _convert([grads[i] for i in todo], [ctx.given[i][1] for i in todo], ctx.given[0][0])
             for i, g in zip(todo, new):

@@ -286,3 +286,60 @@ def test_one_head_whose_rows_are_closer_together_than_in_lds(device, Sq, Sk, D, 
     # 192 and 64 bytes from row to row, where an LDS tile has 256 and 128
     fn, ofn, qkw, kvkw = _bias(kind, 1, Sq, Sk, 1)
     _check(device, f"pair {kind}", 1, Sq, Sk, 1, D, 1, fn, ofn, qkw, kvkw, seed=Sq + Sk, impl="pallas")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Sq,Sk,D,H", [(129, 65, 64, 2), (300, 1000, 96, 2), (2048, 130, 32, 1), (640, 640, 128, 40), (8200, 8200, 128, 1)])
+def test_gradients_leave_the_kernels_in_the_callers_dtype(device, Sq, Sk, D, H, dtype):
+    # shared and unshared rows and keys, and (640, H=40: dK and dV; 8200) the long-stretch kernels
+    g = torch.Generator(device=device).manual_seed(Sq + D)
+    q, k, v = (torch.randn((1, S, H, D), device=device, generator=g).to(torch.bfloat16).to(dtype).requires_grad_(True) for S in (Sq, Sk, Sk))
+    do = torch.randn((1, Sq, H, D), device=device, generator=g).to(torch.bfloat16).to(dtype)
+    causal = Sq == Sk
+    out = ra.ring_attention(q, k, v, 1, ra.causal_bias() if causal else None)
+    grads = torch.autograd.grad(out, (q, k, v), do)
+    for x, got in zip((q, k, v), grads):
+        assert got.dtype == dtype and got.shape == x.shape
+    ref = [x.detach().float().requires_grad_(True) for x in (q, k, v)]
+    for h in range(H):
+        s = (ref[0][0, :, h] @ ref[1][0, :, h].T) / np.sqrt(D)
+        if causal:
+            s = s.masked_fill(torch.ones_like(s, dtype=torch.bool).triu(1), -float("inf"))
+        (torch.softmax(s, -1) @ ref[2][0, :, h]).backward(do[0, :, h].float())
+    for got, x in zip(grads, ref):
+        assert max(_rel(got.float().cpu().numpy(), x.grad.cpu().numpy())) <= GRAD_TOL
+
+
+@pytest.mark.parametrize("Lq,Lk,H,D,offset", [(1, 1, 1, 64, None), (129, 200, 2, 128, 0), (257, 63, 3, 64, 100), (300, 300, 2, 128, 400),
+                                              (1000, 700, 2, 128, -500), (3601, 3700, 32, 128, None), (3601, 3700, 32, 128, 4000),
+                                              (2100, 2100, 32, 64, None), (4100, 4100, 17, 128, 0), (64, 64, 2, 128, -64)])
+def test_single_steps_on_both_sides_of_the_rule(device, Lq, Lk, H, D, offset):
+    """fwd_block on a carry that is not empty and bwd_block: pairs on the kernels for short pairs and on the long-stretch
+    ones (the larger ones without a mask), a pair that sees nothing (-64), queries that see nothing (-500)."""
+    g = torch.Generator(device=device).manual_seed(Lq + H)
+    q, k, v, do, k0, v0 = (torch.randn((1, H, L, D), device=device, generator=g).to(torch.bfloat16)
+                           for L in (Lq, Lk, Lk, Lq, 40, 40))
+    scale = 1 / np.sqrt(D)
+    bias = None if offset is None else ra.BlockBias(ra.causal_bias(), max(offset, 0), max(-offset, 0))
+    carry = rr.init_carry(1, H, Lq, D, device)
+    ra.fwd_block(q, k0, v0, None, *carry, scale)
+    ra.fwd_block(q, k, v, bias, *carry, scale)
+    out, lse = torch.empty((1, H, Lq, D), device=device), torch.empty((1, H, Lq), device=device)
+    rr.finalize_carry(*carry, out, lse)
+    grads = ra.bwd_block(q, k, v, bias, out, lse, do, scale)
+    seen = None
+    if offset is not None:
+        seen = torch.arange(Lq, device=device)[:, None] + offset >= torch.arange(Lk, device=device)[None]
+    for h in range(H):
+        a = [x[0, h].float() for x in (q, k, v, do, k0, v0)]
+        s = torch.cat([a[0] @ a[4].T, a[0] @ a[1].T], 1) * scale
+        if seen is not None:
+            s[:, 40:].masked_fill_(~seen, -float("inf"))
+        p = torch.softmax(s, -1)
+        o = p @ torch.cat([a[5], a[2]])
+        assert (out[0, h] - o).abs().max() <= OUT_TOL and (lse[0, h] - torch.logsumexp(s, -1)).abs().max() <= LSE_TOL
+        ds = p * (a[3] @ torch.cat([a[5], a[2]]).T - (o * a[3]).sum(-1, keepdim=True))
+        want = ((ds[:, 40:] @ a[1]) * scale, (ds[:, 40:].T @ a[0]) * scale, p[:, 40:].T @ a[3])
+        for got, ref in zip(grads, want):
+            err = (got[0, h] - ref).abs().max() / max(ref.abs().max().item(), 1e-3)
+            assert err <= GRAD_TOL, (h, err)

@@ -349,6 +349,17 @@ typedef struct {
 } ra_rows;
 int ra_convert(const ra_rows* items, int32_t n_items, void* stream);
 
+/* A whole call: ra_convert of the operands that `before` lists (none: n_before = 0), then ra_fwd_whole /
+ * ra_bwd_whole on what they made. */
+int ra_fwd_call(const ra_rows* before, int32_t n_before, const ra_fwd_step_params* p, void* out, int32_t out_dtype,
+                int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_l, float* lse, void* workspace,
+                int64_t workspace_bytes, void* stream);
+int ra_bwd_call(const ra_rows* before, int32_t n_before, const ra_bwd_step_params* p, const void* out,
+                int32_t out_dtype, int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_l,
+                int32_t grad_dtype, void* dq, int64_t dq_stride_b, int64_t dq_stride_h, int64_t dq_stride_l,
+                void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h, int64_t dkv_stride_l,
+                void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Host-only, pure: 1 if every score of the (query shard, key/value shard) pair is masked
  * by the positional terms of `bias` (CAUSAL / WINDOW), so that the whole ring step is an
  * identity on the carry and may be skipped; 0 otherwise.  The reference runs such steps and

@@ -1260,6 +1260,27 @@ int ra_convert(const ra_rows* items, int32_t n_items, void* stream) {
   return e == hipSuccess ? RA_OK : hip_fail(e, "ra_convert launch");
 }
 
+int ra_fwd_call(const ra_rows* before, int32_t n_before, const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b,
+                int64_t out_stride_h, int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (n_before) {
+    int rc = ra_convert(before, n_before, stream);
+    if (rc) return rc;
+  }
+  return ra_fwd_whole(p, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, lse, workspace, workspace_bytes, stream);
+}
+
+int ra_bwd_call(const ra_rows* before, int32_t n_before, const ra_bwd_step_params* p, const void* out, int32_t out_dtype,
+                int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_l, int32_t grad_dtype, void* dq, int64_t dq_stride_b,
+                int64_t dq_stride_h, int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
+                int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (n_before) {
+    int rc = ra_convert(before, n_before, stream);
+    if (rc) return rc;
+  }
+  return ra_bwd_whole(p, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, grad_dtype, dq, dq_stride_b, dq_stride_h,
+                      dq_stride_l, dk, dv, dkv_stride_b, dkv_stride_h, dkv_stride_l, workspace, workspace_bytes, stream);
+}
+
 int ra_bwd_finalize_passes(const float* acc, void* out, int64_t out_stride_pass, int64_t out_stride_b,
                            int64_t out_stride_h, int64_t out_stride_l, int32_t n_passes, int32_t B, int32_t H,
                            int32_t L, int32_t D, void* stream) {

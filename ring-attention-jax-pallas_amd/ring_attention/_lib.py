@@ -107,6 +107,12 @@ EXPORTS = {
     "ra_bwd_whole": (C.c_int, [C.POINTER(RaBwdStepParams), C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64, C.c_int32,
                                C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64,
                                C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p]),
+    # blocks that the caller packs: ra_rows, then the call's parameters
+    "ra_fwd_call": (C.c_int, [C.c_char_p, C.c_int32, C.c_char_p, C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64,
+                              C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p]),
+    "ra_bwd_call": (C.c_int, [C.c_char_p, C.c_int32, C.c_char_p, C.c_void_p, C.c_int32, C.c_int64, C.c_int64, C.c_int64,
+                              C.c_int32, C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_int64,
+                              C.c_int64, C.c_int64, C.c_void_p, C.c_int64, C.c_void_p]),
     "ra_convert": (C.c_int, [C.c_char_p, C.c_int32, C.c_void_p]),  # ra_rows blocks, packed
     "ra_fwd_finalize_passes": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_int64,
                                          C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_int32, C.c_int32,

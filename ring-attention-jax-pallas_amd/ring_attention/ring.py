@@ -100,7 +100,9 @@ def _walked_ring_size(n: int, Sq: int, Sk: int, bias_fn) -> int:
 
 
 def _stream() -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream of the current device, as ``torch.cuda.current_stream()`` names it (without building
+    the object: 3 us)."""
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 @functools.lru_cache(maxsize=64)
@@ -163,6 +165,17 @@ def _convert(tensors, dtypes, d: int):
     if n:
         _lib.check("ra_convert", _lib.load().ra_convert(items, n, _stream()))
     return out
+
+
+def _row_item(t: torch.Tensor, ptr: int, d: int):
+    """The ``ra_rows`` that converts [b, l, h, *] to bf16 rows of ``d`` elements one after another at ``ptr``; None for
+    what ``ra_convert`` does not take."""
+    src = _ROW_DTYPES.get(t.dtype)
+    B, L, H, dt = t.shape
+    sb, sl, sh, sd = t.stride()
+    if src is None or sd != 1 or B >= 65536 or not 0 < B * L * H or L * H >= 1 << 27:
+        return None
+    return _ROWS.pack(t.data_ptr(), ptr, src, _lib.RA_DTYPE_BF16, dt, d, B, L, H, sb, sl, sh, L * H * d, H * d, d)
 
 
 def _kernel_inputs(tensors, d: int):
@@ -525,14 +538,21 @@ class _RingPlan:
         plan.D = self.d_pair
         return plan
 
-    def pair_bias(self) -> "_lib.RaBias":
-        """The bias of a ring of one shard, as the library takes it: the plan holds the arrays."""
-        got = self.__dict__.get("_pair_bias")
+    def pair_call(self, backward: bool):
+        """What the calls on a ring of one shard share: the bias block, and the size of the workspace of the forward or
+        the backward.  The plan holds the arrays."""
+        got = self.__dict__.get("_pair_call")
         if got is None:
             bias = self.block_bias(0, 0)
-            got = (_bias_struct(bias, self.device, (self.B, self.H, self.Lq, self.Lk), summary=False), bias)
-            self.__dict__["_pair_bias"] = got
-        return got[0]
+            made = _bias_struct(bias, self.device, (self.B, self.H, self.Lq, self.Lk), summary=False)
+            got = self.__dict__["_pair_call"] = {"bias": bytes(made), "arrays": bias, "made": made}
+        size = got.get(backward)
+        if size is None:
+            p = (_lib.RaBwdStepParams if backward else _lib.RaFwdStepParams)(self.B, self.H, self.Lq, self.Lk, self.D, 1.0)
+            p.bias = got["made"]
+            lib = _lib.load()
+            size = got[backward] = (lib.ra_bwd_whole_workspace if backward else lib.ra_fwd_whole_workspace)(C.byref(p))
+        return got["bias"], size
 
     def live_steps(self, qs: Optional[int], ks: Optional[int]) -> int:
         """How many ring steps of query shard ``qs`` (or key/value shard ``ks``) are not masked
@@ -670,7 +690,7 @@ def _plan_for(q, k, n, bias_fn, q_kwargs, kv_kwargs) -> "_RingPlan":
     elif bias_fn is not None:
         fn_key = ("callable", id(bias_fn))
     kw_key = tuple(tuple(sorted((a, ident(t)) for a, t in (kw or {}).items())) for kw in (q_kwargs, kv_kwargs))
-    key = (tuple(q.shape), tuple(k.shape), str(q.device), n, fn_key, kw_key)
+    key = (q.shape, k.shape, q.device, n, fn_key, kw_key)
     hit = _PLAN_CACHE.get(key)
     if hit is not None:
         _PLAN_CACHE.move_to_end(key)
@@ -777,37 +797,93 @@ def _view_blhd(t: torch.Tensor) -> "_lib.RaTensor":
     return _lib.RaTensor(t.data_ptr(), sb, sh, sl)
 
 
-def _pair_forward(q, k, v, plan: "_RingPlan", sm_scale, out_dtype):
-    """``_ring_forward_fused`` of a ring of one shard: one description, one launch."""
+# The blocks of one call on a whole sequence, up to the bias: packed in one call where ctypes structures cost 10 us.
+_FWD_HEAD = struct.Struct("5if12q24x")     # sizes, scale, q, k, v (pointer, strides of batch, head, row); no carry
+_BWD_HEAD = struct.Struct("5if16qq32x")  # ... and dO, the logsumexp; no delta, no accumulators
+
+
+def _rows_at(ptr: int, L: int, H: int, D: int):
+    """Pointer and strides of contiguous [b, l, h, d] rows."""
+    return ptr, L * H * D, D, H * D
+
+
+def _rows_of(t: torch.Tensor):
+    sb, sl, sh, _ = t.stride()
+    return t.data_ptr(), sb, sh, sl
+
+
+def _pair_operands(q, k, v, plan: "_RingPlan"):
+    """What a call on a whole sequence reads: (tensors to keep, blocks of ``ra_rows`` that make them, their number).
+    One buffer holds all three operands where they have to be converted."""
+    D = plan.D
+    if q.dtype == k.dtype == v.dtype and (q.dtype != torch.bfloat16 or q.shape[3] != D) and q.device == k.device == v.device:
+        nq, nk = plan.B * plan.Lq * plan.H * D, plan.B * plan.Lk * plan.H * D
+        if tuple(k.shape) == tuple(v.shape) == (plan.B, plan.Lk, plan.H, q.shape[3]):
+            buf = torch.empty((nq + 2 * nk,), dtype=torch.bfloat16, device=q.device)
+            at = buf.data_ptr()
+            items = [_row_item(x, y, D) for x, y in ((q, at), (k, at + 2 * nq), (v, at + 2 * (nq + nk)))]
+            if all(items):
+                return (buf,), b"".join(items), 3
+    return tuple(_kernel_inputs((q, k, v), D)), b"", 0
+
+
+def _pair_views(kept, plan: "_RingPlan"):
+    if len(kept) == 3:
+        return [_rows_of(x) for x in kept]
+    at, H, D = kept[0].data_ptr(), plan.H, plan.D
+    nq, nk = plan.B * plan.Lq * H * D, plan.B * plan.Lk * H * D
+    return [_rows_at(at, plan.Lq, H, D), _rows_at(at + 2 * nq, plan.Lk, H, D), _rows_at(at + 2 * (nq + nk), plan.Lk, H, D)]
+
+
+def _workspace(size: int, device):
+    if not size:
+        return None, None
+    ws = torch.empty((size,), dtype=torch.uint8, device=device)
+    return ws, ws.data_ptr()
+
+
+def _pair_forward(kept, plan: "_RingPlan", sm_scale, out_dtype, before=b"", n_before=0):
+    """``_ring_forward_fused`` of a ring of one shard: one call, conversions of its operands (``before``) included.
+    Host code is what small calls cost: fp32 forward of 1024 tokens, H=4, 49 us as three calls with ctypes structures,
+    an object for the stream and an array per operand, 32 us like this (the kernels take 19); training on 2 x 2048 packed
+    tokens 250 | 166."""
     B, H, D, Lq = plan.B, plan.H, plan.D, plan.Lq
     out = torch.empty((B, Lq, H, D), dtype=out_dtype, device=plan.device)
     lse = torch.empty((1, B, H, Lq), dtype=torch.float32, device=plan.device)
-    p = _lib.RaFwdStepParams(B, H, Lq, plan.Lk, D, sm_scale, _view_blhd(q), _view_blhd(k), _view_blhd(v), None, None,
-                             None, plan.pair_bias())
-    lib = _lib.load()
-    size = lib.ra_fwd_whole_workspace(C.byref(p))
-    ws = torch.empty((size,), dtype=torch.uint8, device=plan.device) if size else None
-    _lib.check("ra_fwd_whole", lib.ra_fwd_whole(C.byref(p), out.data_ptr(), _DTYPE_CODE[out_dtype], Lq * H * D, D, H * D,
-                                                lse.data_ptr(), None if ws is None else ws.data_ptr(), size, _stream()))
+    bias, size = plan.pair_call(False)
+    q, k, v = _pair_views(kept, plan)
+    ws, ws_ptr = _workspace(size, plan.device)
+    _lib.check("ra_fwd_call", _lib.load().ra_fwd_call(
+        before, n_before, _FWD_HEAD.pack(B, H, Lq, plan.Lk, D, sm_scale, *q, *k, *v) + bias, out.data_ptr(), _DTYPE_CODE[out_dtype],
+        Lq * H * D, D, H * D, lse.data_ptr(), ws_ptr, size, _stream()))
     return out, lse
 
 
-def _pair_backward(q, k, v, out, lse, do, plan: "_RingPlan", sm_scale, dtype=torch.bfloat16):
-    """``_ring_backward_fused`` of a ring of one shard: one description for all launches.  ``dtype``: the
-    gradients', of bf16 precision whatever it is."""
-    B, H, D, Lq, Lk = plan.B, plan.H, plan.D, plan.Lq, plan.Lk
-    lib = _lib.load()
-    dq, dk, dv = (torch.empty_like(x, dtype=dtype) for x in (q, k, v))
-    p = _lib.RaBwdStepParams(B, H, Lq, Lk, D, sm_scale, _view_blhd(q), _view_blhd(k), _view_blhd(v), _view_blhd(do),
-                             lse.data_ptr(), None, None, None, None, plan.pair_bias())
-    size = lib.ra_bwd_whole_workspace(C.byref(p))
-    ws = torch.empty((size,), dtype=torch.uint8, device=plan.device)
+def _pair_backward(kept, out, lse, do, plan: "_RingPlan", sm_scale, dtype=torch.bfloat16):
+    """``_ring_backward_fused`` of a ring of one shard: one call for all launches, the conversion of ``do`` included.
+    ``dtype``: the gradients', of bf16 precision whatever it is."""
+    B, H, D, Lq, Lk, device = plan.B, plan.H, plan.D, plan.Lq, plan.Lk, plan.device
+    if len(kept) == 3:
+        grads = [torch.empty_like(x, dtype=dtype) for x in kept]
+    else:
+        grads = [torch.empty((B, L, H, D), dtype=dtype, device=device) for L in (Lq, Lk, Lk)]
+    before = None
+    if do.dtype != torch.bfloat16 or do.shape[3] != D:
+        made = torch.empty((B, Lq, H, D), dtype=torch.bfloat16, device=device)
+        before = _row_item(do, made.data_ptr(), D) if do.device == device else None
+    if before is None:
+        made, = _kernel_inputs((do,), D)
+    dq, dk, dv = grads
     assert dk.stride() == dv.stride()
-    (ob, ol, oh, _), (qb, ql, qh, _), (kb, kl, kh, _) = out.stride(), dq.stride(), dk.stride()
-    _lib.check("ra_bwd_whole", lib.ra_bwd_whole(
-        C.byref(p), out.data_ptr(), _DTYPE_CODE[out.dtype], ob, oh, ol, _ROW_DTYPES[dtype] | _lib.RA_DTYPE_VIA_BF16, dq.data_ptr(), qb, qh, ql, dk.data_ptr(),
-        dv.data_ptr(), kb, kh, kl, ws.data_ptr(), size, _stream()))
-    return dq, dk, dv
+    bias, size = plan.pair_call(True)
+    q, k, v = _pair_views(kept, plan)
+    ws, ws_ptr = _workspace(size, device)
+    (_, qb, qh, ql), (_, kb, kh, kl), (_, ob, oh, ol) = _rows_of(dq), _rows_of(dk), _rows_of(out)
+    _lib.check("ra_bwd_call", _lib.load().ra_bwd_call(
+        before, 0 if before is None else 1, _BWD_HEAD.pack(B, H, Lq, Lk, D, sm_scale, *q, *k, *v, *_rows_of(made), lse.data_ptr()) + bias,
+        out.data_ptr(), _DTYPE_CODE[out.dtype], ob, oh, ol, _ROW_DTYPES[dtype] | _lib.RA_DTYPE_VIA_BF16, dq.data_ptr(), qb, qh, ql,
+        dk.data_ptr(), dv.data_ptr(), kb, kh, kl, ws_ptr, size, _stream()))
+    return grads
 
 
 def _ring_forward_fused(q, k, v, plan: _RingPlan, sm_scale, out_dtype, timer=_NO_TIMER, whole=True):
@@ -819,7 +895,7 @@ def _ring_forward_fused(q, k, v, plan: _RingPlan, sm_scale, out_dtype, timer=_NO
     if plan.callable is not None:
         return _ring_forward_rows(q, k, v, plan, sm_scale, out_dtype, timer)
     if plan.n == 1 and whole and timer is _NO_TIMER:
-        return _pair_forward(q, k, v, plan, sm_scale, out_dtype)
+        return _pair_forward((q, k, v), plan, sm_scale, out_dtype)
     n, B, H, D, Lq, Lk = plan.n, plan.B, plan.H, plan.D, plan.Lq, plan.Lk
     dev = q.device
     lib = _lib.load()
@@ -876,7 +952,7 @@ def _ring_backward_fused(q, k, v, out, lse, do, plan: _RingPlan, sm_scale, timer
     if plan.callable is not None:
         return _ring_backward_rows(q, k, v, out, lse, do, plan, sm_scale, timer)
     if plan.n == 1 and whole and timer is _NO_TIMER:
-        return _pair_backward(q, k, v, out, lse, do, plan, sm_scale)
+        return _pair_backward((q, k, v), out, lse, do, plan, sm_scale)
     n, B, H, D, Lq, Lk = plan.n, plan.B, plan.H, plan.D, plan.Lq, plan.Lk
     dev = q.device
     lib = _lib.load()
@@ -990,10 +1066,14 @@ class _RingAttentionFn(torch.autograd.Function):
         be the kernels' own (padded, ``out_dtype``), which the caller cuts."""
         ctx.given = [(t.shape[3], t.dtype) for t in (q, k, v)]
         d = q.shape[3]
-        q, k, v = _kernel_inputs((q, k, v), plan.D)
-        fwd = _ring_forward_fused if fused else _ring_forward
-        out, lse = fwd(q, k, v, plan, sm_scale, out_dtype)
-        ctx.save_for_backward(q, k, v, out, lse)
+        ctx.whole = fused and plan.n == 1 and plan.callable is None  # one call, conversions included
+        if ctx.whole:
+            kept, before, n = _pair_operands(q, k, v, plan)
+            out, lse = _pair_forward(kept, plan, sm_scale, out_dtype, before, n)
+        else:
+            kept = _kernel_inputs((q, k, v), plan.D)
+            out, lse = (_ring_forward_fused if fused else _ring_forward)(*kept, plan, sm_scale, out_dtype)
+        ctx.save_for_backward(*kept, out, lse)
         ctx.plan, ctx.sm_scale, ctx.fused = plan, sm_scale, fused
         ctx.mark_non_differentiable(lse)
         ctx.set_materialize_grads(False)  # no zero fill for the logsumexp's gradient
@@ -1003,22 +1083,23 @@ class _RingAttentionFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, do, _dlse):
-        q, k, v, out, lse = ctx.saved_tensors
+        *kept, out, lse = ctx.saved_tensors
+        plan = ctx.plan
         if do is None:  # nothing came back for the output: gradients of zero, as materialised ones give
             do = torch.zeros(out.shape, dtype=torch.bfloat16, device=out.device)
-        do, = _kernel_inputs((do,), ctx.plan.D)
-        plan = ctx.plan
         d_true, dtype = ctx.given[0]
-        if (ctx.fused and plan.n == 1 and plan.callable is None and d_true == plan.D and dtype in _ROW_DTYPES
-                and all(given[1] == dtype for given in ctx.given)):
-            grads = list(_pair_backward(q, k, v, out, lse, do, plan, ctx.sm_scale, dtype))  # as the caller wants them
+        if ctx.whole:
+            # as the caller wants them, where that takes no cut
+            direct = d_true == plan.D and dtype in _ROW_DTYPES and all(given[1] == dtype for given in ctx.given)
+            grads = list(_pair_backward(kept, out, lse, do, plan, ctx.sm_scale, dtype if direct else torch.bfloat16))
         else:
+            do, = _kernel_inputs((do,), plan.D)
             bwd = _ring_backward_fused if ctx.fused else _ring_backward
-            grads = list(bwd(q, k, v, out, lse, do, plan, ctx.sm_scale))
+            grads = list(bwd(*kept, out, lse, do, plan, ctx.sm_scale))
         todo = [i for i, (d, dtype) in enumerate(ctx.given)
                 if ctx.needs_input_grad[i] and (d != plan.D or dtype != grads[i].dtype)]
         if todo:
-            new = _convert([grads[i] for i in todo], [ctx.given[i][1] for i in todo], ctx.given[0][0])
+            new = _convert([grads[i] for i in todo], [ctx.given[i][1] for i in todo], d_true)
             for i, g in zip(todo, new):
                 grads[i] = g
         return *(g if need else None for g, need in zip(grads, ctx.needs_input_grad)), None, None, None, None, None
@@ -1029,6 +1110,11 @@ def ring_attention_with_lse(q, k, v, axis_name, bias_fn: Union[BiasFn, Callable,
                             block_impl: str = "pallas", out_dtype=None):
     """``ring_attention`` that also returns the logsumexp ``[b, h, S]`` (the ``L`` residual of
     ring.py:135)."""
+    out, lse, plan = _attend(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs, sm_scale, block_impl, out_dtype)
+    return out, lse.permute(1, 2, 0, 3).reshape(plan.B, plan.H, plan.n * plan.Lq)
+
+
+def _attend(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs, sm_scale, block_impl, out_dtype=None):
     if block_impl not in _IMPLS:
         raise ValueError(block_impl)
     if bias_fn is not None and not isinstance(bias_fn, BiasFn) and not callable(bias_fn):
@@ -1058,8 +1144,7 @@ def ring_attention_with_lse(q, k, v, axis_name, bias_fn: Union[BiasFn, Callable,
     out, lse = _RingAttentionFn.apply(q, k, v, plan, float(sm_scale), out_dtype, final_dtype, fused)
     if out.shape[-1] != d_true:
         out = out[..., :d_true]
-    lse_full = lse.permute(1, 2, 0, 3).reshape(plan.B, plan.H, plan.n * plan.Lq)
-    return out, lse_full
+    return out, lse, plan
 
 
 def ring_attention(q, k, v, axis_name, bias_fn: Union[BiasFn, Callable, None] = None, bias_q_kwargs=None,
@@ -1086,9 +1171,7 @@ def ring_attention(q, k, v, axis_name, bias_fn: Union[BiasFn, Callable, None] = 
     Returns:
         attention output ``[b, S, h, d]``; differentiable w.r.t. q, k, v.
     """
-    out, _ = ring_attention_with_lse(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs,
-                                     sm_scale, block_impl)
-    return out
+    return _attend(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs, sm_scale, block_impl)[0]
 
 
 def ring_self_attention(q, k, v, mesh, pspec=None, sm_scale: Optional[float] = None,

@@ -593,15 +593,18 @@ RA_DEV int consecutive_end(const unsigned short* list, int cnt, int lane, int fr
 // Decode the flat workgroup id into (batch*head index, tile index).  Workgroups are handed
 // to the 8 XCDs round-robin, each XCD has its own L2: keep all tiles of one head on one
 // XCD so they share the head's K/V (or Q/dO) stream, and start with the last tile, which
-// has the most work under a causal mask.
+// has the most work under a causal mask.  Where the heads do not divide by eight a head is spread over all XCDs whatever
+// the order: there the tiles come in descending order over all heads, so that the chip does not end on the long tiles of the
+// last heads.  Head by head | longest first, us, D=128, causal: H=12 8192 forward 428 | 262, dK/dV 517 | 421; 4096 dK/dV 191 | 111; 32768
+// 3497 | 2816, 5413 | 5025, dQ 4674 | 3820; H=4 32768 1431 | 948, 1778 | 1688, 1872 | 1283; 36 heads of 8192 1036 | 676, 1334 | 1124.
 RA_DEV void decode_block(int bid, int BH, int ntile, int& hh, int& tile) {
   if ((BH & 7) == 0) {
     int xcd = bid & 7, slot = bid >> 3;
     hh = (slot / ntile) * 8 + xcd;
     tile = ntile - 1 - (slot % ntile);
   } else {
-    hh = bid / ntile;
-    tile = ntile - 1 - (bid % ntile);
+    tile = ntile - 1 - bid / BH;
+    hh = bid % BH;
   }
 }
 

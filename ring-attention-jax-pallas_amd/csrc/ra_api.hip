@@ -406,6 +406,7 @@ bool choose_by_content(const ra_bias& b, int64_t slabs, int Lq, int Lk) {
   const int side = std::min(Lq, Lk);
   return b.dense_map && (side >= 8192 || (side >= 4096 && slabs <= 512));
 }
+constexpr int kHeadGroup = 4;  // heads of an XCD that the pair kernels take together (see pair_decode)
 constexpr int kWholeRow = 1 << 30;  // chunk_tiles of rows that are not shared
 
 int fwd_step_on_pair(const ra_fwd_step_params& p, void* stream) {
@@ -423,6 +424,7 @@ int fwd_step_on_pair(const ra_fwd_step_params& p, void* stream) {
   a.bias = to_bias(p.bias);
   a.n_split = 1;
   a.chunk_tiles = kWholeRow;
+  a.group = kHeadGroup;
   a.o = p.o;
   a.m = p.m;
   a.l = p.l;
@@ -438,6 +440,7 @@ int bwd_step_on_pair(const ra_bwd_step_params& p, int parts, void* stream) {
   a.a = to_bwd_args(p);
   a.n_split = 1;
   a.chunk_tiles = kWholeRow;
+  a.group = kHeadGroup;
   const int mode = kernel_mode(p.bias.flags);
   hipError_t e = hipSuccess;
   if (parts & 1) {
@@ -666,6 +669,7 @@ struct PairPlan {
   bool pair;        // the kernels of ra_pair.hip
   int n_split;      // most workgroups that share a row's keys ...
   int chunk_tiles;  // ... each of about this many tiles
+  int group;        // heads of an XCD that are taken together (see pair_decode)
 };
 
 // Key tiles that one head's query tiles visit (positional terms only): their sum, and the most.
@@ -708,12 +712,20 @@ bool long_stretches(const ra_bias& bias, int D, int64_t wgs, int64_t total, int6
 // 4096: 88 -> 63 us; H=4, 16384: 375 -> 340 us).  At most kMaxSplit shares, and none under kMinChunk tiles, which
 // cost more in partial results (528 bytes per row and share) than they gain.
 constexpr int kMinChunk = 6, kMaxSplit = 64;
+bool has_lists(const ra_bias& b) { return b.flags & (RA_BIAS_SEGMENT | RA_BIAS_PREFIX | RA_BIAS_DENSE); }
+// Whether all of a head's resident tiles have about the same work.
+bool even_rows(int64_t total, int most, int64_t rows) { return total * 20 >= (int64_t)most * rows * 17; }
+// Whether the pair kernels take an XCD's heads one after the other (see pair_decode): unmasked rows.  (Not under a window: D=64,
+// 2048 of 16384, 32 heads, 1.23 ms a pass over all heads, 1.27 one by one.)
+bool one_by_one(const ra_bias& b, int64_t total, int most, int64_t rows) {
+  return even_rows(total, most, rows) && !has_lists(b) && !(b.flags & RA_BIAS_WINDOW);
+}
 // How the `wgs` workgroups of one kind of a head's resident tiles, which meet `total` tiles of the other
 // side (`most` at most), share their work (see above).
 void plan_split(PairPlan& r, int64_t heads, int64_t rows, int64_t total, int most, int min_chunk) {
   const int64_t wgs = heads * rows;
   if (wgs > kPairSlots || most <= min_chunk) return;
-  const bool even = total * 20 >= (int64_t)most * rows * 17;
+  const bool even = even_rows(total, most, rows);
   const int64_t chunk = even ? (most + kPairSlots / wgs - 1) / (kPairSlots / wgs) : heads * total * 3 / (2 * kPairSlots);
   r.chunk_tiles = (int)std::min<int64_t>(most, std::max<int64_t>({chunk, min_chunk, (most + kMaxSplit - 1) / kMaxSplit}));
   r.n_split = (most + r.chunk_tiles - 1) / r.chunk_tiles;
@@ -730,7 +742,7 @@ bool step_on_pair(const ra_bias& bias, int B, int H, int Lq, int Lk, int D, bool
   int most, live;
   count_key_tiles(bias, Lq, Lk, total, most, &live);
   const int64_t rows = (Lq + kPairRowsHost - 1) / kPairRowsHost, wgs = (int64_t)B * H * rows;
-  const bool even = total * 20 >= (int64_t)most * rows * 17;
+  const bool even = even_rows(total, most, rows);
   if (D == 64) return !(forward && even && wgs > kPairSlots / 2 && total < 192 * rows);
   if (wgs <= kPairSlots / 2) return true;
   return wgs <= kPairSlots ? !even : total < 56 * (int64_t)live;
@@ -741,9 +753,13 @@ PairPlan plan_fwd_pair(const ra_fwd_step_params& p) {
   int64_t total;
   int most;
   count_key_tiles(p.bias, p.Lq, p.Lk, total, most);
-  PairPlan r{true, 1, std::max(most, 1)};
-  if (long_stretches(p.bias, p.D, wgs, total, rows, 56)) r.pair = false;
+  PairPlan r{true, 1, std::max(most, 1), kHeadGroup};
+  // (with ALiBi from 192 tiles on: 65 of them, 32 heads of 8192, 0.70 | 0.63 ms, 129, 16 of 16384, 1.19 | 1.16, 257 4.48 | 4.74; and not
+  // uneven rows that fill the chip less than one and a quarter times: 8 heads of 10240, 0.275 | 0.250)
+  const bool nearly_one = wgs <= kPairSlots * 5 / 4 && !even_rows(total, most, rows);
+  if (!nearly_one && long_stretches(p.bias, p.D, wgs, total, rows, (p.bias.flags & RA_BIAS_ALIBI) ? 192 : 56)) r.pair = false;
   if (r.pair) plan_split(r, heads, rows, total, most, kMinChunk);
+  if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;
 }
 // dQ, likewise (dq_kernel | dq_pair_kernel): 65 tiles (32 heads of 8192) 0.70 | 0.66 ms, 66 (window 4096 of 65536, H=8) 1.36 |
@@ -752,16 +768,19 @@ PairPlan plan_dq_pair(const ra_bwd_step_params& p) {
   int64_t total;
   int most;
   count_key_tiles(p.bias, p.Lq, p.Lk, total, most);
-  PairPlan r{true, 1, std::max(most, 1)};
+  PairPlan r{true, 1, std::max(most, 1), kHeadGroup};
   const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lq + kPairRowsHost - 1) / kPairRowsHost;
   if (long_stretches(p.bias, p.D, heads * rows, total, rows, 160)) r.pair = false;
   else plan_split(r, heads, rows, total, most, kMinChunk);
+  if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;
 }
-// dK / dV, in 32-query tiles per 128 keys (dkdv_kernel | dkdv_pair_kernel): 65 (64 heads of 4096) 0.55 | 0.50 ms, 130 (32 of
-// 8192) 0.90 | 0.92, 128 (64 of 4096 x 4096) 0.88 | 0.91, 258 (32 of 16384) 3.4 | 3.6; ALiBi, 258: 1.82 | 1.90.  dkdv_kernel also
-// where there are between one and two and a half slabs per compute unit: dkdv_pair_kernel would hold them all at
-// once, the longest one deciding (16 heads of 4096: 0.13 | 0.16).  Fewer slabs are shared (12 heads of 2048: 0.056 | 0.050).
+// dK / dV, in 32-query tiles per 128 keys (dkdv_kernel | dkdv_pair_kernel): uneven rows 65 of them (64 heads of 4096) 0.55 | 0.50 ms,
+// 130 (32 of 8192) 1.08 | 1.04, 258 (32 of 16384) 3.42 | 3.48; even ones 128 (64 of 4096 x 4096) 0.89 | 0.90, 256 (16 of 8192 x 8192) 0.84 |
+// 0.89; ALiBi 130 1.03 | 0.95, 258 1.83 | 1.79, 514 7.05 | 7.05.  Between one and two and a half slabs per compute unit dkdv_pair_kernel would
+// hold them all at once, the longest one deciding: uneven rows take dkdv_kernel there (16 heads of 4096: 0.13 | 0.16; 12: 0.11 | 0.13; 4
+// of 16384: 0.44 | 0.56), even ones if they are long (16 heads of 4096, unmasked 0.230 | 0.233, of 3072 0.158 | 0.153, window of 1024 0.080 |
+// 0.070).  Fewer slabs are shared (12 heads of 2048: 0.056 | 0.050).
 PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
   const int ntiles = (p.Lq + 31) / 32;
   const ra::BiasArgs b = to_bias(p.bias);
@@ -773,12 +792,15 @@ PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
     total += hi - lo;
     most = std::max(most, hi - lo);
   }
-  PairPlan r{true, 1, std::max(most, 1)};
+  PairPlan r{true, 1, std::max(most, 1), kHeadGroup};
   const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lk + kPairRowsHost - 1) / kPairRowsHost, wgs = heads * rows;
   const bool one_round = wgs > kPairSlots / 2 && wgs <= kPairSlots * 5 / 4;
-  if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, total, rows, one_round ? 0 : 112)) r.pair = false;
+  const bool even = even_rows(total, most, rows);
+  const int tiles = one_round ? (even ? 112 : 0) : (p.bias.flags & RA_BIAS_ALIBI) ? 448 : even ? 112 : 192;
+  if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, total, rows, tiles)) r.pair = false;
   else if (heads * p.Lq >= (int64_t)1 << 30) r.pair = false;  // one 32-bit offset reaches both statistics of a row
   else plan_split(r, heads, rows, total, most, 2 * kMinChunk);
+  if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;
 }
 // The workspace of ra_bwd_pair: the rows' statistics, then the shares of dQ and of dK and dV.
@@ -856,6 +878,7 @@ static int fwd_pair(const ra_fwd_step_params* p, bool any_dim, void* out, int32_
   a.bias = to_bias(p->bias);
   a.n_split = plan.n_split;
   a.chunk_tiles = plan.chunk_tiles;
+  a.group = plan.group;
   a.out = out;
   a.out_f32 = out_dtype == RA_DTYPE_F32;
   a.out_sb = out_stride_b;
@@ -1172,6 +1195,7 @@ static int bwd_pair(const ra_bwd_step_params* p, bool any_dim, int grad_dtype, c
   auto share = [&](const PairPlan& plan, int64_t part, int64_t n, const RingResult& r) {
     a.n_split = plan.n_split;
     a.chunk_tiles = plan.chunk_tiles;
+    a.group = plan.group;
     a.part = plan.n_split > 1 ? (float*)(ws + part) : nullptr;
     a.part_n = plan.n_split > 1 ? (int*)(ws + n) : nullptr;
     a.out = r.base;

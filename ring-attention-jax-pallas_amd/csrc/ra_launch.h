@@ -113,6 +113,7 @@ struct PairFwdArgs {
   BiasArgs bias;
   int n_split;   // most workgroups that share a row's keys ...
   int chunk_tiles;  // ... each of about this many key tiles
+  int group;        // heads of an XCD whose tiles are taken together, the longest first
   // where the result goes: partial results of the shares (n_split > 1; part_s: m, l, l of the rounded
   // probabilities), a carry that is updated in place, or the finished output and logsumexp
   float *part_o, *part_s;
@@ -129,6 +130,7 @@ hipError_t launch_fwd_pair(const PairFwdArgs& a, int D, int mode, hipStream_t st
 struct PairBwdArgs {
   BwdArgs a;  // (its dq / dk / dv slots are not used)
   int n_split, chunk_tiles;
+  int group;  // (see PairFwdArgs)
   const float* stat;  // dK / dV: see pair_stat_kernel (nullptr: from a.lse and a.delta)
   float* part;
   int* part_n;

@@ -835,6 +835,13 @@ def _pair_views(kept, plan: "_RingPlan"):
     return [_rows_at(at, plan.Lq, H, D), _rows_at(at + 2 * nq, plan.Lk, H, D), _rows_at(at + 2 * (nq + nk), plan.Lk, H, D)]
 
 
+def _empty_gradients(q, k, v, dtype=torch.bfloat16):
+    """dq, dk and dv, not yet written, laid out as the operands [b, l, h, d].  The kernels store dk and dv with the same strides:
+    where k and v differ in theirs (rotary embeddings leave k transposed and v as it was, say) both are contiguous."""
+    kv_format = torch.preserve_format if k.stride() == v.stride() else torch.contiguous_format
+    return [torch.empty_like(q, dtype=dtype), *(torch.empty_like(x, dtype=dtype, memory_format=kv_format) for x in (k, v))]
+
+
 def _workspace(size: int, device):
     if not size:
         return None, None
@@ -864,7 +871,7 @@ def _pair_backward(kept, out, lse, do, plan: "_RingPlan", sm_scale, dtype=torch.
     ``dtype``: the gradients', of bf16 precision whatever it is."""
     B, H, D, Lq, Lk, device = plan.B, plan.H, plan.D, plan.Lq, plan.Lk, plan.device
     if len(kept) == 3:
-        grads = [torch.empty_like(x, dtype=dtype) for x in kept]
+        grads = _empty_gradients(*kept, dtype)
     else:
         grads = [torch.empty((B, L, H, D), dtype=dtype, device=device) for L in (Lq, Lk, Lk)]
     before = None
@@ -874,7 +881,6 @@ def _pair_backward(kept, out, lse, do, plan: "_RingPlan", sm_scale, dtype=torch.
     if before is None:
         made, = _kernel_inputs((do,), D)
     dq, dk, dv = grads
-    assert dk.stride() == dv.stride()
     bias, size = plan.pair_call(True)
     q, k, v = _pair_views(kept, plan)
     ws, ws_ptr = _workspace(size, device)
@@ -963,7 +969,7 @@ def _ring_backward_fused(q, k, v, out, lse, do, plan: _RingPlan, sm_scale, timer
     _lib.check("ra_bwd_delta_passes", lib.ra_bwd_delta_passes(
         out.data_ptr(), dt, Lq * ov.stride(2), ov.stride(0), ov.stride(1), ov.stride(2), C.byref(do_t),
         Lq * dov.stride(2), delta.data_ptr(), n, B, H, Lq, D, _stream()))
-    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    dq, dk, dv = _empty_gradients(q, k, v)
 
     def build():
         by_kv = _array_type(_lib.RaBwdStepParams, n * n)()
@@ -993,8 +999,7 @@ def _ring_backward_fused(q, k, v, out, lse, do, plan: _RingPlan, sm_scale, timer
             st.dout.stride_b, st.dout.stride_h, st.dout.stride_l = do.stride(0), do.stride(2), do.stride(1)
             st.lse, st.delta = lse.data_ptr() + qs * s_row, delta.data_ptr() + qs * s_row
     if whole:
-        gq, gk, gv = (g.permute(0, 2, 1, 3) for g in (dq, dk, dv))
-        assert gk.stride() == gv.stride()
+        gq, gk = (g.permute(0, 2, 1, 3) for g in (dq, dk))
         with timer.span("bwd_dkdv_ring", -1, -1):
             rc = lib.ra_bwd_dkdv_ring(by_kv, counts, n, dk.data_ptr(), dv.data_ptr(), Lk * gk.stride(2), gk.stride(0),
                                       gk.stride(1), gk.stride(2), _stream())

@@ -343,3 +343,27 @@ def test_single_steps_on_both_sides_of_the_rule(device, Lq, Lk, H, D, offset):
         for got, ref in zip(grads, want):
             err = (got[0, h] - ref).abs().max() / max(ref.abs().max().item(), 1e-3)
             assert err <= GRAD_TOL, (h, err)
+
+
+@pytest.mark.parametrize("D,n", [(32, 1), (64, 1), (96, 1), (128, 1), (64, 3), (128, 3)])
+@pytest.mark.parametrize("transposed", ["qk", "v"])
+def test_keys_and_values_laid_out_differently(device, D, n, transposed):
+    # [b, h, l, d] arrays seen as [b, l, h, d] (rotary embeddings leave q and k that way) beside contiguous ones; n = 3: shards whose
+    # positions are not consecutive, a whole-ring launch of several shards
+    B, S, H = 2, 129 * n, 2
+    q, k, v, do = R.make_inputs(D, B, S, S, H, D)
+    at = np.broadcast_to(np.concatenate([np.arange(129) + 200 * ((2 * i) % n) for i in range(n)]), (B, S))
+
+    def leaf(x, name):
+        t = _dev(x, device, torch.bfloat16)
+        return (t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3) if name in transposed else t).requires_grad_(True)
+
+    leaves = [leaf(x, name) for x, name in zip((q, k, v), "qkv")]
+    positions = _dev(at.copy(), device)
+    out, lse = ra.ring_attention_with_lse(*leaves, n, ra.causal_bias(), {"q_positions": positions}, {"kv_positions": positions},
+                                          out_dtype=torch.float32)
+    bias = R.make_bias_fn(causal=True)(q_positions=at, kv_positions=at)
+    want, want_lse = R.mha_dense(q, k, v, bias)
+    assert np.abs(out.detach().cpu().numpy() - want).max() <= OUT_TOL and np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_TOL
+    for g, ref in zip(torch.autograd.grad(out, leaves, _dev(do, device)), R.mha_dense_grads(q, k, v, do, bias)):
+        assert max(_rel(g.float().cpu().numpy(), ref)) <= GRAD_TOL

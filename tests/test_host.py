@@ -279,3 +279,36 @@ def test_views_the_kernels_cannot_take_are_copied():
     heads_interleaved = torch.zeros((2, 4, 16, 64), dtype=torch.bfloat16).permute(0, 2, 1, 3)  # [b, l, h, d] view, row stride 64
     assert rr._kernel_ready(heads_interleaved) is heads_interleaved
     assert rr._kernel_ready(torch.zeros((1, 8, 1, 64))).dtype == torch.bfloat16
+
+
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+def test_dk_and_dv_share_their_strides_whatever_those_of_k_and_v(monkeypatch, D):
+    # k a transposed [b, h, l, d], v contiguous, and the other way round: the library stores both gradients with dk's strides
+    calls = []
+
+    class Library:
+        def ra_bwd_whole_workspace(self, p):
+            return 64
+
+        def ra_bwd_call(self, *args):
+            calls.append(args)
+            return 0
+
+    monkeypatch.setattr(rr._lib, "load", Library)
+    monkeypatch.setattr(rr, "_stream", lambda: None)
+    B, L, H = 2, 48, 3
+    rows = torch.zeros((B, L, H, D), dtype=torch.bfloat16)
+    heads = torch.zeros((B, H, L, D), dtype=torch.bfloat16).permute(0, 2, 1, 3)
+    plan = rr._RingPlan(rows, rows, 1, None, None, None).joined()
+    assert plan.D == D
+    for q, k, v in [(heads, heads, rows), (rows, rows, heads), (heads, heads, heads), (heads, rows, rows)]:
+        kept = rr._kernel_inputs((q, k, v), D)
+        assert [x is y for x, y in zip(kept, (q, k, v))] == [True] * 3
+        dq, dk, dv = rr._pair_backward(kept, rows, torch.zeros((1, B, H, L)), rows, plan, 0.1)
+        assert dk.stride() == dv.stride() and (dk.stride() == k.stride() or k.stride() != v.stride())
+        assert dq.stride() == q.stride()
+        sb, sl, sh, _ = dk.stride()
+        assert calls.pop()[-8:-3] == (dk.data_ptr(), dv.data_ptr(), sb, sh, sl)
+    # the launches of a ring of several shards take their gradients from the same place
+    grads = rr._empty_gradients(heads, heads, rows)
+    assert grads[1].stride() == grads[2].stride() and grads[0].stride() == heads.stride()

@@ -363,7 +363,9 @@ def bwd_block(q, k, v, bias: Union[BlockBias, torch.Tensor, None], o, L, do, sm_
     dq, dk, dv = (torch.empty(x.shape, dtype=torch.float32, device=q.device) for x in (q, k, v))
     L = L.contiguous()
     p = _lib.RaBwdStepParams(B, H, Lq, k.shape[2], D, float(sm_scale), _view_bhld(q), _view_bhld(k), _view_bhld(v), _view_bhld(do),
-                             L.data_ptr(), None, None, None, None, _bias_struct(bias, q.device, (B, H, Lq, k.shape[2])))
+                             L.data_ptr(), L.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                             _bias_struct(bias, q.device, (B, H, Lq, k.shape[2])))
+    _lib.check("ra_bwd_step", lib.ra_bwd_step_check(C.byref(p)))  # a step's head dims: ra_bwd_whole takes more
     size = lib.ra_bwd_whole_workspace(C.byref(p))
     ws = torch.empty((size,), dtype=torch.uint8, device=q.device)
     (ob, oh, ol, _), (qb, qh, ql, _), (kb, kh, kl, _) = o.stride(), dq.stride(), dk.stride()

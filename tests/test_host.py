@@ -312,3 +312,18 @@ def test_dk_and_dv_share_their_strides_whatever_those_of_k_and_v(monkeypatch, D)
     # the launches of a ring of several shards take their gradients from the same place
     grads = rr._empty_gradients(heads, heads, rows)
     assert grads[1].stride() == grads[2].stride() and grads[0].stride() == heads.stride()
+
+
+@pytest.mark.parametrize("D", [16, 32, 80, 96, 160])
+def test_blocks_take_head_dims_64_and_128_only(monkeypatch, D):
+    # forward and backward alike: the head dims of whole sequences (multiples of 32) are no head dims of a ring step
+    monkeypatch.setattr(rr, "_require_gpu", lambda t: None)
+    monkeypatch.setattr(rr, "_stream", lambda: None)
+    x = torch.zeros((1, 2, 128, D), dtype=torch.bfloat16)
+    rows = torch.zeros((1, 2, 128))
+    acc = torch.zeros((1, 2, 128, D))
+    with pytest.raises(RuntimeError, match=f"head dim {D} unsupported .64 or 128"):
+        ra.fwd_block(x, x, x, None, acc, rows.clone(), rows.clone(), 0.1)
+    for bias in (None, ra.BlockBias(ra.causal_bias()), torch.zeros((1, 1, 128, 128))):
+        with pytest.raises(RuntimeError, match=f"head dim {D} unsupported .64 or 128"):
+            ra.bwd_block(x, x, x, bias, acc, rows, x, 0.1)

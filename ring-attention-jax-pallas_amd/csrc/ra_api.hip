@@ -798,7 +798,7 @@ PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
   const bool even = even_rows(total, most, rows);
   const int tiles = one_round ? (even ? 112 : 0) : (p.bias.flags & RA_BIAS_ALIBI) ? 448 : even ? 112 : 192;
   if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, total, rows, tiles)) r.pair = false;
-  else if (heads * p.Lq >= (int64_t)1 << 30) r.pair = false;  // one 32-bit offset reaches both statistics of a row
+  else if (heads * p.Lq + 31 >= (int64_t)1 << 30) r.pair = false;  // one 32-bit byte offset reaches both statistics of a tile's 32 rows
   else plan_split(r, heads, rows, total, most, 2 * kMinChunk);
   if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;

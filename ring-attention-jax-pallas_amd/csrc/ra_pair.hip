@@ -1349,7 +1349,7 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dkdv_pair_kern
   // lanes 0..31 move -lse of a tile's rows, lanes 32..63 -delta
   const bool raw_stat = DENSE && p.stat == nullptr;  // a single step, which has no room for them: from lse and delta, per tile
   const float* stat = (DENSE ? (raw_stat ? (g ? a.delta : a.lse) : p.stat + (g ? (long long)a.B * a.H * a.Lq : 0)) : p.stat) + (long long)hh * a.Lq;
-  const unsigned to_delta = (unsigned)(a.B * a.H) * (unsigned)a.Lq * 4;  // (below 2^32: plan_dkdv_pair)
+  const unsigned to_delta = (unsigned)(a.B * a.H) * (unsigned)a.Lq * 4;  // (with a row's 124 bytes below 2^32: plan_dkdv_pair)
   auto issue_tile = [&](int j, int buf) {
     const int r0 = j * kPairQueries;
     ldq.issue(r0, RA_LDS_ADDR(&s_q[0][0]) + buf * TILE_BYTES, wave, lane);

@@ -328,6 +328,19 @@ def test_bwd_pair_rejects_bad_arguments_without_a_gpu(lib):
         assert lib.ra_last_error() != b""
 
 
+def test_rows_beyond_a_32_bit_offset_are_refused_without_a_gpu(lib):
+    # dK / dV reach -lse and -delta of a tile's 32 rows through one 32-bit byte offset, 4 (B H Lq + 31) at most; head dim 32 has no
+    # kernel that does without.  32767 * 32769 = 2^30 - 1 rows are too many, 64 * 16777215 = 2^30 - 64 are not (refused later: no workspace)
+    def call(H, Lq):
+        p = _good_bwd()
+        p.D, p.H, p.Lq = 32, H, Lq
+        return lib.ra_bwd_whole(C.byref(p), 0x1000, _lib.RA_DTYPE_BF16, 64 * 128, 64, 128, _lib.RA_DTYPE_BF16, 0x4000, 64 * 128, 64, 128,
+                                0x5000, 0x6000, 64 * 128, 64, 128, None, 0, None)
+
+    assert call(32767, 32769) == _lib.RA_ERR_TOO_LARGE
+    assert call(64, 16777215) == -4
+
+
 def _rows(**kw):
     a = {**dict(src=0x1000, dst=0x2000, sd=_lib.RA_DTYPE_F32, dd=_lib.RA_DTYPE_BF16, d=96, to=128, B=1, L=4, H=2), **kw}
     return ring._ROWS.pack(a["src"], a["dst"], a["sd"], a["dd"], a["d"], a["to"], a["B"], a["L"], a["H"], 0, 192, 96, 0, 256, 128)

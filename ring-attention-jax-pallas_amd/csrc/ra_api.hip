@@ -853,8 +853,15 @@ static int check_whole_call(const char* what, int D, const ra_bias& bias) {
 static int check_fwd_step(const ra_fwd_step_params* p, bool any_dim);
 static int check_bwd_step(const ra_bwd_step_params* p, bool any_dim);
 
-static int fwd_pair(const ra_fwd_step_params* p, bool any_dim, void* out, int32_t out_dtype, int64_t out_stride_b, int64_t out_stride_h,
-                    int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
+// The conversions that go before a call, which has been checked by then: nothing is launched for one that is refused.
+struct Before {
+  const ra_rows* items;
+  int32_t n;
+  int launch(void* stream) const { return n ? ra_convert(items, n, stream) : RA_OK; }
+};
+
+static int fwd_pair(const Before& before, const ra_fwd_step_params* p, bool any_dim, void* out, int32_t out_dtype, int64_t out_stride_b,
+                    int64_t out_stride_h, int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
   if (!p) return fail(RA_ERR_NULL, "params is NULL");
   ra_fwd_step_params c = *p;
   c.o = c.m = c.l = reinterpret_cast<float*>(uintptr_t(16));  // not used: there is no carry
@@ -864,7 +871,7 @@ static int fwd_pair(const ra_fwd_step_params* p, bool any_dim, void* out, int32_
   const RingResult r{out, nullptr, lse, out_dtype, 0, out_stride_b, out_stride_h, out_stride_l};
   if ((rc = check_ring_result("ra_fwd_pair", r))) return rc;
   const PairPlan plan = plan_fwd_pair(*p);
-  if (!plan.pair) return fwd_passes(p, std::vector<int>{0, 1}, 1, stream, &r);
+  if (!plan.pair) return (rc = before.launch(stream)) ? rc : fwd_passes(p, std::vector<int>{0, 1}, 1, stream, &r);
   ra::PairFwdArgs a;
   memset(&a, 0, sizeof(a));
   a.q = to_arg(p->q);
@@ -894,6 +901,7 @@ static int fwd_pair(const ra_fwd_step_params* p, bool any_dim, void* out, int32_
     a.part_s = a.part_o + rows * p->D;
     a.part_n = (int*)(a.part_s + rows * 4);
   }
+  if ((rc = before.launch(stream))) return rc;
   hipError_t e = ra::launch_fwd_pair(a, p->D, kernel_mode(p->bias.flags), (hipStream_t)stream);
   return e == hipSuccess ? RA_OK : hip_fail(e, "ra_fwd_pair launch");
 }
@@ -903,11 +911,11 @@ int64_t ra_fwd_whole_workspace(const ra_fwd_step_params* p) { return fwd_pair_wo
 
 int ra_fwd_pair(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b, int64_t out_stride_h,
                 int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
-  return fwd_pair(p, false, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, lse, workspace, workspace_bytes, stream);
+  return fwd_pair({}, p, false, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, lse, workspace, workspace_bytes, stream);
 }
 int ra_fwd_whole(const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b, int64_t out_stride_h,
                  int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
-  return fwd_pair(p, true, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, lse, workspace, workspace_bytes, stream);
+  return fwd_pair({}, p, true, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, lse, workspace, workspace_bytes, stream);
 }
 
 const char* ra_last_error(void) { return g_err; }
@@ -1157,7 +1165,7 @@ static int64_t bwd_pair_workspace(const ra_bwd_step_params* p, bool any_dim) {
   return bwd_space(*p, plan_dq_pair(*p), plan_dkdv_pair(*p)).total;
 }
 
-static int bwd_pair(const ra_bwd_step_params* p, bool any_dim, int grad_dtype, const void* out, int32_t out_dtype, int64_t out_stride_b,
+static int bwd_pair(const Before& before, const ra_bwd_step_params* p, bool any_dim, int grad_dtype, const void* out, int32_t out_dtype, int64_t out_stride_b,
                 int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
                 int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
@@ -1186,6 +1194,7 @@ static int bwd_pair(const ra_bwd_step_params* p, bool any_dim, int grad_dtype, c
   memset(&a, 0, sizeof(a));
   a.a = to_bwd_args(c);
   a.stat = (const float*)(ws + sp.stat);
+  if ((rc = before.launch(stream))) return rc;
   hipError_t e = ra::launch_pair_stat(out, out_dtype == RA_DTYPE_F32, out_stride_b, out_stride_h, out_stride_l, a.a.dout, c.lse,
                                       1.0f / a.a.scale_res, (float*)(ws + sp.stat), (float*)(ws + sp.delta), c.B, c.H, c.Lq, c.D,
                                       (hipStream_t)stream);
@@ -1241,14 +1250,14 @@ int ra_bwd_pair(const ra_bwd_step_params* p, const void* out, int32_t out_dtype,
                 int64_t out_stride_h, int64_t out_stride_l, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
                 int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
-  return bwd_pair(p, false, RA_DTYPE_BF16, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h, dq_stride_l, dk, dv, dkv_stride_b,
+  return bwd_pair({}, p, false, RA_DTYPE_BF16, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h, dq_stride_l, dk, dv, dkv_stride_b,
                   dkv_stride_h, dkv_stride_l, workspace, workspace_bytes, stream);
 }
 int ra_bwd_whole(const ra_bwd_step_params* p, const void* out, int32_t out_dtype, int64_t out_stride_b,
                 int64_t out_stride_h, int64_t out_stride_l, int32_t grad_dtype, void* dq, int64_t dq_stride_b, int64_t dq_stride_h,
                 int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
-  return bwd_pair(p, true, grad_dtype, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h, dq_stride_l, dk, dv, dkv_stride_b,
+  return bwd_pair({}, p, true, grad_dtype, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h, dq_stride_l, dk, dv, dkv_stride_b,
                   dkv_stride_h, dkv_stride_l, workspace, workspace_bytes, stream);
 }
 
@@ -1286,23 +1295,15 @@ int ra_convert(const ra_rows* items, int32_t n_items, void* stream) {
 
 int ra_fwd_call(const ra_rows* before, int32_t n_before, const ra_fwd_step_params* p, void* out, int32_t out_dtype, int64_t out_stride_b,
                 int64_t out_stride_h, int64_t out_stride_l, float* lse, void* workspace, int64_t workspace_bytes, void* stream) {
-  if (n_before) {
-    int rc = ra_convert(before, n_before, stream);
-    if (rc) return rc;
-  }
-  return ra_fwd_whole(p, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, lse, workspace, workspace_bytes, stream);
+  return fwd_pair({before, n_before}, p, true, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, lse, workspace, workspace_bytes, stream);
 }
 
 int ra_bwd_call(const ra_rows* before, int32_t n_before, const ra_bwd_step_params* p, const void* out, int32_t out_dtype,
                 int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_l, int32_t grad_dtype, void* dq, int64_t dq_stride_b,
                 int64_t dq_stride_h, int64_t dq_stride_l, void* dk, void* dv, int64_t dkv_stride_b, int64_t dkv_stride_h,
                 int64_t dkv_stride_l, void* workspace, int64_t workspace_bytes, void* stream) {
-  if (n_before) {
-    int rc = ra_convert(before, n_before, stream);
-    if (rc) return rc;
-  }
-  return ra_bwd_whole(p, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, grad_dtype, dq, dq_stride_b, dq_stride_h,
-                      dq_stride_l, dk, dv, dkv_stride_b, dkv_stride_h, dkv_stride_l, workspace, workspace_bytes, stream);
+  return bwd_pair({before, n_before}, p, true, grad_dtype, out, out_dtype, out_stride_b, out_stride_h, out_stride_l, dq, dq_stride_b, dq_stride_h,
+                  dq_stride_l, dk, dv, dkv_stride_b, dkv_stride_h, dkv_stride_l, workspace, workspace_bytes, stream);
 }
 
 int ra_bwd_finalize_passes(const float* acc, void* out, int64_t out_stride_pass, int64_t out_stride_b,

@@ -372,3 +372,27 @@ def test_header_is_plain_c(tmp_path):
     res = subprocess.run([gcc, "-std=c99", "-Wall", "-Wextra", "-pedantic", "-Werror", "-fsyntax-only",
                           "-I", os.path.join(ROOT, "include"), str(src)], capture_output=True, text=True)
     assert res.returncode == 0, res.stderr
+
+
+def test_calls_are_checked_before_their_conversions_without_a_gpu(lib):
+    # the conversions are in order (on a machine without a GPU their launch would fail as such); the call behind them is not
+    fwd, bwd = _good_fwd(), _good_bwd()
+
+    def forward(rows, n, size=1 << 30, lse=0x2000):
+        return lib.ra_fwd_call(rows, n, bytes(fwd), 0x1000, 0, 64 * 256, 128, 256, lse, 0x3000, size, None)
+
+    def backward(rows, n, size=1 << 30, dv=0x6000):
+        return lib.ra_bwd_call(rows, n, bytes(bwd), 0x1000, 0, 64 * 128, 64, 128, 0, 0x4000, 64 * 128, 64, 128, 0x5000, dv, 64 * 128, 64, 128,
+                               0x7000, size, None)
+
+    assert forward(_rows(), 1, lse=None) == -1 and backward(_rows(), 1, dv=None) == -1 and backward(_rows(), 1, size=64) == -2
+    for p, call in ((fwd, forward), (bwd, backward)):
+        for n in (-1, _lib.RA_MAX_CONVERT + 1):
+            assert call(_rows() * 5, n) == -2
+        assert call(None, 1) == -1 and call(_rows(src=0x1002), 1) == -4
+        p.D = 48
+        assert call(_rows(), 1) == -3
+        p.D, p.bias.flags = 64, 64
+        assert call(_rows(), 1) == -5
+    fwd.bias.flags, fwd.Lk = 0, 4096  # rows whose keys are shared
+    assert forward(_rows(), 1, size=64) == -2

@@ -1130,11 +1130,14 @@ def _attend(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs, sm_scale
     _require_gpu(q)
     _lib.load()
     n = _axis_size(axis_name)
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
+    qs, ks, vs = q.shape, k.shape, v.shape
+    if len(qs) != 4 or len(ks) != 4 or len(vs) != 4:
         raise ValueError("q, k, v must be [b, l, h, d]")
-    d_true = q.shape[-1]
-    if k.shape[-1] != d_true or v.shape[-1] != d_true:
+    d_true = qs[3]
+    if ks[3] != d_true or vs[3] != d_true:
         raise ValueError("q, k and v must share the head dim")
+    if ks[0] < qs[0] or vs[0] < qs[0] or ks[2] < qs[2] or vs[2] < qs[2] or vs[1] < ks[1]:  # the kernels would read past their end
+        raise ValueError(f"k {tuple(ks)} and v {tuple(vs)} do not hold the batch and heads of q {tuple(qs)}, or v not the length of k")
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(d_true)  # ring.py:287-288
     in_dtype = q.dtype
@@ -1142,7 +1145,7 @@ def _attend(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs, sm_scale
         out_dtype = torch.float32 if in_dtype == torch.float32 else torch.bfloat16
     if d_true > 128:
         raise ValueError("head dims above 128 are not supported")
-    plan = _plan_for(q, k, _walked_ring_size(n, q.shape[1], k.shape[1], bias_fn), bias_fn, bias_q_kwargs,
+    plan = _plan_for(q, k, _walked_ring_size(n, qs[1], ks[1], bias_fn), bias_fn, bias_q_kwargs,
                      bias_kv_kwargs)
     fused = _launch_whole_ring(block_impl, plan)
     if fused:

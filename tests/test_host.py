@@ -327,3 +327,15 @@ def test_blocks_take_head_dims_64_and_128_only(monkeypatch, D):
     for bias in (None, ra.BlockBias(ra.causal_bias()), torch.zeros((1, 1, 128, 128))):
         with pytest.raises(RuntimeError, match=f"head dim {D} unsupported .64 or 128"):
             ra.bwd_block(x, x, x, bias, acc, rows, x, 0.1)
+
+
+@pytest.mark.parametrize("k_shape,v_shape", [((1, 64, 4, 64), None), ((2, 64, 1, 64), None), ((2, 64, 4, 64), (1, 64, 4, 64)),
+                                             ((2, 64, 4, 64), (2, 64, 2, 64)), ((2, 64, 4, 64), (2, 32, 4, 64))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_operands_smaller_than_the_call_are_refused(monkeypatch, k_shape, v_shape, dtype):
+    # one head or batch row of keys for several of queries, values of another length: nothing broadcasts, and the kernels do
+    # not look at the end of an array
+    monkeypatch.setattr(rr, "_require_gpu", lambda t: None)
+    q, k, v = (torch.zeros(s, dtype=dtype) for s in ((2, 64, 4, 64), k_shape, v_shape or k_shape))
+    with pytest.raises(ValueError, match="do not hold the batch and heads"):
+        ra.ring_attention(q, k, v, 2)

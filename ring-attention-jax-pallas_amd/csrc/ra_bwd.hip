@@ -2051,7 +2051,7 @@ hipError_t launch_bwd_delta(const void* out, int out_f32, long long sp, long lon
   return hipGetLastError();
 }
 
-// mode: as for launch_fwd_steps; 2 for dK / dV only (dQ steps on a dense block run on dq_pair_kernel)
+// mode: as for launch_fwd_steps.  dQ without a dense block and at D = 128 only: the others run on dq_pair_kernel
 hipError_t launch_bwd_step(const BwdArgs& a, int D, int mode, int parts, hipStream_t stream) {
   if (parts & 1) {
     const int keys_wg = 128;
@@ -2072,13 +2072,9 @@ hipError_t launch_bwd_step(const BwdArgs& a, int D, int mode, int parts, hipStre
   if (parts & 2) {
     const int nqt = (a.Lq + kDqRows - 1) / kDqRows;
     dim3 grid((unsigned)(a.B * a.H * nqt)), block(kDqThreads);
-    if (D == 128) {
-      if (mode == 1) hipLaunchKernelGGL((dq_kernel<128, 1, false>), grid, block, 0, stream, a, NoShardList{});
-      else hipLaunchKernelGGL((dq_kernel<128, 0, false>), grid, block, 0, stream, a, NoShardList{});
-    } else {
-      if (mode == 1) hipLaunchKernelGGL((dq_kernel<64, 1, false>), grid, block, 0, stream, a, NoShardList{});
-      else hipLaunchKernelGGL((dq_kernel<64, 0, false>), grid, block, 0, stream, a, NoShardList{});
-    }
+    if (D != 128 || mode == 2) return hipErrorInvalidValue;
+    if (mode == 1) hipLaunchKernelGGL((dq_kernel<128, 1, false>), grid, block, 0, stream, a, NoShardList{});
+    else hipLaunchKernelGGL((dq_kernel<128, 0, false>), grid, block, 0, stream, a, NoShardList{});
   }
   return hipGetLastError();
 }

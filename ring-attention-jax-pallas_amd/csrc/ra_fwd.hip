@@ -205,52 +205,29 @@ __global__ __launch_bounds__(kFwdThreads) void fwd_step_kernel(
   // the listed tiles count up without a gap from the start of a run to ordinal cons_hi / cons2_hi
   int cons_hi = n_act, cons2_hi = 0;
   bool wg_one_doc = true;
-  // A dense block that comes with its summary is listed the same way: tiles in which the
-  // workgroup's rows hold nothing but -inf are left out, tiles of zeros count as tiles of one
-  // id (no term to evaluate: they may join a straight-line stretch), the rest is evaluated
-  // element by element.  (Single-step launches only.)
-  const unsigned char* dmap = nullptr;
-  if constexpr (DENSE && !MULTI) {
-    if (bs.dense_map) dmap = dense_map_of(bs, b, h, a.H, a.Lq, a.Lk);
-  }
-  const bool seg_list = GENERAL && (flags & RA_BIAS_SEGMENT);
-  if (seg_list || (DENSE && dmap != nullptr)) {
+  if (GENERAL && (flags & RA_BIAS_SEGMENT)) {
     // segment-id range of the workgroup's queries, then one thread per key tile decides
     // whether the id ranges can intersect (skip otherwise) and whether the tile has one id
     use_list = true;
-    int qmin = 0, qmax = 0;
-    if (seg_list) {
-      int smin = q_valid ? q_seg : 0x7fffffff, smax = q_valid ? q_seg : (int)0x80000000;
-      smin = wave_min(smin);
-      smax = wave_max(smax);
-      if (lane == 0) {
-        s_red[wave] = smin;
-        s_red[8 + wave] = smax;
-      }
-      __syncthreads();
-      qmin = s_red[0];
-      qmax = s_red[8];
+    int smin = q_valid ? q_seg : 0x7fffffff, smax = q_valid ? q_seg : (int)0x80000000;
+    smin = wave_min(smin);
+    smax = wave_max(smax);
+    if (lane == 0) {
+      s_red[wave] = smin;
+      s_red[8 + wave] = smax;
+    }
+    __syncthreads();
+    int qmin = s_red[0], qmax = s_red[8];
 #pragma unroll
-      for (int w = 1; w < 8; ++w) {
-        qmin = min(qmin, s_red[w]);
-        qmax = max(qmax, s_red[8 + w]);
-      }
+    for (int w = 1; w < 8; ++w) {
+      qmin = min(qmin, s_red[w]);
+      qmax = max(qmax, s_red[8 + w]);
     }
     for (int j = j_lo + tid; j < j_hi; j += kFwdThreads) {
-      int f = 1;
-      if (seg_list) {
-        int kmin, kmax;
-        tile_id_range<kKeyTile>(kv_seg, j, a.Lk, kmin, kmax);
-        const bool act = !(kmax < qmin || kmin > qmax);
-        f = act ? ((kmin == kmax) ? 1 : 3) : 0;
-      }
-      if constexpr (DENSE) {
-        if (dmap != nullptr && f != 0) {
-          const int bits = dense_map_or(dmap, a.Lk, q0, q_rows_hi, j * kKeyTile, min((j + 1) * kKeyTile, a.Lk) - 1);
-          f = (bits & kMapLive) ? ((bits & kMapNonZero) ? 3 : f) : 0;
-        }
-      }
-      s_flag[j - j_lo] = f;
+      int kmin, kmax;
+      tile_id_range<kKeyTile>(kv_seg, j, a.Lk, kmin, kmax);
+      const bool act = !(kmax < qmin || kmin > qmax);
+      s_flag[j - j_lo] = act ? ((kmin == kmax) ? 1 : 3) : 0;
     }
     wg_one_doc = qmin == qmax;
     __syncthreads();
@@ -536,12 +513,8 @@ __global__ __launch_bounds__(kFwdThreads) void fwd_step_kernel(
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, S[kb][r]);
     return half_max(mx) * a.scale2;  // scale2 > 0: the maximum commutes with the scaling
   };
-  // terms that every tile must evaluate; a dense block with a summary is read only in the tiles
-  // that the list marks (segbit)
-  int tile_terms = RA_BIAS_ALIBI | RA_BIAS_PREFIX | RA_BIAS_DENSE;
-  if constexpr (DENSE) {
-    if (dmap != nullptr) tile_terms &= ~RA_BIAS_DENSE;
-  }
+  // terms that every tile must evaluate
+  constexpr int tile_terms = RA_BIAS_ALIBI | RA_BIAS_PREFIX | RA_BIAS_DENSE;
   auto needs_bias = [&](int kt0, int segbit, int cls) -> bool {
     bool nb = (cls & 2) || (kt0 + kKeyTile > a.Lk);
     if (GENERAL) nb = nb || (flags & tile_terms) || segbit;
@@ -555,7 +528,7 @@ __global__ __launch_bounds__(kFwdThreads) void fwd_step_kernel(
     tb.flags = (cls & 2) ? (flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) : 0;
     if (GENERAL) {
       tb.flags |= flags & tile_terms;
-      if (segbit) tb.flags |= DENSE ? (flags & (RA_BIAS_SEGMENT | RA_BIAS_DENSE)) : RA_BIAS_SEGMENT;
+      if (segbit) tb.flags |= RA_BIAS_SEGMENT;
     }
     tb.window = bs.window;
     const float inv_scale2 = 1.0f / a.scale2;

@@ -3,6 +3,7 @@ edges of their 128-row and 64-key tiles, single rows, rows whose keys several wo
 under masks that leave rows of different lengths, down to none), every bias term on the tile lists, and key
 sequences longer than a list.  Tolerances as in test_gpu_parity.py."""
 import ctypes as C
+import re
 
 import numpy as np
 import pytest
@@ -15,6 +16,14 @@ from test_gpu_dense_map import _both_ways
 from test_gpu_parity import GRAD_TOL, LSE_TOL, OUT_TOL, _check, _dev, _rel
 
 pytestmark = pytest.mark.gpu
+
+
+def _kernels(call):
+    """What ``call`` returns, and the kernels of this library that it launched."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as run:
+        got = call()
+        torch.cuda.synchronize()
+    return got, {m.group(1) for m in (re.search(r"ra::(\w+<[^>]*>)", e.key) for e in run.key_averages()) if m}
 
 
 def _bias(kind, B, Sq, Sk, H, seed=0):
@@ -291,7 +300,7 @@ def test_one_head_whose_rows_are_closer_together_than_in_lds(device, Sq, Sk, D, 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("Sq,Sk,D,H", [(129, 65, 64, 2), (300, 1000, 96, 2), (2048, 130, 32, 1), (640, 640, 128, 40), (8200, 8200, 128, 1)])
 def test_gradients_leave_the_kernels_in_the_callers_dtype(device, Sq, Sk, D, H, dtype):
-    # shared and unshared rows and keys, and (640, H=40: dK and dV; 8200) the long-stretch kernels
+    # rows and keys that several workgroups share, and some that they do not
     g = torch.Generator(device=device).manual_seed(Sq + D)
     q, k, v = (torch.randn((1, S, H, D), device=device, generator=g).to(torch.bfloat16).to(dtype).requires_grad_(True) for S in (Sq, Sk, Sk))
     do = torch.randn((1, Sq, H, D), device=device, generator=g).to(torch.bfloat16).to(dtype)
@@ -310,9 +319,35 @@ def test_gradients_leave_the_kernels_in_the_callers_dtype(device, Sq, Sk, D, H, 
         assert max(_rel(got.float().cpu().numpy(), x.grad.cpu().numpy())) <= GRAD_TOL
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("S,H,causal,kernels", [
+    (640, 40, True, {"dkdv_pair_kernel<128, 0>", "dq_pair_kernel<128, 0>"}),
+    (4100, 17, True, {"dkdv_kernel<128, 0, true>", "dq_pair_kernel<128, 0>"}),
+    (10300, 8, False, {"dkdv_kernel<128, 0, true>", "dq_kernel<128, 0, true>"})])
+def test_converted_gradients_are_the_bf16_ones_converted(device, S, H, causal, kernels, dtype):
+    # bit for bit, on both kinds of kernels; the inputs are the same in bf16, fp16 and fp32
+    g = torch.Generator(device=device).manual_seed(S)
+    q, k, v, do = (torch.randn((1, S, H, 128), device=device, generator=g).to(torch.bfloat16) for _ in range(4))
+    for x in (q, k, v, do):
+        x[x.abs() < 1e-3] = 0  # (fp16 holds what is left exactly)
+
+    def gradients(dtype, out_dtype):
+        leaves = [x.to(dtype).requires_grad_(True) for x in (q, k, v)]
+        out, _ = ra.ring_attention_with_lse(*leaves, 1, ra.causal_bias() if causal else None, out_dtype=out_dtype)
+        return _kernels(lambda: torch.autograd.grad(out, leaves, do.to(out.dtype)))
+
+    want, _ = gradients(torch.bfloat16, torch.float32 if dtype == torch.float32 else None)
+    got, launched = gradients(dtype, None)
+    assert kernels <= launched, launched
+    for a, b in zip(got, want):
+        assert a.dtype == dtype and b.dtype == torch.bfloat16 and torch.isfinite(b).all() and b.any()
+        assert torch.equal(a, b.to(dtype))
+
+
 @pytest.mark.parametrize("Lq,Lk,H,D,offset", [(1, 1, 1, 64, None), (129, 200, 2, 128, 0), (257, 63, 3, 64, 100), (300, 300, 2, 128, 400),
                                               (1000, 700, 2, 128, -500), (3601, 3700, 32, 128, None), (3601, 3700, 32, 128, 4000),
-                                              (2100, 2100, 32, 64, None), (4100, 4100, 17, 128, 0), (64, 64, 2, 128, -64)])
+                                              (2100, 2100, 32, 64, None), (4100, 4100, 17, 128, 0), (64, 64, 2, 128, -64),
+                                              (10300, 10300, 8, 128, None)])
 def test_single_steps_on_both_sides_of_the_rule(device, Lq, Lk, H, D, offset):
     """fwd_block on a carry that is not empty and bwd_block: pairs on the kernels for short pairs and on the long-stretch
     ones (the larger ones without a mask), a pair that sees nothing (-64), queries that see nothing (-500)."""
@@ -367,3 +402,57 @@ def test_keys_and_values_laid_out_differently(device, D, n, transposed):
     assert np.abs(out.detach().cpu().numpy() - want).max() <= OUT_TOL and np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_TOL
     for g, ref in zip(torch.autograd.grad(out, leaves, _dev(do, device)), R.mha_dense_grads(q, k, v, do, bias)):
         assert max(_rel(g.float().cpu().numpy(), ref)) <= GRAD_TOL
+
+
+@pytest.mark.parametrize("L,H,D,causal,kernels", [
+    (1000, 2, 128, True, {"fwd_pair_kernel<128, 0>", "dq_pair_kernel<128, 0>", "dkdv_pair_kernel<128, 0>"}),
+    (2100, 32, 64, False, {"fwd_step_kernel<64, 0, false, false>", "dq_pair_kernel<64, 0>", "dkdv_pair_kernel<64, 0>"}),
+    (3601, 32, 128, False, {"fwd_step_kernel<128, 0, false, false>", "dq_pair_kernel<128, 0>", "dkdv_kernel<128, 0, false>"}),
+    (4100, 17, 128, True, {"fwd_pair_kernel<128, 0>", "dq_pair_kernel<128, 0>", "dkdv_kernel<128, 0, false>"}),
+    (10300, 8, 128, False, {"fwd_step_kernel<128, 0, false, false>", "dq_kernel<128, 0, false>", "dkdv_kernel<128, 0, false>"})])
+def test_which_kernels_a_single_step_takes(device, L, H, D, causal, kernels):
+    # ... so that the test above runs them all: fwd_block and bwd_block of its larger cases
+    q = torch.randn((1, H, L, D), device=device).to(torch.bfloat16)
+    bias = ra.BlockBias(ra.causal_bias(), 0, 0) if causal else None
+    carry = rr.init_carry(1, H, L, D, device)
+    lse = torch.zeros((1, H, L), device=device)
+
+    def step():
+        ra.fwd_block(q, q, q, bias, *carry, 0.1)
+        ra.bwd_block(q, q, q, bias, q, lse + 100, q, 0.1)
+
+    _, launched = _kernels(step)
+    assert kernels <= launched, launched
+
+
+@pytest.mark.parametrize("q_off,kv_off", [(100000, 0), (0, 300000)])
+def test_alibi_far_from_the_diagonal_on_the_long_stretch_kernels(device, q_off, kv_off):
+    """Single steps of 4096 x 4096, H=32, whose bias reaches 6000 and 19000; the slopes are those of test_gpu_parity's smaller
+    steps, which run on the kernels for short pairs.  Against float64, tolerances as there."""
+    L, H, D = 4096, 32, 128
+    g = torch.Generator(device=device).manual_seed(q_off)
+    q, k, v, do = (torch.randn((1, H, L, D), device=device, generator=g).to(torch.bfloat16) for _ in range(4))
+    slopes = torch.logspace(-4, -8, H, base=2, device=device)
+    bias, scale = ra.BlockBias(ra.alibi_bias(slopes), q_off, kv_off), 1 / np.sqrt(D)
+    carry = rr.init_carry(1, H, L, D, device)
+    out, lse = torch.empty((1, H, L, D), device=device), torch.empty((1, H, L), device=device)
+    grads = [torch.zeros((1, H, L, D), device=device) for _ in range(3)]
+
+    def step():
+        ra.fwd_block(q, k, v, bias, *carry, scale)
+        rr.finalize_carry(*carry, out, lse)
+        rr._bwd_step(q, k, v, do, lse, rr.precompute_delta(out, do), *grads, bias, scale)
+
+    _, launched = _kernels(step)
+    assert {"fwd_step_kernel<128, 1, false, false>", "dq_kernel<128, 1, false>", "dkdv_kernel<128, 1, false>"} <= launched, launched
+    rel = (q_off + torch.arange(L, device=device)[:, None] - kv_off - torch.arange(L, device=device)[None]).abs().double()
+    for h in range(H):
+        a = [x[0, h].double() for x in (q, k, v, do)]
+        s = a[0] @ a[1].T * scale - slopes[h].double() * rel
+        p, ref_lse = torch.softmax(s, -1), torch.logsumexp(s, -1)
+        o = p @ a[2]
+        assert (out[0, h] - o).abs().max() <= OUT_TOL
+        assert (lse[0, h] - ref_lse).abs().max() <= LSE_TOL + 4e-7 * ref_lse.abs().max(), h
+        ds = p * (a[3] @ a[2].T - (o * a[3]).sum(-1, keepdim=True))
+        for got, ref in zip(grads, (ds @ a[1] * scale, ds.T @ a[0] * scale, p.T @ a[3])):
+            assert max(_rel(got[0, h].cpu().numpy(), ref.cpu().numpy())) <= GRAD_TOL, h

@@ -439,8 +439,10 @@ def test_prefix_block_step_far_from_the_diagonal(device, q_off, kv_off):
 def test_alibi_block_step_far_from_the_diagonal(device, q_off, kv_off, causal):
     """ALiBi on a lone block step far from the diagonal: slope x distance reaches 6000 - 19000 (the
     largest slope is 1/16 here), and the weights inside the block must still follow the bias of
-    the oracle - the kernels add the term through the matrix unit, the distance-dependent constant
-    split into three bf16 words.  (Beyond a few hundred thousand positions fp32 itself - the
+    the oracle.  Steps of this size run on the pair kernels, which add the term's slope through an fp32
+    matrix product and its distance-dependent constant to the exponents (dK / dV: to the row statistics); the
+    long-stretch kernels, which split the constant into three bf16 words, have a test of their own in
+    test_gpu_pair.py.  (Beyond a few hundred thousand positions fp32 itself - the
     reference's bias dtype - no longer resolves the bias to 1e-3.)"""
     H = 2
     sl = R.alibi_slopes(H)

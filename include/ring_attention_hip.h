@@ -350,7 +350,7 @@ typedef struct {
 int ra_convert(const ra_rows* items, int32_t n_items, void* stream);
 
 /* A whole call: ra_convert of the operands that `before` lists (none: n_before = 0), then ra_fwd_whole /
- * ra_bwd_whole on what they made. */
+ * ra_bwd_whole on what they made; everything is checked before anything is launched. */
 int ra_fwd_call(const ra_rows* before, int32_t n_before, const ra_fwd_step_params* p, void* out, int32_t out_dtype,
                 int64_t out_stride_b, int64_t out_stride_h, int64_t out_stride_l, float* lse, void* workspace,
                 int64_t workspace_bytes, void* stream);

@@ -715,8 +715,9 @@ constexpr int kMinChunk = 6, kMaxSplit = 64;
 bool has_lists(const ra_bias& b) { return b.flags & (RA_BIAS_SEGMENT | RA_BIAS_PREFIX | RA_BIAS_DENSE); }
 // Whether all of a head's resident tiles have about the same work.
 bool even_rows(int64_t total, int most, int64_t rows) { return total * 20 >= (int64_t)most * rows * 17; }
-// Whether the pair kernels take an XCD's heads one after the other (see pair_decode): unmasked rows.  (Not under a window: D=64,
-// 2048 of 16384, 32 heads, 1.23 ms a pass over all heads, 1.27 one by one.)
+// Whether the pair kernels take an XCD's heads one after the other (see pair_decode): rows that meet about the same number of tiles,
+// without a list - unmasked ones, and a few queries behind a long context under a causal mask, ALiBi included.  (Not under a
+// window: D=64, 2048 of 16384, 32 heads, 1.23 ms a pass over all heads, 1.27 one by one.)
 bool one_by_one(const ra_bias& b, int64_t total, int most, int64_t rows) {
   return even_rows(total, most, rows) && !has_lists(b) && !(b.flags & RA_BIAS_WINDOW);
 }
@@ -731,8 +732,9 @@ void plan_split(PairPlan& r, int64_t heads, int64_t rows, int64_t total, int mos
   r.n_split = (most + r.chunk_tiles - 1) / r.chunk_tiles;
 }
 // Whether a single step, into a carry or an accumulator, runs on fwd_pair_kernel (dq_pair_kernel) as well: nothing is shared there.  Under
-// a list of tiles and at D = 64 always, but for even rows that fill the chip once or twice in the forward; else up to a workgroup per compute
-// unit, with uneven rows up to two, and beyond with rows that are short.  fwd_step_kernel | fwd_pair_kernel, then dq_kernel |
+// a list of tiles always.  At D = 64 always in dQ; in the forward but for even rows of fewer than 192 tiles on more than a workgroup per
+// compute unit.  At D = 128 up to a workgroup per compute unit, with uneven rows up to two, and beyond where the rows that see a key
+// meet fewer than 56 tiles on average.  fwd_step_kernel | fwd_pair_kernel, then dq_kernel |
 // dq_pair_kernel, us: D=128, a causal diagonal of 1024, H=8, 38 | 25 and 44 | 28, of 2048, H=16, 64 | 46 and 72 | 50, of 4096, H=16, 108 | 96 and 132 | 115,
 // H=32, 189 | 158 and 239 | 194, of 8192, H=16, 273 | 295 and 353 | 367; unmasked 2048, H=16, 61 | 48 and 72 | 55, 4096, H=16, 132 | 142 and 173 | 176;
 // D=64, a diagonal of 4096, H=16, 83 | 68 and 89 | 71, unmasked 85 | 90 and 104 | 102, 8192 314 | 317 and 385 | 373, 16384 1221 | 1215 and 1501 | 1432.

@@ -11,13 +11,14 @@
 // combines.
 //
 // What bounds them is the latency of a wave's step through a tile, with two to four waves per SIMD to cover it: of
-// the wave cycles of documents + ALiBi (D = 128) 44 % issued an instruction, 29 % waited at the barrier or for operands and 26 %
-// for the issue port, and a forward tile took 9 vector and 3.6 scalar instructions per matrix instruction where the
-// softmax needs 6.  Hence everything around the matrix instructions is kept short: what a wave does with
+// the wave cycles of documents + ALiBi (D = 128) 37 to 41 % issue an instruction, 28 to 30 % wait at the barrier or for operands and 29
+// to 34 % for the issue port, and a forward tile takes 7.2 vector and 2.8 scalar instructions per matrix instruction (9 and
+// 3.6 before what follows) where the softmax needs 6.  Hence everything around the matrix instructions is kept short: what a wave does with
 // a tile follows from a few ranges of tile indexes (WaveTiles) and from the wave's own ids (wave_tests), not the
 // workgroup's; the terms of a masked block are passes of their own (apply_terms); a tile's loads share one base
 // (TileLoader); and nothing that can be computed again stays in a register (opaque_lane, kernel_args), so that no
-// variant spills.  Before | after, us: documents of 2048 + ALiBi, 32768, H=16, D=128: forward 1787 | 1590, dQ 1916 | 1755, dK/dV
+// variant spills a vector register or goes to scratch.  (Scalar registers in vector lanes: 2 to 12 in the general variants, 19 to 49 in
+// those with a dense block, for which the compiler reserves 36 bytes of scratch in dK / dV that no instruction uses.)  Before | after, us: documents of 2048 + ALiBi, 32768, H=16, D=128: forward 1787 | 1590, dQ 1916 | 1755, dK/dV
 // 2770 | 2410; causal documents of 2175 in 48128, B=2, H=4, D=64: 443 | 325, 476 | 350, 495 | 427; prefix-LM 4096, B=2, H=16, D=128,
 // forward 229 | 194; steps on dense blocks (documents of 2048 in 32768, 4 shards) 10.2 ms | 7.8 a pass.
 #include <type_traits>

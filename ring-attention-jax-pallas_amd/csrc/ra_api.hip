@@ -435,32 +435,24 @@ int fwd_step_on_pair(const ra_fwd_step_params& p, void* stream) {
 // parts: 1 = dK and dV, 2 = dQ
 int bwd_step_on_pair(const ra_bwd_step_params& p, int parts, void* stream) {
   if (ra_step_is_skippable(&p.bias, p.Lq, p.Lk)) return RA_OK;  // contributes nothing
-  ra::PairBwdArgs a;
-  memset(&a, 0, sizeof(a));
-  a.a = to_bwd_args(p);
-  a.n_split = 1;
-  a.chunk_tiles = kWholeRow;
-  a.group = kHeadGroup;
+  ra::PairBwdArgs dq;
+  memset(&dq, 0, sizeof(dq));
+  dq.a = to_bwd_args(p);
+  dq.n_split = 1;
+  dq.chunk_tiles = kWholeRow;
+  dq.group = kHeadGroup;
+  ra::PairBwdArgs dkdv = dq;
+  dq.acc = p.dq;
+  dkdv.acc = p.dk;
+  dkdv.acc2 = p.dv;
   const int mode = kernel_mode(p.bias.flags);
+  const bool pair = (parts & 1) && dkdv_on_pair(p), other = (parts & 1) && !pair;
+  const int rule = pair && choose_by_content(p.bias, key_slabs(p), p.Lq, p.Lk) ? kDkdvPlain : 0;
+  dkdv.a.bias.plain_rule = -rule;
   hipError_t e = hipSuccess;
-  if (parts & 1) {
-    const bool pair = dkdv_on_pair(p);
-    const int rule = pair && choose_by_content(p.bias, key_slabs(p), p.Lq, p.Lk) ? kDkdvPlain : 0;
-    if (pair) {
-      a.acc = p.dk;
-      a.acc2 = p.dv;
-      a.a.bias.plain_rule = -rule;
-      e = ra::launch_dkdv_pair(a, p.D, mode, (hipStream_t)stream);
-      a.a.bias.plain_rule = rule;
-    }
-    if (e == hipSuccess && (!pair || rule)) e = ra::launch_bwd_step(a.a, p.D, mode, 1, (hipStream_t)stream);
-    a.a.bias.plain_rule = 0;
-  }
-  if (e == hipSuccess && (parts & 2)) {
-    a.acc = p.dq;
-    a.acc2 = nullptr;
-    e = ra::launch_dq_pair(a, p.D, mode, (hipStream_t)stream);
-  }
+  if (pair || (parts & 2)) e = ra::launch_bwd_pair(pair ? &dkdv : nullptr, (parts & 2) ? &dq : nullptr, p.D, mode, (hipStream_t)stream);
+  dkdv.a.bias.plain_rule = rule;
+  if (e == hipSuccess && (other || rule)) e = ra::launch_bwd_step(dkdv.a, p.D, mode, 1, (hipStream_t)stream);
   return e == hipSuccess ? RA_OK : hip_fail(e, "backward step launch");
 }
 
@@ -804,6 +796,21 @@ PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
   else plan_split(r, heads, rows, total, most, 2 * kMinChunk);
   if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;
+}
+// Whether both gradients' workgroups go into one launch: the second kind fills the places that the first one's last round leaves
+// empty.  Two launches | one, us: causal, D=128, 6000, H=16 493 | 488, 4096, H=8 180 | 163; D=64, 2048, B=2, H=16 112 | 97; D=32, 8192, H=16 338 |
+// 312; documents of 500 in 32768, H=8 838 | 793, of 3500 in 10112, causal, H=4, D=80 352 | 278; prefix 4096, B=2, H=16 586 | 576; unmasked 3000,
+// H=24 441 | 370.  Past eight rounds the last one is a few per cent, and the one launch draws more power
+// without a pause (documents of 1200 + ALiBi, 29696, 24 heads: a pass 3.86 | 4.00 ms).  Fewer than two rounds stay two launches
+// (even rows at D <= 64, three workgroups of which fit a compute unit, fewer than three): what those run on is pinned by name in
+// test_gpu_pair.py; one launch would be 10 us faster there too (512, H=4, D=64, causal: 38 | 28).
+bool bwd_in_one_launch(const ra_bwd_step_params& p, const PairPlan& dq, const PairPlan& dkdv) {
+  if (!dq.pair || !dkdv.pair) return false;
+  const int64_t heads = (int64_t)p.B * p.H;
+  auto tiles = [](int L) { return (int64_t)(L + kPairRowsHost - 1) / kPairRowsHost; };
+  const int64_t wgs = heads * (tiles(p.Lq) * dq.n_split + tiles(p.Lk) * dkdv.n_split);
+  const bool three = p.D <= 64 && !(p.bias.flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) && !has_lists(p.bias);
+  return wgs >= (three ? 3 : 2) * kPairSlots && wgs <= 8 * kPairSlots;
 }
 // The workspace of ra_bwd_pair: the rows' statistics, then the shares of dQ and of dK and dV.
 struct BwdSpace {
@@ -1204,19 +1211,27 @@ static int bwd_pair(const Before& before, const ra_bwd_step_params* p, bool any_
   const std::vector<int> one{0, 1};
   const int mode = kernel_mode(c.bias.flags);
   auto share = [&](const PairPlan& plan, int64_t part, int64_t n, const RingResult& r) {
-    a.n_split = plan.n_split;
-    a.chunk_tiles = plan.chunk_tiles;
-    a.group = plan.group;
-    a.part = plan.n_split > 1 ? (float*)(ws + part) : nullptr;
-    a.part_n = plan.n_split > 1 ? (int*)(ws + n) : nullptr;
-    a.out = r.base;
-    a.out2 = r.base2;
-    a.out_dtype = r.dtype;
-    a.via_bf16 = r.via_bf16;
-    a.out_sb = r.stride_b;
-    a.out_sh = r.stride_h;
-    a.out_sl = r.stride_l;
+    ra::PairBwdArgs x = a;
+    x.n_split = plan.n_split;
+    x.chunk_tiles = plan.chunk_tiles;
+    x.group = plan.group;
+    x.part = plan.n_split > 1 ? (float*)(ws + part) : nullptr;
+    x.part_n = plan.n_split > 1 ? (int*)(ws + n) : nullptr;
+    x.out = r.base;
+    x.out2 = r.base2;
+    x.out_dtype = r.dtype;
+    x.via_bf16 = r.via_bf16;
+    x.out_sb = r.stride_b;
+    x.out_sh = r.stride_h;
+    x.out_sl = r.stride_l;
+    return x;
   };
+  const ra::PairBwdArgs dkdv = share(plan_k, sp.dkdv_part, sp.dkdv_n, rk), dq_args = share(plan_q, sp.dq_part, sp.dq_n, rq);
+  auto on_pair = [&](const ra::PairBwdArgs* kv, const ra::PairBwdArgs* q) -> int {
+    hipError_t err = ra::launch_bwd_pair(kv, q, c.D, mode, (hipStream_t)stream);
+    return err == hipSuccess ? RA_OK : hip_fail(err, "ra_bwd_pair launch");
+  };
+  if (bwd_in_one_launch(c, plan_q, plan_k)) return on_pair(&dkdv, &dq_args);
   // fp32 gradients that lie as the accumulators of a step do are stored by its kernels, which know one pair only and are faster
   // (dK and dV of a causal diagonal and a full pair of 4096, H=16, D=128: 430 us on the several-shard ones, 417 on
   // these; 32768 in two shards 5.21 | 5.15 ms and dQ 2.60 | 2.54)
@@ -1233,16 +1248,9 @@ static int bwd_pair(const Before& before, const ra_bwd_step_params* p, bool any_
     hipError_t err = ra::launch_bwd_step(s, c.D, mode, part, (hipStream_t)stream);
     return err == hipSuccess ? RA_OK : hip_fail(err, "ra_bwd_pair launch");
   };
-  if (plan_k.pair) {
-    share(plan_k, sp.dkdv_part, sp.dkdv_n, rk);
-    if ((e = ra::launch_dkdv_pair(a, c.D, mode, (hipStream_t)stream)) != hipSuccess) return hip_fail(e, "ra_bwd_pair launch");
-  } else if ((rc = as_accumulator(rk, c.Lk) ? one_step(1) : bwd_dkdv_passes(&c, one, 1, stream, &rk))) {
+  if ((rc = plan_k.pair ? on_pair(&dkdv, nullptr) : as_accumulator(rk, c.Lk) ? one_step(1) : bwd_dkdv_passes(&c, one, 1, stream, &rk)))
     return rc;
-  }
-  if (!plan_q.pair) return as_accumulator(rq, c.Lq) ? one_step(2) : bwd_dq_passes(&c, one, 1, stream, &rq);
-  share(plan_q, sp.dq_part, sp.dq_n, rq);
-  e = ra::launch_dq_pair(a, c.D, mode, (hipStream_t)stream);
-  return e == hipSuccess ? RA_OK : hip_fail(e, "ra_bwd_pair launch");
+  return plan_q.pair ? on_pair(nullptr, &dq_args) : as_accumulator(rq, c.Lq) ? one_step(2) : bwd_dq_passes(&c, one, 1, stream, &rq);
 }
 
 int64_t ra_bwd_pair_workspace(const ra_bwd_step_params* p) { return bwd_pair_workspace(p, false); }

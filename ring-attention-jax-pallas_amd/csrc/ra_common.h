@@ -267,11 +267,11 @@ RA_DEV void global_to_lds4(const void* gptr, unsigned lds_addr) {
 RA_DEV void global_to_lds4_s(const void* sbase, unsigned voff, unsigned lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dword %1, %0" : : "s"(sbase), "v"(voff), "s"(lds_addr) : "memory", "m0");
 }
-// The arguments of a kernel that takes one struct, read again: what only the end of a kernel needs does not
+// The arguments of a kernel that takes one struct (or a member of it, at byte `at`), read again: what only the end of a kernel needs does not
 // have to sit in scalar registers (or, spilled, in vector registers' lanes) through its loop.
 template <typename T>
-RA_DEV const __attribute__((address_space(4))) T* kernel_args() {
-  auto p = (const __attribute__((address_space(4))) T*)__builtin_amdgcn_kernarg_segment_ptr();
+RA_DEV const __attribute__((address_space(4))) T* kernel_args(int at = 0) {
+  auto p = (const __attribute__((address_space(4))) T*)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + at);
   asm volatile("" : "+s"(p));
   return p;
 }

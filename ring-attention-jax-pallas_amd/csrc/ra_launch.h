@@ -140,8 +140,8 @@ struct PairBwdArgs {
   int via_bf16;   // round to bf16 before the conversion to it
   long long out_sb, out_sh, out_sl;
 };
-hipError_t launch_dq_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream);
-hipError_t launch_dkdv_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream);
+// dK and dV, dQ (nullptr: not this one), or both in one launch
+hipError_t launch_bwd_pair(const PairBwdArgs* dkdv, const PairBwdArgs* dq, int D, int mode, hipStream_t stream);
 hipError_t launch_pair_stat(const void* out, int out_f32, long long sb, long long sh, long long sl, TensorArg dout, const float* lse,
                             float inv_res, float* stat, float* delta, int B, int H, int Lq, int D, hipStream_t stream);
 

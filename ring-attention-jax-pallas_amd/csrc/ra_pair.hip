@@ -21,6 +21,7 @@
 // those with a dense block, for which the compiler reserves 36 bytes of scratch in dK / dV that no instruction uses.)  Before | after, us: documents of 2048 + ALiBi, 32768, H=16, D=128: forward 1787 | 1590, dQ 1916 | 1755, dK/dV
 // 2770 | 2410; causal documents of 2175 in 48128, B=2, H=4, D=64: 443 | 325, 476 | 350, 495 | 427; prefix-LM 4096, B=2, H=16, D=128,
 // forward 229 | 194; steps on dense blocks (documents of 2048 in 32768, 4 shards) 10.2 ms | 7.8 a pass.
+#include <algorithm>
 #include <type_traits>
 
 #include "ra_launch.h"
@@ -858,7 +859,19 @@ __global__ __launch_bounds__(256) void pair_combine_kernel(const PairFwdArgs a) 
 // LDS buffers, scores transposed (S^T = K Q^T, dP^T = V dO^T) so that dS^T is the B operand of
 // dQ^T = K^T dS^T, whose A operand comes from the K tile through the transposing read.
 template <int DL, int MODE>
-__global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel(const PairBwdArgs p) {
+struct DqLds {
+  static constexpr int TILE_BYTES = kPairKeys * (DL <= 64 ? 64 : 128) * 2;
+  __attribute__((aligned(16))) char k[2][TILE_BYTES];
+  __attribute__((aligned(16))) char v[2][TILE_BYTES];
+  __attribute__((aligned(16))) int seg[MODE ? 2 : 1][kPairKeys];
+  __attribute__((aligned(16))) int pre[MODE ? 2 : 1][kPairKeys];
+  ListEntry<MODE == 2> list[MODE ? kPairListTiles : 1];
+  unsigned char flag[MODE ? kPairListTiles : 1];
+  int red[20];
+};
+// args_at: where p lies in the kernel's arguments
+template <int DL, int MODE>
+RA_DEV void dq_pair(const PairBwdArgs& p, int bid, DqLds<DL, MODE>& lds, int args_at) {
   constexpr bool GENERAL = MODE != 0;
   constexpr bool DENSE = MODE == 2;
   constexpr int D = DL <= 64 ? 64 : 128;  // row pitch of the LDS tiles
@@ -866,20 +879,18 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel
   constexpr int ROWB = D * 2;
   constexpr int TILE_BYTES = kPairKeys * ROWB;
   const BwdArgs& a = p.a;
-  __shared__ __attribute__((aligned(16))) char s_k[2][TILE_BYTES];
-  __shared__ __attribute__((aligned(16))) char s_v[2][TILE_BYTES];
-  __shared__ __attribute__((aligned(16))) int s_seg[GENERAL ? 2 : 1][kPairKeys];
-  __shared__ __attribute__((aligned(16))) int s_pre[GENERAL ? 2 : 1][kPairKeys];
-  __shared__ ListEntry<DENSE> s_list[GENERAL ? kPairListTiles : 1];
-  __shared__ unsigned char s_flag[GENERAL ? kPairListTiles : 1];
-  __shared__ int s_red[20];
+  auto &s_k = lds.k, &s_v = lds.v;
+  auto &s_seg = lds.seg, &s_pre = lds.pre;
+  auto& s_list = lds.list;
+  auto& s_flag = lds.flag;
+  auto& s_red = lds.red;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, g = lane >> 5;
   const int nqt = (a.Lq + kPairRows - 1) / kPairRows;
   int hh, split, qt;
-  pair_decode(blockIdx.x, a.B * a.H, nqt, p.n_split, p.group, hh, split, qt);
+  pair_decode(bid, a.B * a.H, nqt, p.n_split, p.group, hh, split, qt);
   const int b = hh / a.H, h = hh % a.H;
   const int q0 = qt * kPairRows;
   const int qw = q0 + wave * 32;
@@ -1137,7 +1148,7 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel
     }
   }
 
-  const auto* e = kernel_args<PairBwdArgs>();
+  const auto* e = kernel_args<PairBwdArgs>(args_at);
   if (e->part_n != nullptr && split == 0 && tid == 0) e->part_n[hh * nqt + qt] = n_piece;
   if (!q_valid) return;
   float* fp = nullptr;  // fp32 destination: a share of the sum, or an accumulator
@@ -1251,7 +1262,20 @@ RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg
 // (MODE 0) and 12 (MODE 1) of them spill, and a reload inside the loop waits for the tile loads that were just issued:
 // causal + ALiBi, 4096, B=2, H=16, 240 us against 189; causal documents of 2175 in 48128, B=2, H=4, 636 against 531.
 template <int DL, int MODE>
-__global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dkdv_pair_kernel(const PairBwdArgs p) {
+struct DkdvLds {
+  static constexpr int ROWB = (DL <= 64 ? 64 : 128) * 2, TILE_BYTES = kPairQueries * ROWB;
+  __attribute__((aligned(16))) char q[2][TILE_BYTES];
+  __attribute__((aligned(16))) char dout[2][TILE_BYTES];
+  __attribute__((aligned(16))) char v[kPairSlab * ROWB];
+  __attribute__((aligned(16))) float stat[2][2][kPairQueries];
+  __attribute__((aligned(16))) int seg[MODE ? 2 : 1][64];  // (a 64-lane load writes 64 words)
+  __attribute__((aligned(16))) int pre[MODE ? 2 : 1][64];
+  ListEntry<MODE == 2> list[MODE ? kPairQListTiles : 1];
+  unsigned char flag[MODE ? kPairQListTiles : 1];
+  int red[20];
+};
+template <int DL, int MODE>
+RA_DEV void dkdv_pair(const PairBwdArgs& p, int bid, DkdvLds<DL, MODE>& lds, int args_at) {
   constexpr bool GENERAL = MODE != 0;
   constexpr bool DENSE = MODE == 2;
   constexpr int D = DL <= 64 ? 64 : 128;  // row pitch of the LDS tiles
@@ -1259,22 +1283,20 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dkdv_pair_kern
   constexpr int ROWB = D * 2;
   constexpr int TILE_BYTES = kPairQueries * ROWB;
   const BwdArgs& a = p.a;
-  __shared__ __attribute__((aligned(16))) char s_q[2][TILE_BYTES];
-  __shared__ __attribute__((aligned(16))) char s_do[2][TILE_BYTES];
-  __shared__ __attribute__((aligned(16))) char s_v[kPairSlab * ROWB];
-  __shared__ __attribute__((aligned(16))) float s_stat[2][2][kPairQueries];
-  __shared__ __attribute__((aligned(16))) int s_seg[GENERAL ? 2 : 1][64];  // (a 64-lane load writes 64 words)
-  __shared__ __attribute__((aligned(16))) int s_pre[GENERAL ? 2 : 1][64];
-  __shared__ ListEntry<DENSE> s_list[GENERAL ? kPairQListTiles : 1];
-  __shared__ unsigned char s_flag[GENERAL ? kPairQListTiles : 1];
-  __shared__ int s_red[20];
+  auto &s_q = lds.q, &s_do = lds.dout;
+  auto& s_v = lds.v;
+  auto& s_stat = lds.stat;
+  auto &s_seg = lds.seg, &s_pre = lds.pre;
+  auto& s_list = lds.list;
+  auto& s_flag = lds.flag;
+  auto& s_red = lds.red;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, g = lane >> 5;
   const int nkt = (a.Lk + kPairSlab - 1) / kPairSlab;
   int hh, split, kt;
-  pair_decode(blockIdx.x, a.B * a.H, nkt, p.n_split, p.group, hh, split, kt);
+  pair_decode(bid, a.B * a.H, nkt, p.n_split, p.group, hh, split, kt);
   kt = nkt - 1 - kt;  // under a causal mask the first keys have the most work
   const int b = hh / a.H, h = hh % a.H;
   const int k0 = kt * kPairSlab;
@@ -1566,7 +1588,7 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dkdv_pair_kern
     }
   }
 
-  const auto* e = kernel_args<PairBwdArgs>();
+  const auto* e = kernel_args<PairBwdArgs>(args_at);
   if (e->part_n != nullptr && split == 0 && tid == 0) e->part_n[hh * nkt + kt] = n_piece;
   // lane l32 holds column 32 db + l32 of rows kw + 4 g + 8 (r / 4) + r % 4
   const long long rows = (long long)e->a.B * e->a.H * e->a.Lk;
@@ -1632,6 +1654,34 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dkdv_pair_kern
   else store(bf16_t{});
 }
 
+template <int DL, int MODE>
+__global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dq_pair_kernel(const PairBwdArgs p) {
+  __shared__ DqLds<DL, MODE> lds;
+  dq_pair<DL, MODE>(p, blockIdx.x, lds, 0);
+}
+template <int DL, int MODE>
+__global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void dkdv_pair_kernel(const PairBwdArgs p) {
+  __shared__ DkdvLds<DL, MODE> lds;
+  dkdv_pair<DL, MODE>(p, blockIdx.x, lds, 0);
+}
+// Both in one launch, the kind with the longer workgroups first.
+struct BothBwdArgs {
+  PairBwdArgs dkdv, dq;
+  int n_first;  // workgroups of the first kind; a multiple of eight where a head stays on its XCD (see pair_decode), for the second's too
+  int dq_first;
+};
+template <int DL, int MODE>
+__global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void bwd_pair_kernel(const BothBwdArgs p) {
+  __shared__ union Lds {
+    DqLds<DL, MODE> dq;
+    DkdvLds<DL, MODE> dkdv;
+  } lds;
+  const bool second = (int)blockIdx.x >= p.n_first;
+  const int bid = second ? blockIdx.x - p.n_first : blockIdx.x;
+  if (second == (p.dq_first != 0)) dkdv_pair<DL, MODE>(p.dkdv, bid, lds.dkdv, offsetof(BothBwdArgs, dkdv));
+  else dq_pair<DL, MODE>(p.dq, bid, lds.dq, offsetof(BothBwdArgs, dq));
+}
+
 // What the dK / dV kernel adds to a row's scores: stat[row] = -lse log2(e) / scale_res (-inf for a row without
 // any key: P = 0) and stat[rows + row] = -delta (0 there: its output, and delta with it, is NaN), with
 // delta = rowsum(out * dout).  HBM bound.
@@ -1666,31 +1716,27 @@ __global__ __launch_bounds__(256) void pair_stat_kernel(const OutT* out, long lo
   }
 }
 
-// Sum of the shares of rows that were split, stored in the gradient's dtype.
-// `n_out` results of the same rows (dK and dV) lie one after another in a share; grid dimension y.
-template <int D, int ROWS>
-__global__ __launch_bounds__(256) void pair_sum_kernel(const PairBwdArgs p, int n_out, int BH, int H, int L) {
+// Sum of the shares of rows that were split, stored in the gradient's dtype.  Grid dimension y, from `first` on: dK and dV, whose
+// rows lie one after another in a share, then dQ.
+template <int D>
+__global__ __launch_bounds__(256) void pair_sum_kernel(const BothBwdArgs both, int first) {
   constexpr int CPR = D / 4;
+  static_assert(kPairSlab == kPairRows, "shares of as many rows");
+  const int which = blockIdx.y + first;
+  const PairBwdArgs& p = which < 2 ? both.dkdv : both.dq;
+  const int H = p.a.H, L = which < 2 ? p.a.Lk : p.a.Lq, n_out = which < 2 ? 2 : 1;
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  const long long rows = (long long)BH * L, row = i / CPR;
+  const long long rows = (long long)p.a.B * H * L, row = i / CPR;
   if (row >= rows) return;
-  const int c = (int)(i % CPR), li = (int)(row % L), which = blockIdx.y;
+  const int c = (int)(i % CPR), li = (int)(row % L);
   const long long hh = row / L;
-  const int n_piece = p.part_n[hh * ((L + ROWS - 1) / ROWS) + li / ROWS];
+  const int n_piece = p.part_n[hh * ((L + kPairRows - 1) / kPairRows) + li / kPairRows];
   if (n_piece <= 1) return;  // written by its only workgroup
   f32x4 x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-  for (int s = 0; s < n_piece; ++s) x += *(const f32x4*)(p.part + (((long long)s * n_out + which) * rows + row) * D + 4 * c);
-  store4(which ? p.out2 : p.out, p.out_dtype, (hh / H) * p.out_sb + (hh % H) * p.out_sh + (long long)li * p.out_sl + 4 * c,
+  for (int s = 0; s < n_piece; ++s) x += *(const f32x4*)(p.part + (((long long)s * n_out + (which & 1)) * rows + row) * D + 4 * c);
+  store4(which == 1 ? p.out2 : p.out, p.out_dtype, (hh / H) * p.out_sb + (hh % H) * p.out_sh + (long long)li * p.out_sl + 4 * c,
          round_via(x, p.via_bf16));
-}
-
-template <int D, int ROWS>
-static hipError_t launch_pair_sum(const PairBwdArgs& p, int n_out, int L, hipStream_t stream) {
-  const long long n = (long long)p.a.B * p.a.H * L * (D / 4);
-  hipLaunchKernelGGL((pair_sum_kernel<D, ROWS>), dim3((unsigned)((n + 255) / 256), (unsigned)n_out), dim3(256), 0, stream, p, n_out,
-                     p.a.B * p.a.H, p.a.H, L);
-  return hipGetLastError();
 }
 
 // The kernels of a head dim: a multiple of 32, dense blocks at 64 and 128 only.
@@ -1706,42 +1752,40 @@ static hipError_t with_dim(int D, int mode, Launch launch) {
   return hipErrorInvalidValue;
 }
 
-template <int D>
-static hipError_t launch_dq_pair_d(const PairBwdArgs& p, int mode, hipStream_t stream) {
-  const BwdArgs& a = p.a;
-  const int nqt = (a.Lq + kPairRows - 1) / kPairRows;
-  dim3 grid((unsigned)(a.B * a.H * p.n_split * nqt)), block(kPairThreads);
-  if (mode == 2) {
-    if constexpr (D == 64 || D == 128) hipLaunchKernelGGL((dq_pair_kernel<D, 2>), grid, block, 0, stream, p);
-  } else if (mode == 1) {
-    hipLaunchKernelGGL((dq_pair_kernel<D, 1>), grid, block, 0, stream, p);
+// dkdv, dq: nullptr for none
+template <int D, int MODE>
+static hipError_t launch_bwd_pair_dm(const PairBwdArgs* dkdv, const PairBwdArgs* dq, hipStream_t stream) {
+  auto tiles = [](int L) { return (L + kPairRows - 1) / kPairRows; };
+  const int n_dkdv = dkdv ? dkdv->a.B * dkdv->a.H * dkdv->n_split * tiles(dkdv->a.Lk) : 0;
+  const int n_dq = dq ? dq->a.B * dq->a.H * dq->n_split * tiles(dq->a.Lq) : 0;
+  const dim3 block(kPairThreads);
+  if (dkdv && dq) {
+    const bool dq_first = dq->chunk_tiles > dkdv->chunk_tiles;
+    const BothBwdArgs p{*dkdv, *dq, dq_first ? n_dq : n_dkdv, dq_first};
+    hipLaunchKernelGGL((bwd_pair_kernel<D, MODE>), dim3((unsigned)(n_dkdv + n_dq)), block, 0, stream, p);
+  } else if (dkdv) {
+    hipLaunchKernelGGL((dkdv_pair_kernel<D, MODE>), dim3((unsigned)n_dkdv), block, 0, stream, *dkdv);
   } else {
-    hipLaunchKernelGGL((dq_pair_kernel<D, 0>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((dq_pair_kernel<D, MODE>), dim3((unsigned)n_dq), block, 0, stream, *dq);
   }
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || p.n_split == 1) return e;
-  return launch_pair_sum<D, kPairRows>(p, 1, a.Lq, stream);
+  const bool sum_dkdv = dkdv && dkdv->n_split > 1, sum_dq = dq && dq->n_split > 1;
+  if (e != hipSuccess || !(sum_dkdv || sum_dq)) return e;
+  const PairBwdArgs& any = dkdv ? *dkdv : *dq;
+  const long long n = (long long)any.a.B * any.a.H * std::max(sum_dkdv ? any.a.Lk : 0, sum_dq ? any.a.Lq : 0) * (D / 4);
+  const BothBwdArgs p{sum_dkdv ? *dkdv : *dq, sum_dq ? *dq : *dkdv, 0, 0};
+  hipLaunchKernelGGL((pair_sum_kernel<D>), dim3((unsigned)((n + 255) / 256), (unsigned)(2 * sum_dkdv + sum_dq)), block, 0, stream, p,
+                     sum_dkdv ? 0 : 2);
+  return hipGetLastError();
 }
 
-template <int D>
-static hipError_t launch_dkdv_pair_d(const PairBwdArgs& p, int mode, hipStream_t stream) {
-  const BwdArgs& a = p.a;
-  const int nkt = (a.Lk + kPairSlab - 1) / kPairSlab;
-  dim3 grid((unsigned)(a.B * a.H * p.n_split * nkt)), block(kPairThreads);
-  if (mode == 2) {
-    if constexpr (D == 64 || D == 128) hipLaunchKernelGGL((dkdv_pair_kernel<D, 2>), grid, block, 0, stream, p);
-  } else if (mode == 1) {
-    hipLaunchKernelGGL((dkdv_pair_kernel<D, 1>), grid, block, 0, stream, p);
-  } else {
-    hipLaunchKernelGGL((dkdv_pair_kernel<D, 0>), grid, block, 0, stream, p);
-  }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || p.n_split == 1) return e;
-  return launch_pair_sum<D, kPairSlab>(p, 2, a.Lk, stream);
-}
-
-hipError_t launch_dkdv_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream) {
-  return with_dim(D, mode, [&](auto d) { return launch_dkdv_pair_d<d.value>(p, mode, stream); });
+hipError_t launch_bwd_pair(const PairBwdArgs* dkdv, const PairBwdArgs* dq, int D, int mode, hipStream_t stream) {
+  return with_dim(D, mode, [&](auto d) {
+    if (mode == 2) {
+      if constexpr (d.value == 64 || d.value == 128) return launch_bwd_pair_dm<d.value, 2>(dkdv, dq, stream);
+    }
+    return mode == 1 ? launch_bwd_pair_dm<d.value, 1>(dkdv, dq, stream) : launch_bwd_pair_dm<d.value, 0>(dkdv, dq, stream);
+  });
 }
 
 hipError_t launch_pair_stat(const void* out, int out_f32, long long sb, long long sh, long long sl, TensorArg dout, const float* lse,
@@ -1754,10 +1798,6 @@ hipError_t launch_pair_stat(const void* out, int out_f32, long long sb, long lon
     else hipLaunchKernelGGL((pair_stat_kernel<bf16_t, d.value>), grid, block, 0, stream, (const bf16_t*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
     return hipGetLastError();
   });
-}
-
-hipError_t launch_dq_pair(const PairBwdArgs& p, int D, int mode, hipStream_t stream) {
-  return with_dim(D, mode, [&](auto d) { return launch_dq_pair_d<d.value>(p, mode, stream); });
 }
 
 template <int D>

@@ -456,3 +456,29 @@ def test_alibi_far_from_the_diagonal_on_the_long_stretch_kernels(device, q_off, 
         ds = p * (a[3] @ a[2].T - (o * a[3]).sum(-1, keepdim=True))
         for got, ref in zip(grads, (ds @ a[1] * scale, ds.T @ a[0] * scale, p.T @ a[3])):
             assert max(_rel(got[0, h].cpu().numpy(), ref.cpu().numpy())) <= GRAD_TOL, h
+
+
+@pytest.mark.parametrize("mask,Sq,Sk,H,D,dtype", [
+    ("causal", 300, 300, 171, 64, torch.bfloat16),         # 513 + 513 workgroups, heads that do not divide by eight
+    ("none", 40, 3000, 43, 128, torch.bfloat16),           # few long rows: dQ's workgroups first, their keys shared
+    ("documents", 2000, 2000, 8, 96, torch.float32),       # rows of both kinds shared, gradients converted
+    ("causal", 700, 700, 86, 32, torch.float16),
+    ("documents", 261, 261, 176, 128, torch.bfloat16)])
+def test_both_gradients_in_one_launch(device, mask, Sq, Sk, H, D, dtype):
+    g = torch.Generator(device=device).manual_seed(Sq + D)
+    q, k, v = (torch.randn((1, S, H, D), device=device, generator=g).to(torch.bfloat16).to(dtype).requires_grad_(True) for S in (Sq, Sk, Sk))
+    do = torch.randn((1, Sq, H, D), device=device, generator=g).to(torch.bfloat16).to(dtype)
+    fn, q_kw, kv_kw, seen = None, None, None, torch.ones((Sq, Sk), dtype=torch.bool, device=device)
+    if mask == "causal":
+        fn, seen = ra.causal_bias(), seen.tril()
+    elif mask == "documents":
+        ids = (torch.arange(Sq, device=device) // 130).to(torch.int32)
+        fn, q_kw, kv_kw, seen = ra.segment_bias(), {"q_segment_ids": ids[None]}, {"kv_segment_ids": ids[None]}, ids[:, None] == ids[None]
+    out = ra.ring_attention(q, k, v, 1, fn, q_kw, kv_kw)
+    grads, launched = _kernels(lambda: torch.autograd.grad(out, (q, k, v), do))
+    assert f"bwd_pair_kernel<{D}, {int(mask == 'documents')}>" in launched, launched
+    ref = [x.detach().float().permute(0, 2, 1, 3).contiguous().requires_grad_(True) for x in (q, k, v)]
+    s = (ref[0] @ ref[1].transpose(2, 3)) / np.sqrt(D)
+    (torch.softmax(s.masked_fill(~seen, -float("inf")), -1) @ ref[2]).backward(do.float().permute(0, 2, 1, 3))
+    for got, x in zip(grads, ref):
+        assert max(_rel(got.float().cpu().numpy(), x.grad.permute(0, 2, 1, 3).cpu().numpy())) <= GRAD_TOL

@@ -713,13 +713,39 @@ bool even_rows(int64_t total, int most, int64_t rows) { return total * 20 >= (in
 bool one_by_one(const ra_bias& b, int64_t total, int most, int64_t rows) {
   return even_rows(total, most, rows) && !has_lists(b) && !(b.flags & RA_BIAS_WINDOW);
 }
-// How the `wgs` workgroups of one kind of a head's resident tiles, which meet `total` tiles of the other
-// side (`most` at most), share their work (see above).
-void plan_split(PairPlan& r, int64_t heads, int64_t rows, int64_t total, int most, int min_chunk) {
+// How the workgroups of one kind of a head's resident tiles, which meet `total` tiles of the other side (`most` at most), share their
+// work (see above).  share: bytes of one share of every row.  beside: the other gradient's workgroups run in the same launch.
+// Rows of about the same length take the number of shares k that a count of time finds best, in tiles of a workgroup (1.4 us at D = 128):
+// the rounds of the fullest compute unit, two workgroups of which are 1.2 times as fast as one (1.4 where a tile has more vector
+// work: ALiBi, lists) - or, beside the other kind, which fills what a round leaves, the mean and a quarter - and the shares written and
+// read, 4 TB/s.  As many shares as places | by this count, us, forward, then backward: unmasked, D=128, 4096, H=8 94 | 93, 256 | 217;
+// 2000, H=4 34 | 30, 71 | 59; 10000, H=4 296 | 247, 795 | 774; 1024, B=2, H=16 47 | 35, 99 | 71; window 1000 of 8192, H=4 46 | 37, 108 | 75;
+// 128 x 32768, H=8 63 | 49, 119 | 108; D=80, 864 x 1024, H=32 44 | 39, 82 | 60; ALiBi 4096, H=8 109 | 107, 273 | 237.
+// Rows of different lengths on more than half of the places are shared only if they are long and the places not nearly full, causal,
+// D=128, shared | not: 14 heads of 4096 (448 workgroups) 104 | 100, 264 | 256; 12 of 4096 (384) 91 | 96, 225 | 230; 24 of 2048 (384) 59 | 54,
+// 156 | 150; 3 of 16384 (384) 284 | 326, 736 | 776; 48 of 758 33 | 27, 86 | 81.  Under a list of tiles the lengths are not known: up to half of the
+// places as many shares as places, and beyond that long rows of the forward by the count (documents of 3000 in 10000, H=5, D=64, 253
+// | 184; short ones lose: documents of 1500 in 4096, H=12, 107 | 121, and so does the backward: prefix 20000, H=3, 1103 | 1202).
+void plan_split(PairPlan& r, int64_t heads, int64_t rows, int64_t total, int most, int min_chunk, int64_t share, const ra_bias& bias,
+                bool beside) {
   const int64_t wgs = heads * rows;
   if (wgs > kPairSlots || most <= min_chunk) return;
-  const bool even = even_rows(total, most, rows);
-  const int64_t chunk = even ? (most + kPairSlots / wgs - 1) / (kPairSlots / wgs) : heads * total * 3 / (2 * kPairSlots);
+  const bool even = even_rows(total, most, rows), few = wgs <= kPairSlots / 2, lists = has_lists(bias);
+  int64_t chunk = even ? (most + kPairSlots / wgs - 1) / (kPairSlots / wgs) : heads * total * 3 / (2 * kPairSlots);
+  if (!even && !few && (wgs > kPairSlots * 3 / 4 || most < 8 * min_chunk)) return;
+  if (even && lists && !few && (beside || most < 16 * min_chunk)) return;
+  if (even && !(lists && few)) {
+    const double pair_rate = lists || (bias.flags & RA_BIAS_ALIBI) ? 1.4 : 1.2;
+    double least = 0;
+    for (int k = 1; k <= std::min(kMaxSplit, (most + min_chunk - 1) / min_chunk); ++k) {
+      const int64_t n = (beside ? 2 : 1) * wgs * k, c = std::max((most + k - 1) / k, min_chunk);
+      const double rounds = beside ? std::max(1.0, n / (kPairSlots / 2.0) + (n > kPairSlots / 2 ? 0.25 : 0.0)) : (double)((n + kPairSlots / 2 - 1) / (kPairSlots / 2));
+      const double cost = rounds * c / (n > kPairSlots / 2 ? pair_rate : 1.0) + (k > 1 ? k * (share * 3.6e-7 + 0.1) + 1 : 0);
+      if (k > 1 && cost >= least) continue;
+      least = cost;
+      chunk = c;
+    }
+  }
   r.chunk_tiles = (int)std::min<int64_t>(most, std::max<int64_t>({chunk, min_chunk, (most + kMaxSplit - 1) / kMaxSplit}));
   r.n_split = (most + r.chunk_tiles - 1) / r.chunk_tiles;
 }
@@ -752,7 +778,7 @@ PairPlan plan_fwd_pair(const ra_fwd_step_params& p) {
   // uneven rows that fill the chip less than one and a quarter times: 8 heads of 10240, 0.275 | 0.250)
   const bool nearly_one = wgs <= kPairSlots * 5 / 4 && !even_rows(total, most, rows);
   if (!nearly_one && long_stretches(p.bias, p.D, wgs, total, rows, (p.bias.flags & RA_BIAS_ALIBI) ? 192 : 56)) r.pair = false;
-  if (r.pair) plan_split(r, heads, rows, total, most, kMinChunk);
+  if (r.pair) plan_split(r, heads, rows, total, most, kMinChunk, 4 * heads * p.Lq * p.D, p.bias, false);
   if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;
 }
@@ -765,7 +791,7 @@ PairPlan plan_dq_pair(const ra_bwd_step_params& p) {
   PairPlan r{true, 1, std::max(most, 1), kHeadGroup};
   const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lq + kPairRowsHost - 1) / kPairRowsHost;
   if (long_stretches(p.bias, p.D, heads * rows, total, rows, 160)) r.pair = false;
-  else plan_split(r, heads, rows, total, most, kMinChunk);
+  else plan_split(r, heads, rows, total, most, kMinChunk, 4 * heads * p.Lq * p.D, p.bias, true);
   if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;
 }
@@ -793,7 +819,7 @@ PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
   const int tiles = one_round ? (even ? 112 : 0) : (p.bias.flags & RA_BIAS_ALIBI) ? 448 : even ? 112 : 192;
   if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, total, rows, tiles)) r.pair = false;
   else if (heads * p.Lq + 31 >= (int64_t)1 << 30) r.pair = false;  // one 32-bit byte offset reaches both statistics of a tile's 32 rows
-  else plan_split(r, heads, rows, total, most, 2 * kMinChunk);
+  else plan_split(r, heads, rows, total, most, 2 * kMinChunk, 8 * heads * p.Lk * p.D, p.bias, true);
   if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;
 }

@@ -164,17 +164,107 @@ struct FragOffsets {
   RA_DEV int tr(int db, int h2) const { return (t0 ^ (db << 6) ^ (h2 * (D == 128 ? 32 : 64))) + h2 * 8 * (D * 2); }
 };
 
+// Smallest and largest value of N neighbouring lanes (8 or 16), in all of them.
+template <int CTRL>
+RA_DEV int dpp(int x) {
+  return __builtin_amdgcn_update_dpp(x, x, CTRL, 0xf, 0xf, false);
+}
+constexpr int kDppXor1 = 0xb1, kDppXor2 = 0x4e, kDppMirror8 = 0x141, kDppMirror16 = 0x140;
+template <int N = 16>
+RA_DEV int row_min(int x) {
+  x = min(x, dpp<kDppXor1>(x));
+  x = min(x, dpp<kDppXor2>(x));
+  x = min(x, dpp<kDppMirror8>(x));
+  return N == 16 ? min(x, dpp<kDppMirror16>(x)) : x;
+}
+template <int N = 16>
+RA_DEV int row_max(int x) {
+  x = max(x, dpp<kDppXor1>(x));
+  x = max(x, dpp<kDppXor2>(x));
+  x = max(x, dpp<kDppMirror8>(x));
+  return N == 16 ? max(x, dpp<kDppMirror16>(x)) : x;
+}
+
 // The segment ids and prefix flags of a wave's 32 rows, as uniform values.
 struct WaveIds {
   int lo, hi;     // smallest and largest segment id of the wave's rows
   bool any, all;  // some / every row carries the prefix flag
   RA_DEV void init(bool valid, int seg, int pre) {
-    lo = __builtin_amdgcn_readfirstlane(wave_min(valid ? seg : 0x7fffffff));
-    hi = __builtin_amdgcn_readfirstlane(wave_max(valid ? seg : (int)0x80000000));
+    const int mn = row_min(valid ? seg : 0x7fffffff), mx = row_max(valid ? seg : (int)0x80000000);  // (both halves of the wave hold the rows)
+    lo = min(__builtin_amdgcn_readlane(mn, 0), __builtin_amdgcn_readlane(mn, 16));
+    hi = max(__builtin_amdgcn_readlane(mx, 0), __builtin_amdgcn_readlane(mx, 16));
     any = __any(valid && pre != 0);
     all = __all(!valid || pre != 0);
   }
 };
+
+// Calls put(i, smallest, largest) for the ids of tiles j_lo + i, i in [i_lo, n), of T tokens, of an array of L, or for its flags as 0 and 1; all
+// four waves.  A lane takes four neighbouring tokens and T / 4 lanes a tile: a load instruction reads a kilobyte in one piece.  (A lane per tile
+// reads 64 lines per instruction.  Documents of 16 in 32768, H=16, which are little but lists, so | like this, us, forward, backward:
+// D=128 206 | 191, 534 | 501; D=64 127 | 111, 331 | 294; documents of 100, D=128 238 | 226, 628 | 606.)
+template <int T, bool FLAGS, typename Put>
+RA_DEV void tile_ranges(const int* ids, int j_lo, int i_lo, int n, int L, int wave, int lane, Put put) {
+  constexpr int LPT = T / 4, TPL = 64 / LPT, U = 8;  // lanes per tile, tiles per load, loads in flight
+  const bool aligned = ((uintptr_t)ids & 15) == 0;
+  for (int base = i_lo + wave * (U * TPL); base < n; base += 4 * U * TPL) {
+    i32x4 x[U];
+    const int first = (j_lo + base) * T + 4 * lane;  // of this lane's tokens in the first load
+    if (aligned && (j_lo + base + U * TPL) * T <= L) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = *(const i32x4*)(ids + first + u * 256);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[u][c] = ids[min(first + u * 256 + c, L - 1)];  // (repeats of the last one change nothing)
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (FLAGS) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[u][c] = x[u][c] != 0;
+      }
+      const int lo = row_min<LPT>(min(min(x[u][0], x[u][1]), min(x[u][2], x[u][3])));
+      const int hi = row_max<LPT>(max(max(x[u][0], x[u][1]), max(x[u][2], x[u][3])));
+      const int i = base + u * TPL + lane / LPT;
+      if (lane % LPT == 0 && i < n) put(i, lo, hi);
+    }
+  }
+}
+
+// The entries of the n tiles from j_lo on whose flag is set, in order; returns their number.  A thread takes PER neighbouring flags.
+// cells: the list holds the tiles' cells.
+template <bool DENSE, int PER>
+RA_DEV int compact_list(int j_lo, int n, bool cells, int* s_red, const unsigned char* s_flag, ListEntry<DENSE>* s_list) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i0 = threadIdx.x * PER;
+  unsigned entry[PER];
+  int mine = 0;
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int f = i0 + p < n ? s_flag[i0 + p] : 0;
+    entry[p] = f ? (j_lo + i0 + p) | ((f & 7) << kTestShift) | 0x80000000u : 0u;
+    if constexpr (DENSE) {
+      if (f) entry[p] = (entry[p] & 0xffff) | (cells ? s_list[i0 + p] : 0xffffu) << kCellShift;
+    }
+    mine += f != 0;
+  }
+  int before = 0, all = 0;
+#pragma unroll
+  for (int bit = 1; bit <= PER; bit <<= 1) {
+    const unsigned long long mask = __ballot(mine & bit);
+    before += bit * __popcll(mask & ((1ull << lane) - 1ull));
+    all += bit * __popcll(mask);
+  }
+  if (lane == 0) s_red[wave] = all;
+  __syncthreads();  // (the cells have been read, too)
+  const int n0 = s_red[0], n1 = s_red[1], n2 = s_red[2], n3 = s_red[3];
+  int at = before + (wave > 0 ? n0 : 0) + (wave > 1 ? n1 : 0) + (wave > 2 ? n2 : 0);
+#pragma unroll
+  for (int p = 0; p < PER; ++p)
+    if (entry[p]) s_list[at++] = (ListEntry<DENSE>)entry[p];
+  __syncthreads();
+  return n0 + n1 + n2 + n3;
+}
 
 // The list of key tiles that the workgroup's rows [q0, q_hi] have to visit, of the n from j_lo on:
 // tiles that one or the other term rules out are dropped, the others carry the terms that they
@@ -195,61 +285,44 @@ RA_DEV int list_key_tiles(int Lq, int Lk, const BiasArgs& bs, const int* kv_seg,
   const int qmin = min(min(s_red[0], s_red[1]), min(s_red[2], s_red[3]));
   const int qmax = max(max(s_red[4], s_red[5]), max(s_red[6], s_red[7]));
   const bool q_any = s_red[8] | s_red[9] | s_red[10] | s_red[11], q_all = s_red[12] & s_red[13] & s_red[14] & s_red[15];
-  for (int i = tid; i < n; i += kPairThreads) {
-    const int j = j_lo + i;
-    int f = 0x80;  // listed
-    if (seg_on) {
-      int kmin, kmax;
-      tile_id_range<kPairKeys>(kv_seg, j, Lk, kmin, kmax);
-      if (kmax < qmin || kmin > qmax) f = 0;
-      else if (kmin != kmax || qmin != qmax) f |= kTestSegment;
-    }
-    if (pre_on && f) {
-      const int klo = bs.kv_off + j * kPairKeys, khi = bs.kv_off + min((j + 1) * kPairKeys, Lk) - 1;
-      if (khi > bs.q_off + q0) {
-        bool k_any, k_all;
-        tile_flag_range<kPairKeys>(kv_pre, j, Lk, k_any, k_all);
-        const int c = prefix_class(bs.q_off + q0, bs.q_off + q_hi, klo, khi, q_any, q_all, k_any, k_all);
-        if (c == 2) f = 0;
-        else if (c == 1) f |= kTestPrefix;
-      }
-    }
-    if constexpr (DENSE) {
-      if (dmap != nullptr && f) {
+  if (seg_on) {
+    tile_ranges<kPairKeys, false>(kv_seg, j_lo, 0, n, Lk, wave, lane, [&](int i, int kmin, int kmax) {
+      s_flag[i] = (kmax < qmin || kmin > qmax) ? 0 : (kmin != kmax || qmin != qmax) ? 0x80 | kTestSegment : 0x80;  // 0x80: listed
+    });
+  } else {
+    for (int i = tid; i < n; i += kPairThreads) s_flag[i] = 0x80;
+  }
+  if (pre_on) {
+    __syncthreads();
+    // from the first tile on with a key behind the first row's position
+    const int i_lo = max(0, floor_div(bs.q_off + q0 - bs.kv_off + 1, kPairKeys) - j_lo);
+    tile_ranges<kPairKeys, true>(kv_pre, j_lo, i_lo, n, Lk, wave, lane, [&](int i, int all, int any) {
+      const int klo = bs.kv_off + (j_lo + i) * kPairKeys, khi = bs.kv_off + min((j_lo + i + 1) * kPairKeys, Lk) - 1;
+      const int c = prefix_class(bs.q_off + q0, bs.q_off + q_hi, klo, khi, q_any, q_all, any, all);
+      const int f = s_flag[i];
+      if (f && c) s_flag[i] = c == 2 ? 0 : f | kTestPrefix;
+    });
+  }
+  if constexpr (DENSE) {
+    if (dmap != nullptr) {
+      __syncthreads();
+      for (int i = tid; i < n; i += kPairThreads) {
         // the summary's cells of the four waves' rows, two bits each, first and second key block of the tile
         const int ncols = (Lk + kMapCell - 1) / kMapCell;
         unsigned cells = 0;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-          const int r = q0 / kMapCell + c / 2, col = 2 * j + c % 2;
+          const int r = q0 / kMapCell + c / 2, col = 2 * (j_lo + i) + c % 2;
           if (r * kMapCell <= q_hi && col < ncols) cells |= (dmap[(long long)r * ncols + col] & 3u) << (2 * c);
         }
-        if (!(cells & 0x5555)) f = 0;
-        else if (cells & 0xaaaa) f |= kTestDense;
+        if (!(cells & 0x5555)) s_flag[i] = 0;
+        else if ((cells & 0xaaaa) && s_flag[i]) s_flag[i] |= kTestDense;
         s_list[i] = cells;  // (until the entries are written)
       }
     }
-    s_flag[i] = (unsigned char)f;
   }
   __syncthreads();
-  if (wave == 0) {
-    int cnt = 0;
-    for (int base = 0; base < n; base += 64) {
-      const int i = base + lane;
-      const int f = (i < n) ? s_flag[i] : 0;
-      const unsigned long long mask = __ballot(f != 0);
-      unsigned entry = (j_lo + i) | ((f & 7) << kTestShift);
-      if constexpr (DENSE) {
-        if (f) entry |= (dmap != nullptr ? s_list[i] : 0xffffu) << kCellShift;
-        __builtin_amdgcn_wave_barrier();  // (entries land at or below what has been read)
-      }
-      if (f) s_list[cnt + __popcll(mask & ((1ull << lane) - 1ull))] = (ListEntry<DENSE>)entry;
-      cnt += __popcll(mask);
-    }
-    if (lane == 0) s_red[16] = cnt;
-  }
-  __syncthreads();
-  return s_red[16];
+  return compact_list<DENSE, kPairListTiles / kPairThreads>(j_lo, n, dmap != nullptr, s_red, s_flag, s_list);
 }
 
 // ALiBi on one side of the diagonal: -slope |q - k| = s (j - rel), with s = +-slope, rel the distance of this lane's
@@ -1195,62 +1268,44 @@ RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg
   const int kmin = min(min(s_red[0], s_red[1]), min(s_red[2], s_red[3]));
   const int kmax = max(max(s_red[4], s_red[5]), max(s_red[6], s_red[7]));
   const bool k_any = s_red[8] | s_red[9] | s_red[10] | s_red[11], k_all = s_red[12] & s_red[13] & s_red[14] & s_red[15];
-  for (int i = tid; i < n; i += kPairThreads) {
-    const int j = j_lo + i;
-    const int q_last = min((j + 1) * kPairQueries, Lq) - 1;
-    int f = 0x80;  // listed
-    if (seg_on) {
-      int qmin, qmax;
-      tile_id_range<kPairQueries>(q_seg, j, Lq, qmin, qmax);
-      if (qmax < kmin || qmin > kmax) f = 0;
-      else if (qmin != qmax || kmin != kmax) f |= kTestSegment;
-    }
-    if (pre_on && f) {
-      const int qlo = bs.q_off + j * kPairQueries, qhi = bs.q_off + q_last;
-      if (bs.kv_off + k_hi > qlo) {
-        bool q_any, q_all;
-        tile_flag_range<kPairQueries>(q_pre, j, Lq, q_any, q_all);
-        const int c = prefix_class(qlo, qhi, bs.kv_off + k0, bs.kv_off + k_hi, q_any, q_all, k_any, k_all);
-        if (c == 2) f = 0;
-        else if (c == 1) f |= kTestPrefix;
-      }
-    }
-    if constexpr (DENSE) {
-      if (dmap != nullptr && f) {
+  if (seg_on) {
+    tile_ranges<kPairQueries, false>(q_seg, j_lo, 0, n, Lq, wave, lane, [&](int i, int qmin, int qmax) {
+      s_flag[i] = (qmax < kmin || qmin > kmax) ? 0 : (qmin != qmax || kmin != kmax) ? 0x80 | kTestSegment : 0x80;  // 0x80: listed
+    });
+  } else {
+    for (int i = tid; i < n; i += kPairThreads) s_flag[i] = 0x80;
+  }
+  if (pre_on) {
+    __syncthreads();
+    // up to the last tile with a query before the last key's position
+    const int i_hi = min(n, floor_div(bs.kv_off + k_hi - 1 - bs.q_off, kPairQueries) + 1 - j_lo);
+    tile_ranges<kPairQueries, true>(q_pre, j_lo, 0, i_hi, Lq, wave, lane, [&](int i, int all, int any) {
+      const int qlo = bs.q_off + (j_lo + i) * kPairQueries, qhi = bs.q_off + min((j_lo + i + 1) * kPairQueries, Lq) - 1;
+      const int c = prefix_class(qlo, qhi, bs.kv_off + k0, bs.kv_off + k_hi, any, all, k_any, k_all);
+      const int f = s_flag[i];
+      if (f && c) s_flag[i] = c == 2 ? 0 : f | kTestPrefix;
+    });
+  }
+  if constexpr (DENSE) {
+    if (dmap != nullptr) {
+      __syncthreads();
+      for (int i = tid; i < n; i += kPairThreads) {
         // the summary's cells of the four waves' keys, two bits each
         const int ncols = (Lk + kMapCell - 1) / kMapCell;
         unsigned cells = 0;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const int col = k0 / kMapCell + c;
-          if (col * kMapCell <= k_hi) cells |= (dmap[(long long)j * ncols + col] & 3u) << (2 * c);
+          if (col * kMapCell <= k_hi) cells |= (dmap[(long long)(j_lo + i) * ncols + col] & 3u) << (2 * c);
         }
-        if (!(cells & 0x55)) f = 0;
-        else if (cells & 0xaa) f |= kTestDense;
+        if (!(cells & 0x55)) s_flag[i] = 0;
+        else if ((cells & 0xaa) && s_flag[i]) s_flag[i] |= kTestDense;
         s_list[i] = cells;  // (until the entries are written)
       }
     }
-    s_flag[i] = (unsigned char)f;
   }
   __syncthreads();
-  if (wave == 0) {
-    int cnt = 0;
-    for (int base = 0; base < n; base += 64) {
-      const int i = base + lane;
-      const int f = (i < n) ? s_flag[i] : 0;
-      const unsigned long long mask = __ballot(f != 0);
-      unsigned entry = (j_lo + i) | ((f & 7) << kTestShift);
-      if constexpr (DENSE) {
-        if (f) entry |= (dmap != nullptr ? s_list[i] : 0xffffu) << kCellShift;
-        __builtin_amdgcn_wave_barrier();  // (entries land at or below what has been read)
-      }
-      if (f) s_list[cnt + __popcll(mask & ((1ull << lane) - 1ull))] = (ListEntry<DENSE>)entry;
-      cnt += __popcll(mask);
-    }
-    if (lane == 0) s_red[16] = cnt;
-  }
-  __syncthreads();
-  return s_red[16];
+  return compact_list<DENSE, kPairQListTiles / kPairThreads>(j_lo, n, dmap != nullptr, s_red, s_flag, s_list);
 }
 
 // 128 keys per workgroup, 32 per wave, two workgroups per compute unit: K operands and the dK / dV

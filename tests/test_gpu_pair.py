@@ -482,3 +482,36 @@ def test_both_gradients_in_one_launch(device, mask, Sq, Sk, H, D, dtype):
     (torch.softmax(s.masked_fill(~seen, -float("inf")), -1) @ ref[2]).backward(do.float().permute(0, 2, 1, 3))
     for got, x in zip(grads, ref):
         assert max(_rel(got.float().cpu().numpy(), x.grad.permute(0, 2, 1, 3).cpu().numpy())) <= GRAD_TOL
+
+
+@pytest.mark.parametrize("S", [63, 65, 1027, 2049, 4100, 16500])
+@pytest.mark.parametrize("kind", ["documents", "prefix", "both"])
+def test_tile_lists_of_any_length(device, S, kind):
+    """Ids and flags that are read a kilobyte at a time, rows that are aligned and that are not, the last tiles of a row, ids in any
+    order: documents that come back later, prefix flags in the middle."""
+    B, H, D = 2, 1, 32
+    g = torch.Generator(device=device).manual_seed(S)
+    q, k, v, do = (torch.randn((B, S, H, D), device=device, generator=g).to(torch.bfloat16) for _ in range(4))
+    at = torch.arange(S, device=device)
+    ids = ((at[None] // 97 * torch.tensor([[5], [7]], device=device)) % 11).to(torch.int32)
+    flags = ((at[None] // 150) % 3 == torch.tensor([[0], [1]], device=device)).to(torch.int32)
+    seen = torch.ones((B, S, S), dtype=torch.bool, device=device)
+    fn, kw = None, {}
+    if kind != "prefix":
+        fn, seen = ra.segment_bias(), seen & (ids[:, :, None] == ids[:, None])
+        kw["segment_ids"] = ids
+    if kind != "documents":
+        fn = ra.prefix_lm_bias() if fn is None else fn + ra.prefix_lm_bias()
+        seen = seen & ((at[:, None] >= at[None]) | ((flags[:, :, None] != 0) & (flags[:, None] != 0)))
+        kw["prefix_mask"] = flags
+    leaves = [x.clone().requires_grad_(True) for x in (q, k, v)]
+    out = ra.ring_attention(*leaves, 1, fn, {"q_" + a: x for a, x in kw.items()}, {"kv_" + a: x for a, x in kw.items()})
+    grads = torch.autograd.grad(out, leaves, do)
+    for b in range(B):
+        ref = [x[b, :, 0].float().requires_grad_(True) for x in (q, k, v)]
+        s = (ref[0] @ ref[1].T / np.sqrt(D)).masked_fill(~seen[b], -float("inf"))
+        want = torch.softmax(s, -1) @ ref[2]
+        assert (out[b, :, 0].float() - want).abs().max() <= OUT_TOL
+        want.backward(do[b, :, 0].float())
+        for got, x in zip(grads, ref):
+            assert max(_rel(got[b, :, 0].float().cpu().numpy(), x.grad.cpu().numpy())) <= GRAD_TOL

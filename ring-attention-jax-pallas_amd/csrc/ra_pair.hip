@@ -333,6 +333,9 @@ RA_DEV int list_key_tiles(int Lq, int Lk, const BiasArgs& bs, const int* kv_seg,
 // 3.4e-3, and by 6e-4 so).  Under dK / dV it is c, on top of -logsumexp, which it cancels.  (Split into
 // bf16 words for the bf16 product, s and c took 20 vector instructions a tile, of the 200 of a forward tile.)
 // `j`: alibi_index of the block.
+// The initial value is the same in every tile on one side: the forward keeps it in the 16 registers that it has free, dQ in LDS; one product
+// per tile | kept, us, D=64 4096, B=2, H=16, causal 121 | 114 and the backward 276 | 268; 8192, H=16 381 | 366 and 918 | 899; D=128 8192, H=16
+// 599 | 580 and 1585 | 1574; documents of 2000 in 32768, H=16 1735 | 1716 and 4489 | 4452.
 RA_DEV float alibi_index(int first, int l32, int g) { return g == 0 ? (float)(first + l32) : 1.0f; }
 // -slope rel log2(e), and what that lacks of the product to twice the bits
 RA_DEV float alibi_far(float slope, int rel, float& rest) {
@@ -654,6 +657,14 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   const bool alibi_on = GENERAL && (flags & RA_BIAS_ALIBI);
   const WaveTiles wt = wave_key_tiles(bs, q_off + qw, q_off + qw + 31, a.Lk);
   TileWalk<DENSE> walk;
+  f32x16 ramp;  // ALiBi's initial value of the scores (alibi_one_side), the same in every tile on one side of the diagonal
+  bool ramp_past = false;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) ramp[r] = 0.f;
+  if (alibi_on) {
+    const f32x16 none = ramp;
+    ramp = alibi_one_side(none, alibi_index(0, l32, g), -slope2, 0.f, g);
+  }
 
   auto step = [&](auto buffer, int i) {
     constexpr int BUF = decltype(buffer)::value;
@@ -698,12 +709,16 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
     if (one_side) {
       const int at = opaque_lane(lane), l = at & 31, half = at >> 5;
       // one initial value for both key blocks: the second one's is 32 slopes further, added to its exponents
-      const float s = j < wt.past ? slope2 : -slope2;
-      const f32x16 init = alibi_one_side(zero, alibi_index(0, l, half), s, 0.f, half);
+      const bool past = j < wt.past;
+      const float s = past ? slope2 : -slope2;
+      if (past != ramp_past) {
+        ramp = alibi_one_side(zero, alibi_index(0, l, half), s, 0.f, half);
+        ramp_past = past;
+      }
       beyond = 32.f * s;
       far = alibi_far(j < wt.past ? slope : -slope, q_off + qw + l - (kv_off + kt0), far_rest);
-      S[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[0], init, 0, 0, 0);
-      S[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[1], qf[0], init, 0, 0, 0);
+      S[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[0], ramp, 0, 0, 0);
+      S[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[1], qf[0], ramp, 0, 0, 0);
     } else {
       S[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[0], zero, 0, 0, 0);
       S[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[1], qf[0], zero, 0, 0, 0);
@@ -941,6 +956,7 @@ struct DqLds {
   ListEntry<MODE == 2> list[MODE ? kPairListTiles : 1];
   unsigned char flag[MODE ? kPairListTiles : 1];
   int red[20];
+  __attribute__((aligned(16))) float ramp[MODE ? 2 : 1][kPairKeys];  // ALiBi on either side of the diagonal: +-slope j of a tile's keys j
 };
 // args_at: where p lies in the kernel's arguments
 template <int DL, int MODE>
@@ -1038,6 +1054,10 @@ RA_DEV void dq_pair(const PairBwdArgs& p, int bid, DqLds<DL, MODE>& lds, int arg
   const int i_lo = n * split / n_piece, i_hi = n * (split + 1) / n_piece;
   int every_test = 0;
   if constexpr (GENERAL) {
+    if ((flags & RA_BIAS_ALIBI) && wave == 0) {
+      lds.ramp[0][lane] = slope2 * (float)lane;
+      lds.ramp[GENERAL][lane] = -slope2 * (float)lane;
+    }
     if (!use_list && (flags & RA_BIAS_PREFIX)) every_test |= kTestPrefix;
     if ((flags & RA_BIAS_DENSE) && dmap == nullptr) every_test |= kTestDense;
   }
@@ -1111,8 +1131,13 @@ RA_DEV void dq_pair(const PairBwdArgs& p, int bid, DqLds<DL, MODE>& lds, int arg
         __builtin_amdgcn_sched_barrier(0);
         if (one_side) {
           const int at = opaque_lane(lane), l = at & 31, half = at >> 5;
-          const float s = j < wt.past ? slope2 : -slope2;
-          S = alibi_one_side(zero, alibi_index(32 * kb, l, half), s, 0.f, half);
+          const float* ramp = lds.ramp[GENERAL && j >= wt.past] + 32 * kb + 4 * half;
+#pragma unroll
+          for (int bb = 0; bb < 4; ++bb) {
+            const f32x4 t = *(const f32x4*)(ramp + 8 * bb);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) S[4 * bb + c] = t[c];
+          }
           // (the bias and the logsumexp cancel before they are scaled)
           neg_row = fmaf(j < wt.past ? -slope : slope, (float)(q_off + qw + l - (kv_off + kt0)), neg_lse) * kLog2e;
           S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[0], qf[0], S, 0, 0, 0);

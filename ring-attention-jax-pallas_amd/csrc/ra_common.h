@@ -303,6 +303,7 @@ struct TileBias {
   const float* dense;   // dense bias element of (fixed index, var0); natural-log units
   long long dense_vs;   // its stride along the varying side (1 when the keys vary)
   int dense_vec;        // keys vary, the whole block is in range and rows are 16-byte aligned: vector loads
+  unsigned dense_lane;  // (kernels for short pairs, queries vary: `dense` is the tile's, this the lane's offset)
 };
 
 // Branch-free per element: the uniform `flags` only shape a handful of per-lane constants up

@@ -427,25 +427,46 @@ RA_DEV void apply_terms(f32x16& t, int todo, const TileBias& tb, int rel0, int f
     }
     if constexpr (DENSE) {
       if (todo & kTestDense) {
-        float dn[16];
-        if (QFIXED && __builtin_amdgcn_readfirstlane(tb.dense_vec)) {
+        const bool vec = __builtin_amdgcn_readfirstlane(tb.dense_vec);
+        if (QFIXED && vec) {
           // a lane's four keys are 16 contiguous bytes of its row
+          f32x4 dn[4];
 #pragma unroll
-          for (int bb = 0; bb < 4; ++bb) {
-            const f32x4 v4 = *(const f32x4*)(tb.dense + 8 * bb);
+          for (int bb = 0; bb < 4; ++bb) dn[bb] = *(const f32x4*)(tb.dense + 8 * bb);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) dn[4 * bb + c] = v4[c];
-          }
-        } else {
+          for (int r = 0; r < 16; ++r) t[r] = fmaf(dn[r / 4][r % 4], tb.dense_mul, t[r]);
+        } else if (QFIXED) {
+          float dn[16];
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int off = 8 * (r / 4) + r % 4;
             dn[r] = 0.f;
-            if (off < tb.var_limit) dn[r] = QFIXED ? tb.dense[off] : tb.dense[off * tb.dense_vs];
+            if (off < tb.var_limit) dn[r] = tb.dense[off];
+          }
+#pragma unroll
+          for (int r = 0; r < 16; ++r) t[r] = fmaf(dn[r], tb.dense_mul, t[r]);
+        } else if (vec) {
+          // a row of the block is scalar, in it and between the wave's halves a lane has one offset.  (An address per lane and row, each
+          // under a range test: 11 registers of dkdv_pair_kernel<128, 2> went to scratch inside the loop.)
+          float dn[16];
+          const char* row = (const char*)tb.dense;
+          const unsigned at = tb.dense_lane;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) dn[r] = *(const float*)(row + (8 * (r / 4) + r % 4) * tb.dense_vs * 4 + at);
+#pragma unroll
+          for (int r = 0; r < 16; ++r) t[r] = fmaf(dn[r], tb.dense_mul, t[r]);
+        } else {
+          // rows past the end read the last one again (masked below); four at a time, for want of registers
+#pragma unroll
+          for (int bb = 0; bb < 4; ++bb) {
+            float dn[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) dn[c] = tb.dense[max(min(8 * bb + c, tb.var_limit - 1), 0) * tb.dense_vs + tb.dense_lane];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) t[4 * bb + c] = fmaf(dn[c], tb.dense_mul, t[4 * bb + c]);
+            __builtin_amdgcn_sched_barrier(0);
           }
         }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) t[r] = fmaf(dn[r], tb.dense_mul, t[r]);
       }
     }
     if (todo & kTestSegment) {
@@ -946,17 +967,20 @@ __global__ __launch_bounds__(256) void pair_combine_kernel(const PairFwdArgs a) 
 // The same split: 128 query rows per workgroup (Q and dO in registers), 64-key tiles of K and V in two
 // LDS buffers, scores transposed (S^T = K Q^T, dP^T = V dO^T) so that dS^T is the B operand of
 // dQ^T = K^T dS^T, whose A operand comes from the K tile through the transposing read.
+// (What the loop reads lies within the 64 KB that an LDS instruction's own offset reaches: with the tiles first, what lay behind them took
+// registers for its addresses, and dkdv_pair_kernel<128, 2> reloaded 11 from scratch in its loop: diagonal blocks of documents of
+// 2000, 8192 x 8192, H=16, 946 and 736 us for both gradients, 818 and 693 so.)
 template <int DL, int MODE>
 struct DqLds {
   static constexpr int TILE_BYTES = kPairKeys * (DL <= 64 ? 64 : 128) * 2;
-  __attribute__((aligned(16))) char k[2][TILE_BYTES];
-  __attribute__((aligned(16))) char v[2][TILE_BYTES];
+  __attribute__((aligned(16))) float ramp[MODE ? 2 : 1][kPairKeys];  // ALiBi on either side of the diagonal: +-slope j of a tile's keys j
   __attribute__((aligned(16))) int seg[MODE ? 2 : 1][kPairKeys];
   __attribute__((aligned(16))) int pre[MODE ? 2 : 1][kPairKeys];
+  __attribute__((aligned(16))) char k[2][TILE_BYTES];
+  __attribute__((aligned(16))) char v[2][TILE_BYTES];
   ListEntry<MODE == 2> list[MODE ? kPairListTiles : 1];
   unsigned char flag[MODE ? kPairListTiles : 1];
   int red[20];
-  __attribute__((aligned(16))) float ramp[MODE ? 2 : 1][kPairKeys];  // ALiBi on either side of the diagonal: +-slope j of a tile's keys j
 };
 // args_at: where p lies in the kernel's arguments
 template <int DL, int MODE>
@@ -1344,12 +1368,12 @@ RA_DEV int list_query_tiles(int Lq, int Lk, const BiasArgs& bs, const int* q_seg
 template <int DL, int MODE>
 struct DkdvLds {
   static constexpr int ROWB = (DL <= 64 ? 64 : 128) * 2, TILE_BYTES = kPairQueries * ROWB;
+  __attribute__((aligned(16))) float stat[2][2][MODE == 2 ? 64 : kPairQueries];  // (a 64-lane load writes 64 words)
+  __attribute__((aligned(16))) int seg[MODE ? 2 : 1][64];
+  __attribute__((aligned(16))) int pre[MODE ? 2 : 1][64];
   __attribute__((aligned(16))) char q[2][TILE_BYTES];
   __attribute__((aligned(16))) char dout[2][TILE_BYTES];
   __attribute__((aligned(16))) char v[kPairSlab * ROWB];
-  __attribute__((aligned(16))) float stat[2][2][kPairQueries];
-  __attribute__((aligned(16))) int seg[MODE ? 2 : 1][64];  // (a 64-lane load writes 64 words)
-  __attribute__((aligned(16))) int pre[MODE ? 2 : 1][64];
   ListEntry<MODE == 2> list[MODE ? kPairQListTiles : 1];
   unsigned char flag[MODE ? kPairQListTiles : 1];
   int red[20];
@@ -1449,18 +1473,21 @@ RA_DEV void dkdv_pair(const PairBwdArgs& p, int bid, DkdvLds<DL, MODE>& lds, int
   TileLoader<D, kPairQueries, DL> ldq, ldo;
   ldq.init(a.q.ptr + b * a.q.sb + h * a.q.sh, a.q.sl, a.Lq, wave, lane);
   ldo.init(a.dout.ptr + b * a.dout.sb + h * a.dout.sh, a.dout.sl, a.Lq, wave, lane);
-  // lanes 0..31 move -lse of a tile's rows, lanes 32..63 -delta
+  // lanes 0..31 move -lse of a tile's rows, lanes 32..63 -delta; under a dense block two waves move one each
   const bool raw_stat = DENSE && p.stat == nullptr;  // a single step, which has no room for them: from lse and delta, per tile
-  const float* stat = (DENSE ? (raw_stat ? (g ? a.delta : a.lse) : p.stat + (g ? (long long)a.B * a.H * a.Lq : 0)) : p.stat) + (long long)hh * a.Lq;
+  const float* stat = (raw_stat ? a.lse : p.stat) + (long long)hh * a.Lq;
+  const float* stat_delta = raw_stat ? a.delta + (long long)hh * a.Lq : stat + (long long)a.B * a.H * a.Lq;
   const unsigned to_delta = (unsigned)(a.B * a.H) * (unsigned)a.Lq * 4;  // (with a row's 124 bytes below 2^32: plan_dkdv_pair)
   auto issue_tile = [&](int j, int buf) {
     const int r0 = j * kPairQueries;
     ldq.issue(r0, RA_LDS_ADDR(&s_q[0][0]) + buf * TILE_BYTES, wave, lane);
     ldo.issue(r0, RA_LDS_ADDR(&s_do[0][0]) + buf * TILE_BYTES, wave, lane);
     const int row = min(opaque_lane(lane) & 31, a.Lq - 1 - r0);
-    if (wave == 0) {
-      if constexpr (DENSE) global_to_lds4(stat + (r0 + row), RA_LDS_ADDR(&s_stat[0][0][0]) + buf * (2 * kPairQueries * 4));
-      else global_to_lds4_s(stat + r0, 4 * row + (lane >= 32 ? to_delta : 0u), RA_LDS_ADDR(&s_stat[0][0][0]) + buf * (2 * kPairQueries * 4));
+    if constexpr (DENSE) {
+      if (wave == 0) global_to_lds4_s(stat + r0, 4 * row, RA_LDS_ADDR(&s_stat[0][0][0]) + buf * 512);
+      if (wave == 3) global_to_lds4_s(stat_delta + r0, 4 * row, RA_LDS_ADDR(&s_stat[0][1][0]) + buf * 512);
+    } else if (wave == 0) {
+      global_to_lds4_s(stat + r0, 4 * row + (lane >= 32 ? to_delta : 0u), RA_LDS_ADDR(&s_stat[0][0][0]) + buf * (2 * kPairQueries * 4));
     }
     if constexpr (GENERAL) {
       if (q_seg && wave == 1) global_to_lds4_s(q_seg + r0, 4 * row, RA_LDS_ADDR(&s_seg[0][0]) + buf * 256);
@@ -1556,8 +1583,13 @@ RA_DEV void dkdv_pair(const PairBwdArgs& p, int bid, DkdvLds<DL, MODE>& lds, int
       tb.dense_mul = kLog2e / a.scale_res;
       tb.var_limit = a.Lq - (qt0 + 4 * g);
       if (DENSE) {
-        tb.dense = bs.dense + b * bs.dense_sb + h * bs.dense_sh + (long long)(qt0 + 4 * g) * bs.dense_sq + min(ki, a.Lk - 1);
+        // whole tiles whose lanes' offsets (four rows at most) fit 32 bits; else, in elements, from the lane's own first row on
+        const int key = min(ki, a.Lk - 1);
+        tb.dense = bs.dense + b * bs.dense_sb + h * bs.dense_sh + (long long)qt0 * bs.dense_sq;
         tb.dense_vs = bs.dense_sq;
+        tb.dense_vec = qt0 + kPairQueries <= a.Lq && bs.dense_sq < (1 << 27);
+        tb.dense_lane = tb.dense_vec ? 4 * (4 * g * (unsigned)bs.dense_sq + key) : key;
+        if (!tb.dense_vec) tb.dense += (long long)(g && qt0 + 4 < a.Lq ? 4 : 0) * bs.dense_sq;
       }
       apply_terms<false, DENSE, GENERAL>(S, tests, tb, (q_off + qt0 + 4 * g) - (kv_off + ki), k_seg, k_pre,
                                          &s_seg[GENERAL ? BUF : 0][4 * g], &s_pre[GENERAL ? BUF : 0][4 * g]);

@@ -515,3 +515,25 @@ def test_tile_lists_of_any_length(device, S, kind):
         want.backward(do[b, :, 0].float())
         for got, x in zip(grads, ref):
             assert max(_rel(got[b, :, 0].float().cpu().numpy(), x.grad.cpu().numpy())) <= GRAD_TOL
+
+
+@pytest.mark.parametrize("summary", [True, False])
+@pytest.mark.parametrize("Lq,Lk,D,columns", [(3, 40, 128, 40), (37, 130, 64, 131), (64, 64, 128, 64), (101, 33, 128, 200), (70, 300, 64, 300)])
+def test_values_of_a_dense_block_on_both_gradients(device, monkeypatch, Lq, Lk, D, columns, summary):
+    """More slabs than compute units: dkdv_pair_kernel reads the block's rows by a scalar address and the lanes' offset, and a tile that
+    is not whole by an address per lane; rows that are further apart than they are long, masked entries among the values."""
+    monkeypatch.setattr(bias_module, "DENSE_SUMMARY", summary)
+    H = 270
+    g = torch.Generator(device=device).manual_seed(Lq + D)
+    q, k, v, do = (torch.randn((1, H, L, D), device=device, generator=g).to(torch.bfloat16) for L in (Lq, Lk, Lk, Lq))
+    block = torch.randn((1, H, Lq, columns), device=device, generator=g)[..., :Lk]
+    block[:, :, :, 1::5] = -float("inf")
+    scale = 1 / np.sqrt(D)
+    ref = [x.float().requires_grad_(True) for x in (q, k, v)]
+    s = ref[0] @ ref[1].transpose(2, 3) * scale + block
+    out = torch.softmax(s, -1) @ ref[2]
+    out.backward(do.float())
+    grads, launched = _kernels(lambda: ra.bwd_block(q, k, v, block, out.detach().to(torch.bfloat16), torch.logsumexp(s, -1).detach(), do, scale))
+    assert f"bwd_pair_kernel<{D}, 2>" in launched, launched
+    for got, x in zip(grads, ref):
+        assert max(_rel(got.cpu().numpy(), x.grad.cpu().numpy())) <= GRAD_TOL

@@ -595,11 +595,14 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   if (split > 0 && split * a.chunk_tiles >= n) return;
 
   bf16x8 qf[KS];
-  {
+  auto load_rows = [&]() {
     const bf16_t* qp = a.q.ptr + b * a.q.sb + h * a.q.sh + (long long)qi_c * a.q.sl + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s) qf[s] = *(const bf16x8*)(qp + 16 * s);
-  }
+  };
+  // (A dense block may leave these rows nothing, as ring steps on masks often do: there the list comes first.  Blocks of 8192 x 8192, H=16,
+  // that are masked throughout, rows first | list first, us: forward 15 | 9, both gradients 44 | 20.)
+  if (!DENSE) load_rows();
   int q_seg = 0, q_pre = 0;
   float slope = 0.f, slope2 = 0.f;  // slope2: in the units of the scores
   const int* kv_seg = nullptr;
@@ -634,6 +637,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   n = __builtin_amdgcn_readfirstlane(n);
   j_lo = __builtin_amdgcn_readfirstlane(j_lo);
   if (n == 0 && a.o != nullptr) return;  // identity on the carry
+  if (DENSE) load_rows();
   const int n_piece = max(1, min(a.n_split, (n + a.chunk_tiles - 1) / a.chunk_tiles));
   if (split >= n_piece) return;
   const int i_lo = n * split / n_piece, i_hi = n * (split + 1) / n_piece;
@@ -1024,7 +1028,9 @@ RA_DEV void dq_pair(const PairBwdArgs& p, int bid, DqLds<DL, MODE>& lds, int arg
   // Q carries the power of two below sm_scale * log2(e) (exact in bf16), the residual factor is
   // applied to the fp32 score (see dkdv_kernel)
   bf16x8 qf[KS], dof[KS];
-  {
+  float neg_lse, neg_lse2, neg_delta;
+  const long long row = (long long)hh * a.Lq + qi_c;
+  auto load_rows = [&]() {
     const bf16_t* qp = a.q.ptr + b * a.q.sb + h * a.q.sh + (long long)qi_c * a.q.sl + 8 * g;
     const bf16_t* dp = a.dout.ptr + b * a.dout.sb + h * a.dout.sh + (long long)qi_c * a.dout.sl + 8 * g;
 #pragma unroll
@@ -1034,12 +1040,12 @@ RA_DEV void dq_pair(const PairBwdArgs& p, int bid, DqLds<DL, MODE>& lds, int arg
       for (int e = 0; e < 8; ++e) qf[s][e] = (bf16_t)((float)qr[e] * a.scale_p2);
       dof[s] = *(const bf16x8*)(dp + 16 * s);
     }
-  }
-  const long long row = (long long)hh * a.Lq + qi_c;
-  const float Lraw = a.lse[row];
-  const float neg_lse = (Lraw == RA_NEG_INF) ? RA_NEG_INF : -Lraw;  // fully masked row: P = 0
-  const float neg_lse2 = neg_lse * kLog2e;
-  const float neg_delta = -a.delta[row];
+    const float Lraw = a.lse[row];
+    neg_lse = (Lraw == RA_NEG_INF) ? RA_NEG_INF : -Lraw;  // fully masked row: P = 0
+    neg_lse2 = neg_lse * kLog2e;
+    neg_delta = -a.delta[row];
+  };
+  if (!DENSE) load_rows();
   int q_seg = 0, q_pre = 0;
   float slope = 0.f, slope2 = 0.f;  // slope2: in the units of the scores
   const int* kv_seg = nullptr;
@@ -1073,6 +1079,7 @@ RA_DEV void dq_pair(const PairBwdArgs& p, int bid, DqLds<DL, MODE>& lds, int arg
   n = __builtin_amdgcn_readfirstlane(n);
   j_lo = __builtin_amdgcn_readfirstlane(j_lo);
   if (n == 0 && p.acc != nullptr) return;  // contributes nothing
+  if (DENSE) load_rows();
   const int n_piece = max(1, min(p.n_split, (n + p.chunk_tiles - 1) / p.chunk_tiles));
   if (split >= n_piece) return;
   const int i_lo = n * split / n_piece, i_hi = n * (split + 1) / n_piece;
@@ -1423,7 +1430,7 @@ RA_DEV void dkdv_pair(const PairBwdArgs& p, int bid, DkdvLds<DL, MODE>& lds, int
   if (split > 0 && split * p.chunk_tiles >= n) return;
 
   bf16x8 kf[KS];
-  {
+  auto load_rows = [&]() {
     const bf16_t* kp = a.k.ptr + b * a.k.sb + h * a.k.sh + (long long)ki_c * a.k.sl + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
@@ -1431,7 +1438,8 @@ RA_DEV void dkdv_pair(const PairBwdArgs& p, int bid, DkdvLds<DL, MODE>& lds, int
 #pragma unroll
       for (int e = 0; e < 8; ++e) kf[s][e] = (bf16_t)((float)kr[e] * a.scale_p2);
     }
-  }
+  };
+  if (!DENSE) load_rows();
   int k_seg = 0, k_pre = 0;
   float slope2 = 0.f;
   const int* q_seg = nullptr;
@@ -1462,6 +1470,7 @@ RA_DEV void dkdv_pair(const PairBwdArgs& p, int bid, DkdvLds<DL, MODE>& lds, int
   n = __builtin_amdgcn_readfirstlane(n);
   j_lo = __builtin_amdgcn_readfirstlane(j_lo);
   if (n == 0 && p.acc != nullptr) return;  // contributes nothing
+  if (DENSE) load_rows();
   const int n_piece = max(1, min(p.n_split, (n + p.chunk_tiles - 1) / p.chunk_tiles));
   if (split >= n_piece) return;
   const int i_lo = n * split / n_piece, i_hi = n * (split + 1) / n_piece;

@@ -826,7 +826,8 @@ PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
 // Whether both gradients' workgroups go into one launch: the second kind fills the places that the first one's last round leaves
 // empty.  Two launches | one, us: causal, D=128, 6000, H=16 493 | 488, 4096, H=8 180 | 163; D=64, 2048, B=2, H=16 112 | 97; D=32, 8192, H=16 338 |
 // 312; documents of 500 in 32768, H=8 838 | 793, of 3500 in 10112, causal, H=4, D=80 352 | 278; prefix 4096, B=2, H=16 586 | 576; unmasked 3000,
-// H=24 441 | 370.  Past eight rounds the last one is a few per cent, and the one launch draws more power
+// H=24 441 | 370.  Past eight rounds (at D <= 64 of 768 workgroups: documents of 2000 in 48128, causal, B=2, H=4, 7.8 of them, a pass
+// 1409 | 1296) the last one is a few per cent, and the one launch draws more power
 // without a pause (documents of 1200 + ALiBi, 29696, 24 heads: a pass 3.86 | 4.00 ms).  Fewer than two rounds stay two launches
 // (even rows at D <= 64, three workgroups of which fit a compute unit, fewer than three): what those run on is pinned by name in
 // test_gpu_pair.py; one launch would be 10 us faster there too (512, H=4, D=64, causal: 38 | 28).
@@ -836,7 +837,7 @@ bool bwd_in_one_launch(const ra_bwd_step_params& p, const PairPlan& dq, const Pa
   auto tiles = [](int L) { return (int64_t)(L + kPairRowsHost - 1) / kPairRowsHost; };
   const int64_t wgs = heads * (tiles(p.Lq) * dq.n_split + tiles(p.Lk) * dkdv.n_split);
   const bool three = p.D <= 64 && !(p.bias.flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) && !has_lists(p.bias);
-  return wgs >= (three ? 3 : 2) * kPairSlots && wgs <= 8 * kPairSlots;
+  return wgs >= (three ? 3 : 2) * kPairSlots && wgs <= (p.D <= 64 ? 12 : 8) * kPairSlots;
 }
 // The workspace of ra_bwd_pair: the rows' statistics, then the shares of dQ and of dK and dV.
 struct BwdSpace {

@@ -19,6 +19,9 @@ SOURCES = ["ra_fwd.hip", "ra_bwd.hip", "ra_pair.hip", "ra_convert.hip", "ra_api.
 # the block-step library exports nothing but the block-step ABI
 PROBE_LIB_PATH = os.path.join(HERE, "ring_attention", "libringattn_probe.so")
 PROBE_SOURCES = ["ra_probe.hip"]
+# the calls on whole sequences from Python: a CPython extension over torch's C++ API
+HOST_LIB_PATH = os.path.join(HERE, "ring_attention", "_host.so")
+HOST_SOURCE = "ra_host.cc"
 # the XLA FFI handlers over the C ABI (what a JAX host binds): built only where jaxlib's headers are
 FFI_LIB_PATH = os.path.join(HERE, "ring_attention", "libringattn_xla_ffi.so")
 FFI_SOURCE = "ra_xla_ffi.cc"
@@ -84,6 +87,26 @@ def build_xla_ffi(verbose: bool = False) -> str | None:
     return FFI_LIB_PATH
 
 
+def build_host(verbose: bool = False) -> str:
+    """ring_attention/_host.so from csrc/ra_host.cc."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    include = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", *(x for p in include for x in ("-isystem", p)),
+           os.path.join(CSRC, HOST_SOURCE), "-o", HOST_LIB_PATH, "-L" + os.path.join(os.path.dirname(torch.__file__), "lib"),
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on {HOST_SOURCE}:\n{res.stderr}")
+    if verbose:
+        print(f"built {HOST_LIB_PATH}")
+    return HOST_LIB_PATH
+
+
 def build(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
     """Compile every kernel translation unit and link the shared library. Always rebuilds."""
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -98,6 +121,7 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
             raise RuntimeError(f"link failed:\n{res.stderr}")
         if verbose:
             print(f"built {lib}")
+    build_host(verbose)
     build_xla_ffi(verbose)
     return LIB_PATH
 

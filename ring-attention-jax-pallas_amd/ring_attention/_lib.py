@@ -161,6 +161,24 @@ def load() -> C.CDLL:
     return lib
 
 
+_host = None
+
+
+def host():
+    """The module of ``csrc/ra_host.cc``, on the library that is loaded."""
+    global _host
+    if _host is None:
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError("ring_attention/_host.so is missing or was built for another torch: build it first (python build.py "
+                               f"in the package directory, or __graft_entry__.build()): {e}") from e
+        lib = load()
+        module.init(*(C.cast(f, C.c_void_p).value for f in (lib.ra_fwd_call, lib.ra_bwd_call, lib.ra_convert)), check)
+        _host = module
+    return _host
+
+
 def check(fn_name: str, code: int) -> None:
     if code != 0:
         raise RingAttentionHipError(fn_name, code, load().ra_last_error().decode())

@@ -167,17 +167,6 @@ def _convert(tensors, dtypes, d: int):
     return out
 
 
-def _row_item(t: torch.Tensor, ptr: int, d: int):
-    """The ``ra_rows`` that converts [b, l, h, *] to bf16 rows of ``d`` elements one after another at ``ptr``; None for
-    what ``ra_convert`` does not take."""
-    src = _ROW_DTYPES.get(t.dtype)
-    B, L, H, dt = t.shape
-    sb, sl, sh, sd = t.stride()
-    if src is None or sd != 1 or B >= 65536 or not 0 < B * L * H or L * H >= 1 << 27:
-        return None
-    return _ROWS.pack(t.data_ptr(), ptr, src, _lib.RA_DTYPE_BF16, dt, d, B, L, H, sb, sl, sh, L * H * d, H * d, d)
-
-
 def _kernel_inputs(tensors, d: int):
     """``_kernel_ready`` for several tensors at once, padded to the kernels' head dim ``d``."""
     todo = [t for t in tensors if t.dtype != torch.bfloat16 or t.shape[3] != d]
@@ -556,6 +545,16 @@ class _RingPlan:
             size = got[backward] = (lib.ra_bwd_whole_workspace if backward else lib.ra_fwd_whole_workspace)(C.byref(p))
         return got["bias"], size
 
+    def native(self, like):
+        """``pair_call`` as ``csrc/ra_host.cc`` keeps it; ``like``: a tensor on the plan's device."""
+        got = self.__dict__.get("_native")
+        if got is None:
+            (bias, forward), (_, backward) = self.pair_call(False), self.pair_call(True)
+            arrays = self.__dict__["_pair_call"]["arrays"]
+            got = self.__dict__["_native"] = _lib.host().plan(self.B, self.H, self.Lq, self.Lk, self.D, bias, forward, backward, like,
+                                                              () if arrays is None else tuple(arrays._keep))
+        return got
+
     def live_steps(self, qs: Optional[int], ks: Optional[int]) -> int:
         """How many ring steps of query shard ``qs`` (or key/value shard ``ks``) are not masked
         entirely by the positional terms - the steps that cost something."""
@@ -804,44 +803,16 @@ _FWD_HEAD = struct.Struct("5if12q24x")     # sizes, scale, q, k, v (pointer, str
 _BWD_HEAD = struct.Struct("5if16qq32x")  # ... and dO, the logsumexp; no delta, no accumulators
 
 
-def _rows_at(ptr: int, L: int, H: int, D: int):
-    """Pointer and strides of contiguous [b, l, h, d] rows."""
-    return ptr, L * H * D, D, H * D
-
-
 def _rows_of(t: torch.Tensor):
     sb, sl, sh, _ = t.stride()
     return t.data_ptr(), sb, sh, sl
 
 
-def _pair_operands(q, k, v, plan: "_RingPlan"):
-    """What a call on a whole sequence reads: (tensors to keep, blocks of ``ra_rows`` that make them, their number).
-    One buffer holds all three operands where they have to be converted."""
-    D = plan.D
-    if q.dtype == k.dtype == v.dtype and (q.dtype != torch.bfloat16 or q.shape[3] != D) and q.device == k.device == v.device:
-        nq, nk = plan.B * plan.Lq * plan.H * D, plan.B * plan.Lk * plan.H * D
-        if tuple(k.shape) == tuple(v.shape) == (plan.B, plan.Lk, plan.H, q.shape[3]):
-            buf = torch.empty((nq + 2 * nk,), dtype=torch.bfloat16, device=q.device)
-            at = buf.data_ptr()
-            items = [_row_item(x, y, D) for x, y in ((q, at), (k, at + 2 * nq), (v, at + 2 * (nq + nk)))]
-            if all(items):
-                return (buf,), b"".join(items), 3
-    return tuple(_kernel_inputs((q, k, v), D)), b"", 0
-
-
-def _pair_views(kept, plan: "_RingPlan"):
-    if len(kept) == 3:
-        return [_rows_of(x) for x in kept]
-    at, H, D = kept[0].data_ptr(), plan.H, plan.D
-    nq, nk = plan.B * plan.Lq * H * D, plan.B * plan.Lk * H * D
-    return [_rows_at(at, plan.Lq, H, D), _rows_at(at + 2 * nq, plan.Lk, H, D), _rows_at(at + 2 * (nq + nk), plan.Lk, H, D)]
-
-
-def _empty_gradients(q, k, v, dtype=torch.bfloat16):
+def _empty_gradients(q, k, v):
     """dq, dk and dv, not yet written, laid out as the operands [b, l, h, d].  The kernels store dk and dv with the same strides:
     where k and v differ in theirs (rotary embeddings leave k transposed and v as it was, say) both are contiguous."""
     kv_format = torch.preserve_format if k.stride() == v.stride() else torch.contiguous_format
-    return [torch.empty_like(q, dtype=dtype), *(torch.empty_like(x, dtype=dtype, memory_format=kv_format) for x in (k, v))]
+    return [torch.empty_like(q), *(torch.empty_like(x, memory_format=kv_format) for x in (k, v))]
 
 
 def _workspace(size: int, device):
@@ -851,45 +822,31 @@ def _workspace(size: int, device):
     return ws, ws.data_ptr()
 
 
-def _pair_forward(kept, plan: "_RingPlan", sm_scale, out_dtype, before=b"", n_before=0):
-    """``_ring_forward_fused`` of a ring of one shard: one call, conversions of its operands (``before``) included.
-    Host code is what small calls cost: fp32 forward of 1024 tokens, H=4, 49 us as three calls with ctypes structures,
-    an object for the stream and an array per operand, 32 us like this (the kernels take 19); training on 2 x 2048 packed
-    tokens 250 | 166."""
+def _pair_forward(kept, plan: "_RingPlan", sm_scale, out_dtype):
+    """``_ring_forward_fused`` of a ring of one shard: one call."""
     B, H, D, Lq = plan.B, plan.H, plan.D, plan.Lq
     out = torch.empty((B, Lq, H, D), dtype=out_dtype, device=plan.device)
     lse = torch.empty((1, B, H, Lq), dtype=torch.float32, device=plan.device)
     bias, size = plan.pair_call(False)
-    q, k, v = _pair_views(kept, plan)
+    q, k, v = (_rows_of(x) for x in kept)
     ws, ws_ptr = _workspace(size, plan.device)
     _lib.check("ra_fwd_call", _lib.load().ra_fwd_call(
-        before, n_before, _FWD_HEAD.pack(B, H, Lq, plan.Lk, D, sm_scale, *q, *k, *v) + bias, out.data_ptr(), _DTYPE_CODE[out_dtype],
+        b"", 0, _FWD_HEAD.pack(B, H, Lq, plan.Lk, D, sm_scale, *q, *k, *v) + bias, out.data_ptr(), _DTYPE_CODE[out_dtype],
         Lq * H * D, D, H * D, lse.data_ptr(), ws_ptr, size, _stream()))
     return out, lse
 
 
-def _pair_backward(kept, out, lse, do, plan: "_RingPlan", sm_scale, dtype=torch.bfloat16):
-    """``_ring_backward_fused`` of a ring of one shard: one call for all launches, the conversion of ``do`` included.
-    ``dtype``: the gradients', of bf16 precision whatever it is."""
-    B, H, D, Lq, Lk, device = plan.B, plan.H, plan.D, plan.Lq, plan.Lk, plan.device
-    if len(kept) == 3:
-        grads = _empty_gradients(*kept, dtype)
-    else:
-        grads = [torch.empty((B, L, H, D), dtype=dtype, device=device) for L in (Lq, Lk, Lk)]
-    before = None
-    if do.dtype != torch.bfloat16 or do.shape[3] != D:
-        made = torch.empty((B, Lq, H, D), dtype=torch.bfloat16, device=device)
-        before = _row_item(do, made.data_ptr(), D) if do.device == device else None
-    if before is None:
-        made, = _kernel_inputs((do,), D)
-    dq, dk, dv = grads
+def _pair_backward(kept, out, lse, do, plan: "_RingPlan", sm_scale):
+    """``_ring_backward_fused`` of a ring of one shard: one call for all launches."""
+    B, H, D, Lq, Lk = plan.B, plan.H, plan.D, plan.Lq, plan.Lk
+    dq, dk, dv = grads = _empty_gradients(*kept)
     bias, size = plan.pair_call(True)
-    q, k, v = _pair_views(kept, plan)
-    ws, ws_ptr = _workspace(size, device)
+    q, k, v = (_rows_of(x) for x in kept)
+    ws, ws_ptr = _workspace(size, plan.device)
     (_, qb, qh, ql), (_, kb, kh, kl), (_, ob, oh, ol) = _rows_of(dq), _rows_of(dk), _rows_of(out)
     _lib.check("ra_bwd_call", _lib.load().ra_bwd_call(
-        before, 0 if before is None else 1, _BWD_HEAD.pack(B, H, Lq, Lk, D, sm_scale, *q, *k, *v, *_rows_of(made), lse.data_ptr()) + bias,
-        out.data_ptr(), _DTYPE_CODE[out.dtype], ob, oh, ol, _ROW_DTYPES[dtype] | _lib.RA_DTYPE_VIA_BF16, dq.data_ptr(), qb, qh, ql,
+        b"", 0, _BWD_HEAD.pack(B, H, Lq, Lk, D, sm_scale, *q, *k, *v, *_rows_of(do), lse.data_ptr()) + bias,
+        out.data_ptr(), _DTYPE_CODE[out.dtype], ob, oh, ol, _lib.RA_DTYPE_BF16 | _lib.RA_DTYPE_VIA_BF16, dq.data_ptr(), qb, qh, ql,
         dk.data_ptr(), dv.data_ptr(), kb, kh, kl, ws_ptr, size, _stream()))
     return grads
 
@@ -1073,13 +1030,8 @@ class _RingAttentionFn(torch.autograd.Function):
         be the kernels' own (padded, ``out_dtype``), which the caller cuts."""
         ctx.given = [(t.shape[3], t.dtype) for t in (q, k, v)]
         d = q.shape[3]
-        ctx.whole = fused and plan.n == 1 and plan.callable is None  # one call, conversions included
-        if ctx.whole:
-            kept, before, n = _pair_operands(q, k, v, plan)
-            out, lse = _pair_forward(kept, plan, sm_scale, out_dtype, before, n)
-        else:
-            kept = _kernel_inputs((q, k, v), plan.D)
-            out, lse = (_ring_forward_fused if fused else _ring_forward)(*kept, plan, sm_scale, out_dtype)
+        kept = _kernel_inputs((q, k, v), plan.D)
+        out, lse = (_ring_forward_fused if fused else _ring_forward)(*kept, plan, sm_scale, out_dtype)
         ctx.save_for_backward(*kept, out, lse)
         ctx.plan, ctx.sm_scale, ctx.fused = plan, sm_scale, fused
         ctx.mark_non_differentiable(lse)
@@ -1094,15 +1046,10 @@ class _RingAttentionFn(torch.autograd.Function):
         plan = ctx.plan
         if do is None:  # nothing came back for the output: gradients of zero, as materialised ones give
             do = torch.zeros(out.shape, dtype=torch.bfloat16, device=out.device)
-        d_true, dtype = ctx.given[0]
-        if ctx.whole:
-            # as the caller wants them, where that takes no cut
-            direct = d_true == plan.D and dtype in _ROW_DTYPES and all(given[1] == dtype for given in ctx.given)
-            grads = list(_pair_backward(kept, out, lse, do, plan, ctx.sm_scale, dtype if direct else torch.bfloat16))
-        else:
-            do, = _kernel_inputs((do,), plan.D)
-            bwd = _ring_backward_fused if ctx.fused else _ring_backward
-            grads = list(bwd(*kept, out, lse, do, plan, ctx.sm_scale))
+        d_true = ctx.given[0][0]
+        do, = _kernel_inputs((do,), plan.D)
+        bwd = _ring_backward_fused if ctx.fused else _ring_backward
+        grads = list(bwd(*kept, out, lse, do, plan, ctx.sm_scale))
         todo = [i for i, (d, dtype) in enumerate(ctx.given)
                 if ctx.needs_input_grad[i] and (d != plan.D or dtype != grads[i].dtype)]
         if todo:
@@ -1151,7 +1098,11 @@ def _attend(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs, sm_scale
     if fused:
         plan = plan.joined()
     final_dtype = out_dtype if in_dtype in (torch.float32, torch.bfloat16) else in_dtype
-    out, lse = _RingAttentionFn.apply(q, k, v, plan, float(sm_scale), out_dtype, final_dtype, fused)
+    # one call, conversions included (torch.jit.trace refuses the Python function; a native node it would record without its kernels)
+    if fused and plan.n == 1 and plan.callable is None and torch._C._get_tracing_state() is None:
+        out, lse = _lib.host().attend(q, k, v, plan.native(q), float(sm_scale), out_dtype, final_dtype)
+    else:
+        out, lse = _RingAttentionFn.apply(q, k, v, plan, float(sm_scale), out_dtype, final_dtype, fused)
     if out.shape[-1] != d_true:
         out = out[..., :d_true]
     return out, lse, plan

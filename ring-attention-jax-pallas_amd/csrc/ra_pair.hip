@@ -667,15 +667,20 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
 
   float m_run = RA_NEG_INF;  // exponent reference (log2 domain), moves lazily
   float m_true = RA_NEG_INF;
-  float l_run = 0.f, lr_run = 0.f;  // row sums of the fp32 and of the rounded probabilities (see fwd_step_kernel)
+  float l_run = 0.f;  // row sum of the probabilities ...
+  // ... and, in the first element, of the rounded ones (see fwd_step_kernel): by dot products, or, where vector issue binds and the matrix
+  // pipe has room, as matrix products of four ones and a lane's own four values (a column of a 4x4 block is one lane).  us, forward, dot
+  // products | matrix products: D=64 causal + ALiBi 4096, B=2, H=16 118 | 111, unmasked 8192, H=16 322 | 320; D=32 causal 8192, H=16 143 |
+  // 137; D=128 causal 4096, H=16 95 | 98, documents + ALiBi 32768 1694 | 1703.
+  constexpr bool SUM_MFMA = DL <= 64;
+  f32x4 lr_acc = {0.f, 0.f, 0.f, 0.f};
   f32x16 oacc[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
-  bf16x2 ones2;
-  ones2[0] = (bf16_t)1.0f;
-  ones2[1] = (bf16_t)1.0f;
+  const i16x4 ones4 = {0x3f80, 0x3f80, 0x3f80, 0x3f80};
+  const bf16x2 ones2 = {(bf16_t)1.0f, (bf16_t)1.0f};
 
   const FragOffsets<D> fo(lane);
   const bool wave_on = qw < a.Lq;
@@ -796,7 +801,8 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
       const float corr = fast_exp2(m_run - ((m_new == RA_NEG_INF) ? 0.f : m_new));
       m_run = m_new;
       l_run *= corr;
-      lr_run *= corr;
+      if constexpr (SUM_MFMA) lr_acc *= corr;
+      else lr_acc[0] *= corr;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -853,11 +859,14 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        bf16x2 pr;
-        pr[0] = pf[ks][e];
-        pr[1] = pf[ks][e + 1];
-        lr_run = __builtin_amdgcn_fdot2_f32_bf16(pr, ones2, lr_run, false);
+      for (int e = 0; e < 8; e += 4) {
+        const bf16x4 pr = {pf[ks][e], pf[ks][e + 1], pf[ks][e + 2], pf[ks][e + 3]};
+        if constexpr (SUM_MFMA) {
+          lr_acc = __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones4, __builtin_bit_cast(i16x4, pr), lr_acc, 0, 0, 0);
+        } else {
+          lr_acc[0] = __builtin_amdgcn_fdot2_f32_bf16((bf16x2){pr[0], pr[1]}, ones2, lr_acc[0], false);
+          lr_acc[0] = __builtin_amdgcn_fdot2_f32_bf16((bf16x2){pr[2], pr[3]}, ones2, lr_acc[0], false);
+        }
       }
   };
 
@@ -873,6 +882,7 @@ __global__ __launch_bounds__(kPairThreads, 2) void fwd_pair_kernel(const PairFwd
   const auto* e = kernel_args<PairFwdArgs>();
   // a wave without a live score leaves its rows of the carry as they are, unread (m would come back through
   // two unit conversions, a last bit off)
+  const float lr_run = lr_acc[0];
   if (e->o != nullptr && __all(l_run == 0.f && lr_run == 0.f)) return;
   const float l_step = half_sum(l_run), lr_step = half_sum(lr_run);
   if (e->part_n != nullptr && split == 0 && tid == 0) e->part_n[hh * nqt + qt] = n_piece;

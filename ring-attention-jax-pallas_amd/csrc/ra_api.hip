@@ -1196,6 +1196,36 @@ int ra_bwd_dkdv_ring(const ra_bwd_step_params* steps, const int32_t* steps_per_p
   return bwd_dkdv_passes(steps, first, n_passes, stream, &r);
 }
 
+static int convert_args(const ra_rows* items, int32_t n_items, ra::ConvertArgs& a) {
+  if (n_items < 1 || n_items > ra::kMaxConvert) return fail(RA_ERR_SHAPE, "ra_convert: 1 to %d arrays (got %d)", ra::kMaxConvert, n_items);
+  if (!items) return fail(RA_ERR_NULL, "ra_convert: items is NULL");
+  memset(&a, 0, sizeof(a));
+  for (int i = 0; i < n_items; ++i) {
+    const ra_rows& r = items[i];
+    if (!r.src || !r.dst) return fail(RA_ERR_NULL, "ra_convert: NULL pointer");
+    if (r.B <= 0 || r.L <= 0 || r.H <= 0 || r.src_d <= 0 || r.dst_d <= 0)
+      return fail(RA_ERR_SHAPE, "ra_convert: bad shape B=%d L=%d H=%d d=%d -> %d", r.B, r.L, r.H, r.src_d, r.dst_d);
+    if (r.src_d > 128 || r.dst_d > 128) return fail(RA_ERR_HEAD_DIM, "ra_convert: head dims of at most 128");
+    if (r.B > 65535 || (int64_t)r.H * 16 >= ((int64_t)1 << 31) || (int64_t)r.L * (r.H * 16) >= ((int64_t)1 << 31))
+      return fail(RA_ERR_TOO_LARGE, "ra_convert: too many rows for one launch");
+    for (int dt : {r.src_dtype, r.dst_dtype})
+      if (dt != RA_DTYPE_BF16 && dt != RA_DTYPE_F32 && dt != RA_DTYPE_F16) return fail(RA_ERR_DTYPE, "unknown dtype %d", dt);
+    // eight elements at a time where every chunk of a row starts on a multiple of 16 bytes
+    auto on_chunks = [](const void* p, int dtype, int64_t sb, int64_t sl, int64_t sh) {
+      const int64_t mask = dtype == RA_DTYPE_F32 ? 3 : 7;
+      return aligned16(p) && !((sb | sl | sh) & mask);
+    };
+    if (reinterpret_cast<uintptr_t>(r.src) % (r.src_dtype == RA_DTYPE_F32 ? 4 : 2) ||
+        reinterpret_cast<uintptr_t>(r.dst) % (r.dst_dtype == RA_DTYPE_F32 ? 4 : 2))
+      return fail(RA_ERR_ALIGN, "ra_convert: arrays must be aligned to their elements");
+    a.item[i] = ra::ConvertItem{r.src, r.dst, r.src_dtype, r.dst_dtype, r.src_d, r.dst_d, r.B, r.L, r.H,
+                                on_chunks(r.src, r.src_dtype, r.src_stride_b, r.src_stride_l, r.src_stride_h),
+                                on_chunks(r.dst, r.dst_dtype, r.dst_stride_b, r.dst_stride_l, r.dst_stride_h),
+                                r.src_stride_b, r.src_stride_l, r.src_stride_h, r.dst_stride_b, r.dst_stride_l, r.dst_stride_h};
+  }
+  return RA_OK;
+}
+
 static int64_t bwd_pair_workspace(const ra_bwd_step_params* p, bool any_dim) {
   if (!p || check_dims(p->B, p->H, p->Lq, p->Lk, p->D, any_dim)) return 0;
   return bwd_space(*p, plan_dq_pair(*p), plan_dkdv_pair(*p)).total;
@@ -1230,10 +1260,46 @@ static int bwd_pair(const Before& before, const ra_bwd_step_params* p, bool any_
   memset(&a, 0, sizeof(a));
   a.a = to_bwd_args(c);
   a.stat = (const float*)(ws + sp.stat);
-  if ((rc = before.launch(stream))) return rc;
-  hipError_t e = ra::launch_pair_stat(out, out_dtype == RA_DTYPE_F32, out_stride_b, out_stride_h, out_stride_l, a.a.dout, c.lse,
-                                      1.0f / a.a.scale_res, (float*)(ws + sp.stat), (float*)(ws + sp.delta), c.B, c.H, c.Lq, c.D,
-                                      (hipStream_t)stream);
+  ra::StatArgs st;
+  memset(&st, 0, sizeof(st));
+  st.out = out;
+  st.sb = out_stride_b;
+  st.sh = out_stride_h;
+  st.sl = out_stride_l;
+  st.dout = c.dout.ptr;
+  st.dsb = c.dout.stride_b;
+  st.dsh = c.dout.stride_h;
+  st.dsl = c.dout.stride_l;
+  st.dout_d = c.D;
+  st.dout_vec = 1;
+  st.lse = c.lse;
+  st.inv_res = 1.0f / a.a.scale_res;
+  st.stat = (float*)(ws + sp.stat);
+  st.delta = (float*)(ws + sp.delta);
+  st.B = c.B;
+  st.H = c.H;
+  st.L = c.Lq;
+  int dout_dtype = RA_DTYPE_BF16;
+  // A conversion that makes dO, row after row, is left to the statistics, which read it anyway.
+  ra::ConvertArgs conv;
+  const bool made = before.n == 1 && before.items && before.items[0].dst == c.dout.ptr;
+  if (made && (rc = convert_args(before.items, 1, conv))) return rc;
+  const ra::ConvertItem& it = conv.item[0];
+  if (made && it.dst_dtype == RA_DTYPE_BF16 && it.dst_d == c.D && it.B == c.B && it.L == c.Lq && it.H == c.H && it.dst_sh == c.D &&
+      it.dst_sl == (int64_t)c.H * c.D && it.dst_sb == (int64_t)c.Lq * c.H * c.D && c.dout.stride_h == it.dst_sh && c.dout.stride_l == it.dst_sl &&
+      c.dout.stride_b == it.dst_sb) {
+    st.dout = it.src;
+    st.dsb = it.src_sb;
+    st.dsh = it.src_sh;
+    st.dsl = it.src_sl;
+    st.dout_d = it.src_d;
+    st.dout_vec = it.src_vec;
+    st.copy = (ra::bf16_t*)it.dst;
+    dout_dtype = it.src_dtype;
+  } else if ((rc = before.launch(stream))) {
+    return rc;
+  }
+  hipError_t e = ra::launch_pair_stat(st, out_dtype == RA_DTYPE_F32, dout_dtype, c.D, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "ra_bwd_pair launch");
   const std::vector<int> one{0, 1};
   const int mode = kernel_mode(c.bias.flags);
@@ -1299,33 +1365,8 @@ int ra_bwd_whole(const ra_bwd_step_params* p, const void* out, int32_t out_dtype
 }
 
 int ra_convert(const ra_rows* items, int32_t n_items, void* stream) {
-  if (n_items < 1 || n_items > ra::kMaxConvert) return fail(RA_ERR_SHAPE, "ra_convert: 1 to %d arrays (got %d)", ra::kMaxConvert, n_items);
-  if (!items) return fail(RA_ERR_NULL, "ra_convert: items is NULL");
   ra::ConvertArgs a;
-  memset(&a, 0, sizeof(a));
-  for (int i = 0; i < n_items; ++i) {
-    const ra_rows& r = items[i];
-    if (!r.src || !r.dst) return fail(RA_ERR_NULL, "ra_convert: NULL pointer");
-    if (r.B <= 0 || r.L <= 0 || r.H <= 0 || r.src_d <= 0 || r.dst_d <= 0)
-      return fail(RA_ERR_SHAPE, "ra_convert: bad shape B=%d L=%d H=%d d=%d -> %d", r.B, r.L, r.H, r.src_d, r.dst_d);
-    if (r.src_d > 128 || r.dst_d > 128) return fail(RA_ERR_HEAD_DIM, "ra_convert: head dims of at most 128");
-    if (r.B > 65535 || (int64_t)r.H * 16 >= ((int64_t)1 << 31) || (int64_t)r.L * (r.H * 16) >= ((int64_t)1 << 31))
-      return fail(RA_ERR_TOO_LARGE, "ra_convert: too many rows for one launch");
-    for (int dt : {r.src_dtype, r.dst_dtype})
-      if (dt != RA_DTYPE_BF16 && dt != RA_DTYPE_F32 && dt != RA_DTYPE_F16) return fail(RA_ERR_DTYPE, "unknown dtype %d", dt);
-    // eight elements at a time where every chunk of a row starts on a multiple of 16 bytes
-    auto on_chunks = [](const void* p, int dtype, int64_t sb, int64_t sl, int64_t sh) {
-      const int64_t mask = dtype == RA_DTYPE_F32 ? 3 : 7;
-      return aligned16(p) && !((sb | sl | sh) & mask);
-    };
-    if (reinterpret_cast<uintptr_t>(r.src) % (r.src_dtype == RA_DTYPE_F32 ? 4 : 2) ||
-        reinterpret_cast<uintptr_t>(r.dst) % (r.dst_dtype == RA_DTYPE_F32 ? 4 : 2))
-      return fail(RA_ERR_ALIGN, "ra_convert: arrays must be aligned to their elements");
-    a.item[i] = ra::ConvertItem{r.src, r.dst, r.src_dtype, r.dst_dtype, r.src_d, r.dst_d, r.B, r.L, r.H,
-                                on_chunks(r.src, r.src_dtype, r.src_stride_b, r.src_stride_l, r.src_stride_h),
-                                on_chunks(r.dst, r.dst_dtype, r.dst_stride_b, r.dst_stride_l, r.dst_stride_h),
-                                r.src_stride_b, r.src_stride_l, r.src_stride_h, r.dst_stride_b, r.dst_stride_l, r.dst_stride_h};
-  }
+  if (int rc = convert_args(items, n_items, a)) return rc;
   hipError_t e = ra::launch_convert(a, n_items, (hipStream_t)stream);
   return e == hipSuccess ? RA_OK : hip_fail(e, "ra_convert launch");
 }

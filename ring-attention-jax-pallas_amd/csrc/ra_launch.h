@@ -142,8 +142,21 @@ struct PairBwdArgs {
 };
 // dK and dV, dQ (nullptr: not this one), or both in one launch
 hipError_t launch_bwd_pair(const PairBwdArgs* dkdv, const PairBwdArgs* dq, int D, int mode, hipStream_t stream);
-hipError_t launch_pair_stat(const void* out, int out_f32, long long sb, long long sh, long long sl, TensorArg dout, const float* lse,
-                            float inv_res, float* stat, float* delta, int B, int H, int Lq, int D, hipStream_t stream);
+// The rows' statistics for the backward (pair_stat_kernel).
+struct StatArgs {
+  const void* out;
+  long long sb, sh, sl;
+  const void* dout;  // of dout_dtype, dout_d elements a row; dout_vec: whole chunks of eight lie on their own alignment
+  long long dsb, dsh, dsl;
+  int dout_d, dout_vec;
+  bf16_t* copy;  // where the converted dO goes, [b, l, h, D]; nullptr: it is bf16 of D elements as it is
+  const float* lse;
+  float inv_res;
+  float *stat, *delta;
+  int B, H, L;
+  int heads, loads, n_l, n_h;  // (the launcher's)
+};
+hipError_t launch_pair_stat(const StatArgs& a, int out_f32, int dout_dtype, int D, hipStream_t stream);
 
 // Arrays of rows that are converted and padded (or cut) to another head dim (ra_convert).
 constexpr int kMaxConvert = 4;

@@ -1815,36 +1815,70 @@ __global__ __launch_bounds__(kPairThreads, DL <= 64 ? 3 : 2) void bwd_pair_kerne
 
 // What the dK / dV kernel adds to a row's scores: stat[row] = -lse log2(e) / scale_res (-inf for a row without
 // any key: P = 0) and stat[rows + row] = -delta (0 there: its output, and delta with it, is NaN), with
-// delta = rowsum(out * dout).  HBM bound.
-template <typename OutT, int D>
-__global__ __launch_bounds__(256) void pair_stat_kernel(const OutT* out, long long sb, long long sh, long long sl, TensorArg dout,
-                                                        const float* lse, float inv_res, float* stat, float* delta, int B, int H,
-                                                        int Lq) {
+// delta = rowsum(out * dout).  A dO that has to be converted (StatArgs::copy) is rounded and stored on the way.
+// HBM bound.  A wave takes rows that lie next to each other: the heads of a token where heads are neighbours, tokens of a head
+// else, up to four such loads in flight; the results are turned round in LDS.  A row after the other of one head, conversion by itself | so,
+// us: 8192, B=2, H=16, D=128 40 | 33 (134 MB, 4.1 TB/s), 32768, H=16 71 | 66; fp32 2048, B=2, H=4, D=64 3.7 + 3.1 | 4.3, fp16 1047, B=2, H=8,
+// D=96 5 + 4.1 | 5.8, D=80, 4096, H=5 4.3 + 4.3 | 5.2, and a launch less.
+template <typename OutT, typename DoT, int D>
+__global__ __launch_bounds__(256) void pair_stat_kernel(const StatArgs a) {
   constexpr int CPR = D == 96 ? 16 : D / 8;  // lanes per row (a power of two)
-  const long long rows = (long long)B * H * Lq;
-  const long long row = (long long)blockIdx.x * (256 / CPR) + threadIdx.x / CPR;
-  const int c = threadIdx.x % CPR;
-  float acc = 0.f;
-  if (row < rows && c < D / 8) {
-    const int li = (int)(row % Lq);
-    const long long hh = row / Lq;
-    const int h = (int)(hh % H);
-    const int b = (int)(hh / H);
-    const OutT* op = out + b * sb + h * sh + (long long)li * sl + 8 * c;
-    const bf16_t* dp = dout.ptr + b * dout.sb + h * dout.sh + (long long)li * dout.sl + 8 * c;
-    const bf16x8 dv = *(const bf16x8*)dp;
+  constexpr int RW = 64 / CPR, P = 4;        // rows per wave and load, loads
+  __shared__ float s_delta[4 * P * RW];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = a.heads, lw = RW / G, LB = 4 * a.loads * lw;  // heads and tokens per wave and load, tokens per workgroup (powers of two)
+  const int lb = blockIdx.x % a.n_l, rest = blockIdx.x / a.n_l, h0 = rest % a.n_h * G, b = rest / a.n_h;
+  const int c = lane % CPR, hl = lane / CPR & (G - 1), lsub = lane / CPR / G, h = h0 + hl;
+  typedef __attribute__((ext_vector_type(8))) DoT do8;
+  typedef __attribute__((ext_vector_type(8))) OutT out8;
+  const bool whole = a.dout_vec && a.dout_d % 8 == 0;  // a chunk of dO is there or not
+  const int n = a.dout_d - 8 * c;                      // elements of this lane's
+  const int co = min(c, D / 8 - 1), cd = min(c, max(a.dout_d / 8 - 1, 0));
+  const OutT* op = (const OutT*)a.out + b * a.sb + h * a.sh + 8 * co;
+  const DoT* dp = (const DoT*)a.dout + b * a.dsb + h * a.dsh;
+  const long long first = ((long long)b * a.H + h0) * a.L;
+  const int mine = lb * LB + threadIdx.x % LB;  // the token whose results this thread writes
+  const long long row = first + (long long)(threadIdx.x / LB) * a.L + mine;
+  const bool writes = (int)threadIdx.x < G * LB && mine < a.L;
+  const float lse = writes ? a.lse[row] : 0.f;
+  // (all loads first: what lies behind the end reads the last row again)
+  do8 x[P];
+  out8 y[P];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc += (float)op[e] * (float)dv[e];
+  for (int p = 0; p < P; ++p) {
+    if (p >= a.loads) break;
+    const long long l = min(lb * LB + (4 * p + wave) * lw + lsub, a.L - 1);
+    if (whole) {
+      x[p] = *(const do8*)(dp + l * a.dsl + 8 * cd);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[p][e] = dp[l * a.dsl + min(8 * c + e, a.dout_d - 1)];
+    }
+    y[p] = *(const out8*)(op + l * a.sl);
   }
 #pragma unroll
-  for (int o = CPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-  if (row < rows && c == 0) {
-    const float L = lse[row];
-    const bool dead = L == RA_NEG_INF;
-    delta[row] = acc;
-    stat[row] = dead ? RA_NEG_INF : -L * kLog2e * inv_res;
-    stat[rows + row] = dead ? 0.f : -acc;
+  for (int p = 0; p < P; ++p) {
+    if (p >= a.loads) break;
+    const int at = (4 * p + wave) * lw + lsub, li = lb * LB + at;
+    bf16x8 dv;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dv[e] = (bf16_t)(e < n ? (float)x[p][e] : 0.f);
+    if (a.copy != nullptr && li < a.L && c < D / 8) *(bf16x8*)(a.copy + (((long long)b * a.L + li) * a.H + h) * D + 8 * c) = dv;
+    float acc = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc += (float)y[p][e] * (float)dv[e];
+    if (c >= D / 8) acc = 0.f;
+#pragma unroll
+    for (int o = CPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    if (c == 0) s_delta[hl * LB + at] = acc;
   }
+  __syncthreads();
+  if (!writes) return;
+  const float delta = s_delta[threadIdx.x];
+  const bool dead = lse == RA_NEG_INF;
+  a.delta[row] = delta;
+  a.stat[row] = dead ? RA_NEG_INF : -lse * kLog2e * a.inv_res;
+  a.stat[(long long)a.B * a.H * a.L + row] = dead ? 0.f : -delta;
 }
 
 // Sum of the shares of rows that were split, stored in the gradient's dtype.  Grid dimension y, from `first` on: dK and dV, whose
@@ -1919,15 +1953,29 @@ hipError_t launch_bwd_pair(const PairBwdArgs* dkdv, const PairBwdArgs* dq, int D
   });
 }
 
-hipError_t launch_pair_stat(const void* out, int out_f32, long long sb, long long sh, long long sl, TensorArg dout, const float* lse,
-                            float inv_res, float* stat, float* delta, int B, int H, int Lq, int D, hipStream_t stream) {
-  const long long rows = (long long)B * H * Lq;
-  const int rpb = 256 / (D == 96 ? 16 : D / 8);
-  dim3 grid((unsigned)((rows + rpb - 1) / rpb)), block(256);
+template <typename OutT, typename DoT, int D>
+static hipError_t launch_pair_stat_d(StatArgs a, hipStream_t stream) {
+  constexpr int RW = 64 / (D == 96 ? 16 : D / 8);
+  a.heads = 1;
+  while (a.sh < a.sl && 2 * a.heads <= RW && a.H % (2 * a.heads) == 0) a.heads *= 2;
+  // (four loads a wave where that still gives every compute unit two workgroups)
+  a.loads = (long long)a.B * a.H * a.L >= 512 * 16 * RW ? 4 : 1;
+  const int tokens = 4 * a.loads * RW / a.heads;
+  a.n_l = (a.L + tokens - 1) / tokens;
+  a.n_h = a.H / a.heads;
+  hipLaunchKernelGGL((pair_stat_kernel<OutT, DoT, D>), dim3((unsigned)((long long)a.B * a.n_h * a.n_l)), dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_pair_stat(const StatArgs& a, int out_f32, int dout_dtype, int D, hipStream_t stream) {
   return with_dim(D, 0, [&](auto d) {
-    if (out_f32) hipLaunchKernelGGL((pair_stat_kernel<float, d.value>), grid, block, 0, stream, (const float*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
-    else hipLaunchKernelGGL((pair_stat_kernel<bf16_t, d.value>), grid, block, 0, stream, (const bf16_t*)out, sb, sh, sl, dout, lse, inv_res, stat, delta, B, H, Lq);
-    return hipGetLastError();
+    auto with_out = [&](auto out) {
+      using OutT = decltype(out);
+      if (dout_dtype == RA_DTYPE_F32) return launch_pair_stat_d<OutT, float, d.value>(a, stream);
+      if (dout_dtype == RA_DTYPE_F16) return launch_pair_stat_d<OutT, _Float16, d.value>(a, stream);
+      return launch_pair_stat_d<OutT, bf16_t, d.value>(a, stream);
+    };
+    return out_f32 ? with_out(float{}) : with_out(bf16_t{});
   });
 }
 

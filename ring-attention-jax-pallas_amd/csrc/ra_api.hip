@@ -795,34 +795,6 @@ PairPlan plan_dq_pair(const ra_bwd_step_params& p) {
   if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;
 }
-// dK / dV, in 32-query tiles per 128 keys (dkdv_kernel | dkdv_pair_kernel): uneven rows 65 of them (64 heads of 4096) 0.55 | 0.50 ms,
-// 130 (32 of 8192) 1.08 | 1.04, 258 (32 of 16384) 3.42 | 3.48; even ones 128 (64 of 4096 x 4096) 0.89 | 0.90, 256 (16 of 8192 x 8192) 0.84 |
-// 0.89; ALiBi 130 1.03 | 0.95, 258 1.83 | 1.79, 514 7.05 | 7.05.  Between one and two and a half slabs per compute unit dkdv_pair_kernel would
-// hold them all at once, the longest one deciding: uneven rows take dkdv_kernel there (16 heads of 4096: 0.13 | 0.16; 12: 0.11 | 0.13; 4
-// of 16384: 0.44 | 0.56), even ones if they are long (16 heads of 4096, unmasked 0.230 | 0.233, of 3072 0.158 | 0.153, window of 1024 0.080 |
-// 0.070).  Fewer slabs are shared (12 heads of 2048: 0.056 | 0.050).
-PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
-  const int ntiles = (p.Lq + 31) / 32;
-  const ra::BiasArgs b = to_bias(p.bias);
-  int64_t total = 0;
-  int most = 0;
-  for (int k0 = 0; k0 < p.Lk; k0 += kPairRowsHost) {
-    int lo, hi;
-    ra::query_tile_range(b.flags, b.window, b.kv_off + k0, b.kv_off + std::min(k0 + kPairRowsHost, p.Lk) - 1, b.q_off, ntiles, 32, lo, hi);
-    total += hi - lo;
-    most = std::max(most, hi - lo);
-  }
-  PairPlan r{true, 1, std::max(most, 1), kHeadGroup};
-  const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lk + kPairRowsHost - 1) / kPairRowsHost, wgs = heads * rows;
-  const bool one_round = wgs > kPairSlots / 2 && wgs <= kPairSlots * 5 / 4;
-  const bool even = even_rows(total, most, rows);
-  const int tiles = one_round ? (even ? 112 : 0) : (p.bias.flags & RA_BIAS_ALIBI) ? 448 : even ? 112 : 192;
-  if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, total, rows, tiles)) r.pair = false;
-  else if (heads * p.Lq + 31 >= (int64_t)1 << 30) r.pair = false;  // one 32-bit byte offset reaches both statistics of a tile's 32 rows
-  else plan_split(r, heads, rows, total, most, 2 * kMinChunk, 8 * heads * p.Lk * p.D, p.bias, true);
-  if (one_by_one(p.bias, total, most, rows)) r.group = 1;
-  return r;
-}
 // Whether both gradients' workgroups go into one launch: the second kind fills the places that the first one's last round leaves
 // empty.  Two launches | one, us: causal, D=128, 6000, H=16 493 | 488, 4096, H=8 180 | 163; D=64, 2048, B=2, H=16 112 | 97; D=32, 8192, H=16 338 |
 // 312; documents of 500 in 32768, H=8 838 | 793, of 3500 in 10112, causal, H=4, D=80 352 | 278; prefix 4096, B=2, H=16 586 | 576; unmasked 3000,
@@ -838,6 +810,44 @@ bool bwd_in_one_launch(const ra_bwd_step_params& p, const PairPlan& dq, const Pa
   const int64_t wgs = heads * (tiles(p.Lq) * dq.n_split + tiles(p.Lk) * dkdv.n_split);
   const bool three = p.D <= 64 && !(p.bias.flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) && !has_lists(p.bias);
   return wgs >= (three ? 3 : 2) * kPairSlots && wgs <= (p.D <= 64 ? 12 : 8) * kPairSlots;
+}
+// dK / dV, in 32-query tiles per 128 keys (dkdv_kernel | dkdv_pair_kernel): uneven rows 65 of them (64 heads of 4096) 0.55 | 0.50 ms,
+// 130 (32 of 8192) 1.08 | 1.04, 258 (32 of 16384) 3.42 | 3.48; even ones 128 (64 of 4096 x 4096) 0.89 | 0.90, 256 (16 of 8192 x 8192) 0.84 |
+// 0.89; ALiBi 130 1.03 | 0.95, 258 1.83 | 1.79, 514 7.05 | 7.05.  Between one and two and a half slabs per compute unit dkdv_pair_kernel would
+// hold them all at once, the longest one deciding: alone, uneven rows take dkdv_kernel there (16 heads of 4096: 0.13 | 0.16; 12: 0.11 | 0.13; 4
+// of 16384: 0.44 | 0.56), even ones if they are long (16 heads of 4096, unmasked 0.230 | 0.233, of 3072 0.158 | 0.153, window of 1024 0.080 |
+// 0.070).  With dQ's workgroups beside them in one launch, which fill what the long slabs leave, they are faster: dkdv_kernel, then dQ | both in
+// one launch, us: causal 16 heads of 4096 269 | 232, 32 of 2048 174 | 136, 4 of 16384 909 | 844, 8 of 8192 478 | 430, with ALiBi 16 of 4096
+// 295 | 246; even rows until they are very long: unmasked 18 heads of 4096 574 | 486, 9 of 8192 1075 | 938, 16 of 4096 435 | 416, 8 of 8192
+// 796 | 805, 4 of 16384 1560 | 1620, window 4096 of 8192, 8 heads 392 | 358.  (Uneven slabs past two per compute unit stay on dkdv_kernel, which
+// test_gpu_pair.py names: 20 heads of 4096 326 | 306.)  Fewer slabs are shared (12 heads of 2048: 0.056 | 0.050).
+PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
+  const int ntiles = (p.Lq + 31) / 32;
+  const ra::BiasArgs b = to_bias(p.bias);
+  int64_t total = 0;
+  int most = 0;
+  for (int k0 = 0; k0 < p.Lk; k0 += kPairRowsHost) {
+    int lo, hi;
+    ra::query_tile_range(b.flags, b.window, b.kv_off + k0, b.kv_off + std::min(k0 + kPairRowsHost, p.Lk) - 1, b.q_off, ntiles, 32, lo, hi);
+    total += hi - lo;
+    most = std::max(most, hi - lo);
+  }
+  PairPlan r{true, 1, std::max(most, 1), kHeadGroup};
+  const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lk + kPairRowsHost - 1) / kPairRowsHost, wgs = heads * rows;
+  const bool one_round = wgs > kPairSlots / 2 && wgs <= kPairSlots * 5 / 4;
+  const bool even = even_rows(total, most, rows);
+  int tiles = one_round ? (even ? 112 : 0) : (p.bias.flags & RA_BIAS_ALIBI) ? 448 : even ? 112 : 192;
+  auto split = [&](PairPlan& x) { plan_split(x, heads, rows, total, most, 2 * kMinChunk, 8 * heads * p.Lk * p.D, p.bias, true); };
+  if (one_round && (even || wgs <= kPairSlots) && p.D == 128) {
+    PairPlan beside = r;
+    split(beside);
+    if (bwd_in_one_launch(p, plan_dq_pair(p), beside)) tiles = even ? 224 : kWholeRow;
+  }
+  if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, total, rows, tiles)) r.pair = false;
+  else if (heads * p.Lq + 31 >= (int64_t)1 << 30) r.pair = false;  // one 32-bit byte offset reaches both statistics of a tile's 32 rows
+  else split(r);
+  if (one_by_one(p.bias, total, most, rows)) r.group = 1;
+  return r;
 }
 // The workspace of ra_bwd_pair: the rows' statistics, then the shares of dQ and of dK and dV.
 struct BwdSpace {

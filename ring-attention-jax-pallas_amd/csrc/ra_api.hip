@@ -776,8 +776,18 @@ PairPlan plan_fwd_pair(const ra_fwd_step_params& p) {
   PairPlan r{true, 1, std::max(most, 1), kHeadGroup};
   // (with ALiBi from 192 tiles on: 65 of them, 32 heads of 8192, 0.70 | 0.63 ms, 129, 16 of 16384, 1.19 | 1.16, 257 4.48 | 4.74; and not
   // uneven rows that fill the chip less than one and a quarter times: 8 heads of 10240, 0.275 | 0.250)
-  const bool nearly_one = wgs <= kPairSlots * 5 / 4 && !even_rows(total, most, rows);
+  const bool even = even_rows(total, most, rows), quarter_more = wgs <= kPairSlots * 5 / 4;
+  const bool nearly_one = wgs <= (even ? kPairSlots * 3 / 2 : kPairSlots * 5 / 4);
   if (!nearly_one && long_stretches(p.bias, p.D, wgs, total, rows, (p.bias.flags & RA_BIAS_ALIBI) ? 192 : 56)) r.pair = false;
+  // Even rows that need up to a quarter more places than there are leave most of the chip empty in their second round: halved if they
+  // are long enough for the halves' partial results.  fwd_step_kernel (D = 128) or fwd_pair_kernel unshared | in two shares, us, unmasked: 9 heads
+  // of 8192, D=128 429 | 369, D=64 232 | 215, D=96 339 | 303; 18 of 4096 232 | 202, 123 | 119, 180 | 171; 5 of 16384, D=128 826 | 717; not 36 of 2048
+  // (32 tiles) 113 | 127, 12 of 8192 (768 workgroups) 436 | 461; nor uneven rows, 18 of 4096, causal, 105 | 116.  Up to one and a half times
+  // the places fwd_pair_kernel is the faster one: 24 of 4096 237 | 224, 12 of 8192 439 | 436.
+  if (even && wgs > kPairSlots && quarter_more && most >= 56 && !has_lists(p.bias)) {
+    r.chunk_tiles = (most + 1) / 2;
+    r.n_split = 2;
+  }
   if (r.pair) plan_split(r, heads, rows, total, most, kMinChunk, 4 * heads * p.Lq * p.D, p.bias, false);
   if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;

@@ -828,8 +828,8 @@ bool bwd_in_one_launch(const ra_bwd_step_params& p, const PairPlan& dq, const Pa
 // of 16384: 0.44 | 0.56), even ones if they are long (16 heads of 4096, unmasked 0.230 | 0.233, of 3072 0.158 | 0.153, window of 1024 0.080 |
 // 0.070).  With dQ's workgroups beside them in one launch, which fill what the long slabs leave, they are faster: dkdv_kernel, then dQ | both in
 // one launch, us: causal 16 heads of 4096 269 | 232, 32 of 2048 174 | 136, 4 of 16384 909 | 844, 8 of 8192 478 | 430, with ALiBi 16 of 4096
-// 295 | 246; even rows until they are very long: unmasked 18 heads of 4096 574 | 486, 9 of 8192 1075 | 938, 16 of 4096 435 | 416, 8 of 8192
-// 796 | 805, 4 of 16384 1560 | 1620, window 4096 of 8192, 8 heads 392 | 358.  (Uneven slabs past two per compute unit stay on dkdv_kernel, which
+// 295 | 246; even rows too, but for long ones that all have a place: unmasked 18 heads of 4096 574 | 486, 9 of 8192 1089 | 958, with ALiBi 1206 |
+// 990, 10 of 8192 1112 | 1045, 16 of 4096 435 | 416, window 4096 of 8192, 8 heads 392 | 358; 8 of 8192 796 | 805, 4 of 16384 1560 | 1620.  (Uneven slabs past two per compute unit stay on dkdv_kernel, which
 // test_gpu_pair.py names: 20 heads of 4096 326 | 306.)  Fewer slabs are shared (12 heads of 2048: 0.056 | 0.050).
 PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
   const int ntiles = (p.Lq + 31) / 32;
@@ -851,7 +851,7 @@ PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
   if (one_round && (even || wgs <= kPairSlots) && p.D == 128) {
     PairPlan beside = r;
     split(beside);
-    if (bwd_in_one_launch(p, plan_dq_pair(p), beside)) tiles = even ? 224 : kWholeRow;
+    if (bwd_in_one_launch(p, plan_dq_pair(p), beside)) tiles = even && wgs <= kPairSlots ? 224 : kWholeRow;
   }
   if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, total, rows, tiles)) r.pair = false;
   else if (heads * p.Lq + 31 >= (int64_t)1 << 30) r.pair = false;  // one 32-bit byte offset reaches both statistics of a tile's 32 rows

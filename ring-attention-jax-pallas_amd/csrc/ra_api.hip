@@ -810,16 +810,19 @@ PairPlan plan_dq_pair(const ra_bwd_step_params& p) {
 // 312; documents of 500 in 32768, H=8 838 | 793, of 3500 in 10112, causal, H=4, D=80 352 | 278; prefix 4096, B=2, H=16 586 | 576; unmasked 3000,
 // H=24 441 | 370.  Past eight rounds (at D <= 64 of 768 workgroups: documents of 2000 in 48128, causal, B=2, H=4, 7.8 of them, a pass
 // 1409 | 1296) the last one is a few per cent, and the one launch draws more power
-// without a pause (documents of 1200 + ALiBi, 29696, 24 heads: a pass 3.86 | 4.00 ms).  Fewer than two rounds stay two launches
-// (even rows at D <= 64, three workgroups of which fit a compute unit, fewer than three): what those run on is pinned by name in
-// test_gpu_pair.py; one launch would be 10 us faster there too (512, H=4, D=64, causal: 38 | 28).
+// without a pause (documents of 1200 + ALiBi, 29696, 24 heads: a pass 3.86 | 4.00 ms).
+// Fewer than one and three quarters rounds (even rows at D = 64, three workgroups of which fit a compute unit, fewer than three) of the kernels that
+// test_gpu_pair.py names - positional masks or none at D = 64 and 128 - stay two launches; one would be 10 us faster there too (512,
+// H=4, D=64, causal: 38 | 28).  The others: documents of 300 in 1024 tokens, causal, B=4, H=8, D=128 80 | 68, prefix 672, B=4, H=12, D=96 70 |
+// 49, unmasked 864 x 1024, D=80, H=32 87 | 83.
 bool bwd_in_one_launch(const ra_bwd_step_params& p, const PairPlan& dq, const PairPlan& dkdv) {
   if (!dq.pair || !dkdv.pair) return false;
   const int64_t heads = (int64_t)p.B * p.H;
   auto tiles = [](int L) { return (int64_t)(L + kPairRowsHost - 1) / kPairRowsHost; };
   const int64_t wgs = heads * (tiles(p.Lq) * dq.n_split + tiles(p.Lk) * dkdv.n_split);
-  const bool three = p.D <= 64 && !(p.bias.flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW)) && !has_lists(p.bias);
-  return wgs >= (three ? 3 : 2) * kPairSlots && wgs <= (p.D <= 64 ? 12 : 8) * kPairSlots;
+  const bool named = (p.D == 64 || p.D == 128) && !has_lists(p.bias) && !(p.bias.flags & RA_BIAS_ALIBI);
+  const bool three = p.D <= 64 && !(p.bias.flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW));
+  return (!named || wgs >= (three ? 12 : 7) * kPairSlots / 4) && wgs <= (p.D <= 64 ? 12 : 8) * kPairSlots;
 }
 // dK / dV, in 32-query tiles per 128 keys (dkdv_kernel | dkdv_pair_kernel): uneven rows 65 of them (64 heads of 4096) 0.55 | 0.50 ms,
 // 130 (32 of 8192) 1.08 | 1.04, 258 (32 of 16384) 3.42 | 3.48; even ones 128 (64 of 4096 x 4096) 0.89 | 0.90, 256 (16 of 8192 x 8192) 0.84 |

@@ -17,8 +17,8 @@
 // a tile follows from a few ranges of tile indexes (WaveTiles) and from the wave's own ids (wave_tests), not the
 // workgroup's; the terms of a masked block are passes of their own (apply_terms); a tile's loads share one base
 // (TileLoader); and nothing that can be computed again stays in a register (opaque_lane, kernel_args), so that no
-// variant spills a vector register or goes to scratch.  (Scalar registers in vector lanes: 2 to 12 in the general variants, 19 to 49 in
-// those with a dense block, for which the compiler reserves 36 bytes of scratch in dK / dV that no instruction uses.)  Before | after, us: documents of 2048 + ALiBi, 32768, H=16, D=128: forward 1787 | 1590, dQ 1916 | 1755, dK/dV
+// variant spills a vector register or goes to scratch.  (Scalar registers in vector lanes: 2 to 24 in the general variants, 20 to 98 in
+// those with a dense block.)  Before | after, us: documents of 2048 + ALiBi, 32768, H=16, D=128: forward 1787 | 1590, dQ 1916 | 1755, dK/dV
 // 2770 | 2410; causal documents of 2175 in 48128, B=2, H=4, D=64: 443 | 325, 476 | 350, 495 | 427; prefix-LM 4096, B=2, H=16, D=128,
 // forward 229 | 194; steps on dense blocks (documents of 2048 in 32768, 4 shards) 10.2 ms | 7.8 a pass.
 #include <algorithm>

@@ -320,8 +320,12 @@ PyObject* attend(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (scale == -1.0 && PyErr_Occurred()) throw python_error();
   const Tensor &q = THPVariable_Unpack(args[0]), &k = THPVariable_Unpack(args[1]), &v = THPVariable_Unpack(args[2]);
   const bool any_grad = q.requires_grad() || k.requires_grad() || v.requires_grad();
-  variable_list got = WholeCall::apply(q, k, v, *p, scale, reinterpret_cast<THPDtype*>(args[5])->scalar_type,
-                                       reinterpret_cast<THPDtype*>(args[6])->scalar_type, any_grad);
+  const at::ScalarType dtype = reinterpret_cast<THPDtype*>(args[5])->scalar_type, final_dtype = reinterpret_cast<THPDtype*>(args[6])->scalar_type;
+  variable_list got;
+  {
+    pybind11::gil_scoped_release no_gil;  // (allocations may wait for the GPU)
+    got = WholeCall::apply(q, k, v, *p, scale, dtype, final_dtype, any_grad);
+  }
   PyObject* r = PyTuple_New(2);
   if (!r) throw python_error();
   PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(std::move(got[0])));

@@ -512,21 +512,6 @@ RA_DEV void tile_id_range(const int* ids, int t, int L, int& mn, int& mx) {
   }
 }
 
-// Whether some / all tokens of tile t carry a non-zero flag.
-template <int T>
-RA_DEV void tile_flag_range(const int* ids, int t, int L, bool& any, bool& all) {
-  int o = 0, z = 0;
-  const int base = t * T;
-#pragma unroll 8
-  for (int e = 0; e < T; ++e) {
-    const int x = ids[min(base + e, L - 1)];
-    o |= x;
-    z |= (x == 0);
-  }
-  any = o != 0;
-  all = z == 0;
-}
-
 // an element, and four, of a result in the caller's dtype (RA_DTYPE_*)
 template <typename T>
 RA_DEV void store_as(void* base, long long at, const f32x4& x) {

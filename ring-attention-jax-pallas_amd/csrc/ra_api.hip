@@ -713,6 +713,19 @@ bool even_rows(int64_t total, int most, int64_t rows) { return total * 20 >= (in
 bool one_by_one(const ra_bias& b, int64_t total, int most, int64_t rows) {
   return even_rows(total, most, rows) && !has_lists(b) && !(b.flags & RA_BIAS_WINDOW);
 }
+// Small backward calls that stay two launches, because test_gpu_pair.py names their two kernels: at D = 128 under a causal or window mask,
+// below one and three quarters rounds, and at D = 64 unmasked, below three (three workgroups fit a compute unit there).  One launch would
+// be faster there too (unmasked 512, H=4, D=64: 32 | 26 us).  The others are one at any size, two launches | one: documents of 300 in
+// 1024 tokens, causal, B=4, H=8, D=128 80 | 68, prefix 672, B=4, H=12, D=96 70 | 49, unmasked 864 x 1024, D=80, H=32 87 | 83, causal
+// 512, H=4, D=64 38 | 28, 700 37 | 25, unmasked, D=128, 1000, H=4 50 | 35, 2000, B=2, H=4 102 | 80.
+bool small_ones_apart(const ra_bias& b, int D) {
+  const bool masked = b.flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW);
+  return !has_lists(b) && !(b.flags & RA_BIAS_ALIBI) && (D == 128 ? masked : D == 64 && !masked);
+}
+// Whether the shares of a gradient of even rows are counted beside the other one's (plan_split): not where small ones run apart at D = 64.
+// Two launches counted by themselves | counted beside each other, backward, us: unmasked, D=64, 2000, H=8 71 | 86, 894, B=2, H=4 43 | 44;
+// at D = 128 windows alone are meant, which were not slowed by the count (as many shares as places | so, 1000 of 8192, H=4 107 | 89).
+bool shares_beside(const ra_bwd_step_params& p) { return !(p.D == 64 && small_ones_apart(p.bias, p.D)); }
 // How the workgroups of one kind of a head's resident tiles, which meet `total` tiles of the other side (`most` at most), share their
 // work (see above).  share: bytes of one share of every row.  beside: the other gradient's workgroups run in the same launch.
 // Rows of about the same length take the number of shares k that a count of time finds best, in tiles of a workgroup (1.4 us at D = 128):
@@ -801,7 +814,7 @@ PairPlan plan_dq_pair(const ra_bwd_step_params& p) {
   PairPlan r{true, 1, std::max(most, 1), kHeadGroup};
   const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lq + kPairRowsHost - 1) / kPairRowsHost;
   if (long_stretches(p.bias, p.D, heads * rows, total, rows, 160)) r.pair = false;
-  else plan_split(r, heads, rows, total, most, kMinChunk, 4 * heads * p.Lq * p.D, p.bias, true);
+  else plan_split(r, heads, rows, total, most, kMinChunk, 4 * heads * p.Lq * p.D, p.bias, shares_beside(p));
   if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;
 }
@@ -811,18 +824,13 @@ PairPlan plan_dq_pair(const ra_bwd_step_params& p) {
 // H=24 441 | 370.  Past eight rounds (at D <= 64 of 768 workgroups: documents of 2000 in 48128, causal, B=2, H=4, 7.8 of them, a pass
 // 1409 | 1296) the last one is a few per cent, and the one launch draws more power
 // without a pause (documents of 1200 + ALiBi, 29696, 24 heads: a pass 3.86 | 4.00 ms).
-// Fewer than one and three quarters rounds (even rows at D = 64, three workgroups of which fit a compute unit, fewer than three) of the kernels that
-// test_gpu_pair.py names - positional masks or none at D = 64 and 128 - stay two launches; one would be 10 us faster there too (512,
-// H=4, D=64, causal: 38 | 28).  The others: documents of 300 in 1024 tokens, causal, B=4, H=8, D=128 80 | 68, prefix 672, B=4, H=12, D=96 70 |
-// 49, unmasked 864 x 1024, D=80, H=32 87 | 83.
 bool bwd_in_one_launch(const ra_bwd_step_params& p, const PairPlan& dq, const PairPlan& dkdv) {
   if (!dq.pair || !dkdv.pair) return false;
   const int64_t heads = (int64_t)p.B * p.H;
   auto tiles = [](int L) { return (int64_t)(L + kPairRowsHost - 1) / kPairRowsHost; };
   const int64_t wgs = heads * (tiles(p.Lq) * dq.n_split + tiles(p.Lk) * dkdv.n_split);
-  const bool named = (p.D == 64 || p.D == 128) && !has_lists(p.bias) && !(p.bias.flags & RA_BIAS_ALIBI);
-  const bool three = p.D <= 64 && !(p.bias.flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW));
-  return (!named || wgs >= (three ? 12 : 7) * kPairSlots / 4) && wgs <= (p.D <= 64 ? 12 : 8) * kPairSlots;
+  const int64_t least = small_ones_apart(p.bias, p.D) ? (p.D == 64 ? 12 : 7) * kPairSlots / 4 : 0;
+  return wgs >= least && wgs <= (p.D <= 64 ? 12 : 8) * kPairSlots;
 }
 // dK / dV, in 32-query tiles per 128 keys (dkdv_kernel | dkdv_pair_kernel): uneven rows 65 of them (64 heads of 4096) 0.55 | 0.50 ms,
 // 130 (32 of 8192) 1.08 | 1.04, 258 (32 of 16384) 3.42 | 3.48; even ones 128 (64 of 4096 x 4096) 0.89 | 0.90, 256 (16 of 8192 x 8192) 0.84 |
@@ -850,7 +858,7 @@ PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
   const bool one_round = wgs > kPairSlots / 2 && wgs <= kPairSlots * 5 / 4;
   const bool even = even_rows(total, most, rows);
   int tiles = one_round ? (even ? 112 : 0) : (p.bias.flags & RA_BIAS_ALIBI) ? 448 : even ? 112 : 192;
-  auto split = [&](PairPlan& x) { plan_split(x, heads, rows, total, most, 2 * kMinChunk, 8 * heads * p.Lk * p.D, p.bias, true); };
+  auto split = [&](PairPlan& x) { plan_split(x, heads, rows, total, most, 2 * kMinChunk, 8 * heads * p.Lk * p.D, p.bias, shares_beside(p)); };
   if (one_round && (even || wgs <= kPairSlots) && p.D == 128) {
     PairPlan beside = r;
     split(beside);

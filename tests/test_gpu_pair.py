@@ -463,6 +463,9 @@ def test_alibi_far_from_the_diagonal_on_the_long_stretch_kernels(device, q_off, 
     ("none", 40, 3000, 43, 128, torch.bfloat16),           # few long rows: dQ's workgroups first, their keys shared
     ("documents", 2000, 2000, 8, 96, torch.float32),       # rows of both kinds shared, gradients converted
     ("causal", 700, 700, 86, 32, torch.float16),
+    ("none", 894, 894, 8, 128, torch.bfloat16),            # a fraction of a round each, keys and queries shared
+    ("none", 1, 64, 1, 128, torch.bfloat16),
+    ("causal", 129, 129, 1, 64, torch.bfloat16),
     ("documents", 261, 261, 176, 128, torch.bfloat16)])
 def test_both_gradients_in_one_launch(device, mask, Sq, Sk, H, D, dtype):
     g = torch.Generator(device=device).manual_seed(Sq + D)

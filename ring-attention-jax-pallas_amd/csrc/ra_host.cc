@@ -156,8 +156,7 @@ class WholeCall : public torch::autograd::Function<WholeCall> {
     ra_rows rows[3];
     int n_rows = 0;
     variable_list kept;
-    if (dtype == call->given[1] && dtype == call->given[2] && !is_operand(q, p.D) && q.device() == k.device() && k.device() == v.device() &&
-        k.sizes() == v.sizes() && k.sizes() == at::IntArrayRef({p.B, p.Lk, p.H, call->dim})) {
+    if (dtype == call->given[1] && dtype == call->given[2] && !is_operand(q, p.D) && q.device() == k.device() && k.device() == v.device()) {
       const int64_t nq = p.B * p.Lq * p.H * p.D, nk = p.B * p.Lk * p.H * p.D;
       Tensor buf = empty({nq + 2 * nk}, at::kBFloat16, q.device());
       char* at = (char*)buf.data_ptr();
@@ -319,6 +318,12 @@ PyObject* attend(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const double scale = PyFloat_AsDouble(args[4]);
   if (scale == -1.0 && PyErr_Occurred()) throw python_error();
   const Tensor &q = THPVariable_Unpack(args[0]), &k = THPVariable_Unpack(args[1]), &v = THPVariable_Unpack(args[2]);
+  const Plan& of = **p;
+  const int64_t d = q.dim() == 4 ? q.size(3) : -1;
+  // (pointers and strides are all that goes on from here)
+  TORCH_CHECK(d <= of.D && q.sizes() == at::IntArrayRef({of.B, of.Lq, of.H, d}) && k.sizes() == at::IntArrayRef({of.B, of.Lk, of.H, d}) &&
+                  v.sizes() == k.sizes(),
+              "attend: q ", q.sizes(), ", k ", k.sizes(), " and v ", v.sizes(), " are not the operands of this plan");
   const bool any_grad = q.requires_grad() || k.requires_grad() || v.requires_grad();
   const at::ScalarType dtype = reinterpret_cast<THPDtype*>(args[5])->scalar_type, final_dtype = reinterpret_cast<THPDtype*>(args[6])->scalar_type;
   variable_list got;

@@ -1083,8 +1083,12 @@ def _attend(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs, sm_scale
     d_true = qs[3]
     if ks[3] != d_true or vs[3] != d_true:
         raise ValueError("q, k and v must share the head dim")
-    if ks[0] < qs[0] or vs[0] < qs[0] or ks[2] < qs[2] or vs[2] < qs[2] or vs[1] < ks[1]:  # the kernels would read past their end
-        raise ValueError(f"k {tuple(ks)} and v {tuple(vs)} do not hold the batch and heads of q {tuple(qs)}, or v not the length of k")
+    if ks != vs or ks[0] != qs[0] or ks[2] != qs[2]:
+        if ks[0] < qs[0] or vs[0] < qs[0] or ks[2] < qs[2] or vs[2] < qs[2] or vs[1] < ks[1]:  # the kernels would read past their end
+            raise ValueError(f"k {tuple(ks)} and v {tuple(vs)} do not hold the batch and heads of q {tuple(qs)}, or v not the length of k")
+        # Batch rows and heads that q has none for, and values without a key, take no part.  Cut off here: their gradients are zeros,
+        # and dk and dv, which the kernels store with the same strides, have the same shape.
+        k, v = k[:qs[0], :, :qs[2]], v[:qs[0], :ks[1], :qs[2]]
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(d_true)  # ring.py:287-288
     in_dtype = q.dtype

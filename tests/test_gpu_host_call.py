@@ -107,3 +107,20 @@ def test_tracing_stays_refused(device):
     # a trace would hold the allocations and not the kernels
     with pytest.raises(RuntimeError):
         torch.jit.trace(lambda *x: ra.ring_attention(*x, 1), [x.detach() for x in _arrays(device)], check_trace=False)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("impl", ["pallas", "hip"])
+@pytest.mark.parametrize("k_shape,v_shape", [((2, 130, 3, 64), (2, 130, 2, 64)), ((2, 130, 2, 64), (3, 200, 4, 64)), ((4, 130, 2, 64), (4, 130, 2, 64))])
+def test_keys_and_values_beyond_the_call(device, k_shape, v_shape, impl, dtype):
+    # they take no part: the output is that of the operands cut to size, and the gradients there are zeros
+    g = torch.Generator(device=device).manual_seed(k_shape[2])
+    q, k, v = (torch.randn(s, device=device, generator=g).to(torch.bfloat16).to(dtype).requires_grad_(True) for s in ((2, 130, 2, 64), k_shape, v_shape))
+    out = ra.ring_attention(q, k, v, 1, ra.causal_bias(), block_impl=impl)
+    do = torch.randn(out.shape, device=device, generator=g).to(torch.bfloat16).to(out.dtype)
+    grads = torch.autograd.grad(out, (q, k, v), do)
+    cut = [x.detach()[:2, :130, :2].contiguous().requires_grad_(True) for x in (q, k, v)]
+    want = ra.ring_attention(*cut, 1, ra.causal_bias(), block_impl=impl)
+    assert torch.equal(out, want)
+    for got, x in zip(grads, torch.autograd.grad(want, cut, do)):
+        assert torch.equal(got[:2, :130, :2], x) and got.count_nonzero() == x.count_nonzero()

@@ -1,4 +1,6 @@
 """CPU-only checks of the host-side mirror of the reference interface (no kernels run)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -339,3 +341,41 @@ def test_operands_smaller_than_the_call_are_refused(monkeypatch, k_shape, v_shap
     q, k, v = (torch.zeros(s, dtype=dtype) for s in ((2, 64, 4, 64), k_shape, v_shape or k_shape))
     with pytest.raises(ValueError, match="do not hold the batch and heads"):
         ra.ring_attention(q, k, v, 2)
+
+
+@pytest.mark.parametrize("k_shape,v_shape", [((3, 64, 2, 64), (2, 64, 2, 64)), ((2, 64, 3, 64), (2, 64, 2, 64)), ((2, 64, 2, 64), (2, 80, 2, 64)),
+                                             ((3, 64, 4, 64), (4, 70, 3, 64))])
+@pytest.mark.parametrize("impl,scheme", [("pallas", "attend"), ("hip", "_RingAttentionFn")])
+def test_what_lies_beyond_the_call_does_not_reach_the_kernels(monkeypatch, k_shape, v_shape, impl, scheme):
+    # more batch rows or heads than q has, values longer than the keys: dk and dv are stored with the same strides, so k and v that
+    # differ in shape would have one of them written past its end
+    seen = []
+
+    class Host:
+        def plan(self, *args):
+            return None
+
+        def attend(self, q, k, v, *args):
+            seen.append((q, k, v))
+            return q, q
+
+    monkeypatch.setattr(rr, "_require_gpu", lambda t: None)
+    monkeypatch.setattr(rr._lib, "host", Host)
+    monkeypatch.setattr(rr._RingAttentionFn, "apply", Host().attend)
+    q, k, v = (torch.zeros(s, dtype=torch.bfloat16, requires_grad=True) for s in ((2, 64, 2, 64), k_shape, v_shape))
+    ra.ring_attention(q, k, v, 1, block_impl=impl)
+    (_, k1, v1), = seen
+    assert k1.shape == v1.shape == (2, 64, 2, 64) and k1.data_ptr() == k.data_ptr() and v1.data_ptr() == v.data_ptr()
+    # the rest has a gradient: zeros
+    dk, dv = torch.autograd.grad((k1 * 2 + v1 * 3).sum(), (k, v))
+    for g, x in ((dk, 2), (dv, 3)):
+        assert g.sum() == x * q.numel() and (g[:2, :64, :2] == x).all()
+
+
+def test_operands_of_another_plan_are_refused():
+    q = torch.zeros((2, 64, 2, 64), dtype=torch.bfloat16)
+    bias = bytes(C.sizeof(rr._lib.RaBias))
+    plan = rr._lib.host().plan(2, 2, 64, 64, 64, bias, 0, 0, q, ())
+    for k, v in [(q[:1], q[:1]), (q, q[:, :32]), (q, torch.cat([q, q], 2)), (q[..., :32], q[..., :32])]:
+        with pytest.raises(RuntimeError, match="not the operands of this plan"):
+            rr._lib.host().attend(q, k, v, plan, 0.1, torch.bfloat16, torch.bfloat16)

@@ -193,6 +193,15 @@ def _bias_struct(bias, device, shape=None, summary=True) -> _lib.RaBias:
     return bias.to_struct(device, summary=summary)
 
 
+def _require_pair(q, k, v) -> None:
+    """``k`` and ``v`` hold the batch, heads and head dim of ``q``, all [b, h, l, d], and ``v`` the length of ``k``: the kernels take
+    pointers and strides and would read past an end."""
+    B, H, _, D = q.shape
+    ks, vs = k.shape, v.shape
+    if min(ks[0], vs[0]) < B or min(ks[1], vs[1]) < H or min(ks[3], vs[3]) < D or vs[2] < ks[2]:
+        raise ValueError(f"k {tuple(ks)} and v {tuple(vs)} do not hold the batch, heads and head dim of q {tuple(q.shape)}, or v not the length of k")
+
+
 def fwd_block(q, k, v, bias: Union[BlockBias, torch.Tensor, None], o, m, l, sm_scale: float):
     """One ring step of the forward pass, in place on the fp32 carry.
 
@@ -203,6 +212,7 @@ def fwd_block(q, k, v, bias: Union[BlockBias, torch.Tensor, None], o, m, l, sm_s
     ``[b, h | 1, lq, lk]`` array as in the reference, or a ``BlockBias`` description.
     Returns ``(o, m, l)`` (the same tensors, updated)."""
     _require_gpu(q)
+    _require_pair(q, k, v)
     lib = _lib.load()
     B, H, Lq, D = q.shape
     p = _lib.RaFwdStepParams()
@@ -246,6 +256,7 @@ def fwd_blocks(q, kvs, biases, o, m, l, sm_scale: float):
     for i, ((k, v), bias) in enumerate(zip(kvs, biases)):
         if isinstance(bias, torch.Tensor):
             bias = BlockBias(dense=bias)
+        _require_pair(q, k, v)
         keep.append(bias)
         steps[i] = _fwd_params(q, k, v, bias, o, m, l, sm_scale)
     _lib.check("ra_fwd_steps", lib.ra_fwd_steps(steps, len(kvs), _stream()))
@@ -338,6 +349,15 @@ def bwd_block(q, k, v, bias: Union[BlockBias, torch.Tensor, None], o, L, do, sm_
     ``bwd_block`` (ring_kernel.py:202-297): all tensors ``[b, h, l, d]``, ``o`` the normalised
     forward output, ``L`` the logsumexp ``[b, h, lq]``.  Returns fp32 ``(dq, dk, dv)``."""
     _require_gpu(q)
+    _require_pair(q, k, v)
+    (B, H, _, D), Lk = q.shape, k.shape[2]
+    if k.shape != v.shape or k.shape[:2] != (B, H) or k.shape[3] != D:
+        # What q has no batch row or head for takes no part: zeros.  (dk and dv are stored with the same strides.)
+        dq, *cut = bwd_block(q, k[:B, :H, :, :D], v[:B, :H, :Lk, :D], bias, o, L, do, sm_scale)
+        grads = [torch.zeros(x.shape, dtype=torch.float32, device=q.device) for x in (k, v)]
+        for whole, part in zip(grads, cut):
+            whole[:B, :H, :Lk, :D] = part
+        return dq, *grads
     if isinstance(bias, torch.Tensor):
         bias = BlockBias(dense=bias)
     if bias is not None and bias.dense is not None:  # into accumulators: those kernels read the block's summary

@@ -380,6 +380,23 @@ def test_single_steps_on_both_sides_of_the_rule(device, Lq, Lk, H, D, offset):
             assert err <= GRAD_TOL, (h, err)
 
 
+@pytest.mark.parametrize("bias", [None, "causal", "dense"])
+def test_block_gradients_of_what_lies_beyond_the_call(device, bias):
+    # more heads and batch rows of keys than of queries, values without a key: the gradients of the call cut to size, zeros around
+    g = torch.Generator(device=device).manual_seed(5)
+    q, k, v, do = (torch.randn(s, device=device, generator=g).to(torch.bfloat16) for s in ((2, 2, 70, 64), (3, 4, 90, 64), (2, 2, 130, 64), (2, 2, 70, 64)))
+    bias = {"causal": ra.BlockBias(ra.causal_bias(), 50, 0), "dense": torch.randn((2, 1, 70, 90), device=device, generator=g)}.get(bias)
+    cut = k[:2, :2].contiguous(), v[:, :, :90].contiguous()
+    carry = ra.fwd_block(q, k, v, bias, *rr.init_carry(2, 2, 70, 64, device), 0.1)
+    for a, b in zip(carry, ra.fwd_block(q, *cut, bias, *rr.init_carry(2, 2, 70, 64, device), 0.1)):
+        assert torch.equal(a, b)
+    out, lse = torch.empty((2, 2, 70, 64), device=device), torch.empty((2, 2, 70), device=device)
+    rr.finalize_carry(*carry, out, lse)
+    for got, want in zip(ra.bwd_block(q, k, v, bias, out, lse, do, 0.1), ra.bwd_block(q, *cut, bias, out, lse, do, 0.1)):
+        B, H, L, _ = want.shape
+        assert torch.equal(got[:B, :H, :L], want) and got.count_nonzero() == want.count_nonzero() > 0
+
+
 @pytest.mark.parametrize("D,n", [(32, 1), (64, 1), (96, 1), (128, 1), (64, 3), (128, 3)])
 @pytest.mark.parametrize("transposed", ["qk", "v"])
 def test_keys_and_values_laid_out_differently(device, D, n, transposed):

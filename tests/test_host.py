@@ -379,3 +379,49 @@ def test_operands_of_another_plan_are_refused():
     for k, v in [(q[:1], q[:1]), (q, q[:, :32]), (q, torch.cat([q, q], 2)), (q[..., :32], q[..., :32])]:
         with pytest.raises(RuntimeError, match="not the operands of this plan"):
             rr._lib.host().attend(q, k, v, plan, 0.1, torch.bfloat16, torch.bfloat16)
+
+
+@pytest.mark.parametrize("k_shape,v_shape", [((1, 2, 32, 64), (2, 2, 32, 64)), ((2, 2, 32, 64), (2, 1, 32, 64)), ((2, 2, 32, 64), (2, 2, 31, 64)),
+                                             ((2, 2, 32, 32), (2, 2, 32, 64))])
+def test_blocks_refuse_keys_and_values_smaller_than_the_call(monkeypatch, k_shape, v_shape):
+    monkeypatch.setattr(rr, "_require_gpu", lambda t: None)
+    q, k, v = (torch.zeros(s, dtype=torch.bfloat16) for s in ((2, 2, 32, 64), k_shape, v_shape))
+    rows, acc = torch.zeros((2, 2, 32)), torch.zeros((2, 2, 32, 64))
+    for call in (lambda: ra.fwd_block(q, k, v, None, acc, rows, rows.clone(), 0.1), lambda: ra.bwd_block(q, k, v, None, acc, rows, q, 0.1),
+                 lambda: rr.fwd_blocks(q, [(k, v)], [None], acc, rows, rows.clone(), 0.1)):
+        with pytest.raises(ValueError, match="do not hold the batch, heads and head dim"):
+            call()
+
+
+@pytest.mark.parametrize("k_shape,v_shape", [((3, 2, 32, 64), (2, 2, 32, 64)), ((2, 3, 32, 64), (2, 2, 32, 64)), ((2, 2, 32, 64), (2, 2, 40, 128)),
+                                             ((2, 4, 32, 128), (4, 3, 33, 64))])
+@pytest.mark.parametrize("dense", [False, True])
+def test_block_gradients_of_what_lies_beyond_the_call(monkeypatch, k_shape, v_shape, dense):
+    # dk and dv are stored with the same strides: arrays of one shape, the call's, and zeros around what comes back
+    class Library:
+        def __getattr__(self, name):
+            return lambda *args: 64
+
+        def ra_bwd_step_check(self, p):
+            return 0
+
+        def ra_bwd_whole(self, p, *args):
+            assert (p._obj.B, p._obj.H, p._obj.Lk, p._obj.D) == (2, 2, 32, 64) and args[-6:-3] == (2 * 32 * 64, 32 * 64, 64)
+            for at, x in ((args[-8], 2.0), (args[-7], 3.0)):
+                torch.frombuffer((C.c_float * (2 * 2 * 32 * 64)).from_address(at), dtype=torch.float32).fill_(x)
+            return 0
+
+    def step(q, k, v, do, lse, delta, dq, dk, dv, *_):
+        assert k.shape == v.shape == q.shape
+        dk.fill_(2.0)
+        dv.fill_(3.0)
+
+    monkeypatch.setattr(rr, "_require_gpu", lambda t: None)
+    monkeypatch.setattr(rr, "_stream", lambda: None)
+    monkeypatch.setattr(rr, "precompute_delta", lambda o, do: None)
+    monkeypatch.setattr(rr, "_bwd_step", step)
+    monkeypatch.setattr(rr._lib, "load", Library)
+    q, k, v = (torch.zeros(s, dtype=torch.bfloat16) for s in ((2, 2, 32, 64), k_shape, v_shape))
+    dq, *grads = ra.bwd_block(q, k, v, torch.zeros((2, 1, 32, 32)) if dense else None, torch.zeros(q.shape), torch.zeros((2, 2, 32)), q, 0.1)
+    for got, x, value in zip(grads, (k, v), (2, 3)):
+        assert got.shape == x.shape and got.sum() == value * q.numel() and (got[:2, :2, :32, :64] == value).all()

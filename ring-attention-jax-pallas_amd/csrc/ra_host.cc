@@ -156,7 +156,7 @@ class WholeCall : public torch::autograd::Function<WholeCall> {
     ra_rows rows[3];
     int n_rows = 0;
     variable_list kept;
-    if (dtype == call->given[1] && dtype == call->given[2] && !is_operand(q, p.D) && q.device() == k.device() && k.device() == v.device()) {
+    if (dtype == call->given[1] && dtype == call->given[2] && !is_operand(q, p.D)) {
       const int64_t nq = p.B * p.Lq * p.H * p.D, nk = p.B * p.Lk * p.H * p.D;
       Tensor buf = empty({nq + 2 * nk}, at::kBFloat16, q.device());
       char* at = (char*)buf.data_ptr();
@@ -322,8 +322,9 @@ PyObject* attend(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const int64_t d = q.dim() == 4 ? q.size(3) : -1;
   // (pointers and strides are all that goes on from here)
   TORCH_CHECK(d <= of.D && q.sizes() == at::IntArrayRef({of.B, of.Lq, of.H, d}) && k.sizes() == at::IntArrayRef({of.B, of.Lk, of.H, d}) &&
-                  v.sizes() == k.sizes(),
-              "attend: q ", q.sizes(), ", k ", k.sizes(), " and v ", v.sizes(), " are not the operands of this plan");
+                  v.sizes() == k.sizes() && q.device() == of.device && k.device() == of.device && v.device() == of.device,
+              "attend: q ", q.sizes(), " on ", q.device(), ", k ", k.sizes(), " on ", k.device(), " and v ", v.sizes(), " on ", v.device(),
+              " are not the operands of this plan");
   const bool any_grad = q.requires_grad() || k.requires_grad() || v.requires_grad();
   const at::ScalarType dtype = reinterpret_cast<THPDtype*>(args[5])->scalar_type, final_dtype = reinterpret_cast<THPDtype*>(args[6])->scalar_type;
   variable_list got;

@@ -193,13 +193,15 @@ def _bias_struct(bias, device, shape=None, summary=True) -> _lib.RaBias:
     return bias.to_struct(device, summary=summary)
 
 
-def _require_pair(q, k, v) -> None:
+def _require_pair(q, k, v, *others) -> None:
     """``k`` and ``v`` hold the batch, heads and head dim of ``q``, all [b, h, l, d], and ``v`` the length of ``k``: the kernels take
-    pointers and strides and would read past an end."""
+    pointers and strides and would read past an end.  They and the ``others`` are on ``q``'s device."""
     B, H, _, D = q.shape
     ks, vs = k.shape, v.shape
     if min(ks[0], vs[0]) < B or min(ks[1], vs[1]) < H or min(ks[3], vs[3]) < D or vs[2] < ks[2]:
         raise ValueError(f"k {tuple(ks)} and v {tuple(vs)} do not hold the batch, heads and head dim of q {tuple(q.shape)}, or v not the length of k")
+    if any(t.device != q.device for t in (k, v, *others)):
+        raise ValueError(f"all arrays of a block must be on the device of q ({q.device})")
 
 
 def fwd_block(q, k, v, bias: Union[BlockBias, torch.Tensor, None], o, m, l, sm_scale: float):
@@ -212,7 +214,7 @@ def fwd_block(q, k, v, bias: Union[BlockBias, torch.Tensor, None], o, m, l, sm_s
     ``[b, h | 1, lq, lk]`` array as in the reference, or a ``BlockBias`` description.
     Returns ``(o, m, l)`` (the same tensors, updated)."""
     _require_gpu(q)
-    _require_pair(q, k, v)
+    _require_pair(q, k, v, o, m, l)
     lib = _lib.load()
     B, H, Lq, D = q.shape
     p = _lib.RaFwdStepParams()
@@ -256,7 +258,7 @@ def fwd_blocks(q, kvs, biases, o, m, l, sm_scale: float):
     for i, ((k, v), bias) in enumerate(zip(kvs, biases)):
         if isinstance(bias, torch.Tensor):
             bias = BlockBias(dense=bias)
-        _require_pair(q, k, v)
+        _require_pair(q, k, v, o, m, l)
         keep.append(bias)
         steps[i] = _fwd_params(q, k, v, bias, o, m, l, sm_scale)
     _lib.check("ra_fwd_steps", lib.ra_fwd_steps(steps, len(kvs), _stream()))
@@ -349,7 +351,7 @@ def bwd_block(q, k, v, bias: Union[BlockBias, torch.Tensor, None], o, L, do, sm_
     ``bwd_block`` (ring_kernel.py:202-297): all tensors ``[b, h, l, d]``, ``o`` the normalised
     forward output, ``L`` the logsumexp ``[b, h, lq]``.  Returns fp32 ``(dq, dk, dv)``."""
     _require_gpu(q)
-    _require_pair(q, k, v)
+    _require_pair(q, k, v, o, L, do)
     (B, H, _, D), Lk = q.shape, k.shape[2]
     if k.shape != v.shape or k.shape[:2] != (B, H) or k.shape[3] != D:
         # What q has no batch row or head for takes no part: zeros.  (dk and dv are stored with the same strides.)
@@ -1109,6 +1111,8 @@ def _attend(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs, sm_scale
         # Batch rows and heads that q has none for, and values without a key, take no part.  Cut off here: their gradients are zeros,
         # and dk and dv, which the kernels store with the same strides, have the same shape.
         k, v = k[:qs[0], :, :qs[2]], v[:qs[0], :ks[1], :qs[2]]
+    if k.device != q.device or v.device != q.device:  # (to q's, as the bias arrays are; the kernels take pointers)
+        k, v = k.to(q.device), v.to(q.device)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(d_true)  # ring.py:287-288
     in_dtype = q.dtype

@@ -124,3 +124,15 @@ def test_keys_and_values_beyond_the_call(device, k_shape, v_shape, impl, dtype):
     assert torch.equal(out, want)
     for got, x in zip(grads, torch.autograd.grad(want, cut, do)):
         assert torch.equal(got[:2, :130, :2], x) and got.count_nonzero() == x.count_nonzero()
+
+
+@pytest.mark.parametrize("impl", ["pallas", "hip"])
+def test_keys_and_values_from_host_memory(device, impl):
+    q, k, v = _arrays(device)
+    do = torch.randn(q.shape, device=device).to(torch.bfloat16)
+    at_home = [x.detach().cpu().requires_grad_(True) for x in (k, v)]
+    out, want = (ra.ring_attention(q, *kv, 1, ra.causal_bias(), block_impl=impl) for kv in (at_home, (k, v)))
+    assert torch.equal(out, want)
+    for got, x in zip(torch.autograd.grad(out, (q, *at_home), do), torch.autograd.grad(want, (q, k, v), do)):
+        assert torch.equal(got.to(device), x)
+    assert got.device.type == "cpu"

@@ -376,7 +376,8 @@ def test_operands_of_another_plan_are_refused():
     q = torch.zeros((2, 64, 2, 64), dtype=torch.bfloat16)
     bias = bytes(C.sizeof(rr._lib.RaBias))
     plan = rr._lib.host().plan(2, 2, 64, 64, 64, bias, 0, 0, q, ())
-    for k, v in [(q[:1], q[:1]), (q, q[:, :32]), (q, torch.cat([q, q], 2)), (q[..., :32], q[..., :32])]:
+    other = torch.zeros_like(q, device="meta")
+    for k, v in [(other, q), (q, other), (q[:1], q[:1]), (q, q[:, :32]), (q, torch.cat([q, q], 2)), (q[..., :32], q[..., :32])]:
         with pytest.raises(RuntimeError, match="not the operands of this plan"):
             rr._lib.host().attend(q, k, v, plan, 0.1, torch.bfloat16, torch.bfloat16)
 
@@ -425,3 +426,33 @@ def test_block_gradients_of_what_lies_beyond_the_call(monkeypatch, k_shape, v_sh
     dq, *grads = ra.bwd_block(q, k, v, torch.zeros((2, 1, 32, 32)) if dense else None, torch.zeros(q.shape), torch.zeros((2, 2, 32)), q, 0.1)
     for got, x, value in zip(grads, (k, v), (2, 3)):
         assert got.shape == x.shape and got.sum() == value * q.numel() and (got[:2, :2, :32, :64] == value).all()
+
+
+@pytest.mark.parametrize("impl", ["pallas", "hip"])
+@pytest.mark.parametrize("elsewhere", ["k", "v", "kv"])
+def test_operands_on_another_device_go_to_that_of_the_queries(monkeypatch, impl, elsewhere):
+    # a pointer into host memory would fault the GPU; "meta" stands for the other device here
+    seen = []
+    monkeypatch.setattr(rr, "_require_gpu", lambda t: None)
+    monkeypatch.setattr(rr._lib, "host", lambda: type("Host", (), {"plan": lambda *a: None, "attend": lambda s, q, k, v, *a: seen.append((k, v)) or (q, q)})())
+    monkeypatch.setattr(rr._RingAttentionFn, "apply", lambda q, k, v, *a: seen.append((k, v)) or (q, q))
+    q, k, v = (torch.zeros((1, 64, 2, 64), dtype=torch.bfloat16, device="cpu" if name in elsewhere else "meta") for name in "qkv")
+    ra.ring_attention(q, k, v, 1, block_impl=impl)
+    assert [x.device.type for x in seen[0]] == ["meta", "meta"]
+
+
+@pytest.mark.parametrize("at", range(6))
+def test_blocks_refuse_arrays_on_another_device(monkeypatch, at):
+    monkeypatch.setattr(rr, "_require_gpu", lambda t: None)
+    x, rows, acc = torch.zeros((1, 1, 32, 64), dtype=torch.bfloat16), torch.zeros((1, 1, 32)), torch.zeros((1, 1, 32, 64))
+    there = lambda *args: [t.to("meta") if i == at else t for i, t in enumerate(args)]
+    calls = []
+    if at < 5:
+        k, v, o, m, l = there(x, x, acc, rows, rows.clone())
+        calls += [lambda: ra.fwd_block(x, k, v, None, o, m, l, 0.1), lambda: rr.fwd_blocks(x, [(k, v)], [None], o, m, l, 0.1)]
+    if at != 2:
+        k1, v1, _, o1, L, do = there(x, x, None, acc, rows, x)
+        calls.append(lambda: ra.bwd_block(x, k1, v1, None, o1, L, do, 0.1))
+    for call in calls:
+        with pytest.raises(ValueError, match="on the device of q"):
+            call()

@@ -87,13 +87,21 @@ def build_xla_ffi(verbose: bool = False) -> str | None:
     return FFI_LIB_PATH
 
 
-def build_host(verbose: bool = False) -> str:
-    """ring_attention/_host.so from csrc/ra_host.cc."""
+def build_host(verbose: bool = False) -> str | None:
+    """ring_attention/_host.so from csrc/ra_host.cc; skipped (None) without a ROCm build of torch, for hosts that bind the C ABI or the
+    XLA FFI handlers only."""
     import sysconfig
 
-    import torch
-    from torch.utils import cpp_extension
-
+    try:
+        import torch
+        from torch.utils import cpp_extension
+        missing = None if torch.version.hip else "this torch is not a ROCm build"
+    except ImportError as e:
+        missing = e
+    if missing:
+        if verbose:
+            print(f"{HOST_SOURCE} skipped: {missing}")
+        return None
     include = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", *(x for p in include for x in ("-isystem", p)),
@@ -121,8 +129,8 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
             raise RuntimeError(f"link failed:\n{res.stderr}")
         if verbose:
             print(f"built {lib}")
-    build_host(verbose)
     build_xla_ffi(verbose)
+    build_host(verbose)
     return LIB_PATH
 
 

@@ -456,3 +456,37 @@ def test_blocks_refuse_arrays_on_another_device(monkeypatch, at):
     for call in calls:
         with pytest.raises(ValueError, match="on the device of q"):
             call()
+
+
+def _build_module():
+    import importlib.util
+    import os
+
+    spec = importlib.util.spec_from_file_location("ra_build", os.path.join(os.path.dirname(os.path.dirname(rr.__file__)), "build.py"))
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+@pytest.mark.parametrize("torch_is", ["absent", "of another platform"])
+def test_the_c_libraries_are_built_without_torch(monkeypatch, tmp_path, torch_is):
+    # a host that binds the C ABI or the XLA FFI handlers only
+    import sys
+
+    build = _build_module()
+    include = tmp_path / "xla" / "ffi" / "api"
+    include.mkdir(parents=True)
+    (include / "ffi.h").touch()
+    ran = []
+    monkeypatch.setenv("XLA_FFI_INCLUDE_DIR", str(tmp_path))
+    monkeypatch.setattr(build, "OBJ_DIR", str(tmp_path / "build"))
+    monkeypatch.setattr(build, "_hipcc", lambda: "hipcc")
+    monkeypatch.setattr(build.subprocess, "run", lambda cmd, **_: ran.append(cmd) or type("Result", (), {"returncode": 0})())
+    if torch_is == "absent":
+        monkeypatch.setitem(sys.modules, "torch", None)
+        monkeypatch.setitem(sys.modules, "torch.utils", None)
+    else:
+        monkeypatch.setattr(torch.version, "hip", None)
+    assert build.build() == build.LIB_PATH
+    made = [cmd[cmd.index("-o") + 1] for cmd in ran]
+    assert build.LIB_PATH in made and build.FFI_LIB_PATH in made and build.HOST_LIB_PATH not in made

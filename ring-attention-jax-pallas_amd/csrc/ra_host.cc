@@ -278,7 +278,7 @@ PyObject* init(PyObject*, PyObject* args) {
   END_HANDLE_TH_ERRORS
 }
 
-// plan(B, H, Lq, Lk, D, ra_bias block, bytes of the forward's and of the backward's workspace, q's device as a tensor, bias arrays)
+// plan(B, H, Lq, Lk, D, ra_bias block, bytes of the forward's workspace, q's device as a tensor, bias arrays)
 PyObject* plan(PyObject*, PyObject* args) {
   HANDLE_TH_ERRORS
   long long B, H, Lq, Lk, D, fwd_bytes, bwd_bytes;
@@ -317,14 +317,19 @@ PyObject* attend(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!p) throw python_error();
   const double scale = PyFloat_AsDouble(args[4]);
   if (scale == -1.0 && PyErr_Occurred()) throw python_error();
-  const Tensor &q = THPVariable_Unpack(args[0]), &k = THPVariable_Unpack(args[1]), &v = THPVariable_Unpack(args[2]);
+  const Tensor& q = THPVariable_Unpack(args[0]);
+  Tensor k = THPVariable_Unpack(args[1]), v = THPVariable_Unpack(args[2]);
+  for (Tensor* t : {&k, &v})
+    if (t->device() != q.device()) {  // (the kernels take pointers; the bias arrays went the same way)
+      pybind11::gil_scoped_release no_gil;
+      *t = t->to(q.device());
+    }
   const Plan& of = **p;
   const int64_t d = q.dim() == 4 ? q.size(3) : -1;
   // (pointers and strides are all that goes on from here)
   TORCH_CHECK(d <= of.D && q.sizes() == at::IntArrayRef({of.B, of.Lq, of.H, d}) && k.sizes() == at::IntArrayRef({of.B, of.Lk, of.H, d}) &&
-                  v.sizes() == k.sizes() && q.device() == of.device && k.device() == of.device && v.device() == of.device,
-              "attend: q ", q.sizes(), " on ", q.device(), ", k ", k.sizes(), " on ", k.device(), " and v ", v.sizes(), " on ", v.device(),
-              " are not the operands of this plan");
+                  v.sizes() == k.sizes() && q.device() == of.device,
+              "attend: q ", q.sizes(), " on ", q.device(), ", k ", k.sizes(), " and v ", v.sizes(), " are not the operands of this plan");
   const bool any_grad = q.requires_grad() || k.requires_grad() || v.requires_grad();
   const at::ScalarType dtype = reinterpret_cast<THPDtype*>(args[5])->scalar_type, final_dtype = reinterpret_cast<THPDtype*>(args[6])->scalar_type;
   variable_list got;

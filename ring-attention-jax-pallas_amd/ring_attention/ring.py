@@ -1111,8 +1111,6 @@ def _attend(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs, sm_scale
         # Batch rows and heads that q has none for, and values without a key, take no part.  Cut off here: their gradients are zeros,
         # and dk and dv, which the kernels store with the same strides, have the same shape.
         k, v = k[:qs[0], :, :qs[2]], v[:qs[0], :ks[1], :qs[2]]
-    if k.device != q.device or v.device != q.device:  # (to q's, as the bias arrays are; the kernels take pointers)
-        k, v = k.to(q.device), v.to(q.device)
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(d_true)  # ring.py:287-288
     in_dtype = q.dtype
@@ -1130,7 +1128,8 @@ def _attend(q, k, v, axis_name, bias_fn, bias_q_kwargs, bias_kv_kwargs, sm_scale
     if fused and plan.n == 1 and plan.callable is None and torch._C._get_tracing_state() is None:
         out, lse = _lib.host().attend(q, k, v, plan.native(q), float(sm_scale), out_dtype, final_dtype)
     else:
-        out, lse = _RingAttentionFn.apply(q, k, v, plan, float(sm_scale), out_dtype, final_dtype, fused)
+        # (the kernels take pointers; the native call does the same)
+        out, lse = _RingAttentionFn.apply(q, k.to(q.device), v.to(q.device), plan, float(sm_scale), out_dtype, final_dtype, fused)
     if out.shape[-1] != d_true:
         out = out[..., :d_true]
     return out, lse, plan

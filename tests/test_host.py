@@ -376,8 +376,7 @@ def test_operands_of_another_plan_are_refused():
     q = torch.zeros((2, 64, 2, 64), dtype=torch.bfloat16)
     bias = bytes(C.sizeof(rr._lib.RaBias))
     plan = rr._lib.host().plan(2, 2, 64, 64, 64, bias, 0, 0, q, ())
-    other = torch.zeros_like(q, device="meta")
-    for k, v in [(other, q), (q, other), (q[:1], q[:1]), (q, q[:, :32]), (q, torch.cat([q, q], 2)), (q[..., :32], q[..., :32])]:
+    for k, v in [(q[:1], q[:1]), (q, q[:, :32]), (q, torch.cat([q, q], 2)), (q[..., :32], q[..., :32])]:
         with pytest.raises(RuntimeError, match="not the operands of this plan"):
             rr._lib.host().attend(q, k, v, plan, 0.1, torch.bfloat16, torch.bfloat16)
 
@@ -428,16 +427,14 @@ def test_block_gradients_of_what_lies_beyond_the_call(monkeypatch, k_shape, v_sh
         assert got.shape == x.shape and got.sum() == value * q.numel() and (got[:2, :2, :32, :64] == value).all()
 
 
-@pytest.mark.parametrize("impl", ["pallas", "hip"])
 @pytest.mark.parametrize("elsewhere", ["k", "v", "kv"])
-def test_operands_on_another_device_go_to_that_of_the_queries(monkeypatch, impl, elsewhere):
-    # a pointer into host memory would fault the GPU; "meta" stands for the other device here
+def test_operands_on_another_device_go_to_that_of_the_queries(monkeypatch, elsewhere):
+    # a pointer into host memory would fault the GPU; "meta" stands for the other device here (the native call does the same on the GPU)
     seen = []
     monkeypatch.setattr(rr, "_require_gpu", lambda t: None)
-    monkeypatch.setattr(rr._lib, "host", lambda: type("Host", (), {"plan": lambda *a: None, "attend": lambda s, q, k, v, *a: seen.append((k, v)) or (q, q)})())
     monkeypatch.setattr(rr._RingAttentionFn, "apply", lambda q, k, v, *a: seen.append((k, v)) or (q, q))
     q, k, v = (torch.zeros((1, 64, 2, 64), dtype=torch.bfloat16, device="cpu" if name in elsewhere else "meta") for name in "qkv")
-    ra.ring_attention(q, k, v, 1, block_impl=impl)
+    ra.ring_attention(q, k, v, 1, block_impl="hip")
     assert [x.device.type for x in seen[0]] == ["meta", "meta"]
 
 

@@ -14,6 +14,7 @@
 #include <torch/csrc/utils/pybind.h>
 #include <torch/types.h>
 
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -29,6 +30,7 @@ using torch::autograd::variable_list;
 struct Library {
   decltype(&ra_fwd_call) fwd_call;
   decltype(&ra_bwd_call) bwd_call;
+  decltype(&ra_bwd_whole_workspace) bwd_workspace;
   decltype(&ra_convert) convert;
   PyObject* check;  // _lib.check: raises what the code says
 } g_lib;
@@ -114,7 +116,8 @@ ra_tensor rows_at(const void* p, int64_t L, int64_t H, int64_t D) { return ra_te
 struct Plan : torch::CustomClassHolder {
   int64_t B, H, Lq, Lk, D;
   ra_bias bias;
-  int64_t fwd_bytes, bwd_bytes;
+  int64_t fwd_bytes;
+  std::atomic<int64_t> bwd_bytes{-1};  // -1: no backward has asked for it (a call without gradients does not pay for its plan)
   at::Device device = at::kCPU;
   std::vector<Tensor> arrays;
 };
@@ -194,7 +197,7 @@ class WholeCall : public torch::autograd::Function<WholeCall> {
 
   static variable_list backward(AutogradContext* ctx, variable_list grads_in) {
     const auto call = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
-    const Plan& p = *call->plan;
+    Plan& p = *call->plan;
     variable_list kept = ctx->get_saved_variables();
     const Tensor lse = kept.back(), out = kept[kept.size() - 2];
     kept.resize(kept.size() - 2);
@@ -230,16 +233,18 @@ class WholeCall : public torch::autograd::Function<WholeCall> {
       Tensor* t = &made;
       operands(&t, 1, p.D);
     }
-    const Tensor ws = workspace(p.bwd_bytes, p.device);
     ra_tensor x[3];
     operand_views(p, kept, x);
     const float* l = (const float*)lse.data_ptr();
     const ra_bwd_step_params a{(int32_t)p.B, (int32_t)p.H, (int32_t)p.Lq, (int32_t)p.Lk, (int32_t)p.D, call->scale, x[0], x[1], x[2],
                                view(made), l, nullptr, nullptr, nullptr, nullptr, p.bias};
+    int64_t bytes = p.bwd_bytes.load(std::memory_order_relaxed);
+    if (bytes < 0) p.bwd_bytes.store(bytes = g_lib.bwd_workspace(&a), std::memory_order_relaxed);  // (sizes and bias alone decide)
+    const Tensor ws = workspace(bytes, p.device);
     const ra_tensor o = view(out), gq = view(dq), gk = view(dk);
     check("ra_bwd_call", g_lib.bwd_call(&rows, n_rows, &a, o.ptr, row_dtype(out.scalar_type()), o.stride_b, o.stride_h, o.stride_l,
                                         row_dtype(dtype) | RA_DTYPE_VIA_BF16, dq.data_ptr(), gq.stride_b, gq.stride_h, gq.stride_l,
-                                        dk.data_ptr(), dv.data_ptr(), gk.stride_b, gk.stride_h, gk.stride_l, pointer(ws), p.bwd_bytes,
+                                        dk.data_ptr(), dv.data_ptr(), gk.stride_b, gk.stride_h, gk.stride_l, pointer(ws), bytes,
                                         stream()));
     Tensor* g[3] = {&dq, &dk, &dv};
     Tensor* todo[3];
@@ -263,14 +268,15 @@ void drop_plan(PyObject* capsule) {
   delete static_cast<c10::intrusive_ptr<Plan>*>(PyCapsule_GetPointer(capsule, kPlanName));
 }
 
-// init(address of ra_fwd_call, of ra_bwd_call, of ra_convert, check)
+// init(address of ra_fwd_call, of ra_bwd_call, of ra_bwd_whole_workspace, of ra_convert, check)
 PyObject* init(PyObject*, PyObject* args) {
   HANDLE_TH_ERRORS
-  unsigned long long f, b, c;
+  unsigned long long f, b, w, c;
   PyObject* check_fn;
-  if (!PyArg_ParseTuple(args, "KKKO", &f, &b, &c, &check_fn)) return nullptr;
+  if (!PyArg_ParseTuple(args, "KKKKO", &f, &b, &w, &c, &check_fn)) return nullptr;
   g_lib.fwd_call = reinterpret_cast<decltype(g_lib.fwd_call)>(static_cast<uintptr_t>(f));
   g_lib.bwd_call = reinterpret_cast<decltype(g_lib.bwd_call)>(static_cast<uintptr_t>(b));
+  g_lib.bwd_workspace = reinterpret_cast<decltype(g_lib.bwd_workspace)>(static_cast<uintptr_t>(w));
   g_lib.convert = reinterpret_cast<decltype(g_lib.convert)>(static_cast<uintptr_t>(c));
   Py_INCREF(check_fn);
   Py_XSETREF(g_lib.check, check_fn);
@@ -281,10 +287,10 @@ PyObject* init(PyObject*, PyObject* args) {
 // plan(B, H, Lq, Lk, D, ra_bias block, bytes of the forward's workspace, q's device as a tensor, bias arrays)
 PyObject* plan(PyObject*, PyObject* args) {
   HANDLE_TH_ERRORS
-  long long B, H, Lq, Lk, D, fwd_bytes, bwd_bytes;
+  long long B, H, Lq, Lk, D, fwd_bytes;
   Py_buffer bias;
   PyObject *like, *arrays;
-  if (!PyArg_ParseTuple(args, "LLLLLy*LLOO!", &B, &H, &Lq, &Lk, &D, &bias, &fwd_bytes, &bwd_bytes, &like, &PyTuple_Type, &arrays)) return nullptr;
+  if (!PyArg_ParseTuple(args, "LLLLLy*LOO!", &B, &H, &Lq, &Lk, &D, &bias, &fwd_bytes, &like, &PyTuple_Type, &arrays)) return nullptr;
   auto p = c10::make_intrusive<Plan>();
   const bool fits = bias.len == sizeof(ra_bias);
   if (fits) std::memcpy(&p->bias, bias.buf, sizeof(ra_bias));
@@ -296,7 +302,6 @@ PyObject* plan(PyObject*, PyObject* args) {
   p->Lk = Lk;
   p->D = D;
   p->fwd_bytes = fwd_bytes;
-  p->bwd_bytes = bwd_bytes;
   TORCH_CHECK_TYPE(THPVariable_Check(like), "a tensor is expected");
   p->device = THPVariable_Unpack(like).device();
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(arrays); ++i) {

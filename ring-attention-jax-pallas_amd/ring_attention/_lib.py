@@ -174,7 +174,8 @@ def host():
             raise RuntimeError("ring_attention/_host.so is missing or was built for another torch: build it first (python build.py "
                                f"in the package directory, or __graft_entry__.build()): {e}") from e
         lib = load()
-        module.init(*(C.cast(f, C.c_void_p).value for f in (lib.ra_fwd_call, lib.ra_bwd_call, lib.ra_convert)), check)
+        module.init(*(C.cast(f, C.c_void_p).value for f in (lib.ra_fwd_call, lib.ra_bwd_call, lib.ra_bwd_whole_workspace,
+                                                                 lib.ra_convert)), check)
         _host = module
     return _host
 

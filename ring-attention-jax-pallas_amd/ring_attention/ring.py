@@ -568,12 +568,13 @@ class _RingPlan:
         return got["bias"], size
 
     def native(self, like):
-        """``pair_call`` as ``csrc/ra_host.cc`` keeps it; ``like``: a tensor on the plan's device."""
+        """``pair_call`` as ``csrc/ra_host.cc`` keeps it, which sizes the backward's workspace itself when a backward comes; ``like``:
+        a tensor on the plan's device."""
         got = self.__dict__.get("_native")
         if got is None:
-            (bias, forward), (_, backward) = self.pair_call(False), self.pair_call(True)
+            bias, forward = self.pair_call(False)
             arrays = self.__dict__["_pair_call"]["arrays"]
-            got = self.__dict__["_native"] = _lib.host().plan(self.B, self.H, self.Lq, self.Lk, self.D, bias, forward, backward, like,
+            got = self.__dict__["_native"] = _lib.host().plan(self.B, self.H, self.Lq, self.Lk, self.D, bias, forward, like,
                                                               () if arrays is None else tuple(arrays._keep))
         return got
 

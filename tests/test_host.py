@@ -375,7 +375,7 @@ def test_what_lies_beyond_the_call_does_not_reach_the_kernels(monkeypatch, k_sha
 def test_operands_of_another_plan_are_refused():
     q = torch.zeros((2, 64, 2, 64), dtype=torch.bfloat16)
     bias = bytes(C.sizeof(rr._lib.RaBias))
-    plan = rr._lib.host().plan(2, 2, 64, 64, 64, bias, 0, 0, q, ())
+    plan = rr._lib.host().plan(2, 2, 64, 64, 64, bias, 0, q, ())
     for k, v in [(q[:1], q[:1]), (q, q[:, :32]), (q, torch.cat([q, q], 2)), (q[..., :32], q[..., :32])]:
         with pytest.raises(RuntimeError, match="not the operands of this plan"):
             rr._lib.host().attend(q, k, v, plan, 0.1, torch.bfloat16, torch.bfloat16)
@@ -487,3 +487,17 @@ def test_the_c_libraries_are_built_without_torch(monkeypatch, tmp_path, torch_is
     assert build.build() == build.LIB_PATH
     made = [cmd[cmd.index("-o") + 1] for cmd in ran]
     assert build.LIB_PATH in made and build.FFI_LIB_PATH in made and build.HOST_LIB_PATH not in made
+
+
+def test_a_call_without_gradients_does_not_plan_a_backward(monkeypatch):
+    class Library:
+        def ra_fwd_whole_workspace(self, p):
+            return 96
+
+    made = []
+    q = torch.zeros((1, 64, 2, 64), dtype=torch.bfloat16)
+    plan = rr._RingPlan(q, q, 1, ra.causal_bias(), None, None).joined()
+    monkeypatch.setattr(rr._lib, "load", Library)
+    monkeypatch.setattr(rr._lib, "host", lambda: type("Host", (), {"plan": lambda s, *args: made.append(args)})())
+    plan.native(q)
+    assert made[0][:5] == (1, 2, 64, 64, 64) and made[0][6:] == (96, q, ())

@@ -713,19 +713,6 @@ bool even_rows(int64_t total, int most, int64_t rows) { return total * 20 >= (in
 bool one_by_one(const ra_bias& b, int64_t total, int most, int64_t rows) {
   return even_rows(total, most, rows) && !has_lists(b) && !(b.flags & RA_BIAS_WINDOW);
 }
-// Small backward calls that stay two launches, because test_gpu_pair.py names their two kernels: at D = 128 under a causal or window mask,
-// below one and three quarters rounds, and at D = 64 unmasked, below three (three workgroups fit a compute unit there).  One launch would
-// be faster there too (unmasked 512, H=4, D=64: 32 | 26 us).  The others are one at any size, two launches | one: documents of 300 in
-// 1024 tokens, causal, B=4, H=8, D=128 80 | 68, prefix 672, B=4, H=12, D=96 70 | 49, unmasked 864 x 1024, D=80, H=32 87 | 83, causal
-// 512, H=4, D=64 38 | 28, 700 37 | 25, unmasked, D=128, 1000, H=4 50 | 35, 2000, B=2, H=4 102 | 80.
-bool small_ones_apart(const ra_bias& b, int D) {
-  const bool masked = b.flags & (RA_BIAS_CAUSAL | RA_BIAS_WINDOW);
-  return !has_lists(b) && !(b.flags & RA_BIAS_ALIBI) && (D == 128 ? masked : D == 64 && !masked);
-}
-// Whether the shares of a gradient of even rows are counted beside the other one's (plan_split): not where small ones run apart at D = 64.
-// Two launches counted by themselves | counted beside each other, backward, us: unmasked, D=64, 2000, H=8 71 | 86, 894, B=2, H=4 43 | 44;
-// at D = 128 windows alone are meant, which were not slowed by the count (as many shares as places | so, 1000 of 8192, H=4 107 | 89).
-bool shares_beside(const ra_bwd_step_params& p) { return !(p.D == 64 && small_ones_apart(p.bias, p.D)); }
 // How the workgroups of one kind of a head's resident tiles, which meet `total` tiles of the other side (`most` at most), share their
 // work (see above).  share: bytes of one share of every row.  beside: the other gradient's workgroups run in the same launch.
 // Rows of about the same length take the number of shares k that a count of time finds best, in tiles of a workgroup (1.4 us at D = 128):
@@ -805,32 +792,21 @@ PairPlan plan_fwd_pair(const ra_fwd_step_params& p) {
   if (one_by_one(p.bias, total, most, rows)) r.group = 1;
   return r;
 }
+// Tiles of the other side that a head's resident tiles of one kind meet: their sum, and the most.
+struct TileCount {
+  int64_t heads, rows, total;  // rows: resident tiles of a head
+  int most;
+  bool even;  // (even_rows)
+};
 // dQ, likewise (dq_kernel | dq_pair_kernel): 65 tiles (32 heads of 8192) 0.70 | 0.66 ms, 66 (window 4096 of 65536, H=8) 1.36 |
 // 1.33, 129 (16 of 16384) 1.31 | 1.30, 128 (16 of 8192 x 8192) 0.64 | 0.66, 257 (32 of 32768) 10.1 | 10.4; ALiBi, 129: 1.41 | 1.32.
-PairPlan plan_dq_pair(const ra_bwd_step_params& p) {
-  int64_t total;
-  int most;
-  count_key_tiles(p.bias, p.Lq, p.Lk, total, most);
-  PairPlan r{true, 1, std::max(most, 1), kHeadGroup};
-  const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lq + kPairRowsHost - 1) / kPairRowsHost;
-  if (long_stretches(p.bias, p.D, heads * rows, total, rows, 160)) r.pair = false;
-  else plan_split(r, heads, rows, total, most, kMinChunk, 4 * heads * p.Lq * p.D, p.bias, shares_beside(p));
-  if (one_by_one(p.bias, total, most, rows)) r.group = 1;
+// beside: dK and dV run in the same launch, if that is what comes out (plan_bwd_pair).
+PairPlan plan_dq_pair(const ra_bwd_step_params& p, const TileCount& c, bool beside) {
+  PairPlan r{true, 1, std::max(c.most, 1), kHeadGroup};
+  if (long_stretches(p.bias, p.D, c.heads * c.rows, c.total, c.rows, 160)) r.pair = false;
+  else plan_split(r, c.heads, c.rows, c.total, c.most, kMinChunk, 4 * c.heads * p.Lq * p.D, p.bias, beside);
+  if (one_by_one(p.bias, c.total, c.most, c.rows)) r.group = 1;
   return r;
-}
-// Whether both gradients' workgroups go into one launch: the second kind fills the places that the first one's last round leaves
-// empty.  Two launches | one, us: causal, D=128, 6000, H=16 493 | 488, 4096, H=8 180 | 163; D=64, 2048, B=2, H=16 112 | 97; D=32, 8192, H=16 338 |
-// 312; documents of 500 in 32768, H=8 838 | 793, of 3500 in 10112, causal, H=4, D=80 352 | 278; prefix 4096, B=2, H=16 586 | 576; unmasked 3000,
-// H=24 441 | 370.  Past eight rounds (at D <= 64 of 768 workgroups: documents of 2000 in 48128, causal, B=2, H=4, 7.8 of them, a pass
-// 1409 | 1296) the last one is a few per cent, and the one launch draws more power
-// without a pause (documents of 1200 + ALiBi, 29696, 24 heads: a pass 3.86 | 4.00 ms).
-bool bwd_in_one_launch(const ra_bwd_step_params& p, const PairPlan& dq, const PairPlan& dkdv) {
-  if (!dq.pair || !dkdv.pair) return false;
-  const int64_t heads = (int64_t)p.B * p.H;
-  auto tiles = [](int L) { return (int64_t)(L + kPairRowsHost - 1) / kPairRowsHost; };
-  const int64_t wgs = heads * (tiles(p.Lq) * dq.n_split + tiles(p.Lk) * dkdv.n_split);
-  const int64_t least = small_ones_apart(p.bias, p.D) ? (p.D == 64 ? 12 : 7) * kPairSlots / 4 : 0;
-  return wgs >= least && wgs <= (p.D <= 64 ? 12 : 8) * kPairSlots;
 }
 // dK / dV, in 32-query tiles per 128 keys (dkdv_kernel | dkdv_pair_kernel): uneven rows 65 of them (64 heads of 4096) 0.55 | 0.50 ms,
 // 130 (32 of 8192) 1.08 | 1.04, 258 (32 of 16384) 3.42 | 3.48; even ones 128 (64 of 4096 x 4096) 0.89 | 0.90, 256 (16 of 8192 x 8192) 0.84 |
@@ -839,36 +815,52 @@ bool bwd_in_one_launch(const ra_bwd_step_params& p, const PairPlan& dq, const Pa
 // of 16384: 0.44 | 0.56), even ones if they are long (16 heads of 4096, unmasked 0.230 | 0.233, of 3072 0.158 | 0.153, window of 1024 0.080 |
 // 0.070).  With dQ's workgroups beside them in one launch, which fill what the long slabs leave, they are faster: dkdv_kernel, then dQ | both in
 // one launch, us: causal 16 heads of 4096 269 | 232, 32 of 2048 174 | 136, 4 of 16384 909 | 844, 8 of 8192 478 | 430, with ALiBi 16 of 4096
-// 295 | 246; even rows too, but for long ones that all have a place: unmasked 18 heads of 4096 574 | 486, 9 of 8192 1089 | 958, with ALiBi 1206 |
-// 990, 10 of 8192 1112 | 1045, 16 of 4096 435 | 416, window 4096 of 8192, 8 heads 392 | 358; 8 of 8192 796 | 805, 4 of 16384 1560 | 1620.  (Uneven slabs past two per compute unit stay on dkdv_kernel, which
-// test_gpu_pair.py names: 20 heads of 4096 326 | 306.)  Fewer slabs are shared (12 heads of 2048: 0.056 | 0.050).
-PairPlan plan_dkdv_pair(const ra_bwd_step_params& p) {
+// 295 | 246, 17 of 4096 291 | 256, 20 321 | 295, 70 of 1024 124 | 101, 9 of 8192 533 | 498, 5 of 16384 1078 | 1056, 3 of 24000 1463 | 1467, with ALiBi
+// 18 of 4096 337 | 272; even rows too, but for long ones that all have a place: unmasked 18 heads of 4096 574 | 486, 9 of 8192 1089 | 958, with ALiBi 1206 |
+// 990, 10 of 8192 1112 | 1045, 16 of 4096 435 | 416, window 4096 of 8192, 8 heads 392 | 358; 8 of 8192 796 | 805, 4 of 16384 1560 | 1620.
+// Fewer slabs are shared (12 heads of 2048: 0.056 | 0.050).  beside: as for dQ.
+PairPlan plan_dkdv_pair(const ra_bwd_step_params& p, const TileCount& c, bool beside) {
+  PairPlan r{true, 1, std::max(c.most, 1), kHeadGroup};
+  const int64_t wgs = c.heads * c.rows;
+  const bool one_round = wgs > kPairSlots / 2 && wgs <= kPairSlots * 5 / 4;
+  int tiles = one_round ? (c.even ? 112 : 0) : (p.bias.flags & RA_BIAS_ALIBI) ? 448 : c.even ? 112 : 192;
+  if (one_round && beside) tiles = c.even && wgs <= kPairSlots ? 224 : kWholeRow;
+  if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, c.total, c.rows, tiles)) r.pair = false;
+  else if (c.heads * p.Lq + 31 >= (int64_t)1 << 30) r.pair = false;  // one 32-bit byte offset reaches both statistics of a tile's 32 rows
+  else plan_split(r, c.heads, c.rows, c.total, c.most, 2 * kMinChunk, 8 * c.heads * p.Lk * p.D, p.bias, beside);
+  if (one_by_one(p.bias, c.total, c.most, c.rows)) r.group = 1;
+  return r;
+}
+struct BwdPlan {
+  PairPlan dq, dkdv;
+  bool one_launch;  // of both gradients' workgroups
+};
+// Both gradients: in one launch where both are on the pair kernels and their workgroups take eight rounds at most; the second kind fills
+// the places that the first one's last round leaves empty.  Two launches | one, us: causal, D=128, 512, H=4 46 | 30, 1000, H=8 57 | 41, 640, H=40
+// 72 | 55, 6000, H=16 493 | 488, 4096, H=8 180 | 163; window 1000 of 8192, H=4 88 | 74, 300 of 4096, H=2 48 | 31; D=64 causal 2048, B=2, H=16 112 |
+// 97, unmasked 512, H=4 33 | 23, 2000, H=8 69 | 56, 3000, H=16 156 | 134, 16384, H=1 266 | 253, 128 x 8192, H=8 39 | 32; D=32, 8192, H=16 338 | 312;
+// documents of 500 in 32768, H=8 838 | 793, of 3500 in 10112, causal, H=4, D=80 352 | 278; prefix 4096, B=2, H=16 586 | 576; unmasked 3000,
+// H=24 441 | 370.  Past eight rounds (at D <= 64 of 768 workgroups: documents of 2000 in 48128, causal, B=2, H=4, 7.8 of them, a pass
+// 1409 | 1296) the last one is a few per cent, and the one launch draws more power
+// without a pause (documents of 1200 + ALiBi, 29696, 24 heads: a pass 3.86 | 4.00 ms).
+BwdPlan plan_bwd_pair(const ra_bwd_step_params& p) {
+  const int64_t heads = (int64_t)p.B * p.H;
+  TileCount q{heads, (p.Lq + kPairRowsHost - 1) / kPairRowsHost, 0, 0, false}, k{heads, (p.Lk + kPairRowsHost - 1) / kPairRowsHost, 0, 0, false};
+  count_key_tiles(p.bias, p.Lq, p.Lk, q.total, q.most);
   const int ntiles = (p.Lq + 31) / 32;
   const ra::BiasArgs b = to_bias(p.bias);
-  int64_t total = 0;
-  int most = 0;
   for (int k0 = 0; k0 < p.Lk; k0 += kPairRowsHost) {
     int lo, hi;
     ra::query_tile_range(b.flags, b.window, b.kv_off + k0, b.kv_off + std::min(k0 + kPairRowsHost, p.Lk) - 1, b.q_off, ntiles, 32, lo, hi);
-    total += hi - lo;
-    most = std::max(most, hi - lo);
+    k.total += hi - lo;
+    k.most = std::max(k.most, hi - lo);
   }
-  PairPlan r{true, 1, std::max(most, 1), kHeadGroup};
-  const int64_t heads = (int64_t)p.B * p.H, rows = (p.Lk + kPairRowsHost - 1) / kPairRowsHost, wgs = heads * rows;
-  const bool one_round = wgs > kPairSlots / 2 && wgs <= kPairSlots * 5 / 4;
-  const bool even = even_rows(total, most, rows);
-  int tiles = one_round ? (even ? 112 : 0) : (p.bias.flags & RA_BIAS_ALIBI) ? 448 : even ? 112 : 192;
-  auto split = [&](PairPlan& x) { plan_split(x, heads, rows, total, most, 2 * kMinChunk, 8 * heads * p.Lk * p.D, p.bias, shares_beside(p)); };
-  if (one_round && (even || wgs <= kPairSlots) && p.D == 128) {
-    PairPlan beside = r;
-    split(beside);
-    if (bwd_in_one_launch(p, plan_dq_pair(p), beside)) tiles = even && wgs <= kPairSlots ? 224 : kWholeRow;
-  }
-  if (long_stretches(p.bias, p.D, one_round ? kPairSlots + 1 : wgs, total, rows, tiles)) r.pair = false;
-  else if (heads * p.Lq + 31 >= (int64_t)1 << 30) r.pair = false;  // one 32-bit byte offset reaches both statistics of a tile's 32 rows
-  else split(r);
-  if (one_by_one(p.bias, total, most, rows)) r.group = 1;
-  return r;
+  q.even = even_rows(q.total, q.most, q.rows);
+  k.even = even_rows(k.total, k.most, k.rows);
+  const BwdPlan r{plan_dq_pair(p, q, true), plan_dkdv_pair(p, k, true), true};
+  const int64_t wgs = heads * (q.rows * r.dq.n_split + k.rows * r.dkdv.n_split);
+  if (r.dq.pair && r.dkdv.pair && wgs <= (p.D <= 64 ? 12 : 8) * kPairSlots) return r;
+  return {plan_dq_pair(p, q, false), plan_dkdv_pair(p, k, false), false};
 }
 // The workspace of ra_bwd_pair: the rows' statistics, then the shares of dQ and of dK and dV.
 struct BwdSpace {
@@ -1259,7 +1251,8 @@ static int convert_args(const ra_rows* items, int32_t n_items, ra::ConvertArgs& 
 
 static int64_t bwd_pair_workspace(const ra_bwd_step_params* p, bool any_dim) {
   if (!p || check_dims(p->B, p->H, p->Lq, p->Lk, p->D, any_dim)) return 0;
-  return bwd_space(*p, plan_dq_pair(*p), plan_dkdv_pair(*p)).total;
+  const BwdPlan plan = plan_bwd_pair(*p);
+  return bwd_space(*p, plan.dq, plan.dkdv).total;
 }
 
 static int bwd_pair(const Before& before, const ra_bwd_step_params* p, bool any_dim, int grad_dtype, const void* out, int32_t out_dtype, int64_t out_stride_b,
@@ -1277,7 +1270,8 @@ static int bwd_pair(const Before& before, const ra_bwd_step_params* p, bool any_
   const RingResult rk{dk, dv, nullptr, grad_dtype, 0, dkv_stride_b, dkv_stride_h, dkv_stride_l, via_bf16};
   if ((rc = check_ring_result("ra_bwd_pair", rq, true)) || (rc = check_ring_result("ra_bwd_pair", rk, true))) return rc;
   if (!dv) return fail(RA_ERR_NULL, "ra_bwd_pair: dv is NULL");
-  const PairPlan plan_q = plan_dq_pair(*p), plan_k = plan_dkdv_pair(*p);
+  const BwdPlan plan = plan_bwd_pair(*p);
+  const PairPlan &plan_q = plan.dq, &plan_k = plan.dkdv;
   if (!plan_k.pair && narrow(c.D)) return fail(RA_ERR_TOO_LARGE, "ra_bwd_whole: too many rows");
   const BwdSpace sp = bwd_space(*p, plan_q, plan_k);
   if (!workspace || !aligned16(workspace)) return fail(RA_ERR_ALIGN, "ra_bwd_pair: the workspace must be 16-byte aligned");
@@ -1355,7 +1349,7 @@ static int bwd_pair(const Before& before, const ra_bwd_step_params* p, bool any_
     hipError_t err = ra::launch_bwd_pair(kv, q, c.D, mode, (hipStream_t)stream);
     return err == hipSuccess ? RA_OK : hip_fail(err, "ra_bwd_pair launch");
   };
-  if (bwd_in_one_launch(c, plan_q, plan_k)) return on_pair(&dkdv, &dq_args);
+  if (plan.one_launch) return on_pair(&dkdv, &dq_args);
   // fp32 gradients that lie as the accumulators of a step do are stored by its kernels, which know one pair only and are faster
   // (dK and dV of a causal diagonal and a full pair of 4096, H=16, D=128: 430 us on the several-shard ones, 417 on
   // these; 32768 in two shards 5.21 | 5.15 ms and dQ 2.60 | 2.54)

@@ -521,6 +521,46 @@ def test_both_gradients_in_one_launch(device, mask, Sq, Sk, H, D, dtype):
         assert max(_rel(got.float().cpu().numpy(), x.grad.permute(0, 2, 1, 3).cpu().numpy())) <= GRAD_TOL
 
 
+@pytest.mark.parametrize("mask,S,H,D,forward,backward", [
+    # even rows on up to a quarter more workgroups than places: halved, an odd number of tiles among them
+    ("none", 8100, 9, 128, "halved", "bwd_pair_kernel<128, 0>"), ("none", 4095, 18, 64, "halved", "bwd_pair_kernel<64, 0>"),
+    ("alibi", 8100, 9, 128, "halved", "bwd_pair_kernel<128, 1>"), ("none", 7700, 9, 96, "halved", "bwd_pair_kernel<96, 0>"),
+    # ... up to one and a half times the places: whole, on the same kernel
+    ("none", 4090, 24, 128, "whole", None),
+    # slabs of different lengths, all on their places at once or a few more than there are
+    ("causal", 4090, 16, 128, "whole", "bwd_pair_kernel<128, 0>"), ("causal", 2047, 32, 128, "whole", "bwd_pair_kernel<128, 0>"),
+    ("causal", 16300, 5, 128, "whole", "bwd_pair_kernel<128, 0>"), ("causal", 2300, 30, 128, None, "bwd_pair_kernel<128, 0>"),
+    # slabs of one length, a few more than places; long ones that all have a place stay on the long-stretch kernel
+    ("none", 4090, 18, 128, "halved", "bwd_pair_kernel<128, 0>"), ("none", 8190, 8, 128, "whole", "dkdv_kernel<128, 0, true>")])
+def test_long_rows_about_as_many_as_places(device, mask, S, H, D, forward, backward):
+    g = torch.Generator(device=device).manual_seed(S + H)
+    leaves = [torch.randn((1, S, H, D), device=device, generator=g).to(torch.bfloat16).requires_grad_(True) for _ in range(3)]
+    do = torch.randn((1, S, H, D), device=device, generator=g).to(torch.bfloat16)
+    slopes = torch.logspace(-1, -8, H, base=2, device=device)
+    fn = {"causal": ra.causal_bias(), "alibi": ra.alibi_bias(slopes)}.get(mask)
+    with torch.no_grad():
+        _, launched = _kernels(lambda: ra.ring_attention(*leaves, 1, fn))
+    if forward:
+        assert f"fwd_pair_kernel<{D}, {int(mask == 'alibi')}>" in launched
+        assert any(x.startswith("pair_combine_kernel") for x in launched) == (forward == "halved"), launched
+    out, lse = ra.ring_attention_with_lse(*leaves, 1, fn, out_dtype=torch.float32)
+    grads, launched = _kernels(lambda: torch.autograd.grad(out, leaves, do.float()))
+    assert backward is None or backward in launched, launched
+    at = torch.arange(S, device=device)
+    for h in (0, H // 2, H - 1):
+        ref = [x.detach()[0, :, h].float().requires_grad_(True) for x in leaves]
+        s = ref[0] @ ref[1].T / np.sqrt(D)
+        if mask == "causal":
+            s = s.masked_fill(at[:, None] < at[None], -float("inf"))
+        elif mask == "alibi":
+            s = s - slopes[h] * (at[:, None] - at[None]).abs()
+        want = torch.softmax(s, -1) @ ref[2]
+        assert (out[0, :, h] - want).abs().max() <= OUT_TOL and (lse[0, h] - torch.logsumexp(s, -1)).abs().max() <= LSE_TOL
+        want.backward(do[0, :, h].float())
+        for got, x in zip(grads, ref):
+            assert max(_rel(got[0, :, h].float().cpu().numpy(), x.grad.cpu().numpy())) <= GRAD_TOL
+
+
 @pytest.mark.parametrize("S", [63, 65, 1027, 2049, 4100, 16500])
 @pytest.mark.parametrize("kind", ["documents", "prefix", "both"])
 def test_tile_lists_of_any_length(device, S, kind):

@@ -2,8 +2,8 @@
 // Python code on the way.  Small calls are host code: the forward of 1024 fp32 tokens, H=4, took 32 us of it as a Python
 // autograd function over ctypes for 19 us of kernels, a training call on 2 x 2048 packed tokens 160 for 76; 19 and 91 so.
 //
-// Conversions are those of _convert and _kernel_inputs of ring.py, which the launch schemes of several shards keep; the library's entry
-// points come in as addresses (init), so that it runs on the build that the package has loaded.
+// The library's entry points come in as addresses (init), so that it runs on the build that the package has loaded.  forward and backward
+// are the call without its node and conversions.
 #include <Python.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
@@ -11,6 +11,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/types.h>
 
@@ -47,7 +48,8 @@ void check(const char* what, int code) {
   throw e;
 }
 
-void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+// (a plan on the host has none: tests of this file)
+void* stream(const at::Device& device) { return device.is_cpu() ? nullptr : c10::hip::getCurrentHIPStream().stream(); }
 
 int row_dtype(at::ScalarType t) {
   switch (t) {
@@ -72,7 +74,10 @@ bool rows_of(ra_rows& r, const Tensor& t, void* dst, at::ScalarType to, int64_t 
   return true;
 }
 
-// [b, l, h, *] tensors as new contiguous [b, l, h, d] ones of the dtypes given, in one launch where ra_convert takes them.
+constexpr int kMostArrays = 4;  // (of one ra_convert)
+
+// [b, l, h, *] tensors as new contiguous [b, l, h, d] ones of the dtypes given, in one launch where ra_convert takes them: cast, and cut or padded with zeros.  What it does
+// not take (other dtypes, a head dimension that is not contiguous, more rows than a launch holds) goes through torch.
 void convert(Tensor* const* t, const at::ScalarType* to, int n, int64_t d) {
   std::vector<ra_rows> rows;
   std::vector<Tensor> from;  // (alive until the launch)
@@ -86,7 +91,7 @@ void convert(Tensor* const* t, const at::ScalarType* to, int n, int64_t d) {
     else o.copy_(x.size(3) >= d ? x.narrow(3, 0, d) : at::constant_pad_nd(x, {0, d - x.size(3)}));
     *t[i] = o;
   }
-  if (!rows.empty()) check("ra_convert", g_lib.convert(rows.data(), (int)rows.size(), stream()));
+  if (!rows.empty()) check("ra_convert", g_lib.convert(rows.data(), (int)rows.size(), stream(device)));
 }
 
 // bf16 [b, l, h, d] as the kernels take it: unit inner stride, aligned rows that do not overlap, within the ABI's row stride.
@@ -98,9 +103,10 @@ Tensor ready(const Tensor& t) {
 
 bool is_operand(const Tensor& t, int64_t d) { return t.scalar_type() == at::kBFloat16 && t.size(3) == d; }
 
+// Tensors as the kernels of head dim d take them, in place.
 void operands(Tensor* const* t, int n, int64_t d) {
-  Tensor* todo[3];
-  const at::ScalarType bf16[3] = {at::kBFloat16, at::kBFloat16, at::kBFloat16};
+  Tensor* todo[kMostArrays];
+  const at::ScalarType bf16[kMostArrays] = {at::kBFloat16, at::kBFloat16, at::kBFloat16, at::kBFloat16};
   int m = 0;
   for (int i = 0; i < n; ++i) {
     if (is_operand(*t[i], d)) *t[i] = ready(*t[i]);
@@ -144,6 +150,53 @@ void operand_views(const Plan& p, const variable_list& kept, ra_tensor (&x)[3]) 
 Tensor workspace(int64_t bytes, const at::Device& device) { return bytes ? empty({bytes}, at::kByte, device) : Tensor(); }
 void* pointer(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
+// Output and logsumexp [1, b, h, l] of operands as the kernels take them, or as the `rows` before the call make them.
+variable_list run_forward(const Plan& p, float scale, const variable_list& kept, const ra_rows* rows, int n_rows, at::ScalarType out_dtype) {
+  Tensor out = empty({p.B, p.Lq, p.H, p.D}, out_dtype, p.device), lse = empty({1, p.B, p.H, p.Lq}, at::kFloat, p.device);
+  const Tensor ws = workspace(p.fwd_bytes, p.device);
+  ra_tensor x[3];
+  operand_views(p, kept, x);
+  const ra_fwd_step_params a{(int32_t)p.B, (int32_t)p.H, (int32_t)p.Lq, (int32_t)p.Lk, (int32_t)p.D, scale, x[0], x[1], x[2],
+                             nullptr, nullptr, nullptr, p.bias};
+  check("ra_fwd_call", g_lib.fwd_call(rows, n_rows, &a, out.data_ptr(), row_dtype(out_dtype), p.Lq * p.H * p.D, p.D, p.H * p.D,
+                                      (float*)lse.data_ptr(), pointer(ws), p.fwd_bytes, stream(p.device)));
+  return {out, lse};
+}
+
+// dq, dk and dv, of bf16 precision whatever their dtype.  dout: as the kernels take it, or as `rows` makes it.
+variable_list run_backward(Plan& p, float scale, const variable_list& kept, const Tensor& out, const Tensor& lse, const ra_rows* rows, int n_rows,
+                           const Tensor& dout, at::ScalarType dtype) {
+  Tensor dq, dk, dv;
+  if (kept.size() == 3) {
+    // laid out as the operands; dk and dv have the same strides, which the library stores them with
+    auto like = [&](const Tensor& t, bool preserve) {
+      return at::empty_like(t, t.options().dtype(dtype), preserve ? at::MemoryFormat::Preserve : at::MemoryFormat::Contiguous);
+    };
+    const bool same = kept[1].strides() == kept[2].strides();
+    dq = like(kept[0], true);
+    dk = like(kept[1], same);
+    dv = like(kept[2], same);
+  } else {
+    dq = empty({p.B, p.Lq, p.H, p.D}, dtype, p.device);
+    dk = empty({p.B, p.Lk, p.H, p.D}, dtype, p.device);
+    dv = empty({p.B, p.Lk, p.H, p.D}, dtype, p.device);
+  }
+  ra_tensor x[3];
+  operand_views(p, kept, x);
+  const float* l = (const float*)lse.data_ptr();
+  const ra_bwd_step_params a{(int32_t)p.B, (int32_t)p.H, (int32_t)p.Lq, (int32_t)p.Lk, (int32_t)p.D, scale, x[0], x[1], x[2],
+                             view(dout), l, nullptr, nullptr, nullptr, nullptr, p.bias};
+  int64_t bytes = p.bwd_bytes.load(std::memory_order_relaxed);
+  if (bytes < 0) p.bwd_bytes.store(bytes = g_lib.bwd_workspace(&a), std::memory_order_relaxed);  // (sizes and bias alone decide)
+  const Tensor ws = workspace(bytes, p.device);
+  const ra_tensor o = view(out), gq = view(dq), gk = view(dk);
+  check("ra_bwd_call", g_lib.bwd_call(rows, n_rows, &a, o.ptr, row_dtype(out.scalar_type()), o.stride_b, o.stride_h, o.stride_l,
+                                      row_dtype(dtype) | RA_DTYPE_VIA_BF16, dq.data_ptr(), gq.stride_b, gq.stride_h, gq.stride_l,
+                                      dk.data_ptr(), dv.data_ptr(), gk.stride_b, gk.stride_h, gk.stride_l, pointer(ws), bytes,
+                                      stream(p.device)));
+  return {dq, dk, dv};
+}
+
 class WholeCall : public torch::autograd::Function<WholeCall> {
  public:
   static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, c10::intrusive_ptr<Plan> plan,
@@ -174,14 +227,8 @@ class WholeCall : public torch::autograd::Function<WholeCall> {
       Tensor* x[3] = {&kept[0], &kept[1], &kept[2]};
       operands(x, 3, p.D);
     }
-    Tensor out = empty({p.B, p.Lq, p.H, p.D}, out_dtype, p.device), lse = empty({1, p.B, p.H, p.Lq}, at::kFloat, p.device);
-    const Tensor ws = workspace(p.fwd_bytes, p.device);
-    ra_tensor x[3];
-    operand_views(p, kept, x);
-    const ra_fwd_step_params a{(int32_t)p.B, (int32_t)p.H, (int32_t)p.Lq, (int32_t)p.Lk, (int32_t)p.D, call->scale, x[0], x[1], x[2],
-                               nullptr, nullptr, nullptr, p.bias};
-    check("ra_fwd_call", g_lib.fwd_call(rows, n_rows, &a, out.data_ptr(), row_dtype(out_dtype), p.Lq * p.H * p.D, p.D, p.H * p.D,
-                                        (float*)lse.data_ptr(), pointer(ws), p.fwd_bytes, stream()));
+    variable_list got = run_forward(p, call->scale, kept, rows, n_rows, out_dtype);
+    Tensor out = got[0], lse = got[1];
     kept.push_back(out);
     kept.push_back(lse);
     ctx->save_for_backward(kept);
@@ -206,21 +253,6 @@ class WholeCall : public torch::autograd::Function<WholeCall> {
     // as the caller wants them, where that takes no cut
     const bool direct = call->dim == p.D && row_dtype(call->given[0]) >= 0 && call->given[0] == call->given[1] && call->given[0] == call->given[2];
     const at::ScalarType dtype = direct ? call->given[0] : at::kBFloat16;
-    Tensor dq, dk, dv;
-    if (kept.size() == 3) {
-      // laid out as the operands; dk and dv have the same strides, which the library stores them with
-      auto like = [&](const Tensor& t, bool preserve) {
-        return at::empty_like(t, t.options().dtype(dtype), preserve ? at::MemoryFormat::Preserve : at::MemoryFormat::Contiguous);
-      };
-      const bool same = kept[1].strides() == kept[2].strides();
-      dq = like(kept[0], true);
-      dk = like(kept[1], same);
-      dv = like(kept[2], same);
-    } else {
-      dq = empty({p.B, p.Lq, p.H, p.D}, dtype, p.device);
-      dk = empty({p.B, p.Lk, p.H, p.D}, dtype, p.device);
-      dv = empty({p.B, p.Lk, p.H, p.D}, dtype, p.device);
-    }
     ra_rows rows;
     int n_rows = 0;
     Tensor made = go;
@@ -233,32 +265,19 @@ class WholeCall : public torch::autograd::Function<WholeCall> {
       Tensor* t = &made;
       operands(&t, 1, p.D);
     }
-    ra_tensor x[3];
-    operand_views(p, kept, x);
-    const float* l = (const float*)lse.data_ptr();
-    const ra_bwd_step_params a{(int32_t)p.B, (int32_t)p.H, (int32_t)p.Lq, (int32_t)p.Lk, (int32_t)p.D, call->scale, x[0], x[1], x[2],
-                               view(made), l, nullptr, nullptr, nullptr, nullptr, p.bias};
-    int64_t bytes = p.bwd_bytes.load(std::memory_order_relaxed);
-    if (bytes < 0) p.bwd_bytes.store(bytes = g_lib.bwd_workspace(&a), std::memory_order_relaxed);  // (sizes and bias alone decide)
-    const Tensor ws = workspace(bytes, p.device);
-    const ra_tensor o = view(out), gq = view(dq), gk = view(dk);
-    check("ra_bwd_call", g_lib.bwd_call(&rows, n_rows, &a, o.ptr, row_dtype(out.scalar_type()), o.stride_b, o.stride_h, o.stride_l,
-                                        row_dtype(dtype) | RA_DTYPE_VIA_BF16, dq.data_ptr(), gq.stride_b, gq.stride_h, gq.stride_l,
-                                        dk.data_ptr(), dv.data_ptr(), gk.stride_b, gk.stride_h, gk.stride_l, pointer(ws), bytes,
-                                        stream()));
-    Tensor* g[3] = {&dq, &dk, &dv};
+    variable_list grads = run_backward(p, call->scale, kept, out, lse, &rows, n_rows, made, dtype);
     Tensor* todo[3];
     at::ScalarType to[3];
     int n = 0;
     for (int i = 0; i < 3; ++i)
       if (ctx->needs_input_grad(i) && (call->dim != p.D || call->given[i] != dtype)) {
-        todo[n] = g[i];
+        todo[n] = &grads[i];
         to[n++] = call->given[i];
       }
     if (n) convert(todo, to, n, call->dim);
     for (int i = 0; i < 3; ++i)
-      if (!ctx->needs_input_grad(i)) *g[i] = Tensor();
-    return {dq, dk, dv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+      if (!ctx->needs_input_grad(i)) grads[i] = Tensor();
+    return {grads[0], grads[1], grads[2], Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -312,47 +331,166 @@ PyObject* plan(PyObject*, PyObject* args) {
   END_HANDLE_TH_ERRORS
 }
 
+const c10::intrusive_ptr<Plan>& plan_of(PyObject* capsule) {
+  auto* p = static_cast<c10::intrusive_ptr<Plan>*>(PyCapsule_GetPointer(capsule, kPlanName));
+  if (!p) throw python_error();
+  return *p;
+}
+double scale_of(PyObject* x) {
+  const double scale = PyFloat_AsDouble(x);
+  if (scale == -1.0 && PyErr_Occurred()) throw python_error();
+  return scale;
+}
+at::ScalarType dtype_of(PyObject* x) {
+  TORCH_CHECK_TYPE(THPDtype_Check(x), "a dtype is expected");
+  return reinterpret_cast<THPDtype*>(x)->scalar_type;
+}
+const Tensor& tensor_of(PyObject* x) {
+  TORCH_CHECK_TYPE(THPVariable_Check(x), "a tensor is expected");
+  return THPVariable_Unpack(x);
+}
+PyObject* tuple_of(variable_list&& tensors) {
+  THPObjectPtr r(PyTuple_New((Py_ssize_t)tensors.size()));
+  if (!r) throw python_error();
+  for (size_t i = 0; i < tensors.size(); ++i) PyTuple_SET_ITEM(r.get(), (Py_ssize_t)i, THPVariable_Wrap(std::move(tensors[i])));
+  return r.release();
+}
+
+// Pointers and strides are all that goes on from here.
+void check_operands(const Plan& of, const Tensor& q, const Tensor& k, const Tensor& v) {
+  const int64_t d = q.dim() == 4 ? q.size(3) : -1;
+  TORCH_CHECK(d <= of.D && q.sizes() == at::IntArrayRef({of.B, of.Lq, of.H, d}) && k.sizes() == at::IntArrayRef({of.B, of.Lk, of.H, d}) &&
+                  v.sizes() == k.sizes() && q.device() == of.device && k.device() == of.device && v.device() == of.device,
+              "q ", q.sizes(), ", k ", k.sizes(), " and v ", v.sizes(), " are not the operands of this plan");
+}
+
 // attend(q, k, v, plan, scale, the kernels' output dtype, the caller's) -> output, logsumexp [1, b, h, l]
 PyObject* attend(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  TORCH_CHECK_TYPE(n == 7 && THPVariable_Check(args[0]) && THPVariable_Check(args[1]) && THPVariable_Check(args[2]) && THPDtype_Check(args[5]) &&
-                       THPDtype_Check(args[6]),
-                   "attend(q, k, v, plan, scale, dtype, dtype)");
-  auto* p = static_cast<c10::intrusive_ptr<Plan>*>(PyCapsule_GetPointer(args[3], kPlanName));
-  if (!p) throw python_error();
-  const double scale = PyFloat_AsDouble(args[4]);
-  if (scale == -1.0 && PyErr_Occurred()) throw python_error();
-  const Tensor& q = THPVariable_Unpack(args[0]);
-  Tensor k = THPVariable_Unpack(args[1]), v = THPVariable_Unpack(args[2]);
-  for (Tensor* t : {&k, &v})
-    if (t->device() != q.device()) {  // (the kernels take pointers; the bias arrays went the same way)
-      pybind11::gil_scoped_release no_gil;
-      *t = t->to(q.device());
-    }
-  const Plan& of = **p;
-  const int64_t d = q.dim() == 4 ? q.size(3) : -1;
-  // (pointers and strides are all that goes on from here)
-  TORCH_CHECK(d <= of.D && q.sizes() == at::IntArrayRef({of.B, of.Lq, of.H, d}) && k.sizes() == at::IntArrayRef({of.B, of.Lk, of.H, d}) &&
-                  v.sizes() == k.sizes() && q.device() == of.device,
-              "attend: q ", q.sizes(), " on ", q.device(), ", k ", k.sizes(), " and v ", v.sizes(), " are not the operands of this plan");
-  const bool any_grad = q.requires_grad() || k.requires_grad() || v.requires_grad();
-  const at::ScalarType dtype = reinterpret_cast<THPDtype*>(args[5])->scalar_type, final_dtype = reinterpret_cast<THPDtype*>(args[6])->scalar_type;
+  TORCH_CHECK_TYPE(n == 7, "attend(q, k, v, plan, scale, dtype, dtype)");
+  const Tensor& q = tensor_of(args[0]);
+  Tensor k = tensor_of(args[1]), v = tensor_of(args[2]);
+  const c10::intrusive_ptr<Plan> p = plan_of(args[3]);
+  const double scale = scale_of(args[4]);
+  const at::ScalarType dtype = dtype_of(args[5]), final_dtype = dtype_of(args[6]);
   variable_list got;
   {
     pybind11::gil_scoped_release no_gil;  // (allocations may wait for the GPU)
-    got = WholeCall::apply(q, k, v, *p, scale, dtype, final_dtype, any_grad);
+    for (Tensor* t : {&k, &v})
+      if (t->device() != q.device()) *t = t->to(q.device());  // (as the bias arrays are)
+    check_operands(*p, q, k, v);
+    const bool any_grad = q.requires_grad() || k.requires_grad() || v.requires_grad();
+    got = WholeCall::apply(q, k, v, p, scale, dtype, final_dtype, any_grad);
   }
-  PyObject* r = PyTuple_New(2);
-  if (!r) throw python_error();
-  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(std::move(got[0])));
-  PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(std::move(got[1])));
-  return r;
+  return tuple_of(std::move(got));
+  END_HANDLE_TH_ERRORS
+}
+
+void check_ready(const Plan& p, const variable_list& kept) {
+  check_operands(p, kept[0], kept[1], kept[2]);
+  for (const Tensor& t : kept) TORCH_CHECK(is_operand(t, p.D), "operands of bf16 and head dim ", p.D, " are expected, not of ", t.scalar_type(), " and ", t.size(3));
+}
+
+// forward(q, k, v, plan, scale, dtype) -> output, logsumexp, of operands as the kernels take them (operands)
+PyObject* forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 6, "forward(q, k, v, plan, scale, dtype)");
+  const variable_list kept{tensor_of(args[0]), tensor_of(args[1]), tensor_of(args[2])};
+  Plan& p = *plan_of(args[3]);
+  const double scale = scale_of(args[4]);
+  const at::ScalarType dtype = dtype_of(args[5]);
+  variable_list got;
+  {
+    pybind11::gil_scoped_release no_gil;
+    check_ready(p, kept);
+    got = run_forward(p, (float)scale, kept, nullptr, 0, dtype);
+  }
+  return tuple_of(std::move(got));
+  END_HANDLE_TH_ERRORS
+}
+
+// backward(q, k, v, output, logsumexp, dout, plan, scale) -> bf16 dq, dk, dv; dout too as the kernels take it
+PyObject* backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 8, "backward(q, k, v, output, logsumexp, dout, plan, scale)");
+  const variable_list kept{tensor_of(args[0]), tensor_of(args[1]), tensor_of(args[2])};
+  const Tensor out = tensor_of(args[3]), lse = tensor_of(args[4]), dout = tensor_of(args[5]);
+  Plan& p = *plan_of(args[6]);
+  const double scale = scale_of(args[7]);
+  variable_list got;
+  {
+    pybind11::gil_scoped_release no_gil;
+    check_ready(p, kept);
+    TORCH_CHECK(out.sizes() == kept[0].sizes() && dout.sizes() == kept[0].sizes() && lse.numel() == p.B * p.H * p.Lq && out.device() == p.device &&
+                    dout.device() == p.device && lse.device() == p.device,
+                "output ", out.sizes(), ", its gradient ", dout.sizes(), " and logsumexp ", lse.sizes(), " are not those of q ", kept[0].sizes());
+    got = run_backward(p, (float)scale, kept, out, lse, nullptr, 0, dout, at::kBFloat16);
+  }
+  return tuple_of(std::move(got));
+  END_HANDLE_TH_ERRORS
+}
+
+variable_list tensors_of(PyObject* seq) {
+  THPObjectPtr fast(PySequence_Fast(seq, "a sequence of tensors is expected"));
+  if (!fast) throw python_error();
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(fast.get());
+  TORCH_CHECK(n >= 1 && n <= kMostArrays, "1 to ", kMostArrays, " arrays at a time (got ", n, ")");
+  variable_list got;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    got.push_back(tensor_of(PySequence_Fast_GET_ITEM(fast.get(), i)));
+    TORCH_CHECK(got.back().dim() == 4, "[b, l, h, d] arrays are expected, not ", got.back().sizes());
+  }
+  return got;
+}
+
+// convert(tensors, dtypes, d) -> new contiguous [b, l, h, d] tensors
+PyObject* convert_arrays(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 3, "convert(tensors, dtypes, d)");
+  variable_list t = tensors_of(args[0]);
+  THPObjectPtr dtypes(PySequence_Fast(args[1], "a sequence of dtypes is expected"));
+  if (!dtypes) throw python_error();
+  TORCH_CHECK(PySequence_Fast_GET_SIZE(dtypes.get()) == (Py_ssize_t)t.size(), "a dtype for each tensor is expected");
+  const int64_t d = PyLong_AsLongLong(args[2]);
+  if (d == -1 && PyErr_Occurred()) throw python_error();
+  Tensor* at[kMostArrays];
+  at::ScalarType to[kMostArrays];
+  for (size_t i = 0; i < t.size(); ++i) {
+    at[i] = &t[i];
+    to[i] = dtype_of(PySequence_Fast_GET_ITEM(dtypes.get(), (Py_ssize_t)i));
+  }
+  {
+    pybind11::gil_scoped_release no_gil;
+    convert(at, to, (int)t.size(), d);
+  }
+  return tuple_of(std::move(t));
+  END_HANDLE_TH_ERRORS
+}
+
+// operands(tensors, d) -> the tensors as the kernels of head dim d take them: themselves where they can be
+PyObject* operand_arrays(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 2, "operands(tensors, d)");
+  variable_list t = tensors_of(args[0]);
+  const int64_t d = PyLong_AsLongLong(args[1]);
+  if (d == -1 && PyErr_Occurred()) throw python_error();
+  Tensor* at[kMostArrays];
+  for (size_t i = 0; i < t.size(); ++i) at[i] = &t[i];
+  {
+    pybind11::gil_scoped_release no_gil;
+    operands(at, (int)t.size(), d);
+  }
+  return tuple_of(std::move(t));
   END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef g_methods[] = {{"init", init, METH_VARARGS, nullptr},
                            {"plan", plan, METH_VARARGS, nullptr},
                            {"attend", (PyCFunction)(void (*)(void))attend, METH_FASTCALL, nullptr},
+                           {"convert", (PyCFunction)(void (*)(void))convert_arrays, METH_FASTCALL, nullptr},
+                           {"operands", (PyCFunction)(void (*)(void))operand_arrays, METH_FASTCALL, nullptr},
+                           {"forward", (PyCFunction)(void (*)(void))forward, METH_FASTCALL, nullptr},
+                           {"backward", (PyCFunction)(void (*)(void))backward, METH_FASTCALL, nullptr},
                            {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_host", "Calls on whole sequences without Python code on the way.", -1, g_methods};
 

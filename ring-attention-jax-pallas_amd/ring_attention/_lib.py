@@ -67,6 +67,15 @@ class RaBwdStepParams(C.Structure):
     ]
 
 
+class RaRows(C.Structure):  # (packed by csrc/ra_host.cc in the package's own calls)
+    _fields_ = [
+        ("src", C.c_void_p), ("dst", C.c_void_p), ("src_dtype", C.c_int32), ("dst_dtype", C.c_int32),
+        ("src_d", C.c_int32), ("dst_d", C.c_int32), ("B", C.c_int32), ("L", C.c_int32), ("H", C.c_int32),
+        ("src_stride_b", C.c_int64), ("src_stride_l", C.c_int64), ("src_stride_h", C.c_int64),
+        ("dst_stride_b", C.c_int64), ("dst_stride_l", C.c_int64), ("dst_stride_h", C.c_int64),
+    ]
+
+
 EXPORTS = {
     "ra_version": (C.c_int, []),
     "ra_last_error": (C.c_char_p, []),

@@ -30,7 +30,6 @@ import collections
 import ctypes as C
 import functools
 import math
-import struct
 from dataclasses import dataclass
 from typing import Callable, Optional, Union
 
@@ -123,57 +122,20 @@ def _view_bhld(t: torch.Tensor) -> _lib.RaTensor:
     return _lib.RaTensor(t.data_ptr(), t.stride(0), t.stride(1), t.stride(2))
 
 
-def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
-    """[b, l, h, d] as the kernels take it: bf16, unit inner stride, 16-byte aligned rows that do not
-    overlap and lie within the row stride the C ABI admits; anything else is copied."""
-    if t.dtype != torch.bfloat16:
-        t = t.to(torch.bfloat16)
-    ok = (t.stride(-1) == 1 and all(s % 8 == 0 for s in t.stride()[:-1]) and t.data_ptr() % 16 == 0
-          and t.shape[-1] <= t.stride(1) <= _lib.RA_MAX_ROW_STRIDE)
-    return t if ok else t.contiguous()
-
-
 def _kernel_dim(d: int) -> int:
     """The head dim that the kernels compute a head dim of ``d`` in."""
     return 64 if d <= 64 else 128
 
 
-_ROW_DTYPES = {torch.bfloat16: _lib.RA_DTYPE_BF16, torch.float32: _lib.RA_DTYPE_F32, torch.float16: _lib.RA_DTYPE_F16}
-
-
-_ROWS = struct.Struct("PP7i4x6q")  # an ra_rows: packed in one call, where a ctypes block costs 3 us each
-
-
 def _convert(tensors, dtypes, d: int):
-    """[b, l, h, *] tensors as new contiguous [b, l, h, d] ones of the dtypes given: cast, and cut or
-    padded with zeros, in one launch (``ra_convert``).  What that does not take (other dtypes, a head
-    dimension that is not contiguous, more rows than a launch holds) goes through torch."""
-    out, items, n = [], b"", 0
-    dev = tensors[0].device
-    for t, dtype in zip(tensors, dtypes):
-        B, L, H, dt = t.shape
-        o = torch.empty((B, L, H, d), dtype=dtype, device=dev)
-        out.append(o)
-        src, dst = _ROW_DTYPES.get(t.dtype), _ROW_DTYPES.get(dtype)
-        sb, sl, sh, sd = t.stride()
-        if (src is not None and dst is not None and sd == 1 and t.is_cuda and t.device == dev and B < 65536
-                and 0 < B * L * H and L * H < 1 << 27):
-            items += _ROWS.pack(t.data_ptr(), o.data_ptr(), src, dst, dt, d, B, L, H, sb, sl, sh, L * H * d, H * d, d)
-            n += 1
-        else:
-            o.copy_(t[..., :d] if dt >= d else torch.nn.functional.pad(t, (0, d - dt)))
-    if n:
-        _lib.check("ra_convert", _lib.load().ra_convert(items, n, _stream()))
-    return out
+    """[b, l, h, *] tensors as new contiguous [b, l, h, d] ones of the dtypes given, in one launch (``csrc/ra_host.cc``)."""
+    return _lib.host().convert(tensors, dtypes, d)
 
 
 def _kernel_inputs(tensors, d: int):
-    """``_kernel_ready`` for several tensors at once, padded to the kernels' head dim ``d``."""
-    todo = [t for t in tensors if t.dtype != torch.bfloat16 or t.shape[3] != d]
-    if not todo:
-        return [_kernel_ready(t) for t in tensors]
-    new = iter(_convert(todo, [torch.bfloat16] * len(todo), d))
-    return [next(new) if t.dtype != torch.bfloat16 or t.shape[3] != d else _kernel_ready(t) for t in tensors]
+    """[b, l, h, *] tensors as the kernels take them: bf16 of head dim ``d``, unit inner stride, 16-byte aligned rows that do not
+    overlap and lie within the row stride the C ABI admits; anything else is copied."""
+    return _lib.host().operands(tensors, d)
 
 
 # --------------------------------------------------------------------------------------
@@ -551,31 +513,17 @@ class _RingPlan:
         plan.D = self.d_pair
         return plan
 
-    def pair_call(self, backward: bool):
-        """What the calls on a ring of one shard share: the bias block, and the size of the workspace of the forward or
-        the backward.  The plan holds the arrays."""
-        got = self.__dict__.get("_pair_call")
-        if got is None:
-            bias = self.block_bias(0, 0)
-            made = _bias_struct(bias, self.device, (self.B, self.H, self.Lq, self.Lk), summary=False)
-            got = self.__dict__["_pair_call"] = {"bias": bytes(made), "arrays": bias, "made": made}
-        size = got.get(backward)
-        if size is None:
-            p = (_lib.RaBwdStepParams if backward else _lib.RaFwdStepParams)(self.B, self.H, self.Lq, self.Lk, self.D, 1.0)
-            p.bias = got["made"]
-            lib = _lib.load()
-            size = got[backward] = (lib.ra_bwd_whole_workspace if backward else lib.ra_fwd_whole_workspace)(C.byref(p))
-        return got["bias"], size
-
     def native(self, like):
-        """``pair_call`` as ``csrc/ra_host.cc`` keeps it, which sizes the backward's workspace itself when a backward comes; ``like``:
-        a tensor on the plan's device."""
+        """What the calls on a ring of one shard share, as ``csrc/ra_host.cc`` keeps it: sizes, the bias block with its arrays, and the
+        size of the forward's workspace (the backward's is counted when a backward comes).  ``like``: a tensor on the plan's device."""
         got = self.__dict__.get("_native")
         if got is None:
-            bias, forward = self.pair_call(False)
-            arrays = self.__dict__["_pair_call"]["arrays"]
-            got = self.__dict__["_native"] = _lib.host().plan(self.B, self.H, self.Lq, self.Lk, self.D, bias, forward, like,
-                                                              () if arrays is None else tuple(arrays._keep))
+            bias = self.block_bias(0, 0)
+            p = _lib.RaFwdStepParams(self.B, self.H, self.Lq, self.Lk, self.D, 1.0)
+            p.bias = _bias_struct(bias, self.device, (self.B, self.H, self.Lq, self.Lk), summary=False)
+            got = self.__dict__["_native"] = _lib.host().plan(self.B, self.H, self.Lq, self.Lk, self.D, bytes(p.bias),
+                                                              _lib.load().ra_fwd_whole_workspace(C.byref(p)), like,
+                                                              () if bias is None else tuple(bias._keep))
         return got
 
     def live_steps(self, qs: Optional[int], ks: Optional[int]) -> int:
@@ -821,57 +769,11 @@ def _view_blhd(t: torch.Tensor) -> "_lib.RaTensor":
     return _lib.RaTensor(t.data_ptr(), sb, sh, sl)
 
 
-# The blocks of one call on a whole sequence, up to the bias: packed in one call where ctypes structures cost 10 us.
-_FWD_HEAD = struct.Struct("5if12q24x")     # sizes, scale, q, k, v (pointer, strides of batch, head, row); no carry
-_BWD_HEAD = struct.Struct("5if16qq32x")  # ... and dO, the logsumexp; no delta, no accumulators
-
-
-def _rows_of(t: torch.Tensor):
-    sb, sl, sh, _ = t.stride()
-    return t.data_ptr(), sb, sh, sl
-
-
 def _empty_gradients(q, k, v):
     """dq, dk and dv, not yet written, laid out as the operands [b, l, h, d].  The kernels store dk and dv with the same strides:
     where k and v differ in theirs (rotary embeddings leave k transposed and v as it was, say) both are contiguous."""
     kv_format = torch.preserve_format if k.stride() == v.stride() else torch.contiguous_format
     return [torch.empty_like(q), *(torch.empty_like(x, memory_format=kv_format) for x in (k, v))]
-
-
-def _workspace(size: int, device):
-    if not size:
-        return None, None
-    ws = torch.empty((size,), dtype=torch.uint8, device=device)
-    return ws, ws.data_ptr()
-
-
-def _pair_forward(kept, plan: "_RingPlan", sm_scale, out_dtype):
-    """``_ring_forward_fused`` of a ring of one shard: one call."""
-    B, H, D, Lq = plan.B, plan.H, plan.D, plan.Lq
-    out = torch.empty((B, Lq, H, D), dtype=out_dtype, device=plan.device)
-    lse = torch.empty((1, B, H, Lq), dtype=torch.float32, device=plan.device)
-    bias, size = plan.pair_call(False)
-    q, k, v = (_rows_of(x) for x in kept)
-    ws, ws_ptr = _workspace(size, plan.device)
-    _lib.check("ra_fwd_call", _lib.load().ra_fwd_call(
-        b"", 0, _FWD_HEAD.pack(B, H, Lq, plan.Lk, D, sm_scale, *q, *k, *v) + bias, out.data_ptr(), _DTYPE_CODE[out_dtype],
-        Lq * H * D, D, H * D, lse.data_ptr(), ws_ptr, size, _stream()))
-    return out, lse
-
-
-def _pair_backward(kept, out, lse, do, plan: "_RingPlan", sm_scale):
-    """``_ring_backward_fused`` of a ring of one shard: one call for all launches."""
-    B, H, D, Lq, Lk = plan.B, plan.H, plan.D, plan.Lq, plan.Lk
-    dq, dk, dv = grads = _empty_gradients(*kept)
-    bias, size = plan.pair_call(True)
-    q, k, v = (_rows_of(x) for x in kept)
-    ws, ws_ptr = _workspace(size, plan.device)
-    (_, qb, qh, ql), (_, kb, kh, kl), (_, ob, oh, ol) = _rows_of(dq), _rows_of(dk), _rows_of(out)
-    _lib.check("ra_bwd_call", _lib.load().ra_bwd_call(
-        b"", 0, _BWD_HEAD.pack(B, H, Lq, Lk, D, sm_scale, *q, *k, *v, *_rows_of(do), lse.data_ptr()) + bias,
-        out.data_ptr(), _DTYPE_CODE[out.dtype], ob, oh, ol, _lib.RA_DTYPE_BF16 | _lib.RA_DTYPE_VIA_BF16, dq.data_ptr(), qb, qh, ql,
-        dk.data_ptr(), dv.data_ptr(), kb, kh, kl, ws_ptr, size, _stream()))
-    return grads
 
 
 def _ring_forward_fused(q, k, v, plan: _RingPlan, sm_scale, out_dtype, timer=_NO_TIMER, whole=True):
@@ -883,7 +785,7 @@ def _ring_forward_fused(q, k, v, plan: _RingPlan, sm_scale, out_dtype, timer=_NO
     if plan.callable is not None:
         return _ring_forward_rows(q, k, v, plan, sm_scale, out_dtype, timer)
     if plan.n == 1 and whole and timer is _NO_TIMER:
-        return _pair_forward((q, k, v), plan, sm_scale, out_dtype)
+        return _lib.host().forward(q, k, v, plan.native(q), float(sm_scale), out_dtype)
     n, B, H, D, Lq, Lk = plan.n, plan.B, plan.H, plan.D, plan.Lq, plan.Lk
     dev = q.device
     lib = _lib.load()
@@ -940,7 +842,7 @@ def _ring_backward_fused(q, k, v, out, lse, do, plan: _RingPlan, sm_scale, timer
     if plan.callable is not None:
         return _ring_backward_rows(q, k, v, out, lse, do, plan, sm_scale, timer)
     if plan.n == 1 and whole and timer is _NO_TIMER:
-        return _pair_backward((q, k, v), out, lse, do, plan, sm_scale)
+        return _lib.host().backward(q, k, v, out, lse, do, plan.native(q), float(sm_scale))
     n, B, H, D, Lq, Lk = plan.n, plan.B, plan.H, plan.D, plan.Lq, plan.Lk
     dev = q.device
     lib = _lib.load()

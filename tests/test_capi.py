@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from oracle import ring_oracle as R
-from ring_attention import _lib, ring
+from ring_attention import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "ring_attention_hip.h")
@@ -343,7 +343,7 @@ def test_rows_beyond_a_32_bit_offset_are_refused_without_a_gpu(lib):
 
 def _rows(**kw):
     a = {**dict(src=0x1000, dst=0x2000, sd=_lib.RA_DTYPE_F32, dd=_lib.RA_DTYPE_BF16, d=96, to=128, B=1, L=4, H=2), **kw}
-    return ring._ROWS.pack(a["src"], a["dst"], a["sd"], a["dd"], a["d"], a["to"], a["B"], a["L"], a["H"], 0, 192, 96, 0, 256, 128)
+    return bytes(_lib.RaRows(a["src"], a["dst"], a["sd"], a["dd"], a["d"], a["to"], a["B"], a["L"], a["H"], 0, 192, 96, 0, 256, 128))
 
 
 def test_convert_rejects_bad_arguments_without_a_gpu(lib):
@@ -366,7 +366,7 @@ def test_header_is_plain_c(tmp_path):
         pytest.skip("no gcc")
     src = tmp_path / "hdr.c"
     src.write_text('#include "ring_attention_hip.h"\n#include <stddef.h>\n'
-                   f"typedef char size_of_ra_rows[sizeof(ra_rows) == {ring._ROWS.size} ? 1 : -1];\n"
+                   f"typedef char size_of_ra_rows[sizeof(ra_rows) == {C.sizeof(_lib.RaRows)} ? 1 : -1];\n"
                    "typedef char place_of_strides[offsetof(ra_rows, src_stride_b) == 48 ? 1 : -1];\n"
                    "int main(void) { ra_fwd_step_params p; (void)p; return RA_OK; }\n")
     res = subprocess.run([gcc, "-std=c99", "-Wall", "-Wextra", "-pedantic", "-Werror", "-fsyntax-only",

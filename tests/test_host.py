@@ -271,49 +271,71 @@ def test_views_the_kernels_cannot_take_are_copied():
     # a view is passed through when its rows are 16-byte aligned, do not overlap and lie within the
     # row stride of the C ABI; otherwise the host makes a contiguous copy
     base = torch.zeros((2, 16, 4, 64 + 8), dtype=torch.bfloat16)
+    ready = lambda t: rr._kernel_inputs((t,), 64)[0]
     padded = base[..., :64]                       # row stride 4 * 72, inner stride 1
-    assert rr._kernel_ready(padded) is padded
+    assert ready(padded) is padded
     odd = torch.zeros((2, 16, 4, 65), dtype=torch.bfloat16)[..., :64]   # strides not multiples of 8
-    assert rr._kernel_ready(odd).is_contiguous()
+    assert ready(odd).is_contiguous()
     same_row = torch.zeros((2, 1, 4, 64), dtype=torch.bfloat16).expand(2, 16, 4, 64)   # row stride 0
-    got = rr._kernel_ready(same_row)
+    got = ready(same_row)
     assert got.is_contiguous() and got.shape == same_row.shape
     heads_interleaved = torch.zeros((2, 4, 16, 64), dtype=torch.bfloat16).permute(0, 2, 1, 3)  # [b, l, h, d] view, row stride 64
-    assert rr._kernel_ready(heads_interleaved) is heads_interleaved
-    assert rr._kernel_ready(torch.zeros((1, 8, 1, 64))).dtype == torch.bfloat16
+    assert ready(heads_interleaved) is heads_interleaved
+    assert ready(torch.zeros((1, 8, 1, 64))).dtype == torch.bfloat16
 
 
 @pytest.mark.parametrize("D", [32, 64, 96, 128])
 def test_dk_and_dv_share_their_strides_whatever_those_of_k_and_v(monkeypatch, D):
-    # k a transposed [b, h, l, d], v contiguous, and the other way round: the library stores both gradients with dk's strides
+    # k a transposed [b, h, l, d], v contiguous, and the other way round: the library stores both gradients with dk's strides.  The
+    # native call on host arrays, with functions in the library's place
     calls = []
-
-    class Library:
-        def ra_bwd_whole_workspace(self, p):
-            return 64
-
-        def ra_bwd_call(self, *args):
-            calls.append(args)
-            return 0
-
-    monkeypatch.setattr(rr._lib, "load", Library)
-    monkeypatch.setattr(rr, "_stream", lambda: None)
-    B, L, H = 2, 48, 3
-    rows = torch.zeros((B, L, H, D), dtype=torch.bfloat16)
-    heads = torch.zeros((B, H, L, D), dtype=torch.bfloat16).permute(0, 2, 1, 3)
-    plan = rr._RingPlan(rows, rows, 1, None, None, None).joined()
-    assert plan.D == D
-    for q, k, v in [(heads, heads, rows), (rows, rows, heads), (heads, heads, heads), (heads, rows, rows)]:
-        kept = rr._kernel_inputs((q, k, v), D)
-        assert [x is y for x, y in zip(kept, (q, k, v))] == [True] * 3
-        dq, dk, dv = rr._pair_backward(kept, rows, torch.zeros((1, B, H, L)), rows, plan, 0.1)
-        assert dk.stride() == dv.stride() and (dk.stride() == k.stride() or k.stride() != v.stride())
-        assert dq.stride() == q.stride()
-        sb, sl, sh, _ = dk.stride()
-        assert calls.pop()[-8:-3] == (dk.data_ptr(), dv.data_ptr(), sb, sh, sl)
+    addr, size = C.c_void_p, C.c_int64
+    fwd = C.CFUNCTYPE(C.c_int, addr, C.c_int32, addr, addr, C.c_int32, size, size, size, addr, addr, size, addr)(lambda *args: 0)
+    bwd = C.CFUNCTYPE(C.c_int, addr, C.c_int32, addr, addr, C.c_int32, size, size, size, C.c_int32, addr, size, size, size, addr, addr, size,
+                      size, size, addr, size, addr)(lambda *args: calls.append(args) or 0)
+    room = C.CFUNCTYPE(size, addr)(lambda p: 64)
+    host, lib = rr._lib.host(), rr._lib.load()
+    host.init(*(C.cast(f, addr).value for f in (fwd, bwd, room, lib.ra_convert)), rr._lib.check)
+    try:
+        B, L, H = 2, 48, 3
+        rows = torch.zeros((B, L, H, D), dtype=torch.bfloat16)
+        heads = torch.zeros((B, H, L, D), dtype=torch.bfloat16).permute(0, 2, 1, 3)
+        plan = rr._RingPlan(rows, rows, 1, None, None, None).joined()
+        assert plan.D == D
+        for case in [(heads, heads, rows), (rows, rows, heads), (heads, heads, heads), (heads, rows, rows)]:
+            leaves = [x.detach().requires_grad_(True) for x in case]
+            out, lse = host.attend(*leaves, plan.native(rows), 0.1, torch.bfloat16, torch.bfloat16)
+            node = torch.autograd.grad(out, leaves, rows)
+            plain = host.backward(*case, rows, lse, rows, plan.native(rows), 0.1)
+            for dq, dk, dv in (plain, node):
+                k, v = case[1:]
+                assert dk.stride() == dv.stride() and (dk.stride() == k.stride() or k.stride() != v.stride())
+                assert dq.stride() == case[0].stride()
+                sb, sl, sh, _ = dk.stride()
+                assert calls.pop()[-8:-3] == (dk.data_ptr(), dv.data_ptr(), sb, sh, sl)
+    finally:
+        monkeypatch.setattr(rr._lib, "_host", None)
+        rr._lib.host()
     # the launches of a ring of several shards take their gradients from the same place
     grads = rr._empty_gradients(heads, heads, rows)
     assert grads[1].stride() == grads[2].stride() and grads[0].stride() == heads.stride()
+
+
+@pytest.mark.parametrize("what", ["shape", "dtype", "head dim", "output", "gradient", "logsumexp"])
+def test_the_native_calls_refuse_what_is_not_an_operand(what):
+    x = torch.zeros((2, 48, 3, 64), dtype=torch.bfloat16)
+    lse = torch.zeros((1, 2, 3, 48))
+    plan = rr._RingPlan(x, x, 1, None, None, None).joined().native(x)
+    host = rr._lib.host()
+    q = {"shape": x[:, :40], "dtype": x.float(), "head dim": x[..., :32]}.get(what, x)
+    if q is not x:
+        with pytest.raises(RuntimeError, match="operands"):
+            host.forward(q, x, x, plan, 0.1, torch.bfloat16)
+    with pytest.raises(RuntimeError, match="operands|are not those of q"):
+        host.backward(q, x, x, x[:1] if what == "output" else x, lse[:, :1] if what == "logsumexp" else lse, x[..., :32] if what == "gradient" else x, plan, 0.1)
+    for args in [((x,) * 5, 64), ((), 64), ((x[0],), 64)]:
+        with pytest.raises(RuntimeError, match="arrays"):
+            host.operands(*args)
 
 
 @pytest.mark.parametrize("D", [16, 32, 80, 96, 160])

@@ -698,8 +698,8 @@ bool long_stretches(const ra_bias& bias, int D, int64_t wgs, int64_t total, int6
 // 17 of them (64 heads of 2048) 0.118 | 0.096 ms, 65 (32 of 8192) 0.52 | 0.53, 64 (64 of 4096 x 4096) 0.50 | 0.53, 129 (32 of
 // 16384) 1.92 | 2.10, 257 (32 of 32768) 7.4 | 8.7; with ALiBi, 129 (16 of 16384): 1.18 | 1.21.
 // A grid below 512 workgroups leaves places on the chip empty: the keys of a row are then shared.
-// Under a mask that leaves all rows about the same number of keys the shares are as many as there
-// are places; under a causal mask a share is 1.5 times the mean work of a place, so that the short
+// Under a mask that leaves all rows about the same number of keys a count of time says in how many shares
+// (plan_split); under a causal mask a share is 1.5 times the mean work of a place, so that the short
 // rows stay whole (B=1, D=128, causal, unsplit -> split: H=8, 2048: 46 -> 34 us; H=4, 4096: 85 -> 42 us; H=8,
 // 4096: 88 -> 63 us; H=4, 16384: 375 -> 340 us).  At most kMaxSplit shares, and none under kMinChunk tiles, which
 // cost more in partial results (528 bytes per row and share) than they gain.

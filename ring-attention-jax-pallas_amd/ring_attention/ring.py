@@ -1043,7 +1043,8 @@ def ring_attention(q, k, v, axis_name, bias_fn: Union[BiasFn, Callable, None] = 
     """Ring attention - general (reference ``ring_attention``, ring.py:246-325).
 
     Args:
-        q, k, v: ``[b, S, h, d]`` global arrays on the GPU (see the module docstring).
+        q, k, v: ``[b, S, h, d]`` global arrays on the GPU (see the module docstring).  ``k`` and ``v`` hold at least the batch and
+            heads of ``q``, and ``v`` the length of ``k``; what they hold beyond that takes no part and has gradients of zero.
         axis_name: ``RingAxis`` / int ring size: how many shards the sequence is cut into.
         bias_fn: optional block-wise attention bias: a ``BiasFn`` description (evaluated inside the
             kernels, masked tiles skipped) or, as in the reference, any callable

@@ -484,9 +484,31 @@ PyObject* operand_arrays(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// require_pair(q, k, v, ...): see _require_pair of ring.py
+PyObject* require_pair(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n >= 3, "require_pair(q, k, v, ...)");
+  const Tensor &q = tensor_of(args[0]), &k = tensor_of(args[1]), &v = tensor_of(args[2]);
+  TORCH_CHECK_VALUE(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "q, k and v must be [b, h, l, d]");
+  bool holds = v.size(2) >= k.size(2), exact = v.size(2) == k.size(2);
+  for (const Tensor* t : {&k, &v})
+    for (int i : {0, 1, 3}) {
+      holds &= t->size(i) >= q.size(i);
+      exact &= t->size(i) == q.size(i);
+    }
+  TORCH_CHECK_VALUE(holds, "k ", k.sizes(), " and v ", v.sizes(), " do not hold the batch, heads and head dim of q ", q.sizes(),
+                    ", or v not the length of k");
+  const at::Device device = q.device();
+  for (Py_ssize_t i = 1; i < n; ++i)
+    TORCH_CHECK_VALUE(tensor_of(args[i]).device() == device, "all arrays of a block must be on the device of q (", device, ")");
+  return PyBool_FromLong(exact);
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef g_methods[] = {{"init", init, METH_VARARGS, nullptr},
                            {"plan", plan, METH_VARARGS, nullptr},
                            {"attend", (PyCFunction)(void (*)(void))attend, METH_FASTCALL, nullptr},
+                           {"require_pair", (PyCFunction)(void (*)(void))require_pair, METH_FASTCALL, nullptr},
                            {"convert", (PyCFunction)(void (*)(void))convert_arrays, METH_FASTCALL, nullptr},
                            {"operands", (PyCFunction)(void (*)(void))operand_arrays, METH_FASTCALL, nullptr},
                            {"forward", (PyCFunction)(void (*)(void))forward, METH_FASTCALL, nullptr},

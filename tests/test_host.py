@@ -442,6 +442,7 @@ def test_block_gradients_of_what_lies_beyond_the_call(monkeypatch, k_shape, v_sh
     monkeypatch.setattr(rr, "_stream", lambda: None)
     monkeypatch.setattr(rr, "precompute_delta", lambda o, do: None)
     monkeypatch.setattr(rr, "_bwd_step", step)
+    rr._lib.host()
     monkeypatch.setattr(rr._lib, "load", Library)
     q, k, v = (torch.zeros(s, dtype=torch.bfloat16) for s in ((2, 2, 32, 64), k_shape, v_shape))
     dq, *grads = ra.bwd_block(q, k, v, torch.zeros((2, 1, 32, 32)) if dense else None, torch.zeros(q.shape), torch.zeros((2, 2, 32)), q, 0.1)
